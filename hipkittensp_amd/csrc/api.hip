@@ -176,6 +176,18 @@ bool apply_choice(mxfp6::GemmArgs& g, const mxfp6::KernelChoice& c, hipStream_t 
   }
 }
 
+// A call that no candidate takes: the block kernel's instantiations for ragged sizes and any alignment, with or without its K
+// split, or (false) the generic kernel.
+bool apply_ragged(mxfp6::GemmArgs& g, hipStream_t s) {
+  int shares = mxfp6::ragged_shares(g, g_ksplit, true);
+  uint8_t* pp = shares > 1 ? stream_workspace(s, 2, (size_t)shares * g.M * mxfp6::ragged_pitch(g.N) * sizeof(float)) : nullptr;
+  if (shares > 1 && !pp) shares = mxfp6::ragged_shares(g, g_ksplit, false);
+  if (shares < 1) return false;
+  g.ragged = 1;
+  if (pp) g.ksplit = shares, g.ks_part = reinterpret_cast<float*>(pp);
+  return true;
+}
+
 // A forced kernel family with this thread's K-split setting: 0 = the family's split where the model prefers it to the
 // family's unsplit form, -1 / n = the split wherever the shape has one, 1 = never.  The tile shape of a forced tiled kernel
 // without one (mxfp6_set_kernel 2) is the model's choice as well.
@@ -368,7 +380,7 @@ int gemm_common(const void* A, const void* B, const void* As, const void* Bs, vo
       case mxfp6::kCandBlock: case mxfp6::kCandBlockWide: case mxfp6::kCandBlockSplit: e = mxfp6::launch_gemm_block(g, s); break;
       case mxfp6::kCandSkinny: e = mxfp6::launch_gemm_skinny(g, s); break;
       case mxfp6::kCandRing: e = mxfp6::launch_gemm_ring(g, s); break;
-      default: e = mxfp6::launch_gemm_generic(g, s); break;
+      default: e = K != 0 && apply_ragged(g, s) ? mxfp6::launch_gemm_block(g, s) : mxfp6::launch_gemm_generic(g, s); break;
     }
   }
   return e == hipSuccess ? MXFP6_OK : (int)e;
@@ -585,7 +597,12 @@ int mxfp6_kernel_choice(int M, int N, int K, int layouts) {
   // aligned stand-ins for the pointers: the choice looks at their alignment only
   const uint8_t* p = reinterpret_cast<const uint8_t*>((uintptr_t)4096);
   mxfp6::GemmArgs g{p, p, p, p, const_cast<uint8_t*>(p), M, N, K, 2, 2, false, layout_a, layout_b};
-  return choice_code(auto_choice(g, 0, true));
+  const mxfp6::KernelChoice c = auto_choice(g, 0, true);
+  if (c.cand < 0 && K > 0) {
+    const int shares = mxfp6::ragged_shares(g, g_ksplit, true);
+    return shares > 1 ? kChoiceBlockKsplit : shares == 1 ? kChoiceBlock : kChoiceGeneric;
+  }
+  return choice_code(c);
 }
 
 #ifdef MXFP6_PROBES  // ---- measurement entry points (include/mxfp6_probes.h)

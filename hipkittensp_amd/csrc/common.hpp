@@ -138,6 +138,9 @@ __host__ __device__ __forceinline__ int ksplit_order(int bid, int total, int xcd
   return ksplit_by_share(total, xcd_remap) ? (bid & 7) * (total >> 3) + (bid >> 3) : bid;
 }
 
+// Floats per row of the partial matrices that a K split of a ragged product leaves (rows of whole, aligned 16 bytes)
+__host__ __device__ __forceinline__ size_t ragged_pitch(int n) { return ((size_t)n + 3) & ~(size_t)3; }
+
 // Byte offset, inside a tile-major operand, of byte `b` (0 .. 3K/4) of row `row`; nkt = K / 128.
 // Tiles are 32 rows x 96 bytes in the kernels' LDS image order (16-byte pieces, pairs swapped in
 // rows with bit 3 set).

@@ -45,18 +45,36 @@ struct BlockArgs {
 // WN: waves side by side along N, 2 (tile of 128 x 128, four waves) or 4 (128 x 256, eight waves: waves 0-3 load A's tile
 // and half of B's, six loads per K-tile, waves 4-7 the other half of B's, three loads).
 // FUSED: the epilogue applies args.ep (a separate instantiation, so that unfused calls carry none of it).
-template <int FA, int FB, typename Out, int STAGES, int WN, bool FUSED>
+// RAGGED: any M, N, K (K % 32 == 0) and any alignment the entry points take.  What differs from the aligned instantiations:
+//   * rows of 24 bytes per K-block start at multiples of 8 (4 at least), which a direct load of 16 bytes accepts; the
+//     K-tile's offset rides in the per-lane offset, so that the last K-tile of the last row is cut off at the end of the
+//     resource.  Elsewhere a partial last K-tile brings in the head of the next row, and the reader puts 0 for both
+//     operands' scale bytes of the K-blocks past K: the products of what stands there, 28 * 28 * 32 * 2^-254 at most, are
+//     nothing to an fp32 sum, whose last place is 2^-149 at least.  (Zeroing A's fragments instead: 24 v_and a K-tile behind
+//     the wait for the LDS reads, 3 us of 20 at 500 x 5003 x 2880, and in a branch the compiler spills them.)
+//   * a row's scales start at any byte: a lane fetches the 20 bytes of aligned dwords around its 16 (one load of 16 bytes and
+//     one of 4) and the reader shifts them into place (v_alignbyte_b32, once per four K-tiles).  Up to four slots one scale
+//     buffer serves (a group's scales are in registers before the next group's are fetched): three slots are 77 KB
+//   * C's rows start at any element: 16-byte stores at element alignment, and single elements where a run of eight (bf16) or
+//     four (fp32) outputs crosses N
+// 500 x 5003 x 2880: 19.3 us against 148.5 on the one-wave-per-tile kernel, which fetches every operand row again for each of
+// its 32 x 32 tiles, 4 bytes per lane.
+template <int FA, int FB, typename Out, int STAGES, int WN, bool FUSED, bool RAGGED = false>
 __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_block_kernel(const BlockArgs args) {
   typedef typename Out::type OutT;
   static_assert(STAGES >= 3 && STAGES <= 6 && (WN == 2 || WN == 4), "ring depth, tile width");
-  constexpr int NW = 2 * WN, kBN = WN * 64, kSlot = kATile + kBN * 96, kScBuf = kScA + kBN * 16;
+  static_assert(!RAGGED || (WN == 2 && FUSED), "one tile width, one epilogue");
+  constexpr int NW = 2 * WN, kBN = WN * 64, kSlot = kATile + kBN * 96, kScRows = kScA + kBN * 16;
+  constexpr int kScBuf = kScRows + (RAGGED ? (kBM + kBN) * 4 : 0);  // RAGGED: 4 more bytes per row behind the rows' 16
   constexpr int kStages = STAGES, E = STAGES > 4 ? 1 : 0;  // E: extra groups of four K-tiles the scale loads run ahead
-  constexpr int kScBase = kStages * kSlot, kLdsBytes = kScBase + 2 * kScBuf;
+  constexpr int kScBufs = RAGGED && !E ? 1 : 2;
+  constexpr int kScLoads = RAGGED ? 2 : 1;  // loads per group of scales
+  constexpr int kScBase = kStages * kSlot, kLdsBytes = kScBase + kScBufs * kScBuf;
   static_assert(kLdsBytes <= (STAGES <= 3 && WN == 2 ? 81920 : 163840), "LDS budget");
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kLdsBytes];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(MXFP6_LDS uint8_t*)smem;
   const int K = args.K, layout_a = args.layout_a, layout_b = args.layout_b;
-  const int rowbytes = K / 4 * 3, sbytes = K / 32, nkt_all = K / kBK, nk4_all = (nkt_all + 3) / 4;  // tile-major scales: one 512-byte chunk per 32 rows and group of four K-tiles, the last one padded
+  const int rowbytes = K / 32 * 24, sbytes = K / 32, nkt_all = RAGGED ? (K + kBK - 1) / kBK : K / kBK, nk4_all = (nkt_all + 3) / 4;  // tile-major scales: one 512-byte chunk per 32 rows and group of four K-tiles, the last one padded
   // K split: workgroup b takes share l / tiles of tile l % tiles, l = ksplit_order(b) -- the same number of whole groups
   // of four K-tiles for every share, the last one what is left of K (at least one K-tile: the launcher sees to that) --
   // and leaves its fp32 sums in matrix `share` of args.C, then a workspace of nsplit matrices [M, N]
@@ -93,13 +111,18 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   const uint8_t* sp = sc_a ? args.As : args.Bs;
   const int sheight = sc_a ? kBM : kBN;  // rows per tile of the operand whose scales these are
   const uint32_t os = (uint32_t)(kt0 >> 2) * (slay ? 512 : 16);  // the share's first group of four K-tiles
-  const __amdgpu_buffer_rsrc_t rS = slay ? make_rsrc(sp + (size_t)stile * (sheight / 32) * nk4_all * 512 + os, (uint32_t)((srows + 31) / 32) * nk4_all * 512 - os)
-                                         : make_rsrc(sp + (size_t)stile * sheight * sbytes + os, (uint32_t)srows * sbytes - os);
+  const uint8_t* const sbase = sp + (size_t)stile * (sheight / 32) * (slay ? nk4_all * 512 : 32 * sbytes) + os;
+  const uint32_t slen = (uint32_t)(slay ? (srows + 31) / 32 * nk4_all * 512 : srows * sbytes) - os;
+  // RAGGED: the resource starts and ends at aligned dwords (which hold at least one byte of the tensor each)
+  const uint32_t smis = RAGGED ? (uint32_t)(uintptr_t)sbase & 3 : 0;
+  const __amdgpu_buffer_rsrc_t rS = RAGGED ? make_rsrc(sbase - smis, (slen + smis + 3) & ~3u) : make_rsrc(sbase, slen);
   const int spart = sc_a ? wave & 1 : wave - NW / 2;  // which 64 rows
   const int srow = spart * 64 + lane;
-  const int voff_s = slay ? (srow >> 5) * nk4_all * 512 + (srow & 31) * 16 : srow * sbytes;
+  const int voff_row = slay ? (srow >> 5) * nk4_all * 512 + (srow & 31) * 16 : srow * sbytes;
+  const int voff_s = RAGGED ? (voff_row + (int)smis) & ~3 : voff_row;
   const int sstep = slay ? 512 : 16;
   const uint32_t sdst = lds0 + kScBase + (sc_a ? 0 : kScA) + spart * 1024;
+  const uint32_t sdst_tail = lds0 + kScBase + kScRows + (sc_a ? 0 : kBM * 4) + spart * 256;  // RAGGED: bytes 16 .. 19 of a row's dwords
 
   // per-lane global byte offsets of the direct loads: load q = 3 wave + i fills LDS bytes [q * 1024, + 1024) of an
   // operand's tile.  Row-major: 16-byte slot o holds piece (o % 6) ^ ((row >> 3) & 1) of row o / 6.  Tile-major: the
@@ -136,15 +159,22 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   v12i fa[2][2], fb[2][2];  // [set][tile]: a lane's 48 bytes of a 32-row tile, dwords 0-5 the first MFMA's operand, 6-11 the second's
   int sca[2][4], scb[2][4];  // [tile][K-tile of the group]: scale bytes in bytes 0, 1
   v4i raw_a[2], raw_b[2];
+  [[maybe_unused]] int tail_a[2], tail_b[2];
+  // RAGGED: how many bytes a row's scales start behind the aligned dwords fetched for it (v_alignbyte_b32 takes it modulo 4;
+  // rows 32 apart share it)
+  [[maybe_unused]] const uint32_t shift_a = (uint32_t)(uintptr_t)args.As + (layout_a ? 0 : r32 * sbytes);
+  [[maybe_unused]] const uint32_t shift_b = (uint32_t)(uintptr_t)args.Bs + (layout_b ? 0 : r32 * sbytes);
 
   // load n of this wave's for K-tile t: 0-2 the three of row-tile `wave` of A's tile (LA: this wave loads A at all), 3-5 of B's
   auto load_one = [&]<bool LA>(int t, int slot, int n) __attribute__((always_inline)) {
     const bool in = t < nkt;
     const uint32_t dst = lds0 + slot * kSlot + wave * 3072;
     if (n < 3) {
-      if constexpr (LA) dma16(in ? rA : rZ, dst + n * 1024, voff_a[n], t * kstep_a);
+      if constexpr (LA) dma16(in ? rA : rZ, dst + n * 1024, voff_a[n], RAGGED ? 0 : t * kstep_a);
+      if constexpr (RAGGED) voff_a[n] += kstep_a;  // the loads come in the order of t
     } else {
-      dma16(in ? rB : rZ, dst + kATile + (n - 3) * 1024, voff_b[n - 3], t * kstep_b);
+      dma16(in ? rB : rZ, dst + kATile + (n - 3) * 1024, voff_b[n - 3], RAGGED ? 0 : t * kstep_b);
+      if constexpr (RAGGED) voff_b[n - 3] += kstep_b;
     }
   };
   auto load_tile = [&]<bool LA>(int t, int slot) __attribute__((always_inline)) {
@@ -155,7 +185,8 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   // K % 512 != 0 the last group of a row-major row is shorter than 16 bytes, and the last row's must not read past the tensor)
   auto load_scales = [&](int grp) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rs = grp < nk4 ? rS : rZ;
-    dma16(rs, sdst + (grp & 1) * kScBuf, voff_s + grp * sstep, 0);
+    dma16(rs, sdst + (grp & (kScBufs - 1)) * kScBuf, voff_s + grp * sstep, 0);
+    if constexpr (RAGGED) dma4(rs, sdst_tail + (grp & (kScBufs - 1)) * kScBuf, voff_s + grp * sstep + 16, 0);
   };
   auto read_tile = [&]<int SET>(int slot) __attribute__((always_inline)) {
     const uint8_t* st = smem + slot * kSlot;
@@ -177,13 +208,35 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
       }
   };
   auto read_scales = [&](int grp) __attribute__((always_inline)) {
-    const uint8_t* sc = smem + (grp & 1) * kScBuf;
+    const uint8_t* sc = smem + (grp & (kScBufs - 1)) * kScBuf;
 #pragma unroll
     for (int i = 0; i < 2; i++) raw_a[i] = *reinterpret_cast<const v4i*>(sc + sa_rd + i * 512);
 #pragma unroll
     for (int j = 0; j < 2; j++) raw_b[j] = *reinterpret_cast<const v4i*>(sc + sb_rd + j * 512);
+    if constexpr (RAGGED) {
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        tail_a[i] = *reinterpret_cast<const int*>(sc + kScBase + kScRows + (wm * 64 + i * 32 + r32) * 4);
+        tail_b[i] = *reinterpret_cast<const int*>(sc + kScBase + kScRows + kBM * 4 + (wn * 64 + i * 32 + r32) * 4);
+      }
+    }
   };
-  auto take_scales = [&]() __attribute__((always_inline)) {
+  auto take_scales = [&]([[maybe_unused]] int grp) __attribute__((always_inline)) {
+    if constexpr (RAGGED) {
+#pragma unroll
+      for (int km = 0; km < 4; km++) {
+        // K-blocks this K-tile has; a lane's two are blocks 2h, 2h + 1
+        const int nvalid = sbytes - ((kt0 >> 2) + grp) * 16 - 4 * km;
+        const uint32_t keep = (2 * h < nvalid ? 0xffu : 0u) | (2 * h + 1 < nvalid ? 0xff00u : 0u);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          const uint32_t wa = __builtin_amdgcn_alignbyte(km < 3 ? raw_a[i][km + 1] : tail_a[i], raw_a[i][km], shift_a);
+          const uint32_t wb = __builtin_amdgcn_alignbyte(km < 3 ? raw_b[i][km + 1] : tail_b[i], raw_b[i][km], shift_b);
+          sca[i][km] = (int)(wa >> sc_shift & keep), scb[i][km] = (int)(wb >> sc_shift & keep);
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
@@ -243,11 +296,11 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
     for (int i = 0; i < 2; i++) asm volatile("" : "+v"(fa[NXT][i]));
 #pragma unroll
     for (int j = 0; j < 2; j++) asm volatile("" : "+v"(fb[NXT][j]));
-    if (KM == 3) take_scales();
+    if (KM == 3) take_scales((k >> 2) + 1);
     // K-tile k + 2 has landed: everything older than the loads of the last STAGES - 2 steps (six each, and a scale load
     // in steps with KM == 0)
     constexpr int kScalesInFlight = (KM % 4 == 0) + (STAGES >= 4 && (KM + 3) % 4 == 0) + (STAGES >= 5 && (KM + 2) % 4 == 0) + (STAGES >= 6 && (KM + 1) % 4 == 0);
-    wait_vmcnt<(LA ? 6 : 3) * (STAGES - 2) + kScalesInFlight>();
+    wait_vmcnt<(LA ? 6 : 3) * (STAGES - 2) + kScLoads * kScalesInFlight>();
     barrier();
     const int t = slot[0];
 #pragma unroll
@@ -267,7 +320,7 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
     read_tile.template operator()<0>(0);
     read_scales(0);
     wait_lds_reads();
-    take_scales();
+    take_scales(0);
     wait_vmcnt<NL * (STAGES - 2)>();
     barrier();  // K-tile 1 is in place, and every wave has K-tile 0 in registers: its slot is free
     int k = 0;
@@ -312,7 +365,14 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
         for (int q = 0; q < 4; q++) {
           const long n = n0 + j * 32 + q * 8;
           v4f cs = {1.f, 1.f, 1.f, 1.f}, bi = {0.f, 0.f, 0.f, 0.f};
-          if (n < N) {
+          if constexpr (RAGGED) {  // a run of four may cross N
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              const long ne = n + e < N ? n + e : N - 1;
+              if (col_scale) cs[e] = col_scale[ne];
+              if (bias) bi[e] = bias_bf16 ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(bias)[ne]) : reinterpret_cast<const float*>(bias)[ne];
+            }
+          } else if (n < N) {
             if (col_scale) cs = *reinterpret_cast<const v4f*>(col_scale + n);
             if (bias && bias_bf16) {
               const u32x2 b2 = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(bias) + n);
@@ -327,15 +387,43 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
             for (int e = 0; e < 4; e++) acc[i][j][4 * q + e] = fmaf(acc[i][j][4 * q + e] * rs[i], cs[e], bi[e]);
         }
       }
+      // one branch per activation and tile, not one per element (that took 2 us of a 20 us call, with or without an activation)
 #pragma unroll
-      for (int i = 0; i < 2; i++)
+      for (int i = 0; i < 2; i++) {
+        if (act == 1) {
 #pragma unroll
-        for (int e = 0; e < 16; e++) acc[i][j][e] = epilogue_act(acc[i][j][e], act);
+          for (int e = 0; e < 16; e++) acc[i][j][e] = act_relu(acc[i][j][e]);
+        } else if (act == 2) {
+#pragma unroll
+          for (int e = 0; e < 16; e++) acc[i][j][e] = act_gelu(acc[i][j][e]);
+        } else if (act == 3) {
+#pragma unroll
+          for (int e = 0; e < 16; e++) acc[i][j][e] = act_silu(acc[i][j][e]);
+        }
+        asm volatile("" : "+v"(acc[i][j]));
+      }
     }
   }
+  // RAGGED with a K split: the shares' matrices have rows of a multiple of four floats
+  [[maybe_unused]] const size_t ldc = RAGGED && args.nsplit > 1 ? ragged_pitch(N) : N;
   const __amdgpu_buffer_rsrc_t rC = make_rsrc((OutT*)args.C + (size_t)share * args.M * N + (size_t)pm * kBM * N + (size_t)pn * kBN,
                                               (uint32_t)((rows_a - 1) * N + rows_b) * (uint32_t)sizeof(OutT));
   const int row_l = wm * 64 + r32;
+  // RAGGED: `n` consecutive outputs of a row, 16 bytes of them at C's element alignment or, across N, one by one
+  [[maybe_unused]] auto store_run = [&](v4i v, int row, int col) __attribute__((always_inline)) {
+    constexpr int kRun = 16 / (int)sizeof(OutT);
+    if (row >= rows_a || col >= rows_b) return;
+    OutT* const p = (OutT*)args.C + ((size_t)share * args.M + (size_t)pm * kBM + row) * ldc + (size_t)pn * kBN + col;
+    if (col + kRun <= rows_b) {
+      __builtin_memcpy(p, &v, 16);
+    } else {
+      OutT o[kRun];
+      __builtin_memcpy(o, &v, 16);
+#pragma unroll
+      for (int e = 0; e + 1 < kRun; e++)
+        if (col + e < rows_b) p[e] = o[e];
+    }
+  };
   if constexpr (sizeof(OutT) == 2) {
     const int col_l = wn * 64 + 8 * h;
     const int voff = row_l * N2 + col_l * 2;
@@ -361,7 +449,8 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
 #pragma unroll
         for (int t = 0; t < 2; t++) {
           const v4i v = {(int)pk[j][4 * t], (int)pk[j][4 * t + 1], (int)pk[j][4 * t + 2], (int)pk[j][4 * t + 3]};
-          if (!edge || (row_l + i * 32 < rows_a && col_l + j * 32 + t * 16 < rows_b))
+          if constexpr (RAGGED) store_run(v, row_l + i * 32, col_l + j * 32 + t * 16);
+          else if (!edge || (row_l + i * 32 < rows_a && col_l + j * 32 + t * 16 < rows_b))
             __builtin_amdgcn_raw_buffer_store_b128(v, rC, voff + j * 64 + t * 32, i * 32 * N2, 0);
         }
     }
@@ -375,7 +464,8 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
 #pragma unroll
         for (int gq = 0; gq < 4; gq++) {
           const v4f f = {acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]};
-          if (!edge || (row_l + i * 32 < rows_a && col_l + j * 32 + gq * 8 < rows_b))
+          if constexpr (RAGGED) store_run(__builtin_bit_cast(v4i, f), row_l + i * 32, col_l + j * 32 + gq * 8);
+          else if (!edge || (row_l + i * 32 < rows_a && col_l + j * 32 + gq * 8 < rows_b))
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, f), rC, voff + j * 128 + gq * 32, i * 32 * N2, 0);
         }
   }
@@ -421,6 +511,20 @@ hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, 
   }
   return hipGetLastError();
 }
+// RAGGED instantiations: three or six slots by the same rule, the fused epilogue applied or not inside
+template <int FA, int FB>
+hipError_t launch_ragged(const GemmArgs& g, const BlockArgs& a, int tiles, hipStream_t s) {
+  const int grid = tiles * a.nsplit, cus = cu_count_of_device();
+  const bool deep = grid <= cus && g.K > 2048;
+  if (g.f32out || a.nsplit > 1) {
+    if (deep) gemm_block_kernel<FA, FB, OutF32, 6, 2, true, true><<<grid, 256, 0, s>>>(a);
+    else gemm_block_kernel<FA, FB, OutF32, 3, 2, true, true><<<grid, 256, 0, s>>>(a);
+  } else {
+    if (deep) gemm_block_kernel<FA, FB, OutBf16, 6, 2, true, true><<<grid, 256, 0, s>>>(a);
+    else gemm_block_kernel<FA, FB, OutBf16, 3, 2, true, true><<<grid, 256, 0, s>>>(a);
+  }
+  return hipGetLastError();
+}
 template <int FA, int FB>
 hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, hipStream_t s) {
   // a split leaves the epilogue to the reduction
@@ -439,6 +543,12 @@ bool gemm_block_supports(const GemmArgs& g) {
          !g.no_alloc;
 }
 
+// The RAGGED instantiations: whatever the entry points take, up to 32-bit offsets inside a tile
+bool gemm_block_ragged_supports(const GemmArgs& g) {
+  return g.M > 0 && g.N > 0 && g.K >= 32 && g.K % 32 == 0 && (long)128 * (g.K / 4 * 3) < (1L << 31) - 32768 && (long)((g.M + 127) / 128) <= 65535 &&
+         (long)((g.N + 127) / 128) <= 32767 && (long)((g.M + 127) / 128) * ((g.N + 127) / 128) < (1L << 31) && !g.fmt_c;
+}
+
 // g.ksplit > 1 (with g.ks_part): the K range of every output tile split between that many workgroups, then
 // ksplit_reduce_kernel (gemm_tiled.hip), which also applies a fused epilogue.  The caller has checked that the last share
 // is not empty (block_split_shares, dispatch.hip).
@@ -448,7 +558,13 @@ hipError_t launch_gemm_block(const GemmArgs& g, hipStream_t s) {
               g.raster_group_m > 0 ? g.raster_group_m : kGroupM, g.raster_no_xcd_remap == 1 ? 0 : g.raster_no_xcd_remap == 2 ? 2 : 1, nsplit, g.ep};
   const int tiles = a.tiles_m * a.tiles_n, stages = g.tile_rows == 3 || g.tile_rows == 6 ? g.tile_rows : 0;
   hipError_t e;
-  if (g.fmt_a == 2 && g.fmt_b == 2) e = launch<2, 2>(g, a, tiles, stages, s);
+  if (g.ragged) {
+    if (nsplit > 1) a.ep = Epilogue{};  // the reduction applies it
+    if (g.fmt_a == 2 && g.fmt_b == 2) e = launch_ragged<2, 2>(g, a, tiles, s);
+    else if (g.fmt_a == 2 && g.fmt_b == 3) e = launch_ragged<2, 3>(g, a, tiles, s);
+    else if (g.fmt_a == 3 && g.fmt_b == 2) e = launch_ragged<3, 2>(g, a, tiles, s);
+    else e = launch_ragged<3, 3>(g, a, tiles, s);
+  } else if (g.fmt_a == 2 && g.fmt_b == 2) e = launch<2, 2>(g, a, tiles, stages, s);
   else if (g.fmt_a == 2 && g.fmt_b == 3) e = launch<2, 3>(g, a, tiles, stages, s);
   else if (g.fmt_a == 3 && g.fmt_b == 2) e = launch<3, 2>(g, a, tiles, stages, s);
   else e = launch<3, 3>(g, a, tiles, stages, s);

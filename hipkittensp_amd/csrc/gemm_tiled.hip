@@ -792,7 +792,31 @@ __global__ __launch_bounds__(256) void ksplit_reduce_kernel(const float* __restr
   }
 }
 
+// The same for a C of any shape and alignment (the block kernel's ragged instantiations), whose shares' rows are padded to
+// four floats: a thread adds four columns of a row, of which those past N are padding.
+template <typename T>
+__global__ __launch_bounds__(64) void ksplit_reduce_ragged_kernel(const float* __restrict__ part, int nsplit, T* __restrict__ C, int M, int N, const Epilogue ep) {
+  const size_t ld = ragged_pitch(N), mn = (size_t)M * ld;
+  const int n = (blockIdx.x * 64 + threadIdx.x) * 4;
+  if (n >= N) return;
+  for (int m = blockIdx.y; m < M; m += gridDim.y) {
+    const float* p = part + (size_t)m * ld + n;
+    v4f acc = *reinterpret_cast<const v4f*>(p);
+    for (int s = 1; s < nsplit; s++) acc += *reinterpret_cast<const v4f*>(p + s * mn);
+    const bool has_ep = epilogue_any(ep);
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (n + e < N) store1(C + (size_t)m * N + n + e, has_ep ? epilogue_apply(ep, acc[e], m, n + e) : acc[e]);
+  }
+}
+
 hipError_t launch_ksplit_reduce(const GemmArgs& g, hipStream_t s) {
+  if (g.ragged) {
+    const dim3 blocks((unsigned)(g.N + 255) / 256, (unsigned)(g.M < 65535 ? g.M : 65535));
+    if (g.f32out) ksplit_reduce_ragged_kernel<float><<<blocks, 64, 0, s>>>(g.ks_part, g.ksplit, (float*)g.C, g.M, g.N, g.ep);
+    else ksplit_reduce_ragged_kernel<uint16_t><<<blocks, 64, 0, s>>>(g.ks_part, g.ksplit, (uint16_t*)g.C, g.M, g.N, g.ep);
+    return hipGetLastError();
+  }
   const size_t quads = (size_t)g.M * g.N / 4;
   const unsigned blocks = (unsigned)((quads + 255) / 256);
   if (g.f32out) ksplit_reduce_kernel<float><<<blocks, 256, 0, s>>>(g.ks_part, g.ksplit, (float*)g.C, g.M, g.N, g.ep);

@@ -22,6 +22,7 @@ struct GemmArgs {
   int raster_group_m = 0, raster_no_xcd_remap = 0;  // tiled kernel, measurement only: tile rows per raster group (0 = the default, 4), XCD remap off (1), or on with a K split's workgroups in tile-by-tile order (2)
   int ablation = 0;  // tiled kernel, measurement only: leave out LDS reads (1), loads (2), MFMAs (4); results are then meaningless
   uint32_t* clock_stamps = nullptr;  // tiled kernel, measurement only: four words for workgroup 0's clock / real-time counters at start and end
+  int ragged = 0;                  // block kernel: its instantiations for any size and alignment (gemm_block_ragged_supports)
   int no_alloc = 0;                // skinny kernel: the K split keeps its partial tiles in the library's static scratch array instead of an allocated workspace
   int force_split = 0;             // skinny kernel, M <= 32: split K between this many workgroups (1, 2, 4, 8); 0 = by shape
   int ksplit = 0;                  // tiled kernel: workgroups that share an output tile (from tiled_ksplit_plan, which also gives tile_rows); needs ks_part
@@ -37,7 +38,7 @@ inline bool operands_aligned16(const GemmArgs& g) {
 // ---- kernel choice (dispatch.hip): candidates of the automatic path, a time model per candidate, a calibration table
 enum Candidate : int { kCandTiled256 = 0, kCandTiled128x256, kCandTiled128x128, kCandBlock, kCandBlockWide, kCandSkinny, kCandTiledSplit256, kCandTiledSplit128, kCandBlockSplit, kCandRing, kNumCandidates };
 struct KernelChoice {
-  int cand;    // a Candidate, or -1: none of them takes the shape (the generic kernel does)
+  int cand;    // a Candidate, or -1: none of them takes the shape (ragged_shares says what does)
   int shares;  // K split: workgroups per output tile (1 = none)
   int rows;    // tiled kernel's split: rows of A per tile
   double us;   // modelled time x calibration factor
@@ -46,6 +47,7 @@ int device_cus();
 double candidate_model_us(const GemmArgs& g, int cand, int want_split, int cus, int* shares, int* rows);  // modelled microseconds; < 0: the candidate does not take the shape
 KernelChoice choose_kernel(const GemmArgs& g, int want_split, bool allow_split, unsigned mask = ~0u);  // mask: bit per Candidate that may be chosen; want_split: 0 = by the model, 1 = never, n = n shares where a candidate splits; allow_split: a workspace is to be had
 int tiled_split_shares(const GemmArgs& g, int want, int cus, int bm);  // the tiled kernel's K split with tiles of bm (256 or 128) rows when it is to split: shares (1 = the shape has none)
+int ragged_shares(const GemmArgs& g, int want, bool allow_split);  // shapes no candidate takes: shares of the block kernel's K split (1 = unsplit), 0 = the generic kernel
 int block_split_shares(const GemmArgs& g, int want, int cus);             // ... the block kernel's
 
 hipError_t launch_gemm_generic(const GemmArgs& g, hipStream_t s);
@@ -54,6 +56,7 @@ hipError_t launch_gemm_tiled(const GemmArgs& g, hipStream_t s);
 bool gemm_tiled4_supports(const GemmArgs& g);  // the 4-wave variant of the tiled kernel (selectable, never chosen automatically)
 hipError_t launch_gemm_tiled4(const GemmArgs& g, hipStream_t s);
 bool gemm_block_supports(const GemmArgs& g);  // 128 x 128 tiles, four waves in step (a few hundred to a few thousand rows of A)
+bool gemm_block_ragged_supports(const GemmArgs& g);  // with GemmArgs::ragged: any M, N, K % 32 == 0 and alignment
 hipError_t launch_gemm_block(const GemmArgs& g, hipStream_t s);
 hipError_t launch_ksplit_reduce(const GemmArgs& g, hipStream_t s);  // sums g.ksplit partial matrices at g.ks_part into g.C, with the epilogue
 bool gemm_ring_supports(const GemmArgs& g);  // batched decode: private streams of B per wave, A through a flag-guarded ring (no barrier per K-tile)

@@ -18,6 +18,13 @@ __device__ __forceinline__ void dma16(const __amdgpu_buffer_rsrc_t& rsrc, uint32
                : "s"(lds_base), "v"(voff), "s"(rsrc), "s"(soff)
                : "memory");
 }
+// the same with 4 bytes per lane, to lds_base + 4 * lane
+__device__ __forceinline__ void dma4(const __amdgpu_buffer_rsrc_t& rsrc, uint32_t lds_base, int voff, int soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+               :
+               : "s"(lds_base), "v"(voff), "s"(rsrc), "s"(soff)
+               : "memory");
+}
 // at most N of this wave's loads (and stores) may still be in flight; they retire in order
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {

@@ -43,8 +43,8 @@
  *
  * Alignment.  Pointers are accepted from 4-byte alignment on (C: its element size).  The fast kernels
  * fetch 16 bytes per lane: they run when A_packed, B_packed, both scale tensors and C are 16-byte aligned
- * (any tensor PyTorch allocates is); otherwise the call is served by the generic kernel, with the same
- * results and a fraction of the speed.
+ * (any tensor PyTorch allocates is); otherwise the call is served by the block kernel's instantiations for any size and
+ * alignment (or, where it is small, by the generic kernel), with the same results.
  *
  * Accuracy.  Products of dequantised values are exact in fp32; with an e2m3 operand on either side the
  * accumulators agree with an fp64 dequantise-and-matmul to fp32 rounding (relative error < 1e-6 of the

@@ -1,0 +1,73 @@
+"""Sizes and alignments that the aligned kernels do not take (N % 8, K % 128, pointers off 16 bytes), through the automatic
+path: the block kernel's ragged instantiations against the CPU oracle, at the edges of their tiles and K-tiles.  Bound: every
+product and partial sum of these inputs is exact in fp32 up to the sum's own rounding, so the fp32 result is held to 1e-5 of
+the oracle's (its metric), the bf16 result to the rounding of that fp32 result, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import c_oracle as co
+from oracle import mxfp6_oracle as o
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hk():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import hipkittensp_amd as m
+
+    return m
+
+
+def at(a, off):
+    """`a` on the GPU at a pointer `off` bytes past 256-byte alignment, NaN bit patterns (0xff) around it."""
+    raw = np.ascontiguousarray(a).view(np.uint8).reshape(-1)
+    buf = torch.full((raw.size + 1024,), 255, dtype=torch.uint8, device="cuda")
+    buf[256 + off:256 + off + raw.size] = torch.from_numpy(raw).cuda()
+    return buf[256 + off:256 + off + raw.size].view(*a.shape)
+
+
+def call(hk, A, B, As, Bs, M, N, fa, fb, dtype, off_c=0, shares=0, **kw):
+    guard = torch.full((M * N + 64,), 7.0, dtype=dtype, device="cuda")
+    C = guard[16 + off_c:16 + off_c + M * N].view(M, N)
+    prev = hk.tk_kernel.set_k_split(shares)
+    try:
+        hk.dispatch_micro(A, B, As, Bs, C, fa, fb, **kw)
+        torch.cuda.synchronize()
+    finally:
+        hk.tk_kernel.set_k_split(prev)
+    assert bool((guard[:16 + off_c] == 7.0).all()) and bool((guard[16 + off_c + M * N:] == 7.0).all())
+    return C
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 160), (128, 128, 160), (129, 127, 288), (127, 129, 224), (5, 131, 2080), (257, 255, 1056), (130, 1001, 992),
+                                   (64, 8, 4064), (33, 4, 8224), (300, 12, 640), (200, 260, 384), (1, 5003, 2880), (500, 515, 2880), (1000, 1001, 96)])
+@pytest.mark.parametrize("fa,fb,shares", [(2, 2, 0), (2, 2, 1), (3, 2, 2), (2, 3, -1)])
+def test_ragged_sizes_vs_oracle(hk, M, N, K, fa, fb, shares):
+    ap, asc = co.quantise(o.make_source("normal", (M, K), np.random.default_rng(M + K)), fa)
+    bp, bsc = co.quantise(o.make_source("weights_outliers", (N, K), np.random.default_rng(N + K)), fb)
+    ref = o.gemm_ref(ap, bp, asc, bsc, fa, fb, acc=np.float64)
+    ops = [at(x, 0) for x in (ap, bp, asc, bsc)]
+    got = call(hk, *ops, M, N, fa, fb, torch.float32, shares=shares).cpu().numpy()
+    assert np.isfinite(got).all() and o.rel_err(got, ref) <= 1e-5
+    c16 = call(hk, *ops, M, N, fa, fb, torch.bfloat16, shares=shares)
+    assert np.array_equal(c16.view(torch.int16).cpu().numpy().view(np.uint16), o.f32_to_bf16_bits(got))
+
+
+@pytest.mark.parametrize("M,N,K,la", [(70, 136, 640, 0), (64, 136, 640, 1), (200, 96, 1056, 0)])
+def test_ragged_alignment_and_fused_epilogue(hk, M, N, K, la):
+    """Operands at every alignment the entry points take (4 bytes, scales and C any element), tile-major A, fused epilogue."""
+    ap, asc = co.quantise(o.make_source("normal", (M, K), np.random.default_rng(1)), 2)
+    bp, bsc = co.quantise(o.make_source("weights", (N, K), np.random.default_rng(2)), 2)
+    ref = o.gemm_ref(ap, bp, asc, bsc, acc=np.float64)
+    tiled = (o.tile_operand(ap), o.tile_scales(asc)) if la else (ap, asc)
+    for oa, ob, osa, osb, oc in ((4, 0, 0, 0, 0), (0, 12, 0, 0, 1), (0, 0, 1, 2, 3), (8, 4, 3, 1, 5)):
+        ops = [at(tiled[0], oa), at(bp, ob), at(tiled[1], osa), at(bsc, osb)]
+        got = call(hk, *ops, M, N, 2, 2, torch.float32, off_c=oc, layout_a=la).cpu().numpy()
+        assert o.rel_err(got, ref) <= 1e-5, (oa, ob, osa, osb, oc)
+        bias = torch.randn(N, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
+        fused = call(hk, *ops, M, N, 2, 2, torch.float32, off_c=oc, layout_a=la, bias=bias, activation="relu").cpu().numpy()
+        want = np.maximum(got + bias.cpu().numpy(), 0)  # one fp32 addition: exact to its rounding
+        assert np.array_equal(fused, want.astype(np.float32)), (oa, ob, osa, osb, oc)
