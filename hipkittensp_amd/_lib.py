@@ -46,6 +46,8 @@ def _bind(L: ctypes.CDLL) -> ctypes.CDLL:
     L.mxfp6_gemm_fused.argtypes = [vp, vp, vp, vp, vp, ci, ci, ci, ci, ci, ci, ci, ci, vp, ci, vp, vp, ci, vp]
     L.mxfp6_gemm_fused_fp6.restype = ci
     L.mxfp6_gemm_fused_fp6.argtypes = [vp, vp, vp, vp, vp, vp, ci, ci, ci, ci, ci, ci, ci, ci, vp, ci, vp, vp, ci, vp]
+    L.mxfp6_linear.restype = ci
+    L.mxfp6_linear.argtypes = [vp, ci, vp, vp, vp, ci, ci, ci, ci, ci, ci, vp, ci, ci, vp]
     L.mxfp6_quantize_ex.restype = ci
     L.mxfp6_quantize_ex.argtypes = [vp, vp, vp, ci, ci, ci, ci, vp]
     L.mxfp6_quantize_bf16.restype = ci
@@ -91,6 +93,18 @@ def lib() -> ctypes.CDLL:
     if _lib is None:
         _lib = _bind(_load(LIB_PATH))
     return _lib
+
+
+def native():
+    """The native binding of the operator's hot calls (csrc/binding.cpp), linked against the operator's library."""
+    import torch  # noqa: F401  (the binding's symbols are torch's)
+
+    lib()
+    try:
+        from . import _native
+    except ImportError as e:
+        raise Mxfp6LibraryMissing(f"hipkittensp_amd._native is not built ({e}); run `python -m hipkittensp_amd.build`.") from e
+    return _native
 
 
 def probes() -> ctypes.CDLL:

@@ -1,4 +1,5 @@
-"""Builds hipkittensp_amd/libmxfp6_gemm.so (gfx950 only) from csrc/*.hip with hipcc, and libmxfp6_probes.so beside it.
+"""Builds hipkittensp_amd/libmxfp6_gemm.so (gfx950 only) from csrc/*.hip with hipcc, libmxfp6_probes.so beside it, and the
+Python binding of the hot calls (_native.so, csrc/binding.cpp) with the host compiler.
 
     python -m hipkittensp_amd.build            # rebuild everything
 The libraries are built in-tree; nothing is installed.  No GPU is needed to build.
@@ -19,6 +20,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libmxfp6_gemm.so")
+NATIVE = os.path.join(HERE, "_native.so")
 PROBES_LIB = os.path.join(HERE, "libmxfp6_probes.so")
 SOURCES = ["api.hip", "dispatch.hip", "gemm_generic.hip", "gemm_tiled.hip", "gemm_tiled4.hip", "gemm_block.hip", "gemm_mid.hip", "gemm_skinny.hip", "gemm_ring.hip", "quantize.hip"]
 # (source, object name, extra flags).  gemm_tiled.hip gives five objects: its host-side part, and the kernel
@@ -49,6 +51,23 @@ def _compile(unit) -> str:
     return obj
 
 
+def _build_native() -> str:
+    """The Python binding of the hot calls: host code against torch's headers, linked to the operator's library beside it."""
+    import sysconfig
+
+    import torch
+
+    t = os.path.dirname(torch.__file__)
+    cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-isystem", os.path.join(t, "include"), "-isystem", "/opt/rocm/include",
+           "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, "binding.cpp"), "-o", NATIVE,
+           "-L", HERE, "-lmxfp6_gemm", "-L", os.path.join(t, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode:
+        raise RuntimeError(f"g++ failed on binding.cpp:\n{r.stderr}")
+    return NATIVE
+
+
 def build(verbose: bool = True) -> str:
     os.makedirs(OBJ, exist_ok=True)
     # the units that take longest first
@@ -65,6 +84,9 @@ def build(verbose: bool = True) -> str:
             raise RuntimeError(f"link failed:\n{r.stderr}")
         if verbose:
             print(f"built {lib}")
+    _build_native()
+    if verbose:
+        print(f"built {NATIVE}")
     return LIB
 
 

@@ -62,7 +62,8 @@ bool stream_is_capturing(hipStream_t s) {
 }
 
 // kind 0: pre-pass copies, kind 1: fp32 result of mxfp6_gemm_fused_fp6, kind 2: partial sums of a K split, kind 3: arrival
-// counters of the ring kernel's K split (zeroed when allocated; the kernels leave them zero).
+// counters of the ring kernel's K split (zeroed when allocated; the kernels leave them zero), kind 4: packed activations of
+// mxfp6_linear.
 // nullptr: no workspace (capture without one, table full of pinned entries, out of memory).
 uint8_t* stream_workspace(hipStream_t s, int kind, size_t bytes, bool zeroed = false) {
   int dev = 0;
@@ -313,10 +314,10 @@ int check_gemm_args(const void* A, const void* B, const void* As, const void* Bs
 
 int gemm_common(const void* A, const void* B, const void* As, const void* Bs, void* C, int M, int N, int K, int fmt_a,
                 int fmt_b, bool f32out, int layout_a, int layout_b, void* stream, const mxfp6::Epilogue& ep = mxfp6::Epilogue(),
-                int no_alloc = 0, int force_split = 0) {
+                int no_alloc = 0, int force_split = 0, bool checked = false) {
   bool empty;
-  int rc = check_gemm_args(A, B, As, Bs, C, M, N, K, fmt_a, fmt_b, f32out ? 3 : 1, layout_a, layout_b, ep, &empty);
-  if (rc || empty) return rc;
+  int rc = checked ? MXFP6_OK : check_gemm_args(A, B, As, Bs, C, M, N, K, fmt_a, fmt_b, f32out ? 3 : 1, layout_a, layout_b, ep, &empty);
+  if (rc || (!checked && empty)) return rc;
   rc = check_device();
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
@@ -412,6 +413,33 @@ int mxfp6_gemm_fused(const void* A, const void* B, const void* As, const void* B
   mxfp6::Epilogue ep;
   ep.bias = bias, ep.bias_bf16 = bias_bf16 != 0, ep.row_scale = row_scale, ep.col_scale = col_scale, ep.act = activation;
   return gemm_common(A, B, As, Bs, C, M, N, K, fmt_a, fmt_b, out_f32 != 0, layout_a, layout_b, stream, ep);
+}
+
+int mxfp6_linear(const void* X, int x_bf16, const void* W, const void* Ws, void* C, int M, int N, int K, int fmt_x, int fmt_w, int layout_w,
+                 const void* bias, int bias_bf16, int activation, void* stream) {
+  mxfp6::Epilogue ep;
+  ep.bias = bias, ep.bias_bf16 = bias_bf16 != 0, ep.act = activation;
+  bool empty;
+  int rc = check_gemm_args(X, W, X, Ws, C, M, N, K, fmt_x, fmt_w, 1, 0, layout_w, ep, &empty);
+  if (rc || empty) return rc;
+  if ((uintptr_t)X & 15) return MXFP6_EINVAL_ALIGN;
+  rc = check_device();
+  if (rc) return rc;
+  hipStream_t s = (hipStream_t)stream;
+  // Tile-major from 64 rows on, whatever M is (the workspace has whole 32-row tiles; what stands in the rows past M reaches
+  // nothing but outputs that are not stored): whole cache lines for every load of the GEMM.  Fewer rows stay row-major for the
+  // skinny kernel.
+  const int layout_x = M >= 64 && K % 128 == 0 ? MXFP6_LAYOUT_TILE : MXFP6_LAYOUT_ROW;
+  const size_t rows = ((size_t)M + 31) & ~(size_t)31;
+  const size_t nx = (rows * (K / 32) * 24 + 255) & ~(size_t)255, ns = rows * ((K + 511) / 512) * 16;
+  std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
+  uint8_t* xp = K > 0 ? stream_workspace(s, 4, nx + ns) : nullptr;
+  if (K > 0) {
+    if (!xp) return MXFP6_EWORKSPACE;
+    const hipError_t e = mxfp6::launch_quantize(X, x_bf16 != 0, xp, xp + nx, M, K, fmt_x, layout_x, s);
+    if (e != hipSuccess) return (int)e;
+  }
+  return gemm_common(xp, W, xp ? xp + nx : nullptr, Ws, C, M, N, K, fmt_x, fmt_w, false, layout_x, layout_w, stream, ep, 0, 0, true);
 }
 
 int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const void* Bs, void* C_packed, void* C_scale, int M, int N,

@@ -27,7 +27,7 @@ constexpr int kQWaves = 4;  // waves per workgroup; a wave fetches 64 blocks at 
 // v_cvt_scalef32_pk32_{fp6,bf6}_bf16 was checked against the fp32 one on 1 M values per format, no difference).
 template <int FMT, typename In>
 __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __restrict__ X, uint8_t* __restrict__ packed,
-                                                              uint8_t* __restrict__ scales, long nblocks, int nkb, int layout) {
+                                                              uint8_t* __restrict__ scales, long nblocks, int nkb, int layout, int rows) {
   constexpr int EMAX = FMT == 2 ? 2 : 4;
   constexpr int BB = 32 * (int)sizeof(In), P = BB / 16;  // bytes and 16-byte pieces of a block
   constexpr int kChunk = 64 * BB, NLD = kChunk / 1024;   // bytes and direct loads of a chunk
@@ -35,10 +35,10 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t buf = (uint32_t)(uintptr_t)(MXFP6_LDS uint8_t*)smem + wave * kChunk;
-  const long nchunks = (nblocks + 63) / 64;
+  const int nkt = nkb / 4;  // tile-major only: K-tiles per row
+  const long nchunks = layout ? (long)((rows + 15) / 16) * nkt : (nblocks + 63) / 64;
   const long stride = (long)gridDim.x * kQWaves;
   long chunk = (long)blockIdx.x * kQWaves + wave;
-  const int nkt = nkb / 4;  // tile-major only: K-tiles per row
 
   // slot s = q * 64 + lane of load q holds piece (s % P) ^ (b % P) of the chunk's block b = s / P; tile-major:
   // block b is K-block b % 4 of row b / 4 of the chunk
@@ -52,7 +52,7 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
     // the resource covers this chunk only (the whole input may exceed 4 GB); bytes past the end read as zero
     if (layout) {
       const long g16 = ch / nkt, kt = ch - g16 * nkt;
-      const __amdgpu_buffer_rsrc_t r = make_rsrc(reinterpret_cast<const uint8_t*>(X) + (g16 * 16 * nkb + kt * 4) * BB, (uint32_t)(15 * nkb * BB + 4 * BB));
+      const __amdgpu_buffer_rsrc_t r = make_rsrc(reinterpret_cast<const uint8_t*>(X) + (g16 * 16 * nkb + kt * 4) * BB, (uint32_t)((min(16, rows - (int)g16 * 16) - 1) * nkb * BB + 4 * BB));  // rows past the last read as zeros
 #pragma unroll
       for (int q = 0; q < NLD; q++) dma16(r, buf + q * 1024, voff[q], 0);
     } else {
@@ -124,7 +124,10 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
 #pragma unroll
       for (int i = 0; i < 3; i++)
         *reinterpret_cast<u32x2*>(packed + tile_major_offset(row, kb * 24 + 8 * i, nkt)) = u32x2{w[2 * i], w[2 * i + 1]};
-      scales[tile_major_scale_offset(row, kb, (nkb + 15) / 16)] = (uint8_t)sb;
+      uint8_t* const sp = scales + tile_major_scale_offset(row, kb, (nkb + 15) / 16);
+      *sp = (uint8_t)sb;
+      if (kt == nkt - 1)  // the bytes of K-blocks past K (K % 512 != 0) are zeros
+        for (int b = 4; b < 16 - ((nkb - 4) & 15); b += 4) sp[b] = 0;
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -133,9 +136,9 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
 hipError_t launch_quantize(const void* X, int x_bf16, uint8_t* packed, uint8_t* scales, int rows, int K, int fmt, int layout, hipStream_t s) {
   const long nblocks = (long)rows * (K / 32);
   if (nblocks == 0) return hipSuccess;
-  const long nchunks = (nblocks + 63) / 64, want = (nchunks + kQWaves - 1) / kQWaves;
+  const long nchunks = layout ? (long)((rows + 15) / 16) * (K / 128) : (nblocks + 63) / 64, want = (nchunks + kQWaves - 1) / kQWaves;
   const unsigned grid = (unsigned)(want < 256 * 5 ? want : 256 * 5);  // five workgroups of 32 KB LDS fit a CU
-#define MXFP6_Q(FMT, T) quantize_kernel<FMT, T><<<grid, kQWaves * 64, 0, s>>>((const T*)X, packed, scales, nblocks, K / 32, layout)
+#define MXFP6_Q(FMT, T) quantize_kernel<FMT, T><<<grid, kQWaves * 64, 0, s>>>((const T*)X, packed, scales, nblocks, K / 32, layout, rows)
   if (fmt == 2) { if (x_bf16) MXFP6_Q(2, uint16_t); else MXFP6_Q(2, float); }
   else { if (x_bf16) MXFP6_Q(3, uint16_t); else MXFP6_Q(3, float); }
 #undef MXFP6_Q

@@ -117,20 +117,15 @@ ACT_NONE, ACT_RELU, ACT_GELU, ACT_SILU = 0, 1, 2, 3
 _ACTS = {None: 0, "none": 0, "relu": 1, "gelu": 2, "silu": 3, 0: 0, 1: 1, 2: 2, 3: 3}
 
 
-_torch = None
-_fast = None  # (Tensor type, uint8, bfloat16, float32, raw-stream getter, current_device, the library's mxfp6_gemm_fused)
+_native_module = None
 
 
-def _fast_state():
-    global _torch, _fast
-    import torch
-
-    _torch = torch
-    get_raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if get_raw is None:
-        get_raw = lambda index: torch.cuda.current_stream(index).cuda_stream
-    _fast = (torch.Tensor, torch.uint8, torch.bfloat16, torch.float32, get_raw, torch.cuda.current_device, _lib.lib().mxfp6_gemm_fused)
-    return _fast
+def _native():
+    """The native binding (csrc/binding.cpp): the usual calls without Python and ctypes between them and the library."""
+    global _native_module
+    if _native_module is None:
+        _native_module = _lib.native()
+    return _native_module
 
 
 def dispatch_micro(A, B, A_scale, B_scale, C, fmt_a: int = E2M3, fmt_b: int = E2M3, layout_a: int = LAYOUT_ROW,
@@ -138,37 +133,13 @@ def dispatch_micro(A, B, A_scale, B_scale, C, fmt_a: int = E2M3, fmt_b: int = E2
                    fmt_c: int = E2M3) -> None:
     """C = dq(A) @ dq(B).T (the full description is _dispatch_micro_checked's, which this is a short cut in front of).
 
-    The usual call -- five contiguous 2-D torch tensors of the right dtypes and shapes on the current GPU, no fused
-    epilogue -- is recognised here with one read of each tensor's metadata and goes straight to the library (a few
-    microseconds of host time, which is what a small GEMM's launch rate is bound by); everything else, including every
-    call that is wrong in some way, takes the checked path below, which handles the general cases and raises the
-    reference binding's errors."""
-    f = _fast or _fast_state()
-    T, u8 = f[0], f[1]
-    if (bias is None and row_scale is None and col_scale is None and activation is None and C_scale is None
-            and type(A) is T and type(B) is T and type(A_scale) is T and type(B_scale) is T and type(C) is T
-            and A.dtype is u8 and B.dtype is u8 and A_scale.dtype is u8 and B_scale.dtype is u8):
-        cd = C.dtype
-        sa, sb, sas, sbs, sc = A.shape, B.shape, A_scale.shape, B_scale.shape, C.shape
-        dev = C.get_device()
-        if ((cd is f[2] or cd is f[3]) and len(sa) == 2 and len(sb) == 2 and len(sas) == 2 and len(sbs) == 2 and len(sc) == 2
-                and dev >= 0 and dev == f[5]() and A.get_device() == dev and B.get_device() == dev
-                and A_scale.get_device() == dev and B_scale.get_device() == dev
-                and A.is_contiguous() and B.is_contiguous() and A_scale.is_contiguous() and B_scale.is_contiguous() and C.is_contiguous()
-                and (fmt_a == 2 or fmt_a == 3) and (fmt_b == 2 or fmt_b == 3) and (layout_a == 0 or layout_a == 1) and (layout_b == 0 or layout_b == 1)):
-            M, wa = sa
-            N = sb[0]
-            K = wa // 3 * 4
-            if (wa == sb[1] and wa % 24 == 0 and sc[0] == M and sc[1] == N and sas[0] == M and sbs[0] == N
-                    and sas[1] == (K // 32 if layout_a == 0 else (K + 511) // 512 * 16)
-                    and sbs[1] == (K // 32 if layout_b == 0 else (K + 511) // 512 * 16)
-                    and (layout_a == 0 or (M % 32 == 0 and K % 128 == 0)) and (layout_b == 0 or (N % 32 == 0 and K % 128 == 0))):
-                rc = f[6](A.data_ptr(), B.data_ptr(), A_scale.data_ptr(), B_scale.data_ptr(), C.data_ptr(), M, N, K,
-                          fmt_a, fmt_b, layout_a, layout_b, 1 if cd is f[3] else 0, 0, 0, 0, 0, 0, f[4](dev))
-                if rc:
-                    _lib.check(rc, "dispatch_micro")
-                return
-    _dispatch_micro_checked(A, B, A_scale, B_scale, C, fmt_a, fmt_b, layout_a, layout_b, bias, row_scale, col_scale, activation, C_scale, fmt_c)
+    The usual call -- contiguous 2-D torch tensors of the right dtypes and shapes on the current GPU -- is recognised and
+    made by the native binding in about a microsecond of host time (which is what a small GEMM's launch rate is bound
+    by); everything else, including every call that is wrong in some way, takes the checked path below, which handles the
+    general cases and raises the reference binding's errors."""
+    act = 0 if activation is None else _ACTS.get(activation, -1) if isinstance(activation, (str, int)) else -1
+    if (_native_module or _native()).gemm(A, B, A_scale, B_scale, C, fmt_a, fmt_b, layout_a, layout_b, bias, row_scale, col_scale, act, C_scale, fmt_c) is None:
+        _dispatch_micro_checked(A, B, A_scale, B_scale, C, fmt_a, fmt_b, layout_a, layout_b, bias, row_scale, col_scale, activation, C_scale, fmt_c)
 
 
 def _dispatch_micro_checked(A, B, A_scale, B_scale, C, fmt_a: int = E2M3, fmt_b: int = E2M3, layout_a: int = LAYOUT_ROW,
@@ -262,6 +233,9 @@ def quantize(X, fmt: int = E2M3, layout: int = LAYOUT_ROW):
     """fp32 or bf16 [rows, K] on the GPU -> (packed uint8 [rows, 3K/4], scales uint8 [rows, K/32]).
     With layout=LAYOUT_TILE packed bytes and scales are written tile-major (rows % 32 == 0, K % 128 == 0;
     scales [rows, ceil(K/512) * 16], padding zero)."""
+    out = (_native_module or _native()).quantize(X, fmt, layout)
+    if out is not None:
+        return out
     import torch
 
     X = _as_tensor(X, "X")
@@ -276,8 +250,7 @@ def quantize(X, fmt: int = E2M3, layout: int = LAYOUT_ROW):
     if layout not in (LAYOUT_ROW, LAYOUT_TILE):
         raise RuntimeError("layout must be LAYOUT_ROW (0) or LAYOUT_TILE (1)")
     sw = scale_width(K, layout)
-    alloc = torch.zeros if sw != K // 32 else torch.empty  # the quantiser does not write padding bytes
-    scales = alloc(*X.shape[:-1], sw, dtype=torch.uint8, device=X.device)
+    scales = torch.empty(*X.shape[:-1], sw, dtype=torch.uint8, device=X.device)
     with _on_device(X.device):
         fn = _lib.lib().mxfp6_quantize_bf16 if X.dtype == torch.bfloat16 else _lib.lib().mxfp6_quantize_ex
         rc = fn(X.data_ptr(), packed.data_ptr(), scales.data_ptr(), rows, K, fmt, layout, _stream())

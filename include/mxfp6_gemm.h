@@ -19,12 +19,13 @@
  * Work is queued on `hip_stream` (a hipStream_t; NULL = the null stream); no function synchronises the
  * device or the stream.
  *
- * Device memory.  Four uses take a workspace from the stream-ordered allocator
+ * Device memory.  Five uses take a workspace from the stream-ordered allocator
  * (hipMallocAsync on `hip_stream`), at most once per (device, stream) and use (regrown when a later call
  * needs more), and keep it until mxfp6_release_workspaces():
  *   - the gemm entry points on large row-major problems (re-layout pre-pass, see mxfp6_set_relayout):
  *     up to 0.78 (M + N) K bytes;
  *   - mxfp6_gemm_fused_fp6 on shapes the LDS-tiled kernel does not run: 4 M N bytes;
+ *   - mxfp6_linear: 0.79 M K bytes, M rounded up to 32;
  *   - the gemm entry points on decode shapes whose K range is split between workgroups (M <= 32, N <= 2048,
  *     K >= 24576): 2 MB;
  *   - the gemm entry points on problems of few output tiles and long K (up to a few hundred rows of A; see
@@ -228,7 +229,7 @@ int mxfp6_gemm_ex(const void *A_packed, const void *B_packed, const void *A_scal
                   void *hip_stream);
 
 /* mxfp6_quantize writing the packed operand and its scales in the given layout (tile-major scales: rows *
- * ceil(K/512) * 16 bytes, of which the padding bytes are not written). */
+ * ceil(K/512) * 16 bytes; the bytes of K-blocks past K are written as 0). */
 int mxfp6_quantize_ex(const float *X, void *packed, void *scales, int rows, int K, int fmt, int layout,
                       void *hip_stream);
 
@@ -269,6 +270,18 @@ int mxfp6_gemm_fused_fp6(const void *A_packed, const void *B_packed, const void 
                          void *C_packed, void *C_scale, int M, int N, int K, int fmt_a, int fmt_b, int layout_a,
                          int layout_b, int fmt_c, const void *bias, int bias_bf16, const float *row_scale,
                          const float *col_scale, int activation, void *hip_stream);
+
+/*
+ * A linear layer on unquantised activations: X [M, K] (fp32, or bf16 with x_bf16 != 0; 16-byte aligned) is quantised to
+ * MXFP6 (fmt_x) as mxfp6_quantize_ex / mxfp6_quantize_bf16 would, and
+ *   C[m][n] = act((dq(X) . dq(W)^T)[m][n] + bias[n])         bf16
+ * as mxfp6_gemm_fused would compute it from that operand.  W_packed [N, 3K/4], W_scale: the weights in layout_w; bias as in
+ * mxfp6_gemm_fused (NULL = none).  The packed activations live in a workspace of this stream (0.79 bytes per element of X,
+ * rows rounded up to 32), in the layout the GEMM prefers.  MXFP6_EWORKSPACE, and nothing launched, where it cannot be had
+ * (first use under capture).  No counterpart in the reference.
+ */
+int mxfp6_linear(const void *X, int x_bf16, const void *W_packed, const void *W_scale, void *C_bf16, int M, int N, int K,
+                 int fmt_x, int fmt_w, int layout_w, const void *bias, int bias_bf16, int activation, void *hip_stream);
 
 /*
  * Returns every workspace this library holds (see "Device memory" above) to the stream-ordered allocator, each in

@@ -1,0 +1,90 @@
+"""The linear layer's single native call (mxfp6_linear) against the two public calls it stands for, quantise then GEMM: the same
+packed activations and the same kernels' sums, so the same bits wherever those are exact (these inputs' sums are), at the
+edges of its layouts: below and above 64 rows, row counts that are no multiple of the 16 and 32 rows of a tile-major
+chunk, K-tiles that fill no group of four."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hk():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import hipkittensp_amd as m
+
+    return m
+
+
+def steps(hk, layer, x):
+    tk = hk.tk_kernel
+    rows = x.numel() // x.shape[-1]
+    xp, xs = tk.quantize(x.reshape(rows, -1), layer.fmt_x)
+    C = torch.empty(rows, layer.out_features, dtype=torch.bfloat16, device="cuda")
+    tk.dispatch_micro(xp, layer.weight_packed, xs, layer.weight_scale, C, layer.fmt_x, layer.fmt_w, 0, layer.layout_w, bias=layer.bias, activation=layer.activation)
+    return C.view(*x.shape[:-1], -1)
+
+
+@pytest.mark.parametrize("M", [1, 17, 63, 64, 65, 79, 80, 81, 97, 200, 257, 700])
+@pytest.mark.parametrize("N,K", [(256, 512), (96, 640), (1000, 1152), (160, 96), (33, 512)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_linear_is_quantise_then_gemm(hk, M, N, K, dtype):
+    from hipkittensp_amd.torch_op import MXFP6Linear
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    layer = MXFP6Linear(torch.randn(N, K, device="cuda", generator=g) * 0.02, bias=torch.randn(N, device="cuda", generator=g).to(torch.bfloat16), activation="relu")
+    for x in (torch.randn(M, K, device="cuda", generator=g).to(dtype), torch.randn(2, M, K, device="cuda", generator=g).to(dtype)):
+        y = layer(x)
+        assert y.shape == (*x.shape[:-1], N) and y.dtype == torch.bfloat16
+        assert torch.equal(y, steps(hk, layer, x)), (M, N, K, x.shape)
+
+
+def test_linear_streams_graphs_and_general_cases(hk):
+    from hipkittensp_amd.torch_op import MXFP6Linear
+
+    g = torch.Generator(device="cuda").manual_seed(5)
+    layer = MXFP6Linear(torch.randn(512, 1024, device="cuda", generator=g) * 0.02)
+    xs = [torch.randn(96, 1024, device="cuda", generator=g) for _ in range(2)]
+    want = [steps(hk, layer, x) for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in xs]   # a workspace per stream
+    out = [[], []]
+    for _ in range(8):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                out[i].append(layer(xs[i]))
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, want[i]) for i in range(2) for y in out[i])
+    assert torch.equal(layer(xs[0].t().contiguous().t()), want[0])      # a view that is not contiguous
+    assert torch.equal(layer(xs[0].to(torch.float16).to(torch.float32)), steps(hk, layer, xs[0].to(torch.float16).float()))
+    # captured on a stream with a workspace and on one without; replayed with other work in between
+    x = xs[0].clone()
+    for s in (streams[0], torch.cuda.Stream()):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            y = layer(x)
+        for i in (1, 0, 1):
+            x.copy_(xs[i])
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want[i])
+            layer(xs[0])
+            torch.cuda.synchronize()
+    with pytest.raises(RuntimeError):
+        layer(torch.randn(4, 1000, device="cuda"))   # K of another layer
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,K", [(32, 128), (64, 640), (32, 896), (96, 1152)])
+def test_tile_major_scales_are_padded_with_zeros(hk, rows, K, dtype):
+    from hipkittensp_amd import _lib
+
+    x = torch.randn(rows, K, device="cuda", generator=torch.Generator(device="cuda").manual_seed(K)).to(dtype)
+    w = (K + 511) // 512 * 16
+    p = torch.empty(rows, K // 4 * 3, dtype=torch.uint8, device="cuda")
+    s = torch.full((rows, w), 255, dtype=torch.uint8, device="cuda")
+    fn = _lib.lib().mxfp6_quantize_bf16 if dtype == torch.bfloat16 else _lib.lib().mxfp6_quantize_ex
+    assert fn(x.data_ptr(), p.data_ptr(), s.data_ptr(), rows, K, 2, 1, torch.cuda.current_stream().cuda_stream) == 0
+    pr, sr = hk.quantize(x, 2)
+    assert torch.equal(s, hk.tile_scales(sr, K)) and torch.equal(p, hk.tile_operand(pr))
