@@ -44,6 +44,7 @@ struct RingArgs {
   float* part;   // nsplit > 1: partial tiles, [tile][share][wave][TA][4][64 lanes][4] floats
   int* counters; // nsplit > 1: one arrival counter per tile, zero between launches
   int M, N, K, layout_a, layout_b, col_tiles, m_blocks, nsplit;
+  int stream;  // B is read with the non-temporal bit (kStreamBytes)
   Epilogue ep;
 };
 
@@ -125,8 +126,13 @@ __global__ __launch_bounds__((kRingNC + 1) * 64) void gemm_ring_kernel(const Rin
       const uint32_t pb = __builtin_amdgcn_readfirstlane(par);
       dma16(rBs, bsbuf + pb * 1024, voff_bs, __builtin_amdgcn_readfirstlane(layout_b ? chunk * 512 : chunk * 16));
       const int so = __builtin_amdgcn_readfirstlane(layout_b ? chunk * (KT * 3072) : chunk * (KT * 96));
+      if (args.stream) {
 #pragma unroll
-      for (int i = 0; i < NL; i++) dma16(rB, bbuf + pb * kSlot + i * 1024, voff_b[i], so);
+        for (int i = 0; i < NL; i++) dma16_nt(rB, bbuf + pb * kSlot + i * 1024, voff_b[i], so);
+      } else {
+#pragma unroll
+        for (int i = 0; i < NL; i++) dma16(rB, bbuf + pb * kSlot + i * 1024, voff_b[i], so);
+      }
     };
     issue_b(c0, 0);
     if (nmine > 1) issue_b(c0 + 1, 1);
@@ -370,7 +376,8 @@ static hipError_t launch(const GemmArgs& g, hipStream_t s) {
   const bool split = g.ksplit > 1 && g.ks_part && g.ks_counters;
   RingPlan p = ring_plan(g, split ? g.ksplit : 1);
   if (split && p.nsplit != g.ksplit) return hipErrorInvalidValue;
-  RingArgs ra = {g.A, g.B, g.As, g.Bs, g.C, g.ks_part, g.ks_counters, g.M, g.N, g.K, g.layout_a, g.layout_b, p.col_tiles, p.m_blocks, p.nsplit, g.ep};
+  RingArgs ra = {g.A, g.B, g.As, g.Bs, g.C, g.ks_part, g.ks_counters, g.M, g.N, g.K, g.layout_a, g.layout_b, p.col_tiles, p.m_blocks, p.nsplit,
+                 p.m_blocks == 1 && (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes, g.ep};
   const unsigned grid = (unsigned)p.col_tiles * p.m_blocks * p.nsplit;
   constexpr int threads = (kRingNC + 1) * 64;
   if (p.ta == 1) gemm_ring_kernel<FA, FB, Out, 1><<<grid, threads, 0, s>>>(ra);

@@ -50,7 +50,7 @@ template <int FA, int FB, typename Out, int AR, int NW, int BR, int DB>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                                                               const uint8_t* __restrict__ As, const uint8_t* __restrict__ Bs,
                                                               typename Out::type* __restrict__ C, int M, int N, int K, int layout_b,
-                                                              const Epilogue ep, int nsplit, float* ws_part, int* ws_cnt) {
+                                                              const Epilogue ep, int nsplit, float* ws_part, int* ws_cnt, int stream) {
   static_assert(BR == 64 || BR == 32 || BR == 16, "rows of B per workgroup");
   static_assert(AR == 16 || AR == 32 || AR == 64 || AR == 128, "rows of A");
   constexpr int TA = AR > 32 ? AR / 32 : 1;   // 32-row tiles of A per wave
@@ -144,8 +144,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
     const uint32_t pb = __builtin_amdgcn_readfirstlane(par);
     dma16(rBs, buf + kScOff + pb * 1024, voff_bs, sosb);
     const int sob = __builtin_amdgcn_readfirstlane(layout_b ? chunk * (KT * 3072) : chunk * kRow);
+    if (stream) {  // B is read with the non-temporal bit (kStreamBytes)
 #pragma unroll
-    for (int i = 0; i < NBL; i++) dma16(rB, buf + pb * kBBuf + i * 1024, voff_b[i], sob);
+      for (int i = 0; i < NBL; i++) dma16_nt(rB, buf + pb * kBBuf + i * 1024, voff_b[i], sob);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NBL; i++) dma16(rB, buf + pb * kBBuf + i * 1024, voff_b[i], sob);
+    }
   };
   auto issue_a = [&](int chunk) __attribute__((always_inline)) {
     const int sg = KT == 4 ? chunk : chunk >> 1;
@@ -461,7 +466,7 @@ static hipError_t launch(const GemmArgs& g, hipStream_t s) {
 #define MXFP6_SK(AR, NW, BR) MXFP6_SKD(AR, NW, BR, 1)
 #define MXFP6_SKD(AR, NW, BR, DB) \
   gemm_skinny_kernel<FA, FB, Out, AR, NW, BR, DB><<<(g.N + BR - 1) / BR * nsplit, NW * 64, 0, s>>>( \
-      g.A, g.B, g.As, g.Bs, (T*)g.C, g.M, g.N, g.K, g.layout_b, g.ep, nsplit, ws.part, ws.cnt)
+      g.A, g.B, g.As, g.Bs, (T*)g.C, g.M, g.N, g.K, g.layout_b, g.ep, nsplit, ws.part, ws.cnt, (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes)
   // two chunks of B per wave (17 - 32 and 65 - 128 rows of A: measured 3 - 15 % and 3 - 6 %); forced geometry 1: one
   const bool db = g.skinny_geometry != 1;
   if (geo == 6) {

@@ -35,6 +35,14 @@ inline bool operands_aligned16(const GemmArgs& g) {
   return (((uintptr_t)g.A | (uintptr_t)g.B | (uintptr_t)g.As | (uintptr_t)g.Bs) & 15) == 0;
 }
 
+// Streams of this many bytes and more are read with the non-temporal bit: half of the 256 MB last-level cache, so that little of
+// the stream would be found there by the next read.  us, plain / non-temporal, weights of 184 MB: ring kernel at 16 x 8192 x 28672
+// 36.5 / 33.6 (tile-major 35.0 / 31.7), 64 rows 41.8 / 39.7 (40.0 / 38.1); skinny kernel at 16 rows 36.7 / 34.3 (33.9 / 31.1);
+// quantiser, 8192 x 28672 fp32 in and packed out: 214 / 185.  A smaller stream may stay in that cache from one call to the next, where the bit
+// costs more than it gives: skinny kernel, 32 x 4096 x 14336 (46 MB), weights found in the cache 11.8 / 14.5, from memory
+// 15.5 / 15.1.
+constexpr size_t kStreamBytes = (size_t)128 << 20;
+
 // ---- kernel choice (dispatch.hip): candidates of the automatic path, a time model per candidate, a calibration table
 enum Candidate : int { kCandTiled256 = 0, kCandTiled128x256, kCandTiled128x128, kCandBlock, kCandBlockWide, kCandSkinny, kCandTiledSplit256, kCandTiledSplit128, kCandBlockSplit, kCandRing, kNumCandidates };
 struct KernelChoice {

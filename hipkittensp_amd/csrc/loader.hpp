@@ -18,7 +18,14 @@ __device__ __forceinline__ void dma16(const __amdgpu_buffer_rsrc_t& rsrc, uint32
                : "s"(lds_base), "v"(voff), "s"(rsrc), "s"(soff)
                : "memory");
 }
-// the same with 4 bytes per lane, to lds_base + 4 * lane
+// dma16 with the non-temporal bit: for a stream that is read once and larger than the caches
+__device__ __forceinline__ void dma16_nt(const __amdgpu_buffer_rsrc_t& rsrc, uint32_t lds_base, int voff, int soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+               :
+               : "s"(lds_base), "v"(voff), "s"(rsrc), "s"(soff)
+               : "memory");
+}
+// dma16 with 4 bytes per lane, to lds_base + 4 * lane
 __device__ __forceinline__ void dma4(const __amdgpu_buffer_rsrc_t& rsrc, uint32_t lds_base, int voff, int soff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
                :
