@@ -18,8 +18,13 @@ namespace mxfp6 {
 // instructions per element, the kernel was ALU-bound at 4.4 TB/s.)
 // Row-major output: a wave's 64 blocks are consecutive (1536 contiguous output bytes).  Tile-major output: they are
 // 16 rows x one K-tile (512 input bytes per row, four whole lines), which is half of a 3 KB output tile and again
-// 1536 contiguous bytes; a block's 24 bytes are three 8-byte stores (an aligned 8-byte run never straddles the
-// 16-byte pieces the tile-major order permutes).
+// 1536 contiguous bytes.  The 1536 bytes are put together in the wave's buffer (a block's 24 bytes are three 8-byte writes:
+// an aligned 8-byte run never straddles the 16-byte pieces the tile-major order permutes) and leave as 16 bytes per lane, whole
+// lines in one and a half store instructions instead of three that touch every line three times.
+// What bounds it is memory: 8192 x 28672 fp32 (940 MB in, 183 MB out) took 224 us (5.0 TB/s; a copy reaches 4.8, a
+// read-only stream 6.05) with five workgroups per CU that each took many chunks in turn, the next one's loads under the
+// stores; one chunk per wave and as many workgroups as that takes, so that the CUs' scheduler fills every gap: 214; past the last-level
+// cache the input read and the output written with the non-temporal bit: 185 (6.1 TB/s; each alone 196 and 205).
 constexpr int kQWaves = 4;  // waves per workgroup; a wave fetches 64 blocks at a time (8 KB of fp32, 4 KB of bf16)
 
 
@@ -27,7 +32,7 @@ constexpr int kQWaves = 4;  // waves per workgroup; a wave fetches 64 blocks at 
 // v_cvt_scalef32_pk32_{fp6,bf6}_bf16 was checked against the fp32 one on 1 M values per format, no difference).
 template <int FMT, typename In>
 __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __restrict__ X, uint8_t* __restrict__ packed,
-                                                              uint8_t* __restrict__ scales, long nblocks, int nkb, int layout, int rows) {
+                                                              uint8_t* __restrict__ scales, long nblocks, int nkb, int layout, int rows, int stream_in, int stream_out) {
   constexpr int EMAX = FMT == 2 ? 2 : 4;
   constexpr int BB = 32 * (int)sizeof(In), P = BB / 16;  // bytes and 16-byte pieces of a block
   constexpr int kChunk = 64 * BB, NLD = kChunk / 1024;   // bytes and direct loads of a chunk
@@ -50,26 +55,33 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
   }
   auto fetch = [&](long ch) __attribute__((always_inline)) {
     // the resource covers this chunk only (the whole input may exceed 4 GB); bytes past the end read as zero
+    const uint8_t* base;
+    uint32_t len;
     if (layout) {
       const long g16 = ch / nkt, kt = ch - g16 * nkt;
-      const __amdgpu_buffer_rsrc_t r = make_rsrc(reinterpret_cast<const uint8_t*>(X) + (g16 * 16 * nkb + kt * 4) * BB, (uint32_t)((min(16, rows - (int)g16 * 16) - 1) * nkb * BB + 4 * BB));  // rows past the last read as zeros
-#pragma unroll
-      for (int q = 0; q < NLD; q++) dma16(r, buf + q * 1024, voff[q], 0);
+      base = reinterpret_cast<const uint8_t*>(X) + (g16 * 16 * nkb + kt * 4) * BB;
+      len = (uint32_t)((min(16, rows - (int)g16 * 16) - 1) * nkb * BB + 4 * BB);  // rows past the last read as zeros
     } else {
       const long left = nblocks * BB - ch * kChunk;
-      const __amdgpu_buffer_rsrc_t r = make_rsrc(reinterpret_cast<const uint8_t*>(X) + ch * kChunk, (uint32_t)(left < kChunk ? left : kChunk));
+      base = reinterpret_cast<const uint8_t*>(X) + ch * kChunk;
+      len = (uint32_t)(left < kChunk ? left : kChunk);
+    }
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(base, len);
+    if (stream_in) {
+#pragma unroll
+      for (int q = 0; q < NLD; q++) dma16_nt(r, buf + q * 1024, voff[q], 0);
+    } else {
 #pragma unroll
       for (int q = 0; q < NLD; q++) dma16(r, buf + q * 1024, voff[q], 0);
     }
   };
-  if (chunk < nchunks) fetch(chunk);
-  for (; chunk < nchunks; chunk += stride) {
+  for (; chunk < nchunks; chunk += stride) {  // once, unless the chunks outnumber the largest grid
+    fetch(chunk);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     v4i x[P];
 #pragma unroll
     for (int c = 0; c < P; c++) x[c] = *reinterpret_cast<const v4i*>(smem + wave * kChunk + lane * BB + ((c ^ (lane % P)) * 16));
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (chunk + stride < nchunks) fetch(chunk + stride);  // the buffer is free again: the next chunk streams in under the arithmetic
 
     float amax = 0.f;
 #pragma unroll
@@ -110,35 +122,51 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
       if constexpr (FMT == 2) w = __builtin_amdgcn_cvt_scalef32_pk32_fp6_bf16(xb, scale);
       else w = __builtin_amdgcn_cvt_scalef32_pk32_bf6_bf16(xb, scale);
     }
+    // the chunk's 1536 output bytes in order, in the buffer its input has left
+    uint8_t* const image = smem + wave * kChunk;
+    const long g16 = layout ? chunk / nkt : 0;
+    const int kt = layout ? (int)(chunk - g16 * nkt) : 0, row = (int)(g16 * 16) + (lane >> 2);
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const int byte = (lane & 3) * 24 + 8 * i, c = byte >> 4;
+      const int at = layout ? (lane >> 2) * 96 + (c ^ ((row >> 3) & 1)) * 16 + (byte & 15) : lane * 24 + 8 * i;
+      *reinterpret_cast<u32x2*>(image + at) = u32x2{w[2 * i], w[2 * i + 1]};
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    v4i out0 = *reinterpret_cast<const v4i*>(image + lane * 16), out1 = *reinterpret_cast<const v4i*>(image + 1024 + (lane & 31) * 16);
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(out0), "+v"(out1)::"memory");
+    uint8_t* const dst = layout ? packed + ((g16 >> 1) * nkt + kt) * 3072 + (g16 & 1) * 1536 : packed + chunk * 1536;
+    if (layout || (chunk + 1) * 64 <= nblocks) {
+      v4i* const d = reinterpret_cast<v4i*>(dst) + lane;
+      if (stream_out) {
+        __builtin_nontemporal_store(out0, d);
+        if (lane < 32) __builtin_nontemporal_store(out1, d + 64);
+      } else {
+        d[0] = out0;
+        if (lane < 32) d[64] = out1;
+      }
+    } else if (chunk * 64 + lane < nblocks) {  // the last chunk's blocks one by one
+#pragma unroll
+      for (int i = 0; i < 3; i++) *reinterpret_cast<u32x2*>(dst + lane * 24 + 8 * i) = u32x2{w[2 * i], w[2 * i + 1]};
+    }
     if (layout == 0) {
-      const long b = chunk * 64 + lane;
-      if (b >= nblocks) continue;
-      u32x2* dst = reinterpret_cast<u32x2*>(packed + b * 24);
-#pragma unroll
-      for (int i = 0; i < 3; i++) dst[i] = u32x2{w[2 * i], w[2 * i + 1]};
-      scales[b] = (uint8_t)sb;
+      if (chunk * 64 + lane < nblocks) scales[chunk * 64 + lane] = (uint8_t)sb;
     } else {
-      const long g16 = chunk / nkt;
-      const int kt = (int)(chunk - g16 * nkt);
-      const int row = (int)(g16 * 16) + (lane >> 2), kb = kt * 4 + (lane & 3);
-#pragma unroll
-      for (int i = 0; i < 3; i++)
-        *reinterpret_cast<u32x2*>(packed + tile_major_offset(row, kb * 24 + 8 * i, nkt)) = u32x2{w[2 * i], w[2 * i + 1]};
-      uint8_t* const sp = scales + tile_major_scale_offset(row, kb, (nkb + 15) / 16);
+      uint8_t* const sp = scales + tile_major_scale_offset(row, kt * 4 + (lane & 3), (nkb + 15) / 16);
       *sp = (uint8_t)sb;
       if (kt == nkt - 1)  // the bytes of K-blocks past K (K % 512 != 0) are zeros
         for (int b = 4; b < 16 - ((nkb - 4) & 15); b += 4) sp[b] = 0;
     }
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 hipError_t launch_quantize(const void* X, int x_bf16, uint8_t* packed, uint8_t* scales, int rows, int K, int fmt, int layout, hipStream_t s) {
   const long nblocks = (long)rows * (K / 32);
   if (nblocks == 0) return hipSuccess;
   const long nchunks = layout ? (long)((rows + 15) / 16) * (K / 128) : (nblocks + 63) / 64, want = (nchunks + kQWaves - 1) / kQWaves;
-  const unsigned grid = (unsigned)(want < 256 * 5 ? want : 256 * 5);  // five workgroups of 32 KB LDS fit a CU
-#define MXFP6_Q(FMT, T) quantize_kernel<FMT, T><<<grid, kQWaves * 64, 0, s>>>((const T*)X, packed, scales, nblocks, K / 32, layout, rows)
+  const unsigned grid = (unsigned)(want < (1L << 30) ? want : 1L << 30);
+  const int stream_in = (size_t)rows * K * (x_bf16 ? 2 : 4) >= kStreamBytes, stream_out = (size_t)rows * (K / 4 * 3) >= kStreamBytes;
+#define MXFP6_Q(FMT, T) quantize_kernel<FMT, T><<<grid, kQWaves * 64, 0, s>>>((const T*)X, packed, scales, nblocks, K / 32, layout, rows, stream_in, stream_out)
   if (fmt == 2) { if (x_bf16) MXFP6_Q(2, uint16_t); else MXFP6_Q(2, float); }
   else { if (x_bf16) MXFP6_Q(3, uint16_t); else MXFP6_Q(3, float); }
 #undef MXFP6_Q
