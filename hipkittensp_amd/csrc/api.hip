@@ -157,7 +157,7 @@ bool apply_choice(mxfp6::GemmArgs& g, const mxfp6::KernelChoice& c, hipStream_t 
     case mxfp6::kCandTiled128x128: g.tile_rows = 128, g.tile_cols = 128; return true;
     case mxfp6::kCandBlockWide: g.tile_cols = 256; return true;
     case mxfp6::kCandTiledSplit256: case mxfp6::kCandTiledSplit128: case mxfp6::kCandBlockSplit: {
-      uint8_t* pp = stream_workspace(s, 2, (size_t)c.shares * g.M * g.N * sizeof(float));
+      uint8_t* pp = stream_workspace(s, 2, mxfp6::partial_offset(c.shares, 0, 0, g.M, g.N));
       if (!pp) return false;
       g.ksplit = c.shares, g.ks_part = reinterpret_cast<float*>(pp);
       if (c.cand != mxfp6::kCandBlockSplit) g.tile_rows = c.rows, g.tile_cols = 256;

@@ -77,8 +77,7 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   const int rowbytes = K / 32 * 24, sbytes = K / 32, nkt_all = RAGGED ? (K + kBK - 1) / kBK : K / kBK, nk4_all = (nkt_all + 3) / 4;  // tile-major scales: one 512-byte chunk per 32 rows and group of four K-tiles, the last one padded
   // K split: workgroup b takes share l / tiles of tile l % tiles, l = ksplit_order(b) -- the same number of whole groups
   // of four K-tiles for every share, the last one what is left of K (at least one K-tile: the launcher sees to that) --
-  // and leaves its fp32 sums in matrix `share` of args.C, then a workspace of nsplit matrices [M, N]
-  // (ksplit_reduce_kernel adds them up)
+  // and leaves its fp32 sums in args.C, then a workspace (partial_offset; RAGGED: nsplit matrices; the reduction adds them up)
   const int ntiles = args.tiles_m * args.tiles_n;
   const bool by_share = args.nsplit > 1 && ksplit_by_share(ntiles * args.nsplit, args.xcd_remap);  // the XCDs are dealt by ksplit_order, not by tile_order
   const int order = args.nsplit > 1 ? ksplit_order(blockIdx.x, ntiles * args.nsplit, args.xcd_remap) : blockIdx.x, share = order / ntiles;
@@ -455,6 +454,20 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
             __builtin_amdgcn_raw_buffer_store_b128(v, rC, voff + j * 64 + t * 32, i * 32 * N2, 0);
         }
     }
+  } else if (!RAGGED && args.nsplit > 1) {
+    // this share's partial sums, in the accumulators' order (partial_offset)
+    const int band0 = pm * (kBM / 32) + wm * 2, ct0 = pn * (kBN / 32) + wn * 2;
+    float* const base = (float*)args.C + partial_offset(share, band0, ct0, args.M, N) / 4 + lane * 4;
+    const size_t band_stride = ((size_t)N + 31) / 32 * 1024;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+        if ((band0 + i) * 32 + r32 < args.M && (ct0 + j) * 32 < N) {
+#pragma unroll
+          for (int gq = 0; gq < 4; gq++)
+            *reinterpret_cast<v4f*>(base + i * band_stride + j * 1024 + gq * 256) = v4f{acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]};
+        }
   } else {
     const int col_l = wn * 64 + 4 * h;
     const int voff = row_l * N2 + col_l * 4;

@@ -132,8 +132,8 @@ struct TiledArgs {
 // tile; bit 3 leaves everything in and adds idle clocks (a wave sleeps 128 clocks after every fourth MFMA).  What the remaining parts of the kernel take, in time and in shader clocks, is how bench.py splits the kernel's
 // time between the matrix cores, the LDS reads and the loads.
 // KSPLIT: the K range of an output tile is split between args.nsplit workgroups (few output tiles, long K: M of a few
-// hundred rows).  Share s of a tile multiplies K-tiles [s, s + 1) * nkt / nsplit and stores its fp32 sums into matrix s of
-// args.C, which is then a workspace of nsplit matrices [M, N]; ksplit_reduce_kernel adds them in share order and applies
+// hundred rows).  Share s of a tile multiplies K-tiles [s, s + 1) * nkt / nsplit and stores its fp32 sums into args.C, which is
+// then a workspace (partial_offset); ksplit_reduce_kernel adds them in share order and applies
 // the epilogue.  (Summed inside this kernel instead -- partial tiles and arrival counters at device scope, the last
 // wave to arrive adds -- the few waves that end up adding read nsplit tiles each past the L2s: 30 us for 32 MB.)
 template <int FA, int FB, typename Out, int TM, int TN, bool FUSED, int ABL = 0, bool KSPLIT = false>
@@ -614,9 +614,24 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
       return;
     }
     const int N = g->N, N2 = N * (int)sizeof(OutT);  // N2: bytes per row of C
+    if constexpr (KSPLIT) {
+      // this share's partial sums, in the accumulators' order (partial_offset); bands and column tiles past M and N have no place
+      const int M = g->M, band0 = (tile_cur & 0xffff) * (kBM / 32) + wm * TM, ct0 = (tile_cur >> 16) * (kBN / 32) + wn * TN;
+      float* const base = (float*)g->C + partial_offset(share_of(bid_cur), band0, ct0, M, N) / 4 + lane * 4;
+      const size_t band_stride = ((size_t)N + 31) / 32 * 1024;
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+          if (!EDGE || ((band0 + i) * 32 + r32 < M && (ct0 + j) * 32 < N)) {
+#pragma unroll
+            for (int gq = 0; gq < 4; gq++)
+              *reinterpret_cast<v4f*>(base + i * band_stride + j * 1024 + gq * 256) = v4f{acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]};
+          }
+      return;
+    }
     // the resource ends with the tile's last valid element
     OutT* cbase = (OutT*)g->C;
-    if constexpr (KSPLIT) cbase += (size_t)share_of(bid_cur) * g->M * N;  // this share's matrix
     const __amdgpu_buffer_rsrc_t rC = make_rsrc(cbase + (size_t)(tile_cur & 0xffff) * kBM * N + (size_t)(tile_cur >> 16) * kBN,
                                                 (uint32_t)((rows_a - 1) * N + rows_b) * (uint32_t)sizeof(OutT));
     const int row_l = wm * (TM * 32) + r32;
@@ -771,25 +786,76 @@ int tiled_grid_size(const GemmArgs& g, int tiles, int per_cu) {
   return tiles < cus ? tiles : cus;
 }
 
-// Sum of the K split's partial matrices, in share order, with the epilogue: 4 consecutive outputs per thread.
+// Sum of a K split's partial sums (partial_offset), in share order, with the epilogue: a wave adds one 32 x 32 tile of C, all
+// loads of up to eight shares in flight at once, and stores it as the GEMM kernels do (bf16: lanes l and l + 32 trade halves,
+// 16 bytes per lane).
 template <typename T>
 __global__ __launch_bounds__(256) void ksplit_reduce_kernel(const float* __restrict__ part, int nsplit, T* __restrict__ C, int M, int N, const Epilogue ep) {
-  const size_t mn = (size_t)M * N, i4 = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
-  if (i4 >= mn) return;
-  v4f acc = *reinterpret_cast<const v4f*>(part + i4);
-  for (int s = 1; s < nsplit; s++) {
-    const v4f p = *reinterpret_cast<const v4f*>(part + s * mn + i4);
-    acc += p;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int cts = (N + 31) / 32, groups = (cts + 3) / 4;  // a workgroup's four waves take column tiles side by side
+  const int band = blockIdx.x / groups, ct = (blockIdx.x - band * groups) * 4 + wave;
+  const int h = lane >> 5, r32 = lane & 31;
+  const long m = (long)band * 32 + r32;
+  if (ct >= cts || m >= M) return;
+  const float* const p = part + partial_offset(0, band, ct, M, N) / 4 + lane * 4;
+  const size_t share_stride = partial_offset(1, 0, 0, M, N) / 4;
+  v4f acc[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) acc[q] = *reinterpret_cast<const v4f*>(p + q * 256);
+  int s = 1;
+  for (; s + 3 < nsplit; s += 4) {
+    v4f v[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) v[u][q] = *reinterpret_cast<const v4f*>(p + (s + u) * share_stride + q * 256);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) acc[q] += v[u][q];
   }
-  const long m = (long)(i4 / N), n = (long)(i4 % N);
+  if (s < nsplit) {  // up to three more
+    v4f v[3][4];
+#pragma unroll
+    for (int u = 0; u < 3; u++)
+      if (s + u < nsplit) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[u][q] = *reinterpret_cast<const v4f*>(p + (s + u) * share_stride + q * 256);
+      }
+#pragma unroll
+    for (int u = 0; u < 3; u++)
+      if (s + u < nsplit) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) acc[q] += v[u][q];
+      }
+  }
+  const long n0 = (long)ct * 32 + 4 * h;  // quad q: columns n0 + 8 q .. + 3 (N % 8 == 0: inside or outside N as a whole)
   if (epilogue_any(ep)) {
 #pragma unroll
-    for (int e = 0; e < 4; e++) acc[e] = epilogue_apply(ep, acc[e], m, n + e);
+    for (int q = 0; q < 4; q++)
+      if (n0 + 8 * q < N) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[q][e] = epilogue_apply(ep, acc[q][e], m, n0 + 8 * q + e);
+      }
   }
+  T* const c = C + (size_t)m * N;
   if constexpr (sizeof(T) == 2) {
-    *reinterpret_cast<u32x2*>(C + i4) = u32x2{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])};
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      uint32_t lo[2] = {pack_bf16x2(acc[2 * t][0], acc[2 * t][1]), pack_bf16x2(acc[2 * t][2], acc[2 * t][3])};
+      uint32_t hi[2] = {pack_bf16x2(acc[2 * t + 1][0], acc[2 * t + 1][1]), pack_bf16x2(acc[2 * t + 1][2], acc[2 * t + 1][3])};
+#pragma unroll
+      for (int k = 0; k < 2; k++) {  // lower lanes keep run 2t and get the partner's half of it, upper lanes run 2t + 1
+        const auto sw = __builtin_amdgcn_permlane32_swap(lo[k], hi[k], false, false);
+        lo[k] = sw[0], hi[k] = sw[1];
+      }
+      const long n = (long)ct * 32 + 16 * t + 8 * h;
+      if (n < N) *reinterpret_cast<u32x4*>(c + n) = u32x4{lo[0], lo[1], hi[0], hi[1]};
+    }
   } else {
-    *reinterpret_cast<v4f*>(C + i4) = acc;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      if (n0 + 8 * q < N) *reinterpret_cast<v4f*>(c + n0 + 8 * q) = acc[q];
   }
 }
 
@@ -818,8 +884,7 @@ hipError_t launch_ksplit_reduce(const GemmArgs& g, hipStream_t s) {
     else ksplit_reduce_ragged_kernel<uint16_t><<<blocks, 64, 0, s>>>(g.ks_part, g.ksplit, (uint16_t*)g.C, g.M, g.N, g.ep);
     return hipGetLastError();
   }
-  const size_t quads = (size_t)g.M * g.N / 4;
-  const unsigned blocks = (unsigned)((quads + 255) / 256);
+  const unsigned blocks = (unsigned)(((g.M + 31) / 32) * (((g.N + 31) / 32 + 3) / 4));
   if (g.f32out) ksplit_reduce_kernel<float><<<blocks, 256, 0, s>>>(g.ks_part, g.ksplit, (float*)g.C, g.M, g.N, g.ep);
   else ksplit_reduce_kernel<uint16_t><<<blocks, 256, 0, s>>>(g.ks_part, g.ksplit, (uint16_t*)g.C, g.M, g.N, g.ep);
   return hipGetLastError();

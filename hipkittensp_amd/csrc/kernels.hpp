@@ -26,7 +26,7 @@ struct GemmArgs {
   int no_alloc = 0;                // skinny kernel: the K split keeps its partial tiles in the library's static scratch array instead of an allocated workspace
   int force_split = 0;             // skinny kernel, M <= 32: split K between this many workgroups (1, 2, 4, 8); 0 = by shape
   int ksplit = 0;                  // tiled kernel: workgroups that share an output tile (from tiled_ksplit_plan, which also gives tile_rows); needs ks_part
-  float* ks_part = nullptr;        // ... their partial sums: ksplit matrices [M, N] of floats (ring kernel: partial tiles)
+  float* ks_part = nullptr;        // ... their partial sums: ksplit sets of 32 x 32 tiles (partial_offset), ragged: matrices [M, ragged_pitch(N)] of floats (ring kernel: partial tiles)
   int* ks_counters = nullptr;      // ring kernel's K split: one arrival counter per tile of C, zero between launches
 };
 
@@ -66,7 +66,7 @@ hipError_t launch_gemm_tiled4(const GemmArgs& g, hipStream_t s);
 bool gemm_block_supports(const GemmArgs& g);  // 128 x 128 tiles, four waves in step (a few hundred to a few thousand rows of A)
 bool gemm_block_ragged_supports(const GemmArgs& g);  // with GemmArgs::ragged: any M, N, K % 32 == 0 and alignment
 hipError_t launch_gemm_block(const GemmArgs& g, hipStream_t s);
-hipError_t launch_ksplit_reduce(const GemmArgs& g, hipStream_t s);  // sums g.ksplit partial matrices at g.ks_part into g.C, with the epilogue
+hipError_t launch_ksplit_reduce(const GemmArgs& g, hipStream_t s);  // sums g.ksplit shares' partial sums at g.ks_part into g.C, with the epilogue
 bool gemm_ring_supports(const GemmArgs& g);  // batched decode: private streams of B per wave, A through a flag-guarded ring (no barrier per K-tile)
 int ring_ksplit_plan(const GemmArgs& g, int want, size_t* part_bytes, size_t* counters);  // its K split for this problem (want: 0 = by shape, 1 = none, n = n shares): shares (1 = none), bytes of partial tiles, arrival counters
 hipError_t launch_gemm_ring(const GemmArgs& g, hipStream_t s);
