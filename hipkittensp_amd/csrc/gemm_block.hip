@@ -39,9 +39,16 @@ struct BlockArgs {
   Epilogue ep;  // FUSED instantiations: scales / bias / activation on the accumulators before the output rounding
 };
 
-// STAGES: ring slots, 3 (80 KB of LDS, two workgroups per CU) to 6 (152 KB, one).  Loads run STAGES K-tiles ahead of the
-// MFMAs and have STAGES - 1 steps to land; from five slots on the scales are fetched two groups ahead instead of one, so
-// that they are older than every load a step's wait leaves in flight.
+// STAGES: ring slots, 3 (80 KB of LDS, two workgroups per CU), 4 (128 x 256 tiles) or 6, which is PAIR.  Loads run STAGES K-tiles
+// ahead of the MFMAs and have STAGES - 1 steps to land.
+// PAIR: three slots of two K-tiles (a chunk) each, 152 KB, one workgroup per CU.  What it is for is a row-major operand: the 96
+// bytes that a row has in one K-tile straddle 128-byte lines, six line requests for the three lines of four K-tiles, and requests
+// are what bounds the way from L2; 192 bytes at a time are four.  A's part of a chunk is loaded in one step and B's in the next,
+// three chunks ahead, and there is one wait and one barrier per chunk.  LDS image of a row-major part: rows of 192 bytes, 16-byte
+// pieces permuted inside groups of four (piece p of row r at r * 192 + (p ^ ((r >> 2) & 3)) * 16: the 16 rows of a ds_read_b128
+// phase fall into different banks); of a tile-major one: two sets of four 3 KB tiles.  us, six slots of one K-tile / PAIR,
+// both operands row-major, B tile-major, both: 512 x 8192 x 8192 49.5 / 39.8, 42.4 / 34.6, 33.4 / 31.6; 1024 x 4096 x 14336
+// 80.2 / 65.2, 67.5 / 58.9, 52.3 / 51.3; 512 x 2048 x 2048 15.6 / 12.7, 13.6 / 11.6, 11.2 / 10.8.
 // WN: waves side by side along N, 2 (tile of 128 x 128, four waves) or 4 (128 x 256, eight waves: waves 0-3 load A's tile
 // and half of B's, six loads per K-tile, waves 4-7 the other half of B's, three loads).
 // FUSED: the epilogue applies args.ep (a separate instantiation, so that unfused calls carry none of it).
@@ -53,21 +60,23 @@ struct BlockArgs {
 //     nothing to an fp32 sum, whose last place is 2^-149 at least.  (Zeroing A's fragments instead: 24 v_and a K-tile behind
 //     the wait for the LDS reads, 3 us of 20 at 500 x 5003 x 2880, and in a branch the compiler spills them.)
 //   * a row's scales start at any byte: a lane fetches the 20 bytes of aligned dwords around its 16 (one load of 16 bytes and
-//     one of 4) and the reader shifts them into place (v_alignbyte_b32, once per four K-tiles).  Up to four slots one scale
-//     buffer serves (a group's scales are in registers before the next group's are fetched): three slots are 77 KB
+//     one of 4) and the reader shifts them into place (v_alignbyte_b32, once per four K-tiles).  With three slots one scale
+//     buffer serves (a group's scales are in registers, and a barrier passed, before the next group's are fetched): 77 KB
 //   * C's rows start at any element: 16-byte stores at element alignment, and single elements where a run of eight (bf16) or
 //     four (fp32) outputs crosses N
-// 500 x 5003 x 2880: 19.3 us against 148.5 on the one-wave-per-tile kernel, which fetches every operand row again for each of
+// 500 x 5003 x 2880: 17.0 us against 148.5 on the one-wave-per-tile kernel, which fetches every operand row again for each of
 // its 32 x 32 tiles, 4 bytes per lane.
 template <int FA, int FB, typename Out, int STAGES, int WN, bool FUSED, bool RAGGED = false>
 __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_block_kernel(const BlockArgs args) {
   typedef typename Out::type OutT;
-  static_assert(STAGES >= 3 && STAGES <= 6 && (WN == 2 || WN == 4), "ring depth, tile width");
+  static_assert((STAGES == 3 || STAGES == 4 || STAGES == 6) && (WN == 2 || WN == 4), "ring depth, tile width");
+  constexpr bool PAIR = STAGES == 6;
   static_assert(!RAGGED || (WN == 2 && FUSED), "one tile width, one epilogue");
+  static_assert(!PAIR || WN == 2, "three slots of two K-tiles");
   constexpr int NW = 2 * WN, kBN = WN * 64, kSlot = kATile + kBN * 96, kScRows = kScA + kBN * 16;
   constexpr int kScBuf = kScRows + (RAGGED ? (kBM + kBN) * 4 : 0);  // RAGGED: 4 more bytes per row behind the rows' 16
-  constexpr int kStages = STAGES, E = STAGES > 4 ? 1 : 0;  // E: extra groups of four K-tiles the scale loads run ahead
-  constexpr int kScBufs = RAGGED && !E ? 1 : 2;
+  constexpr int kStages = STAGES;
+  constexpr int kScBufs = RAGGED && !PAIR ? 1 : 2;
   constexpr int kScLoads = RAGGED ? 2 : 1;  // loads per group of scales
   constexpr int kScBase = kStages * kSlot, kLdsBytes = kScBase + kScBufs * kScBuf;
   static_assert(kLdsBytes <= (STAGES <= 3 && WN == 2 ? 81920 : 163840), "LDS budget");
@@ -127,9 +136,19 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   // per-lane global byte offsets of the direct loads: load q = 3 wave + i fills LDS bytes [q * 1024, + 1024) of an
   // operand's tile.  Row-major: 16-byte slot o holds piece (o % 6) ^ ((row >> 3) & 1) of row o / 6.  Tile-major: the
   // 3072-byte tile of 32 rows is stored in this order; wave w loads row-tile w.
-  int voff_a[3], voff_b[3];
+  // PAIR: load q = 6 wave + i of two K-tiles: slot o holds piece (o % 12) ^ ((row >> 2) & 3) of row o / 12; tile-major: K-tile
+  // q / 12's four tiles one after the other.
+  constexpr int kLoads = PAIR ? 6 : 3;
+  int voff_a[kLoads], voff_b[kLoads];
 #pragma unroll
-  for (int i = 0; i < 3; i++) {
+  for (int i = 0; i < kLoads; i++) {
+    if constexpr (PAIR) {
+      const int q = wave * 6 + i, o = q * 64 + lane, r = o / 12, c = (o - r * 12) ^ ((r >> 2) & 3);
+      const int vrow = r * rowbytes + c * 16, vtile = (q % 12 / 3) * (nkt_all * 3072) + (q / 12) * 3072 + (q % 3) * 1024 + lane * 16;
+      voff_a[i] = layout_a ? vtile : vrow;
+      voff_b[i] = layout_b ? vtile : vrow;
+      continue;
+    }
     const int q = wave * 3 + i, o = q * 64 + lane;
     const int r = o / 6, c = (o - r * 6) ^ ((r >> 3) & 1);
     const int vrow = r * rowbytes + c * 16, vtile = wave * (nkt_all * 3072) + i * 1024 + lane * 16;
@@ -145,6 +164,19 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   for (int c = 0; c < 3; c++) {
     a_rd[c] = (wm * 64 + r32) * 96 + ((3 * h + c) ^ sw) * 16;
     b_rd[c] = kATile + (wn * 64 + r32) * 96 + ((3 * h + c) ^ sw) * 16;
+  }
+  // PAIR: pieces 6 u + 3 h .. + 2 of the row's two K-tiles (u: which), and the step from a 32-row tile to the next
+  [[maybe_unused]] int a_rd2[2][3], b_rd2[2][3];
+  [[maybe_unused]] const int a_next = layout_a ? 3072 : 6144, b_next = layout_b ? 3072 : 6144;
+  if constexpr (PAIR) {
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        const int row = r32 * 192 + ((6 * u + 3 * h + c) ^ ((r32 >> 2) & 3)) * 16, tile = u * 12288 + r32 * 96 + ((3 * h + c) ^ sw) * 16;
+        a_rd2[u][c] = wm * 2 * a_next + (layout_a ? tile : row);
+        b_rd2[u][c] = 2 * kATile + wn * 2 * b_next + (layout_b ? tile : row);
+      }
   }
   const int sa_rd = kScBase + (wm * 64 + r32) * 16, sb_rd = kScBase + kScA + (wn * 64 + r32) * 16;
   const int sc_shift = 16 * h;  // a lane's two scale bytes of a K-tile: bytes 2h, 2h + 1 of the K-tile's four
@@ -177,6 +209,14 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
       if constexpr (RAGGED) voff_b[n - 3] += kstep_b;
     }
   };
+  // PAIR: load n of this wave's six of A's or B's part of chunk c (K-tiles 2c, 2c + 1).  The chunk's offset rides in the per-lane
+  // offset, which the hardware checks against the end of the resource: past the last row's last K-tile it fetches nothing.
+  [[maybe_unused]] const int nchunks = (nkt + 1) / 2;
+  auto load_pair = [&]<bool OF_A>(int c, int slot, int n) __attribute__((always_inline)) {
+    const uint32_t dst = lds0 + slot * (2 * kSlot) + (OF_A ? 0 : 2 * kATile) + (wave * 6 + n) * 1024;
+    if constexpr (OF_A) dma16(c < nchunks ? rA : rZ, dst, voff_a[PAIR ? n : 0] + c * (2 * kstep_a), 0);
+    else dma16(c < nchunks ? rB : rZ, dst, voff_b[PAIR ? n : 0] + c * (2 * kstep_b), 0);
+  };
   auto load_tile = [&]<bool LA>(int t, int slot) __attribute__((always_inline)) {
 #pragma unroll
     for (int n = 0; n < 6; n++) load_one.template operator()<LA>(t, slot, n);
@@ -203,6 +243,25 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
 #pragma unroll
       for (int c = 0; c < 3; c++) {
         const v4i p = *reinterpret_cast<const v4i*>(st + a_rd[c] + i * 3072);
+#pragma unroll
+        for (int e = 0; e < 4; e++) fa[SET][i][4 * c + e] = p[e];
+      }
+  };
+  auto read_pair = [&]<int SET, int U>(int slot) __attribute__((always_inline)) {  // PAIR: K-tile U of a chunk
+    const uint8_t* st = smem + slot * (2 * kSlot);
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        const v4i p = *reinterpret_cast<const v4i*>(st + b_rd2[U][c] + j * b_next);
+#pragma unroll
+        for (int e = 0; e < 4; e++) fb[SET][j][4 * c + e] = p[e];
+      }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        const v4i p = *reinterpret_cast<const v4i*>(st + a_rd2[U][c] + i * a_next);
 #pragma unroll
         for (int e = 0; e < 4; e++) fa[SET][i][4 * c + e] = p[e];
       }
@@ -279,14 +338,21 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
     // LDS reads of K-tile k + 1 first, then the MFMAs of K-tile k with the direct loads of K-tile k + STAGES (into K-tile
     // k's slot) between them, one after each of the first six, and after the seventh the scales of a later group of four
     // (with a group's first K-tile): the loads wait for the address unit behind an MFMA instead of in front of the LDS reads
-    read_tile.template operator()<NXT>(slot[1]);
+    // PAIR: slot[0 .. 2] hold chunks k / 2 .. + 2
+    if constexpr (PAIR) read_pair.template operator()<NXT, NXT>(slot[KM & 1]);
+    else read_tile.template operator()<NXT>(slot[1]);
     if (KM == 3) read_scales((k >> 2) + 1);
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(1);
     mma_tile.template operator()<CUR, KM>([&](int q) __attribute__((always_inline)) {
       __builtin_amdgcn_sched_barrier(0);
-      if (q < 6) load_one.template operator()<LA>(k + kStages, slot[0], q);
-      if (q == 6 && KM == 0) load_scales((k >> 2) + 1 + E);
+      if constexpr (PAIR) {  // B's part of chunk k / 2 + 2 in even steps, A's of chunk k / 2 + 3 in odd ones
+        if (q < 6 && (KM & 1) == 0) load_pair.template operator()<false>((k >> 1) + 2, slot[2], q);
+        if (q < 6 && (KM & 1) == 1) load_pair.template operator()<true>((k >> 1) + 3, slot[0], q);
+      } else {
+        if (q < 6) load_one.template operator()<LA>(k + kStages, slot[0], q);
+      }
+      if (q == 6 && KM == 0) load_scales((k >> 2) + 1);
       __builtin_amdgcn_sched_barrier(0);
     });
     __builtin_amdgcn_s_setprio(0);
@@ -297,9 +363,22 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
 #pragma unroll
     for (int j = 0; j < 2; j++) asm volatile("" : "+v"(fb[NXT][j]));
     if (KM == 3) take_scales((k >> 2) + 1);
+    if constexpr (PAIR) {
+      // Chunk c's places are free once its second K-tile is in registers (the barrier of step 2c), and chunk c + 1 must be there
+      // for step 2c + 1: one wait and barrier per chunk.  Younger than the last of chunk c + 1's loads (step 2c - 2): A's of step
+      // 2c - 1, B's of this step, six each, and this step's scales; those of step 2c - 2 must have landed (read in step 2c + 1).
+      if constexpr ((KM & 1) == 0) {
+        wait_vmcnt<12 + (KM == 0 ? kScLoads : 0)>();
+        barrier();
+      } else {
+        const int t = slot[0];
+        slot[0] = slot[1], slot[1] = slot[2], slot[2] = t;
+      }
+      return;
+    }
     // K-tile k + 2 has landed: everything older than the loads of the last STAGES - 2 steps (six each, and a scale load
     // in steps with KM == 0)
-    constexpr int kScalesInFlight = (KM % 4 == 0) + (STAGES >= 4 && (KM + 3) % 4 == 0) + (STAGES >= 5 && (KM + 2) % 4 == 0) + (STAGES >= 6 && (KM + 1) % 4 == 0);
+    constexpr int kScalesInFlight = (KM % 4 == 0) + (STAGES == 4 && (KM + 3) % 4 == 0);
     wait_vmcnt<(LA ? 6 : 3) * (STAGES - 2) + kScLoads * kScalesInFlight>();
     barrier();
     const int t = slot[0];
@@ -312,17 +391,32 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   auto run = [&]<bool LA>() __attribute__((always_inline)) {
     constexpr int NL = LA ? 6 : 3;
     load_scales(0);
-    if (E) load_scales(1);
+    if constexpr (PAIR) {  // chunks 0, 1 and A's part of chunk 2; step 0 goes on with B's
 #pragma unroll
-    for (int t = 0; t < kStages; t++) load_tile.template operator()<LA>(t, t);
-    wait_vmcnt<NL * (STAGES - 1)>();
-    barrier();
-    read_tile.template operator()<0>(0);
-    read_scales(0);
-    wait_lds_reads();
-    take_scales(0);
-    wait_vmcnt<NL * (STAGES - 2)>();
-    barrier();  // K-tile 1 is in place, and every wave has K-tile 0 in registers: its slot is free
+      for (int t = 0; t < 5; t++)
+#pragma unroll
+        for (int n = 0; n < 6; n++) {
+          if (t & 1) load_pair.template operator()<false>(t >> 1, t >> 1, n);
+          else load_pair.template operator()<true>(t >> 1, t >> 1, n);
+        }
+      wait_vmcnt<18>();
+      barrier();
+      read_pair.template operator()<0, 0>(0);
+      read_scales(0);
+      wait_lds_reads();
+      take_scales(0);
+    } else {
+#pragma unroll
+      for (int t = 0; t < kStages; t++) load_tile.template operator()<LA>(t, t);
+      wait_vmcnt<NL * (STAGES - 1)>();
+      barrier();
+      read_tile.template operator()<0>(0);
+      read_scales(0);
+      wait_lds_reads();
+      take_scales(0);
+      wait_vmcnt<NL * (STAGES - 2)>();
+      barrier();  // K-tile 1 is in place, and every wave has K-tile 0 in registers: its slot is free
+    }
     int k = 0;
     for (; k + 4 <= nkt; k += 4) {
       step.template operator()<0, LA>(k);
@@ -497,14 +591,20 @@ int cu_count_of_device() {
   return cus[dev];
 }
 
-// Ring depth: six slots (one workgroup per CU) while the tiles fill at most five eighths of the CUs -- a workgroup is alone
-// on its CU anyway, and loads that run six K-tiles ahead cover the way from HBM (256 x 8192 x 8192: 23.0 us against 24.7,
-// 1024 x 2048 x 8192: 23.5 against 25.1); three slots beyond, where two workgroups may share a CU and one's waits are the
-// other's work (256 tiles: 1024 x 4096 x 4096 18.6 against 20.0, 512 x 8192 x 2048 11.9 against 13.6, 2048 x 2048 x 8192
-// 28.8 against 31.2) -- except with K from 6144 on while a CU is left over (512 x 6144 x 16384: six slots 46.0 against
-// 51.9, 64 x 28672 x 8192: 34.9 against 38.2, 1 x 27136 x 7680: 30.5 against 34.1; at K = 5120 three: 96 x 20480 x 5120 22.5 against 23.6; between the two six with one row of tiles, 1 x 25600 x 5632 21.2 against 24.6, 32 x 20608 x 5632 19.8 against 22.6, three with more, 512 x 7552 x 5504 23.9 against 24.9), and three slots for K up to 2048, where filling six takes a good part of
-// the 8 - 16 K-tiles there are (384 x 2048 x 1024: 6.3 against 7.2, 512 x 4096 x 2048: 10.2 against 11.1, 24 shapes of 384 -
-// 1024 rows x N = 2048 .. 6144 all 7 - 14 % ahead).  stages = 3 or 6 forces one (measurement).
+// Chunks of two K-tiles (PAIR, one workgroup per CU) or three slots of one K-tile (two workgroups per CU, one's waits are the
+// other's work).  While no CU gets a second workgroup: PAIR, but for K up to 1024, where filling its slots takes a good part of
+// the eight K-tiles there are (us, three slots / PAIR: 256 x 4096 x 512 5.9 / 6.4, 256^3 4.4 / 5.0, 384 x 2048 x 1024 7.4 / 7.4 and
+// 6.7 / 7.1 tile-major; 256 x 8192 x 1536 12.1 / 11.0, 512 x 4096 x 2048 15.4 / 13.3, tile-major 11.7 / 11.5; 32 x 20608 x 5632
+// 27.6 / 23.4 and 22.2 / 18.4), and up to 2048 with both operands tile-major (512 x 8192 x 2048 12.9 / 13.3, 512 x 4096 x 4096 17.9 /
+// 16.8).  Beyond: PAIR where its fewer line requests outweigh the second workgroup, with both operands row-major from K = 4096 on
+// (2048 x 4096 x 4096 49.5 / 43.8, 1536 x 4096 x 4096 41.2 / 41.1, 640 x 8192 x 2048 23.6 / 25.1), with one from 8192 on (1024 x 8192 x 8192
+// 70.1 / 64.9, 256 x 28672 x 8192 81.0 / 73.0, 2048 x 4096 x 4096 39.2 / 40.3), with none never (31.5 / 36.4).
+// stages = 3 or 6 forces one (measurement).
+int block_stages(const GemmArgs& g, int grid, int cus) {
+  const int row_major = !g.layout_a + !g.layout_b;
+  const int min_k = grid <= cus ? (row_major ? 1025 : 2049) : row_major == 2 ? 4096 : row_major == 1 ? 8192 : 0x7fffffff;
+  return g.K >= min_k ? 6 : 3;
+}
 template <int FA, int FB, bool FUSED>
 hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, hipStream_t s) {
   const int cus = cu_count_of_device();
@@ -515,7 +615,7 @@ hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, 
     else gemm_block_kernel<FA, FB, OutBf16, 4, 4, FUSED><<<grid, 512, 0, s>>>(a);
     return hipGetLastError();
   }
-  if (stages == 0) stages = ((long)grid * 8 <= (long)cus * 5 && g.K > 2048) || ((g.K >= 6144 || (g.K > 5120 && a.tiles_m == 1) || a.nsplit > 1) && grid < cus) ? 6 : 3;
+  if (stages == 0) stages = block_stages(g, grid, cus);
   if (stages == 6) {
     if (f32) gemm_block_kernel<FA, FB, OutF32, 6, 2, FUSED><<<grid, 256, 0, s>>>(a);
     else gemm_block_kernel<FA, FB, OutBf16, 6, 2, FUSED><<<grid, 256, 0, s>>>(a);
@@ -525,11 +625,13 @@ hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, 
   }
   return hipGetLastError();
 }
-// RAGGED instantiations: three or six slots by the same rule, the fused epilogue applied or not inside
+// RAGGED instantiations, the fused epilogue applied or not inside.  PAIR from K = 1920 on while no CU gets a second workgroup (us,
+// three slots / PAIR: 64 x 3001 x 1888 11.1 / 11.1, 500 x 5003 x 1056 13.2 / 13.6, 100 x 5003 x 2016 17.8 / 16.1), from 6144 on
+// beyond (2000 x 8191 x 4128 107.5 / 105.0, 1000 x 4097 x 4128 47.3 / 48.6, 572 x 22563 x 13760 295 / 266).
 template <int FA, int FB>
 hipError_t launch_ragged(const GemmArgs& g, const BlockArgs& a, int tiles, hipStream_t s) {
   const int grid = tiles * a.nsplit, cus = cu_count_of_device();
-  const bool deep = grid <= cus && g.K > 2048;
+  const bool deep = g.K >= (grid <= cus ? 1920 : 6144);
   if (g.f32out || a.nsplit > 1) {
     if (deep) gemm_block_kernel<FA, FB, OutF32, 6, 2, true, true><<<grid, 256, 0, s>>>(a);
     else gemm_block_kernel<FA, FB, OutF32, 3, 2, true, true><<<grid, 256, 0, s>>>(a);

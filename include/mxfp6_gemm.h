@@ -136,7 +136,7 @@ int mxfp6_gemm_f32out(const void *A_packed, const void *B_packed, const void *A_
  *   22  block kernel: output tiles of 128 x 128, four waves in step with the operand fragments double-buffered in
  *       registers, one barrier per K-tile (needs N % 8 == 0, K % 128 == 0); typically chosen for a few hundred to a few
  *       thousand rows of A;
- *       23 / 24: with an operand ring of three slots (two workgroups per CU) / six slots (one); 26: with tiles of
+ *       23 / 24: with an operand ring of three K-tiles (two workgroups per CU) / three pairs of K-tiles (one); 26: with tiles of
  *       128 x 256 and eight waves.  22 - 24 split K between workgroups by the thread's mxfp6_set_k_split setting
  *       (0: where the library's time model prefers the split; the same per-stream workspace as the tiled kernel's split)
  * No counterpart in the reference, whose shapes are compile-time constants per binary
