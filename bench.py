@@ -536,7 +536,7 @@ def dispatch_sweep(hk, torch, grid):
 
 def calibration_sweep(hk, torch):
     """The sweep behind the kernel choice's calibration table (hipkittensp_amd/csrc/dispatch_table.inc): every candidate of the
-    choice, forced, on a grid of shapes x three layout pairs, timed on the GPU's side with weights rotating through 400 MB
+    choice, forced, on a grid of shapes x four layout pairs, timed on the GPU's side with weights rotating through 400 MB
     (probe_time_us), twice (the better counts).  `python -m hipkittensp_amd.calibrate` turns the JSON this prints into the
     table: per shape and candidate, measured time / the time model's figure."""
     import ctypes
@@ -555,13 +555,14 @@ def calibration_sweep(hk, torch):
     g = torch.Generator(device="cuda")
     g.manual_seed(1)
     for N, K in shapes:
+        print(f"N = {N}, K = {K}", file=sys.stderr, flush=True)
         sets, row, tile = weight_sets(hk, torch, N, K, g)
         for M in rows_of_a:
             if M * N > 1 << 28:
                 continue
             a, asc = hk.quantize(torch.randn(M, K, device="cuda", generator=g), 2)
             C = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
-            for la, lb in ((0, 0), (0, 1), (1, 1)):
+            for la, lb in ((0, 0), (1, 0), (0, 1), (1, 1)):
                 if la and (M % 32 or K % 128):
                     continue
                 at, ast = (hk.tile_operand(a), hk.tile_scales(asc, K)) if la else (a, asc)
