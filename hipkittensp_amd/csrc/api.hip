@@ -426,6 +426,16 @@ int mxfp6_linear(const void* X, int x_bf16, const void* W, const void* Ws, void*
   rc = check_device();
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
+  // Up to four rows of bf16 the skinny kernel quantises itself where it is the choice: one launch instead of two, nothing in the workspace
+  if (x_bf16 && K > 0 && g_force == 0) {
+    mxfp6::GemmArgs g{(const uint8_t*)X, (const uint8_t*)W, (const uint8_t*)X, (const uint8_t*)Ws, C, M, N, K, fmt_x, fmt_w, false, 0, layout_w};
+    g.X = X;
+    if (mxfp6::gemm_skinny_takes_x(g) && auto_choice(g, 0, true).cand == mxfp6::kCandSkinny) {
+      g.ep = ep;
+      const hipError_t e = mxfp6::launch_gemm_skinny(g, s);
+      return e == hipSuccess ? MXFP6_OK : (int)e;
+    }
+  }
   // Tile-major from 64 rows on, whatever M is (the workspace has whole 32-row tiles; what stands in the rows past M reaches
   // nothing but outputs that are not stored): whole cache lines for every load of the GEMM.  Fewer rows stay row-major for the
   // skinny kernel.

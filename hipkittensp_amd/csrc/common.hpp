@@ -32,6 +32,31 @@ __device__ __forceinline__ int e8m0_of_amax(float amax, int emax) {
   return sb < 0 ? 0 : (sb > 254 ? 254 : sb);
 }
 
+// A 32-block of bf16 (64 bytes) quantised to FMT: six dwords and its E8M0 byte.  The instruction divides by the power of two and
+// rounds (nearest even, saturating).
+typedef uint32_t u32x6 __attribute__((ext_vector_type(6)));
+template <int FMT>
+__device__ __forceinline__ u32x6 quantise_block_bf16(const v4i (&x)[4], int& sb) {
+  float amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      amax = fmaxf(amax, fabsf(__int_as_float(x[i][j] << 16)));
+      amax = fmaxf(amax, fabsf(__int_as_float(x[i][j] & (int)0xffff0000)));
+    }
+  sb = e8m0_of_amax(amax, FMT == 2 ? 2 : 4);
+  const float scale = __uint_as_float((uint32_t)sb << 23);  // 2^(sb - 127); the instruction uses the exponent field
+  typedef __bf16 v32bf __attribute__((ext_vector_type(32)));
+  typedef int v16i __attribute__((ext_vector_type(16)));
+  v16i raw;
+#pragma unroll
+  for (int i = 0; i < 16; i++) raw[i] = x[i / 4][i & 3];
+  const v32bf xb = __builtin_bit_cast(v32bf, raw);
+  if constexpr (FMT == 2) return __builtin_amdgcn_cvt_scalef32_pk32_fp6_bf16(xb, scale);
+  else return __builtin_amdgcn_cvt_scalef32_pk32_bf6_bf16(xb, scale);
+}
+
 // fp32 -> bf16, round to nearest even (v_cvt_pk_bf16_f32 on gfx950).
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   typedef __bf16 bf2 __attribute__((ext_vector_type(2)));

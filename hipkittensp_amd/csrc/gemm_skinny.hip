@@ -46,7 +46,13 @@ namespace mxfp6 {
 // BR = rows of B per workgroup (32; 16 so that a narrow N still gives every CU a workgroup: the MFMA's other 16
 // rows then mirror the first and their outputs are dropped; 64 = two 32-row tiles of B against every fragment of A,
 // which halves the bytes of A a workgroup pulls from L2 per byte of B)
-template <int FA, int FB, typename Out, int AR, int NW, int BR, int DB>
+// XQ: A is bf16 activations of up to kXqRows rows, which every wave quantises for itself: a chunk's 1 KB per row comes into LDS in
+// front of the chunk's B, and while B is on its way every lane quantises one 32-block of it into the A image (AR is 16, of which
+// kXqRows rows are staged; the accumulator tile's other rows mirror them and are never stored).  What it saves is a launch: for one
+// token the quantiser's 2.2 us and the gap behind it, of 10 us in all; every workgroup reads the activations anew, 1 KB per row
+// against the 6 or 12 KB of B a wave reads per chunk.
+constexpr int kXqRows = 4;
+template <int FA, int FB, typename Out, int AR, int NW, int BR, int DB, bool XQ = false>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                                                               const uint8_t* __restrict__ As, const uint8_t* __restrict__ Bs,
                                                               typename Out::type* __restrict__ C, int M, int N, int K, int layout_b,
@@ -61,12 +67,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
   // a wave's buffer: DB chunks of B (DB = 2: the chunk after the next is on its way from HBM while the next one's A, which
   // comes from L2 in a fraction of that time, is fetched one chunk ahead), one chunk of A, then the scales:
   static_assert(DB == 1 || DB == 2, "chunks of B per wave");
-  constexpr int kBBuf = BR * kRow, kABuf = AR * kRow, kAOff = DB * kBBuf, kScOff = kAOff + kABuf;
+  static_assert(!XQ || (AR == 16 && DB == 1), "quantised activations: one tile of A, one chunk of B");
+  constexpr int kBBuf = BR * kRow, kABuf = (XQ ? kXqRows : AR) * kRow, kAOff = DB * kBBuf, kScOff = kAOff + kABuf;
   constexpr int kASc = AR <= 64 ? 1024 : AR * 16;                              // 1 KB per chunk of B, 16 bytes per row of A
   constexpr int kAScOff = kScOff + DB * 1024;
-  constexpr int kBuf = kAScOff + kASc;
+  constexpr int kXOff = kAScOff + (XQ ? 64 : kASc);  // XQ: kXqRows rows x 16 scale bytes, then the chunk's activations
+  constexpr int kBuf = XQ ? kXOff + kXqRows * 1024 : kAScOff + kASc;
   constexpr int NBL = kBBuf / 1024, NAL = kABuf / 1024, NAS = kASc / 1024;  // direct loads per chunk: 12 or 6; 6, 12 or 24; 1 or 2
-  static_assert(kBBuf % 1024 == 0 && kABuf % 1024 == 0, "whole direct loads");
+  static_assert(kBBuf % 1024 == 0 && (XQ || kABuf % 1024 == 0), "whole direct loads");
   __shared__ __attribute__((aligned(1024))) uint8_t smem[NW * kBuf];
   static_assert(NW * kBuf <= 163840 && NW * kBuf >= NW * TT * 16 * 64 * 4 + 64, "LDS budget (the buffers double as the reduction buffer)");
 
@@ -86,7 +94,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
   // rows that do not exist (n >= N, m >= M) lie past the end of the resource and read as zeros
   const __amdgpu_buffer_rsrc_t rB = layout_b ? make_rsrc(B + (size_t)rt * 32 * rowbytes, (uint32_t)nrt * 32 * rowbytes)
                                              : make_rsrc(B + (size_t)n0 * rowbytes, (uint32_t)nrows * rowbytes);
-  const __amdgpu_buffer_rsrc_t rA = make_rsrc(A, (uint32_t)M * rowbytes);
+  const __amdgpu_buffer_rsrc_t rA = make_rsrc(A, XQ ? (uint32_t)M * K * 2 : (uint32_t)M * rowbytes);
   // tile-major B: this workgroup's 32 rows are one row-tile, whose scales are nk4 chunks of 512 bytes (row r at r * 16)
   const int nk4 = nkt / 4;
   const __amdgpu_buffer_rsrc_t rBs = layout_b ? make_rsrc(Bs + (size_t)rt * nk4 * 512, (uint32_t)nrt * nk4 * 512)
@@ -114,7 +122,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
   }
   // scale loads: lane l fetches the 16 bytes (four K-tiles) of row l % 32 (both halves of the wave fetch the same rows;
   // 64 or more rows of A: of row l, l + 64; 64 rows of B: of row l)
-  const int ra = AR == 16 ? (r32 & 15) : r32;  // AR = 16: lanes 16-31 mirror rows 0-15 (their outputs are never stored)
+  const int ra = XQ ? r32 & (kXqRows - 1) : AR == 16 ? (r32 & 15) : r32;  // AR = 16: lanes 16-31 mirror rows 0-15 (their outputs are never stored)
   const int rb = BR == 16 ? (r32 & 15) : r32;  // BR = 16: likewise for B
   const int voff_bs = BR == 64 ? (layout_b ? h * (nk4 * 512) + r32 * 16 : lane * sbytes) : layout_b ? (half * 16 + rb) * 16 : rb * sbytes;
   const int voff_as = (AR >= 64 ? lane : r32) * sbytes;
@@ -153,6 +161,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
     }
   };
   auto issue_a = [&](int chunk) __attribute__((always_inline)) {
+    if constexpr (XQ) {  // lane l fetches piece (l % 4) ^ (l / 4 % 4) of block l / 4: a ds_read_b128 of every lane's block is spread over the banks
+      const int so = __builtin_amdgcn_readfirstlane(chunk * 1024), piece = (lane & ~3) | ((lane ^ (lane >> 2)) & 3);
+#pragma unroll
+      for (int m = 0; m < kXqRows; m++) dma16(rA, buf + kXOff + m * 1024, m * K * 2 + piece * 16, so);  // rows past M read as zeros
+      return;
+    }
     const int sg = KT == 4 ? chunk : chunk >> 1;
     const int sos = __builtin_amdgcn_readfirstlane(sg * 16);
 #pragma unroll
@@ -160,6 +174,24 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
     const int so = __builtin_amdgcn_readfirstlane(chunk * kRow);
 #pragma unroll
     for (int i = 0; i < NAL; i++) dma16(rA, buf + kAOff + i * 1024, voff_a[i], so);
+  };
+
+  // XQ: lane l quantises block l % 16 of row l / 16 of the chunk
+  [[maybe_unused]] auto quantise_a = [&]() __attribute__((always_inline)) {
+    const int m = lane >> 4, b = lane & 15;
+    uint8_t* const own = smem + wave * kBuf;
+    v4i x[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) x[c] = *reinterpret_cast<const v4i*>(own + kXOff + m * 1024 + b * 64 + ((c ^ b) & 3) * 16);
+    int sb;
+    const u32x6 w = quantise_block_bf16<FA>(x, sb);
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const int byte = b * 24 + 8 * i;
+      *reinterpret_cast<u32x2*>(own + kAOff + m * kRow + swz(byte >> 4, m) * 16 + (byte & 15)) = u32x2{w[2 * i], w[2 * i + 1]};
+    }
+    own[kAScOff + m * 16 + b] = (uint8_t)sb;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   };
 
   v16f acc[TT];
@@ -171,10 +203,16 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
   if (mine > 0) {
     // queue order: B(0), A(0), B(1), A(1), B(2), ...: with DB = 2 chunk j is read once everything up to A(j) has landed,
     // while B(j+1), the youngest batch, stays in flight
+    // (XQ: A(j) before B(j), so that A can be quantised while B is in flight)
+    if (XQ) issue_a(c0 + wave);
     issue_b(c0 + wave, 0);
-    issue_a(c0 + wave);
+    if (!XQ) issue_a(c0 + wave);
     if (DB == 2 && mine > 1) issue_b(c0 + wave + NW, 1);
     for (int j = 0; j < mine; j++) {
+      if constexpr (XQ) {
+        wait_vmcnt<NBL + 1>();
+        quantise_a();
+      }
       if (DB == 2 && j + 1 < mine) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NBL + 1) : "memory");
       else wait_vmcnt<0>();
       const int par = DB == 2 ? j & 1 : 0;
@@ -202,8 +240,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
         if (j + 1 < mine) issue_a(c0 + wave + (j + 1) * NW);
         if (j + 2 < mine) issue_b(c0 + wave + (j + 2) * NW, par);
       } else if (j + 1 < mine) {
+        if (XQ) issue_a(c0 + wave + (j + 1) * NW);
         issue_b(c0 + wave + (j + 1) * NW, 0);
-        issue_a(c0 + wave + (j + 1) * NW);
+        if (!XQ) issue_a(c0 + wave + (j + 1) * NW);
       }
 #pragma unroll
       for (int u = 0; u < KT; u++)
@@ -282,6 +321,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
 bool gemm_skinny_supports(const GemmArgs& g) {
   // K % 512: chunks of four K-tiles are whole (three 128-byte lines per row, 16 scale bytes per row)
   return g.layout_a == 0 && g.M >= 1 && g.M <= 128 && g.N >= 1 && g.K >= 512 && g.K % 512 == 0 && (long)128 * (g.K / 4 * 3) < (1L << 31) && operands_aligned16(g);
+}
+
+bool gemm_skinny_takes_x(const GemmArgs& g) {
+  return g.M >= 1 && g.M <= kXqRows && g.K >= 512 && g.K % 512 == 0 && ((uintptr_t)g.X & 15) == 0 && !g.no_alloc && !g.f32out;
 }
 
 // Workspace of the K split: 4 KB of partial tile per (tile, split) and a counter per tile that is zero between
@@ -467,6 +510,17 @@ static hipError_t launch(const GemmArgs& g, hipStream_t s) {
 #define MXFP6_SKD(AR, NW, BR, DB) \
   gemm_skinny_kernel<FA, FB, Out, AR, NW, BR, DB><<<(g.N + BR - 1) / BR * nsplit, NW * 64, 0, s>>>( \
       g.A, g.B, g.As, g.Bs, (T*)g.C, g.M, g.N, g.K, g.layout_b, g.ep, nsplit, ws.part, ws.cnt, (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes)
+  if (g.X) {
+    if constexpr (sizeof(T) == 2) {
+#define MXFP6_SKX(NW, BR)                                                                                                       \
+  gemm_skinny_kernel<FA, FB, Out, 16, NW, BR, 1, true><<<(g.N + BR - 1) / BR * nsplit, NW * 64, 0, s>>>(                          \
+      (const uint8_t*)g.X, g.B, nullptr, g.Bs, (T*)g.C, g.M, g.N, g.K, g.layout_b, g.ep, nsplit, ws.part, ws.cnt, (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes)
+      if (geo == 2) MXFP6_SKX(8, 16); else if (geo == 3) MXFP6_SKX(4, 32); else if (geo == 5) MXFP6_SKX(2, 32); else MXFP6_SKX(8, 32);
+#undef MXFP6_SKX
+      return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
+  }
   // two chunks of B per wave (17 - 32 and 65 - 128 rows of A: measured 3 - 15 % and 3 - 6 %); forced geometry 1: one
   const bool db = g.skinny_geometry != 1;
   if (geo == 6) {

@@ -19,6 +19,7 @@ struct GemmArgs {
   Epilogue ep;                     // fused bias / scales / activation (all optional)
   uint8_t* C_scale = nullptr;      // fp6 output (tiled kernel): C is the packed operand [M, 3N/4], this its E8M0 bytes [M, N/32]
   int fmt_c = 0;                   // 2 / 3: format of the fp6 output; 0: bf16 / fp32 output
+  const void* X = nullptr;         // skinny kernel: bf16 activations [M, K] that it quantises to fmt_a itself, in place of A and As (gemm_skinny_takes_x)
   int raster_group_m = 0, raster_no_xcd_remap = 0;  // tiled kernel, measurement only: tile rows per raster group (0 = the default, 4), XCD remap off (1), or on with a K split's workgroups in tile-by-tile order (2)
   int ablation = 0;  // tiled kernel, measurement only: leave out LDS reads (1), loads (2), MFMAs (4); results are then meaningless
   uint32_t* clock_stamps = nullptr;  // tiled kernel, measurement only: four words for workgroup 0's clock / real-time counters at start and end
@@ -73,6 +74,7 @@ hipError_t launch_gemm_ring(const GemmArgs& g, hipStream_t s);
 bool gemm_mid_supports(const GemmArgs& g);
 hipError_t launch_gemm_mid(const GemmArgs& g, hipStream_t s);
 bool gemm_skinny_supports(const GemmArgs& g);
+bool gemm_skinny_takes_x(const GemmArgs& g);  // M and K of a call whose activations the kernel can quantise itself
 hipError_t launch_gemm_skinny(const GemmArgs& g, hipStream_t s);
 bool gemm_skinny_scratch_fits(const GemmArgs& g);  // no_alloc: the K split this call would use fits the static scratch array
 hipError_t release_split_workspaces();             // returns every K-split workspace to the stream-ordered allocator

@@ -33,7 +33,6 @@ constexpr int kQWaves = 4;  // waves per workgroup; a wave fetches 64 blocks at 
 template <int FMT, typename In>
 __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __restrict__ X, uint8_t* __restrict__ packed,
                                                               uint8_t* __restrict__ scales, long nblocks, int nkb, int layout, int rows, int stream_in, int stream_out) {
-  constexpr int EMAX = FMT == 2 ? 2 : 4;
   constexpr int BB = 32 * (int)sizeof(In), P = BB / 16;  // bytes and 16-byte pieces of a block
   constexpr int kChunk = 64 * BB, NLD = kChunk / 1024;   // bytes and direct loads of a chunk
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kQWaves * kChunk];
@@ -83,44 +82,23 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
     for (int c = 0; c < P; c++) x[c] = *reinterpret_cast<const v4i*>(smem + wave * kChunk + lane * BB + ((c ^ (lane % P)) * 16));
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
-    float amax = 0.f;
-#pragma unroll
-    for (int i = 0; i < P; i++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        if constexpr (sizeof(In) == 4) {
-          amax = fmaxf(amax, fabsf(__int_as_float(x[i][j])));
-        } else {
-          amax = fmaxf(amax, fabsf(__int_as_float(x[i][j] << 16)));
-          amax = fmaxf(amax, fabsf(__int_as_float(x[i][j] & (int)0xffff0000)));
-        }
-      }
-    int sb = 0;
-    if (amax > 0.f) {
-      const uint32_t u = __float_as_uint(amax);
-      const int be = (int)(u >> 23);
-      const int fl = be ? be - 127 : (31 - __clz((int)u)) - 149;  // floor(log2(amax)), fp32 subnormals included
-      sb = fl - EMAX + 127;
-      sb = sb < 0 ? 0 : (sb > 254 ? 254 : sb);
-    }
-    const float scale = __uint_as_float((uint32_t)sb << 23);  // 2^(sb - 127); the instruction uses the exponent field
-    typedef unsigned v6u __attribute__((ext_vector_type(6)));
-    v6u w;
+    int sb;
+    u32x6 w;
     if constexpr (sizeof(In) == 4) {
+      float amax = 0.f;
+#pragma unroll
+      for (int i = 0; i < P; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) amax = fmaxf(amax, fabsf(__int_as_float(x[i][j])));
+      sb = e8m0_of_amax(amax, FMT == 2 ? 2 : 4);
+      const float scale = __uint_as_float((uint32_t)sb << 23);  // 2^(sb - 127); the instruction uses the exponent field
       v16f ev, od;
 #pragma unroll
       for (int i = 0; i < 16; i++) ev[i] = __int_as_float(x[i / 2][(2 * i) & 3]), od[i] = __int_as_float(x[i / 2][(2 * i + 1) & 3]);
       if constexpr (FMT == 2) w = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ev, od, scale);
       else w = __builtin_amdgcn_cvt_scalef32_2xpk16_bf6_f32(ev, od, scale);
     } else {
-      typedef __bf16 v32bf __attribute__((ext_vector_type(32)));
-      typedef int v16i __attribute__((ext_vector_type(16)));
-      v16i raw;
-#pragma unroll
-      for (int i = 0; i < 16; i++) raw[i] = x[i / 4][i & 3];
-      const v32bf xb = __builtin_bit_cast(v32bf, raw);
-      if constexpr (FMT == 2) w = __builtin_amdgcn_cvt_scalef32_pk32_fp6_bf16(xb, scale);
-      else w = __builtin_amdgcn_cvt_scalef32_pk32_bf6_bf16(xb, scale);
+      w = quantise_block_bf16<FMT>(x, sb);
     }
     // the chunk's 1536 output bytes in order, in the buffer its input has left
     uint8_t* const image = smem + wave * kChunk;

@@ -88,3 +88,28 @@ def test_tile_major_scales_are_padded_with_zeros(hk, rows, K, dtype):
     assert fn(x.data_ptr(), p.data_ptr(), s.data_ptr(), rows, K, 2, 1, torch.cuda.current_stream().cuda_stream) == 0
     pr, sr = hk.quantize(x, 2)
     assert torch.equal(s, hk.tile_scales(sr, K)) and torch.equal(p, hk.tile_operand(pr))
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("N,K", [(40, 512), (4096, 4096), (1000, 1536), (512, 16384), (5000, 1024), (8200, 1024), (16384, 512), (33000, 512)])
+@pytest.mark.parametrize("fmt_x,fmt_w", [(2, 2), (3, 2), (2, 3)])
+def test_few_rows_quantised_inside_the_gemm(hk, M, N, K, fmt_x, fmt_w):
+    """bf16 activations of up to four rows, which the decode kernel quantises itself: the bits of quantise, then GEMM, for every
+    workgroup shape it has (few and many rows of weights, K split between workgroups), for blocks of zeros, for subnormal
+    and very large values and for NaN (each block's own)."""
+    from hipkittensp_amd.torch_op import MXFP6Linear
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    layer = MXFP6Linear(torch.randn(N, K, device="cuda", generator=g) * 0.02, fmt_w=fmt_w, fmt_x=fmt_x, bias=torch.randn(N, device="cuda", generator=g), activation="silu")
+    guard = torch.randn(M * K + 4096, device="cuda", generator=g).to(torch.bfloat16)
+    guard[M * K:] = float("nan")
+    x = guard[:M * K].view(M, K)
+    assert torch.equal(layer(x), steps(hk, layer, x))
+    x[0, 32:64] = 0
+    x[M - 1, 64:96] *= 1e-39
+    x[M - 1, K - 32:] *= 1e30
+    y, want = layer(x), steps(hk, layer, x)
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+    x[0, 5] = float("nan")
+    y, want = layer(x), steps(hk, layer, x)
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
