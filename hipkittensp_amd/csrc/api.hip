@@ -470,8 +470,7 @@ int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const voi
   // small there) the product goes to an fp32 workspace of the stream-ordered allocator and through the quantiser
   mxfp6::GemmArgs g{(const uint8_t*)A, (const uint8_t*)B, (const uint8_t*)As, (const uint8_t*)Bs, C_packed, M, N, K, fmt_a, fmt_b, false, layout_a, layout_b};
   const int force = g_force;
-  // the tiled kernel's own fp6 epilogue only where the automatic choice is that kernel (unsplit); any other choice runs as
-  // it would for an fp32 output, into the workspace, and the quantiser follows
+  // the tiled kernel's own fp6 epilogue only where the automatic choice is that kernel (unsplit)
   const bool tiled = K > 0 && mxfp6::gemm_tiled_supports(g) &&
                      (force == 2 || force == 5 || force == 6 || force == 17 || (force == 0 && choice_code(auto_choice(g, 0, true)) == kChoiceTiled));
   if (tiled) {
@@ -483,6 +482,22 @@ int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const voi
     return e == hipSuccess ? MXFP6_OK : (int)e;
   }
   std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
+  // So do the block kernel and the reduction of a K split (us, through the fp32 workspace / here: 256 x 2560 x 2304
+  // 16.7 / 13.0, 500 x 8192 x 8192 38.3 / 30.6, 2048 x 4096 x 4096 41.4 / 32.0, 3000 x 2048 x 1024 24.9 / 11.6).  Skinny, ring, ragged and generic products, and a split without its workspace, go through the workspace.
+  if (K > 0 && (force == 0 || (force >= 22 && force <= 24) || force == 26)) {
+    mxfp6::GemmArgs t = g;
+    t.C = nullptr, t.f32out = true;  // the kernel of the same call with fp32 output, whose bits these are (fp6 itself is stored 8 bytes at a time)
+    const mxfp6::KernelChoice c = force == 0    ? auto_choice(t, 0, true)
+                                  : force == 26 ? mxfp6::choose_kernel(t, 1, false, 1u << mxfp6::kCandBlockWide)
+                                                : family_choice(t, 1u << mxfp6::kCandBlock, 1u << mxfp6::kCandBlockSplit);
+    const bool block = c.cand == mxfp6::kCandBlock || c.cand == mxfp6::kCandBlockWide || c.cand == mxfp6::kCandBlockSplit;
+    if ((block || c.cand == mxfp6::kCandTiledSplit256 || c.cand == mxfp6::kCandTiledSplit128) && apply_choice(t, c, s)) {
+      t.C = C_packed, t.f32out = false, t.ep = ep, t.C_scale = (uint8_t*)C_scale, t.fmt_c = fmt_c;
+      if (force) t.tile_rows = force == 23 ? 3 : force == 24 ? 6 : 0;
+      const hipError_t e = block ? mxfp6::launch_gemm_block(t, s) : mxfp6::launch_gemm_tiled(t, s);
+      return e == hipSuccess ? MXFP6_OK : (int)e;
+    }
+  }
   float* tmp = reinterpret_cast<float*>(stream_workspace(s, 1, (size_t)M * N * 4));
   if (!tmp) return stream_is_capturing(s) ? (int)hipErrorStreamCaptureUnsupported : MXFP6_EWORKSPACE;
   rc = gemm_common(A, B, As, Bs, tmp, M, N, K, fmt_a, fmt_b, true, layout_a, layout_b, stream, ep);

@@ -20,7 +20,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // unrounded accumulators, used to state the accuracy contract before the bf16 rounding).
 struct OutBf16 { typedef uint16_t type; };
 struct OutF32 { typedef float type; };
-struct OutFp6 { typedef uint8_t type; };  // C re-quantised to MXFP6: packed [M, 3N/4] + E8M0 [M, N/32] (tiled kernel only)
+struct OutFp6 { typedef uint8_t type; };  // C re-quantised to MXFP6: packed [M, 3N/4] + E8M0 [M, N/32] (tiled and block kernels, reduction of a K split)
 
 // E8M0 byte of a 32-block with largest magnitude amax (floor(log2(amax)) - emax, clamped; 0 for an all-zero block)
 __device__ __forceinline__ int e8m0_of_amax(float amax, int emax) {
@@ -55,6 +55,56 @@ __device__ __forceinline__ u32x6 quantise_block_bf16(const v4i (&x)[4], int& sb)
   const v32bf xb = __builtin_bit_cast(v32bf, raw);
   if constexpr (FMT == 2) return __builtin_amdgcn_cvt_scalef32_pk32_fp6_bf16(xb, scale);
   else return __builtin_amdgcn_cvt_scalef32_pk32_bf6_bf16(xb, scale);
+}
+
+// The same for a 32-block of fp32 as two lanes of an MFMA tile hold it: column 8 (k / 4) + k % 4 of the block in p0[k], that + 4 in
+// p1[k].  fmt (2 or 3) is uniform.
+__device__ __forceinline__ u32x6 quantise_block_acc(const float (&p0)[16], const float (&p1)[16], int fmt, int& sb) {
+  float amax = 0.f;
+#pragma unroll
+  for (int k = 0; k < 16; k++) amax = fmaxf(amax, fmaxf(fabsf(p0[k]), fabsf(p1[k])));
+  sb = e8m0_of_amax(amax, fmt == 2 ? 2 : 4);
+  const float scale = __uint_as_float((uint32_t)sb << 23);
+  v16f ev, od;  // even and odd columns: column n = 8 q + r is p0[4 q + r] for r < 4, p1[4 q + r - 4] otherwise
+#pragma unroll
+  for (int t = 0; t < 16; t++) {
+    const int ne = 2 * t, no = 2 * t + 1;
+    ev[t] = (ne & 4) ? p1[4 * (ne >> 3) + (ne & 3)] : p0[4 * (ne >> 3) + (ne & 3)];
+    od[t] = (no & 4) ? p1[4 * (no >> 3) + (no & 3)] : p0[4 * (no >> 3) + (no & 3)];
+  }
+  // a real branch (the empty asm keeps it one): with both conversions issued on the same sources and a select
+  // behind them, the second one's result came out wrong from the third dword on
+  u32x6 w;
+  if (fmt == 2) {
+    w = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ev, od, scale);
+    asm volatile("" : "+v"(w));
+  } else {
+    w = __builtin_amdgcn_cvt_scalef32_2xpk16_bf6_f32(ev, od, scale);
+    asm volatile("" : "+v"(w));
+  }
+  return w;
+}
+
+// Two 32 x 32 accumulator tiles side by side (a band of 32 rows), re-quantised along N and stored as blocks blk0 and blk0 + 1 of
+// row m of an fp6 operand with nkb blocks a row.  A 32-block of row m is the 16 values of lane (m, h = 0) and the 16 of lane
+// (m, h = 1) of one tile.  The two tiles are traded with v_permlane32_swap, register by register, after which the lower lane holds
+// all of the first block and the upper lane all of the second: then exactly the quantiser, 24 bytes and a scale byte per lane.
+__device__ __forceinline__ void store_fp6_band(const v16f& c0, const v16f& c1, int fmt, uint8_t* packed, uint8_t* scales, long m, int M, int blk0, int nkb) {
+  float p0[16], p1[16];
+#pragma unroll
+  for (int k = 0; k < 16; k++) {
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(c0[k]), __float_as_uint(c1[k]), false, false);
+    p0[k] = __uint_as_float(sw[0]), p1[k] = __uint_as_float(sw[1]);
+  }
+  int sb;
+  const u32x6 w = quantise_block_acc(p0, p1, fmt, sb);
+  const int blk = blk0 + ((threadIdx.x >> 5) & 1);
+  if (m < M && blk < nkb) {
+    u32x2* dst = reinterpret_cast<u32x2*>(packed + (m * nkb + blk) * 24);
+#pragma unroll
+    for (int c = 0; c < 3; c++) dst[c] = u32x2{w[2 * c], w[2 * c + 1]};
+    scales[m * nkb + blk] = (uint8_t)sb;
+  }
 }
 
 // fp32 -> bf16, round to nearest even (v_cvt_pk_bf16_f32 on gfx950).

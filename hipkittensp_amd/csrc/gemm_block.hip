@@ -37,6 +37,8 @@ struct BlockArgs {
   int M, N, K, tiles_m, tiles_n, layout_a, layout_b, group_m, xcd_remap;
   int nsplit;  // workgroups that share an output tile, each over the same number of whole groups of four K-tiles (the last one over what is left); 1 = no split
   Epilogue ep;  // FUSED instantiations: scales / bias / activation on the accumulators before the output rounding
+  uint8_t* C_scale;  // fp6 output only
+  int fmt_c;
 };
 
 // STAGES: ring slots, 3 (80 KB of LDS, two workgroups per CU), 4 (128 x 256 tiles) or 6, which is PAIR.  Loads run STAGES K-tiles
@@ -73,6 +75,7 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   constexpr bool PAIR = STAGES == 6;
   static_assert(!RAGGED || (WN == 2 && FUSED), "one tile width, one epilogue");
   static_assert(!PAIR || WN == 2, "three slots of two K-tiles");
+  static_assert(sizeof(OutT) != 1 || (FUSED && !RAGGED), "fp6 output: one epilogue, whole 32-blocks");
   constexpr int NW = 2 * WN, kBN = WN * 64, kSlot = kATile + kBN * 96, kScRows = kScA + kBN * 16;
   constexpr int kScBuf = kScRows + (RAGGED ? (kBM + kBN) * 4 : 0);  // RAGGED: 4 more bytes per row behind the rows' 16
   constexpr int kStages = STAGES;
@@ -498,6 +501,12 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
       }
     }
   }
+  if constexpr (sizeof(OutT) == 1) {  // C re-quantised to MXFP6 along N (the next GEMM's K): a wave's two tiles of a band at a time
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+      store_fp6_band(acc[i][0], acc[i][1], args.fmt_c, (uint8_t*)args.C, args.C_scale, (long)pm * kBM + wm * 64 + i * 32 + r32, args.M, pn * (kBN / 32) + wn * 2, N / 32);
+    return;
+  }
   // RAGGED with a K split: the shares' matrices have rows of a multiple of four floats
   [[maybe_unused]] const size_t ldc = RAGGED && args.nsplit > 1 ? ragged_pitch(N) : N;
   const __amdgpu_buffer_rsrc_t rC = make_rsrc((OutT*)args.C + (size_t)share * args.M * N + (size_t)pm * kBM * N + (size_t)pn * kBN,
@@ -641,8 +650,18 @@ hipError_t launch_ragged(const GemmArgs& g, const BlockArgs& a, int tiles, hipSt
   }
   return hipGetLastError();
 }
+// fp6 output, the fused epilogue applied or not inside
+template <int FA, int FB>
+hipError_t launch_fp6(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, hipStream_t s) {
+  if (stages == 0) stages = block_stages(g, tiles, cu_count_of_device());
+  if (g.tile_cols == 256) gemm_block_kernel<FA, FB, OutFp6, 4, 4, true><<<tiles, 512, 0, s>>>(a);
+  else if (stages == 6) gemm_block_kernel<FA, FB, OutFp6, 6, 2, true><<<tiles, 256, 0, s>>>(a);
+  else gemm_block_kernel<FA, FB, OutFp6, 3, 2, true><<<tiles, 256, 0, s>>>(a);
+  return hipGetLastError();
+}
 template <int FA, int FB>
 hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, hipStream_t s) {
+  if (g.fmt_c && a.nsplit == 1) return launch_fp6<FA, FB>(g, a, tiles, stages, s);
   // a split leaves the epilogue to the reduction
   if (a.nsplit == 1 && epilogue_any(g.ep)) return launch<FA, FB, true>(g, a, tiles, stages, s);
   return launch<FA, FB, false>(g, a, tiles, stages, s);
@@ -671,7 +690,7 @@ bool gemm_block_ragged_supports(const GemmArgs& g) {
 hipError_t launch_gemm_block(const GemmArgs& g, hipStream_t s) {
   const int bn = g.tile_cols == 256 ? 256 : 128, nsplit = g.ksplit > 1 ? g.ksplit : 1;
   BlockArgs a{g.A, g.B, g.As, g.Bs, nsplit > 1 ? (void*)g.ks_part : g.C, g.M, g.N, g.K, (g.M + kBM - 1) / kBM, (g.N + bn - 1) / bn, g.layout_a, g.layout_b,
-              g.raster_group_m > 0 ? g.raster_group_m : kGroupM, g.raster_no_xcd_remap == 1 ? 0 : g.raster_no_xcd_remap == 2 ? 2 : 1, nsplit, g.ep};
+              g.raster_group_m > 0 ? g.raster_group_m : kGroupM, g.raster_no_xcd_remap == 1 ? 0 : g.raster_no_xcd_remap == 2 ? 2 : 1, nsplit, g.ep, g.C_scale, g.fmt_c};
   const int tiles = a.tiles_m * a.tiles_n, stages = g.tile_rows == 3 || g.tile_rows == 6 ? g.tile_rows : 0;
   hipError_t e;
   if (g.ragged) {

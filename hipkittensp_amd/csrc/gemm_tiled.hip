@@ -561,56 +561,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
   auto epilogue = [&]<bool EDGE>(int rows_a, int rows_b) __attribute__((always_inline)) {
     const auto g = fresh_args();
     if constexpr (sizeof(OutT) == 1) {
-      // C re-quantised to MXFP6 along N (the next GEMM's K): a 32-block of row m is the 16 values of lane (m, h = 0)
-      // and the 16 of lane (m, h = 1) of one 32x32 tile.  The wave's two tiles of a band (j = 0, 1) are traded with
-      // v_permlane32_swap, register by register, after which the lower lane holds all of block j = 0 and the upper
-      // lane all of block j = 1: P0[k] = column 8 (k / 4) + k % 4, P1[k] = that + 4.  Then exactly the quantiser:
-      // amax -> E8M0 -> hardware conversion -> 24 bytes and a scale byte per lane.
-      const int N = g->N, nkb = N / 32, fmt_c = g->fmt_c;
+      // C re-quantised to MXFP6 along N (the next GEMM's K): a wave's two tiles of a band at a time
       const long m0 = (long)(tile_cur & 0xffff) * kBM + wm * (TM * 32) + r32;
-      const int blk = (tile_cur >> 16) * (kBN / 32) + wn * TN + h;  // 32-block index along N of this lane's block
-      uint8_t* cp = reinterpret_cast<uint8_t*>(g->C);
-      uint8_t* sp = g->C_scale;
-      const int M = g->M;
+      const int blk0 = (tile_cur >> 16) * (kBN / 32) + wn * TN, nkb = g->N / 32, fmt_c = g->fmt_c, M = g->M;
+      uint8_t *cp = reinterpret_cast<uint8_t*>(g->C), *sp = g->C_scale;
 #pragma unroll
-      for (int i = 0; i < TM; i++) {
-        float p0[16], p1[16];
-#pragma unroll
-        for (int k = 0; k < 16; k++) {
-          const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[i][0][k]), __float_as_uint(acc[i][1][k]), false, false);
-          p0[k] = __uint_as_float(sw[0]), p1[k] = __uint_as_float(sw[1]);
-        }
-        float amax = 0.f;
-#pragma unroll
-        for (int k = 0; k < 16; k++) amax = fmaxf(amax, fmaxf(fabsf(p0[k]), fabsf(p1[k])));
-        const int sb = e8m0_of_amax(amax, fmt_c == 2 ? 2 : 4);
-        const float scale = __uint_as_float((uint32_t)sb << 23);
-        v16f ev, od;  // even and odd columns of the block: column n = 8 q + r is p0[4 q + r] for r < 4, p1[4 q + r - 4] otherwise
-#pragma unroll
-        for (int t = 0; t < 16; t++) {
-          const int ne = 2 * t, no = 2 * t + 1;
-          ev[t] = (ne & 4) ? p1[4 * (ne >> 3) + (ne & 3)] : p0[4 * (ne >> 3) + (ne & 3)];
-          od[t] = (no & 4) ? p1[4 * (no >> 3) + (no & 3)] : p0[4 * (no >> 3) + (no & 3)];
-        }
-        typedef unsigned v6u __attribute__((ext_vector_type(6)));
-        // a real branch (the empty asm keeps it one): with both conversions issued on the same sources and a select
-        // behind them, the second one's result came out wrong from the third dword on
-        v6u w;
-        if (fmt_c == 2) {
-          w = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ev, od, scale);
-          asm volatile("" : "+v"(w));
-        } else {
-          w = __builtin_amdgcn_cvt_scalef32_2xpk16_bf6_f32(ev, od, scale);
-          asm volatile("" : "+v"(w));
-        }
-        const long m = m0 + i * 32;
-        if (m < M && blk < nkb) {
-          u32x2* dst = reinterpret_cast<u32x2*>(cp + (m * nkb + blk) * 24);
-#pragma unroll
-          for (int c = 0; c < 3; c++) dst[c] = u32x2{w[2 * c], w[2 * c + 1]};
-          sp[m * nkb + blk] = (uint8_t)sb;
-        }
-      }
+      for (int i = 0; i < TM; i++) store_fp6_band(acc[i][0], acc[i][1], fmt_c, cp, sp, m0 + i * 32, M, blk0, nkb);
       return;
     }
     const int N = g->N, N2 = N * (int)sizeof(OutT);  // N2: bytes per row of C
@@ -789,8 +745,11 @@ int tiled_grid_size(const GemmArgs& g, int tiles, int per_cu) {
 // Sum of a K split's partial sums (partial_offset), in share order, with the epilogue: a wave adds one 32 x 32 tile of C, all
 // loads of up to eight shares in flight at once, and stores it as the GEMM kernels do (bf16: lanes l and l + 32 trade halves,
 // 16 bytes per lane).
+// T = uint8_t: C re-quantised to MXFP6 along N (N % 32 == 0).  Lanes l and l + 32 hold a block's halves; both get all of it, and one stores the 24
+// bytes, the other the scale.
 template <typename T>
-__global__ __launch_bounds__(256) void ksplit_reduce_kernel(const float* __restrict__ part, int nsplit, T* __restrict__ C, int M, int N, const Epilogue ep) {
+__global__ __launch_bounds__(256) void ksplit_reduce_kernel(const float* __restrict__ part, int nsplit, T* __restrict__ C, int M, int N, const Epilogue ep,
+                                                            uint8_t* __restrict__ C_scale, int fmt_c) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int cts = (N + 31) / 32, groups = (cts + 3) / 4;  // a workgroup's four waves take column tiles side by side
   const int band = blockIdx.x / groups, ct = (blockIdx.x - band * groups) * 4 + wave;
@@ -837,6 +796,25 @@ __global__ __launch_bounds__(256) void ksplit_reduce_kernel(const float* __restr
 #pragma unroll
         for (int e = 0; e < 4; e++) acc[q][e] = epilogue_apply(ep, acc[q][e], m, n0 + 8 * q + e);
       }
+  }
+  if constexpr (sizeof(T) == 1) {
+    float p0[16], p1[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+      const uint32_t x = __float_as_uint(acc[k >> 2][k & 3]);
+      const auto sw = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+      p0[k] = __uint_as_float(sw[0]), p1[k] = __uint_as_float(sw[1]);
+    }
+    int sb;
+    const u32x6 w = quantise_block_acc(p0, p1, fmt_c, sb);
+    const size_t blk = (size_t)m * cts + ct;
+    if (h == 0) {
+#pragma unroll
+      for (int i = 0; i < 3; i++) reinterpret_cast<u32x2*>(C + blk * 24)[i] = u32x2{w[2 * i], w[2 * i + 1]};
+    } else {
+      C_scale[blk] = (uint8_t)sb;
+    }
+    return;
   }
   T* const c = C + (size_t)m * N;
   if constexpr (sizeof(T) == 2) {
@@ -885,8 +863,9 @@ hipError_t launch_ksplit_reduce(const GemmArgs& g, hipStream_t s) {
     return hipGetLastError();
   }
   const unsigned blocks = (unsigned)(((g.M + 31) / 32) * (((g.N + 31) / 32 + 3) / 4));
-  if (g.f32out) ksplit_reduce_kernel<float><<<blocks, 256, 0, s>>>(g.ks_part, g.ksplit, (float*)g.C, g.M, g.N, g.ep);
-  else ksplit_reduce_kernel<uint16_t><<<blocks, 256, 0, s>>>(g.ks_part, g.ksplit, (uint16_t*)g.C, g.M, g.N, g.ep);
+  if (g.fmt_c) ksplit_reduce_kernel<uint8_t><<<blocks, 256, 0, s>>>(g.ks_part, g.ksplit, (uint8_t*)g.C, g.M, g.N, g.ep, g.C_scale, g.fmt_c);
+  else if (g.f32out) ksplit_reduce_kernel<float><<<blocks, 256, 0, s>>>(g.ks_part, g.ksplit, (float*)g.C, g.M, g.N, g.ep, nullptr, 0);
+  else ksplit_reduce_kernel<uint16_t><<<blocks, 256, 0, s>>>(g.ks_part, g.ksplit, (uint16_t*)g.C, g.M, g.N, g.ep, nullptr, 0);
   return hipGetLastError();
 }
 
@@ -964,7 +943,8 @@ static hipError_t launch(const GemmArgs& g, hipStream_t s) {
 hipError_t MXFP6_PASTE(launch_gemm_tiled_fmt, MXFP6_TILED_FMT)(const GemmArgs& g, hipStream_t s) {
   constexpr int FA = MXFP6_TILED_FMT / 10, FB = MXFP6_TILED_FMT % 10;
   static_assert((FA == 2 || FA == 3) && (FB == 2 || FB == 3), "MXFP6_TILED_FMT: 22, 23, 32 or 33");
-  return g.fmt_c ? launch<FA, FB, OutFp6>(g, s) : g.f32out ? launch<FA, FB, OutF32>(g, s) : launch<FA, FB, OutBf16>(g, s);
+  const bool ksplit = g.ksplit > 1 && g.ks_part;  // the shares are fp32 whatever the output is; the reduction makes it
+  return g.fmt_c && !ksplit ? launch<FA, FB, OutFp6>(g, s) : g.f32out ? launch<FA, FB, OutF32>(g, s) : launch<FA, FB, OutBf16>(g, s);
 }
 #undef MXFP6_PASTE
 #undef MXFP6_PASTE2

@@ -113,3 +113,38 @@ def test_few_rows_quantised_inside_the_gemm(hk, M, N, K, fmt_x, fmt_w):
     x[0, 5] = float("nan")
     y, want = layer(x), steps(hk, layer, x)
     assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("kernel,shares,M,N,K,tile_b", [(23, 1, 129, 4096, 640, True), (24, 1, 500, 1056, 2176, False), (26, 1, 300, 2080, 640, True), (26, 1, 128, 96, 128, False),
+                                                        (22, 3, 257, 2048, 4096, False), (22, 5, 90, 1056, 2816, True), (0, 0, 256, 8192, 28672, True),
+                                                        (0, 0, 300, 12064, 4096, False), (0, 0, 384, 4096, 640, True), (0, 0, 700, 8896, 640, False)])
+@pytest.mark.parametrize("fmt_c", [2, 3])
+def test_fp6_output_of_the_block_kernel_and_the_k_splits(hk, kernel, shares, M, N, K, tile_b, fmt_c):
+    """Bit for bit the quantiser applied to the fp32 result of the same call, which the same kernel computes: edge tiles, an
+    odd number of 32-column tiles, several shares; blocks of zeros, of NaN and of infinities; outputs that start 8 bytes past a
+    multiple of 16; nothing written around them."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, asc = hk.quantize(torch.randn(M, K, device="cuda", generator=g))
+    lb = hk.LAYOUT_TILE if tile_b else hk.LAYOUT_ROW
+    b, bsc = hk.quantize(torch.randn(N, K, device="cuda", generator=g) * 0.05, 2, lb)
+    bias = torch.randn(N, device="cuda", generator=g)
+    cs = torch.rand(N, device="cuda", generator=g) + 0.5
+    rs = torch.rand(M, device="cuda", generator=g) + 0.5
+    cs[:32], rs[M - 1] = 0.0, float("nan")
+    cs[64:65] = float("inf")
+    prev, prev_split = hk.tk_kernel.set_kernel(kernel), hk.tk_kernel.set_k_split(shares)
+    try:
+        for kw in (dict(), dict(bias=bias, row_scale=rs, activation="gelu"), dict(col_scale=cs, row_scale=rs, activation="relu")):
+            C = torch.empty(M, N, dtype=torch.float32, device="cuda")
+            hk.dispatch_micro(a, b, asc, bsc, C, 2, 2, hk.LAYOUT_ROW, lb, **kw)
+            want, want_s = hk.quantize(C, fmt_c)
+            n, m = M * (N // 4 * 3), M * (N // 32)
+            raw, raw_s = torch.full((n + 64,), 0xAA, dtype=torch.uint8, device="cuda"), torch.full((m + 64,), 0xAA, dtype=torch.uint8, device="cuda")
+            P, S = raw[8:8 + n].view(M, -1), raw_s[8:8 + m].view(M, -1)
+            hk.dispatch_micro(a, b, asc, bsc, P, 2, 2, hk.LAYOUT_ROW, lb, C_scale=S, fmt_c=fmt_c, **kw)
+            assert torch.equal(S, want_s) and torch.equal(P, want)
+            for r, k in ((raw, n), (raw_s, m)):
+                assert (r[:8] == 0xAA).all() and (r[8 + k:] == 0xAA).all()
+    finally:
+        hk.tk_kernel.set_kernel(prev)
+        hk.tk_kernel.set_k_split(prev_split)
