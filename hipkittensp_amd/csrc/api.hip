@@ -466,37 +466,38 @@ int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const voi
   rc = check_device();
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  // the tiled kernel quantises its accumulators itself; where another kernel is the better one (few rows of A: C is
-  // small there) the product goes to an fp32 workspace of the stream-ordered allocator and through the quantiser
-  mxfp6::GemmArgs g{(const uint8_t*)A, (const uint8_t*)B, (const uint8_t*)As, (const uint8_t*)Bs, C_packed, M, N, K, fmt_a, fmt_b, false, layout_a, layout_b};
+  // The tiled and the block kernel and the reduction of a K split quantise their sums themselves (us, block kernel through the fp32
+  // workspace and the quantiser / here: 256 x 2560 x 2304 16.7 / 13.0, 500 x 8192 x 8192 38.3 / 30.6, 2048 x 4096 x 4096 41.4 / 32.0,
+  // 3000 x 2048 x 1024 24.9 / 11.6).  Skinny, ring, ragged and generic products, and a split without its workspace, go through the
+  // workspace.  The choice is that of the same call with fp32 output, whose bits these are; where that is the tiled kernel's 128 x
+  // 128 tile, which has no fp6 form, the best of the kernels that add up in the same order.
+  mxfp6::GemmArgs g{(const uint8_t*)A, (const uint8_t*)B, (const uint8_t*)As, (const uint8_t*)Bs, nullptr, M, N, K, fmt_a, fmt_b, true, layout_a, layout_b};
+  g.ep = ep;
   const int force = g_force;
-  // the tiled kernel's own fp6 epilogue only where the automatic choice is that kernel (unsplit)
-  const bool tiled = K > 0 && mxfp6::gemm_tiled_supports(g) &&
-                     (force == 2 || force == 5 || force == 6 || force == 17 || (force == 0 && choice_code(auto_choice(g, 0, true)) == kChoiceTiled));
-  if (tiled) {
-    g.ep = ep, g.C_scale = (uint8_t*)C_scale, g.fmt_c = fmt_c;
-    g.tile_rows = force == 5 || force == 17 ? 128 : force == 6 ? 256 : 0, g.tile_cols = force == 17 ? 128 : 0;
-    if (force == 0 || force == 2) (void)apply_choice(g, mxfp6::choose_kernel(g, 1, false, kTiledUnsplit), s);  // the tile height (the fp6 epilogue needs 256 columns)
-    hipError_t e;
-    if (force != 0 || !relayout_then_tiled(g, s, e)) e = mxfp6::launch_gemm_tiled(g, s);
-    return e == hipSuccess ? MXFP6_OK : (int)e;
-  }
   std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
-  // So do the block kernel and the reduction of a K split (us, through the fp32 workspace / here: 256 x 2560 x 2304
-  // 16.7 / 13.0, 500 x 8192 x 8192 38.3 / 30.6, 2048 x 4096 x 4096 41.4 / 32.0, 3000 x 2048 x 1024 24.9 / 11.6).  Skinny, ring, ragged and generic products, and a split without its workspace, go through the workspace.
-  if (K > 0 && (force == 0 || (force >= 22 && force <= 24) || force == 26)) {
-    mxfp6::GemmArgs t = g;
-    t.C = nullptr, t.f32out = true;  // the kernel of the same call with fp32 output, whose bits these are (fp6 itself is stored 8 bytes at a time)
-    const mxfp6::KernelChoice c = force == 0    ? auto_choice(t, 0, true)
-                                  : force == 26 ? mxfp6::choose_kernel(t, 1, false, 1u << mxfp6::kCandBlockWide)
-                                                : family_choice(t, 1u << mxfp6::kCandBlock, 1u << mxfp6::kCandBlockSplit);
-    const bool block = c.cand == mxfp6::kCandBlock || c.cand == mxfp6::kCandBlockWide || c.cand == mxfp6::kCandBlockSplit;
-    if ((block || c.cand == mxfp6::kCandTiledSplit256 || c.cand == mxfp6::kCandTiledSplit128) && apply_choice(t, c, s)) {
-      t.C = C_packed, t.f32out = false, t.ep = ep, t.C_scale = (uint8_t*)C_scale, t.fmt_c = fmt_c;
-      if (force) t.tile_rows = force == 23 ? 3 : force == 24 ? 6 : 0;
-      const hipError_t e = block ? mxfp6::launch_gemm_block(t, s) : mxfp6::launch_gemm_tiled(t, s);
-      return e == hipSuccess ? MXFP6_OK : (int)e;
-    }
+  mxfp6::KernelChoice c{-1, 1, 0, 0.0};
+  if (K > 0 && force == 0) {
+    c = auto_choice(g, 0, true);
+    if (c.cand == mxfp6::kCandTiled128x128)
+      c = mxfp6::choose_kernel(g, 1, false, auto_mask(g, 0) & (1u << mxfp6::kCandTiled256 | 1u << mxfp6::kCandTiled128x256 | 1u << mxfp6::kCandBlock | 1u << mxfp6::kCandBlockWide));
+  } else if (K > 0 && (force == 2 || force == 5 || force == 6 || force == 17)) {
+    c = mxfp6::choose_kernel(g, 1, false, force == 2 ? 1u << mxfp6::kCandTiled256 | 1u << mxfp6::kCandTiled128x256 : 1u << (force == 6 ? mxfp6::kCandTiled256 : mxfp6::kCandTiled128x256));
+  } else if (K > 0 && force == 26) {
+    c = mxfp6::choose_kernel(g, 1, false, 1u << mxfp6::kCandBlockWide);
+  } else if (K > 0 && force >= 22 && force <= 24) {
+    c = family_choice(g, 1u << mxfp6::kCandBlock, 1u << mxfp6::kCandBlockSplit);
+  }
+  const bool block = c.cand == mxfp6::kCandBlock || c.cand == mxfp6::kCandBlockWide || c.cand == mxfp6::kCandBlockSplit;
+  const bool split = c.cand == mxfp6::kCandTiledSplit256 || c.cand == mxfp6::kCandTiledSplit128;
+  // (the unsplit tiled kernel: C on 16 bytes, as ever; the others store fp6 8 bytes at a time)
+  const bool tiled = (c.cand == mxfp6::kCandTiled256 || c.cand == mxfp6::kCandTiled128x256) && ((uintptr_t)C_packed & 15) == 0;
+  if ((block || split || tiled) && apply_choice(g, c, s)) {
+    g.C = C_packed, g.f32out = false, g.C_scale = (uint8_t*)C_scale, g.fmt_c = fmt_c;
+    if (force == 23 || force == 24) g.tile_rows = force == 23 ? 3 : 6;
+    hipError_t e;
+    if (block) e = mxfp6::launch_gemm_block(g, s);
+    else if (split || force != 0 || !relayout_then_tiled(g, s, e)) e = mxfp6::launch_gemm_tiled(g, s);
+    return e == hipSuccess ? MXFP6_OK : (int)e;
   }
   float* tmp = reinterpret_cast<float*>(stream_workspace(s, 1, (size_t)M * N * 4));
   if (!tmp) return stream_is_capturing(s) ? (int)hipErrorStreamCaptureUnsupported : MXFP6_EWORKSPACE;

@@ -117,7 +117,7 @@ def test_few_rows_quantised_inside_the_gemm(hk, M, N, K, fmt_x, fmt_w):
 
 @pytest.mark.parametrize("kernel,shares,M,N,K,tile_b", [(23, 1, 129, 4096, 640, True), (24, 1, 500, 1056, 2176, False), (26, 1, 300, 2080, 640, True), (26, 1, 128, 96, 128, False),
                                                         (22, 3, 257, 2048, 4096, False), (22, 5, 90, 1056, 2816, True), (0, 0, 256, 8192, 28672, True),
-                                                        (0, 0, 300, 12064, 4096, False), (0, 0, 384, 4096, 640, True), (0, 0, 700, 8896, 640, False)])
+                                                        (0, 0, 300, 12064, 4096, False), (0, 0, 384, 4096, 640, True), (0, 0, 700, 8896, 640, False), (0, 0, 1500, 11008, 4096, True), (0, 0, 4096, 2048, 512, True)])
 @pytest.mark.parametrize("fmt_c", [2, 3])
 def test_fp6_output_of_the_block_kernel_and_the_k_splits(hk, kernel, shares, M, N, K, tile_b, fmt_c):
     """Bit for bit the quantiser applied to the fp32 result of the same call, which the same kernel computes: edge tiles, an
