@@ -64,7 +64,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled4_kernel(const uint8_t* __r
 
   const int rowbytes = K / 4 * 3, sbytes = K / 32, nkt = K / kBK;
   const int rows_a = min(kBM, M - pm * kBM), rows_b = min(kBN, N - pn * kBN);
-  const __amdgpu_buffer_rsrc_t rA = make_rsrc(A + (size_t)pm * kBM * rowbytes, (uint32_t)rows_a * rowbytes);
+  // (a tile-major A may end in a partial row-tile: its rows past M are there, of no meaning)
+  const __amdgpu_buffer_rsrc_t rA = make_rsrc(A + (size_t)pm * kBM * rowbytes, (uint32_t)(layout_a ? (rows_a + 31) & ~31 : rows_a) * rowbytes);
   const __amdgpu_buffer_rsrc_t rB = make_rsrc(B + (size_t)pn * kBN * rowbytes, (uint32_t)rows_b * rowbytes);
   const int nk4 = (nkt + 3) / 4;
   const __amdgpu_buffer_rsrc_t rSA = layout_a ? make_rsrc(As + (size_t)pm * (kBM / 32) * nk4 * 512, (uint32_t)((rows_a + 31) / 32) * nk4 * 512) : make_rsrc(As + (size_t)pm * kBM * sbytes, (uint32_t)rows_a * sbytes);

@@ -148,3 +148,20 @@ def test_fp6_output_of_the_block_kernel_and_the_k_splits(hk, kernel, shares, M, 
     finally:
         hk.tk_kernel.set_kernel(prev)
         hk.tk_kernel.set_k_split(prev_split)
+
+
+@pytest.mark.parametrize("M", [65, 97, 257, 300])
+@pytest.mark.parametrize("N,K", [(256, 512), (96, 640)])
+def test_linear_on_the_four_wave_kernel(hk, M, N, K):
+    """Row counts that end in a partial row-tile of the packed activations: the last tile's rows are multiplied whole."""
+    from hipkittensp_amd.torch_op import MXFP6Linear
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    layer = MXFP6Linear(torch.randn(N, K, device="cuda", generator=g) * 0.02)
+    x = torch.randn(M, K, device="cuda", generator=g)
+    want = steps(hk, layer, x)
+    prev = hk.tk_kernel.set_kernel(hk.tk_kernel.KERNEL_TILED_4WAVE)
+    try:
+        assert torch.equal(layer(x), want)
+    finally:
+        hk.tk_kernel.set_kernel(prev)
