@@ -71,3 +71,18 @@ def test_ragged_alignment_and_fused_epilogue(hk, M, N, K, la):
         fused = call(hk, *ops, M, N, 2, 2, torch.float32, off_c=oc, layout_a=la, bias=bias, activation="relu").cpu().numpy()
         want = np.maximum(got + bias.cpu().numpy(), 0)  # one fp32 addition: exact to its rounding
         assert np.array_equal(fused, want.astype(np.float32)), (oa, ob, osa, osb, oc)
+
+
+@pytest.mark.parametrize("N,first_is_odd_c", [(328, True), (344, False)])
+def test_choice_is_per_alignment(hk, N, first_is_odd_c):
+    """One shape twice: operands on 16 bytes with a C off 16 bytes (the decode kernel takes it), then scales one byte off with
+    a C on 16 bytes (it does not), and in the other order: the first call's choice is not the second one's."""
+    M, K = 16, 1536
+    ap, asc = co.quantise(o.make_source("normal", (M, K), np.random.default_rng(4)), 2)
+    bp, bsc = co.quantise(o.make_source("weights", (N, K), np.random.default_rng(5)), 2)
+    ref = o.gemm_ref(ap, bp, asc, bsc, acc=np.float64)
+    odd_c = ([at(x, 0) for x in (ap, bp, asc, bsc)], 1)
+    odd_scales = ([at(ap, 0), at(bp, 0), at(asc, 1), at(bsc, 3)], 0)
+    for ops, off_c in (odd_c, odd_scales) if first_is_odd_c else (odd_scales, odd_c):
+        got = call(hk, *ops, M, N, 2, 2, torch.float32, off_c=off_c).cpu().numpy()
+        assert o.rel_err(got, ref) <= 1e-5
