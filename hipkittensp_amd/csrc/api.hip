@@ -438,8 +438,9 @@ int mxfp6_linear(const void* X, int x_bf16, const void* W, const void* Ws, void*
   }
   // Tile-major from 64 rows on, whatever M is (the workspace has whole 32-row tiles; what stands in the rows past M reaches
   // nothing but outputs that are not stored): whole cache lines for every load of the GEMM.  Fewer rows stay row-major for the
-  // skinny kernel.
-  const int layout_x = M >= 64 && K % 128 == 0 ? MXFP6_LAYOUT_TILE : MXFP6_LAYOUT_ROW;
+  // skinny kernel, and so does a partial last tile for a forced kernel that takes a row-major A only (skinny, mid).
+  const bool forced_row = g_force == 3 || g_force == 4 || (g_force >= 7 && g_force <= 16) || (g_force >= 19 && g_force <= 21);
+  const int layout_x = M >= 64 && K % 128 == 0 && (M % 32 == 0 || !forced_row) ? MXFP6_LAYOUT_TILE : MXFP6_LAYOUT_ROW;
   const size_t rows = ((size_t)M + 31) & ~(size_t)31;
   const size_t nx = (rows * (K / 32) * 24 + 255) & ~(size_t)255, ns = rows * ((K + 511) / 512) * 16;
   std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);

@@ -165,3 +165,21 @@ def test_linear_on_the_four_wave_kernel(hk, M, N, K):
         assert torch.equal(layer(x), want)
     finally:
         hk.tk_kernel.set_kernel(prev)
+
+
+@pytest.mark.parametrize("M", [65, 97, 127])
+@pytest.mark.parametrize("kernel", [3, 4, 7, 16, 21])
+def test_linear_on_forced_kernels_of_row_major_activations(hk, M, kernel):
+    """Kernels that take a row-major A only run the layer at row counts that fill no row-tile.  (Sums of 1024 products of
+    4-bit significands are exact in any order.)"""
+    from hipkittensp_amd.torch_op import MXFP6Linear
+
+    g = torch.Generator(device="cuda").manual_seed(M)
+    layer = MXFP6Linear(torch.randn(256, 1024, device="cuda", generator=g) * 0.02, activation="relu")
+    x = torch.randn(M, 1024, device="cuda", generator=g)
+    want = steps(hk, layer, x)
+    prev = hk.tk_kernel.set_kernel(kernel)
+    try:
+        assert torch.equal(layer(x), want)
+    finally:
+        hk.tk_kernel.set_kernel(prev)
