@@ -443,6 +443,8 @@ int mxfp6_linear(const void* X, int x_bf16, const void* W, const void* Ws, void*
   const int layout_x = M >= 64 && K % 128 == 0 && (M % 32 == 0 || !forced_row) ? MXFP6_LAYOUT_TILE : MXFP6_LAYOUT_ROW;
   const size_t rows = ((size_t)M + 31) & ~(size_t)31;
   const size_t nx = (rows * (K / 32) * 24 + 255) & ~(size_t)255, ns = rows * ((K + 511) / 512) * 16;
+  // A graph's activations live in its own memory plan: graphs captured on one stream may be replayed side by side on others
+  if (K > 0 && stream_is_capturing(s)) return MXFP6_EWORKSPACE;
   std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
   uint8_t* xp = K > 0 ? stream_workspace(s, 4, nx + ns) : nullptr;
   if (K > 0) {
@@ -821,7 +823,7 @@ const char* mxfp6_strerror(int code) {
     case MXFP6_EINVAL_EPILOGUE: return "mxfp6: activation must be 0 (none), 1 (relu), 2 (gelu) or 3 (silu)";
     case MXFP6_ESCRATCH: return "mxfp6: the K split of this call needs more than the static scratch memory holds (256 partial tiles: rows of C tiles times nsplit)";
     case MXFP6_EINVAL_KERNEL: return "mxfp6: unknown kernel code";
-    case MXFP6_EWORKSPACE: return "mxfp6: no workspace for this call (the allocator refused, or every workspace slot is held by a captured graph)";
+    case MXFP6_EWORKSPACE: return "mxfp6: no workspace for this call (the allocator refused, every workspace slot is held by a captured graph, or a linear layer is being captured)";
     case MXFP6_EACCURACY: return "mxfp6: e3m2 x e3m2 can exceed the 2e-3 accuracy bar (up to 1e-4 of sum |a||b| per output); call mxfp6_allow_e3m2_pair(1) to accept that";
     case MXFP6_EBLOB: return "mxfp6: not a tile-major operand blob this library reads (magic, version, format, layout or shape)";
     default: break;

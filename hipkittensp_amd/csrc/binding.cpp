@@ -171,7 +171,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_BEGIN_ALLOW_THREADS;
     rc = mxfp6_linear(X->data_ptr(), bf16, W->data_ptr(), Ws->data_ptr(), C.data_ptr(), (int)rows, (int)N, (int)K, fx, fw, lw, bias, bias_bf16, act, s);
     Py_END_ALLOW_THREADS;
-    // no workspace to be had (a stream under capture, the allocator): the two steps with tensors of the caller's allocator
+    // no workspace (a stream under capture, whose graph owns its activations; the allocator's refusal): the two steps with tensors of the caller's allocator
     if (rc == MXFP6_EWORKSPACE) Py_RETURN_NONE;
     if (rc) return done(rc, "linear");
     return THPVariable_Wrap(std::move(C));

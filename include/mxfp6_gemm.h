@@ -34,7 +34,9 @@
  *     256 x 256 fp32), one workspace for the three kernels, and for the ring kernel one counter per output tile.
  * While `hip_stream` is being captured nothing is allocated: the pre-pass and the K splits are left out
  * (same results up to the order of fp32 sums, other kernels) unless their workspace exists already, and mxfp6_gemm_fused_fp6 returns
- * hipErrorStreamCaptureUnsupported where it would need a new one.  A workspace that a capture did use is recorded in the
+ * hipErrorStreamCaptureUnsupported where it would need a new one.  mxfp6_linear records no packed activations
+ * of its own in a graph: where it needs a workspace for them it returns MXFP6_EWORKSPACE under capture (quantise into the
+ * graph's own memory and call the GEMM).  A workspace that a capture did use is recorded in the
  * graph: the library never frees such a block again (when a later call needs a larger one, or at
  * mxfp6_release_workspaces(), it is kept allocated until the process ends), so the graph stays valid.  Replay it on the
  * stream it was captured on, or on another one only while no call of this library runs on the capture stream: the
@@ -81,7 +83,7 @@ extern "C" {
 #define MXFP6_EINVAL_KERNEL (-9) /* mxfp6_set_kernel: unknown kernel code                        */
 #define MXFP6_EBLOB (-10)       /* not a tile-major operand blob of a version this library reads */
 #define MXFP6_EACCURACY (-12)   /* e3m2 x e3m2 without mxfp6_allow_e3m2_pair(1): the pair can miss the 2e-3 accuracy bar */
-#define MXFP6_EWORKSPACE (-11)  /* a call that cannot run without a workspace did not get one (allocator, or all slots held by graphs) */
+#define MXFP6_EWORKSPACE (-11)  /* a call that cannot run without a workspace did not get one (allocator, all slots held by graphs, mxfp6_linear under capture) */
 
 /* Activations of mxfp6_gemm_fused. */
 #define MXFP6_ACT_NONE 0
@@ -277,8 +279,9 @@ int mxfp6_gemm_fused_fp6(const void *A_packed, const void *B_packed, const void 
  *   C[m][n] = act((dq(X) . dq(W)^T)[m][n] + bias[n])         bf16
  * as mxfp6_gemm_fused would compute it from that operand.  W_packed [N, 3K/4], W_scale: the weights in layout_w; bias as in
  * mxfp6_gemm_fused (NULL = none).  The packed activations live in a workspace of this stream (0.79 bytes per element of X,
- * rows rounded up to 32), in the layout the GEMM prefers.  MXFP6_EWORKSPACE, and nothing launched, where it cannot be had
- * (first use under capture).  No counterpart in the reference.
+ * rows rounded up to 32), in the layout the GEMM prefers.  MXFP6_EWORKSPACE, and nothing launched, where it cannot be had,
+ * and while the stream is being captured (two graphs captured on one stream would share it).  Up to four bf16 rows on the
+ * decode kernel need none and are captured.  No counterpart in the reference.
  */
 int mxfp6_linear(const void *X, int x_bf16, const void *W_packed, const void *W_scale, void *C_bf16, int M, int N, int K,
                  int fmt_x, int fmt_w, int layout_w, const void *bias, int bias_bf16, int activation, void *hip_stream);

@@ -183,3 +183,65 @@ def test_linear_on_forced_kernels_of_row_major_activations(hk, M, kernel):
         assert torch.equal(layer(x), want)
     finally:
         hk.tk_kernel.set_kernel(prev)
+
+
+def test_graphs_of_one_stream_share_no_activations(hk):
+    """Two graphs of a layer captured on one stream that has run it before, replayed side by side on two others, beside the layer
+    itself on the capture stream: the packed activations of each are its own."""
+    from hipkittensp_amd import _lib
+    from hipkittensp_amd.torch_op import MXFP6Linear
+
+    g = torch.Generator(device="cuda").manual_seed(8)
+    M, N, K = 200, 512, 8192
+    layer = MXFP6Linear(torch.randn(N, K, device="cuda", generator=g) * 0.02)
+    xs = [torch.randn(M, K, device="cuda", generator=g) for _ in range(3)]
+    want = [steps(hk, layer, x) for x in xs]
+    capture, streams = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    prev = hk.tk_kernel.set_k_split(1)   # a K split's partial sums are the stream's, as the header says
+    try:
+        with torch.cuda.stream(capture):
+            layer(xs[2])
+        torch.cuda.synchronize()
+        graphs, ys = [], []
+        for i in range(2):
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=capture):
+                if i == 0:
+                    C = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+                    assert _lib.lib().mxfp6_linear(xs[0].data_ptr(), 0, layer.weight_packed.data_ptr(), layer.weight_scale.data_ptr(), C.data_ptr(), M, N, K,
+                                                   2, 2, layer.layout_w, None, 0, 0, torch.cuda.current_stream().cuda_stream) == -11   # MXFP6_EWORKSPACE
+                ys.append(layer(xs[i]))
+            graphs.append(graph)
+        for _ in range(20):
+            for s, graph in zip(streams, graphs):
+                with torch.cuda.stream(s):
+                    graph.replay()
+            with torch.cuda.stream(capture):
+                y = layer(xs[2])
+            torch.cuda.synchronize()
+            for got, w in zip((*ys, y), want):
+                assert torch.equal(got, w)
+    finally:
+        hk.tk_kernel.set_k_split(prev)
+
+
+@pytest.mark.parametrize("M", [1, 4])
+def test_decode_rows_are_captured_in_one_launch(hk, M):
+    """Up to four bf16 rows need no workspace for their activations: mxfp6_linear itself is captured, on a stream that has none."""
+    from hipkittensp_amd import _lib
+    from hipkittensp_amd.torch_op import MXFP6Linear
+
+    g = torch.Generator(device="cuda").manual_seed(9)
+    layer = MXFP6Linear(torch.randn(512, 1024, device="cuda", generator=g) * 0.02)
+    x = torch.randn(M, 1024, device="cuda", generator=g).to(torch.bfloat16)
+    C, graph = torch.zeros(M, 512, dtype=torch.bfloat16, device="cuda"), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        assert _lib.lib().mxfp6_linear(x.data_ptr(), 1, layer.weight_packed.data_ptr(), layer.weight_scale.data_ptr(), C.data_ptr(), M, 512, 1024,
+                                       2, 2, layer.layout_w, None, 0, 0, torch.cuda.current_stream().cuda_stream) == 0
+    for _ in range(3):
+        x.copy_(torch.randn(M, 1024, device="cuda", generator=g))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C, steps(hk, layer, x))
