@@ -478,11 +478,14 @@ int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const voi
   g.ep = ep;
   const int force = g_force;
   std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
+  constexpr unsigned same_order = 1u << mxfp6::kCandTiled256 | 1u << mxfp6::kCandTiled128x256 | 1u << mxfp6::kCandBlock | 1u << mxfp6::kCandBlockWide;
+  auto choose = [&](bool allow_split) {
+    const mxfp6::KernelChoice c = auto_choice(g, 0, allow_split);
+    return c.cand == mxfp6::kCandTiled128x128 ? mxfp6::choose_kernel(g, 1, false, auto_mask(g, 0) & same_order) : c;
+  };
   mxfp6::KernelChoice c{-1, 1, 0, 0.0};
   if (K > 0 && force == 0) {
-    c = auto_choice(g, 0, true);
-    if (c.cand == mxfp6::kCandTiled128x128)
-      c = mxfp6::choose_kernel(g, 1, false, auto_mask(g, 0) & (1u << mxfp6::kCandTiled256 | 1u << mxfp6::kCandTiled128x256 | 1u << mxfp6::kCandBlock | 1u << mxfp6::kCandBlockWide));
+    c = choose(true);
   } else if (K > 0 && (force == 2 || force == 5 || force == 6 || force == 17)) {
     c = mxfp6::choose_kernel(g, 1, false, force == 2 ? 1u << mxfp6::kCandTiled256 | 1u << mxfp6::kCandTiled128x256 : 1u << (force == 6 ? mxfp6::kCandTiled256 : mxfp6::kCandTiled128x256));
   } else if (K > 0 && force == 26) {
@@ -490,19 +493,30 @@ int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const voi
   } else if (K > 0 && force >= 22 && force <= 24) {
     c = family_choice(g, 1u << mxfp6::kCandBlock, 1u << mxfp6::kCandBlockSplit);
   }
-  const bool block = c.cand == mxfp6::kCandBlock || c.cand == mxfp6::kCandBlockWide || c.cand == mxfp6::kCandBlockSplit;
-  const bool split = c.cand == mxfp6::kCandTiledSplit256 || c.cand == mxfp6::kCandTiledSplit128;
-  // (the unsplit tiled kernel: C on 16 bytes, as ever; the others store fp6 8 bytes at a time)
-  const bool tiled = (c.cand == mxfp6::kCandTiled256 || c.cand == mxfp6::kCandTiled128x256) && ((uintptr_t)C_packed & 15) == 0;
-  if ((block || split || tiled) && apply_choice(g, c, s)) {
-    g.C = C_packed, g.f32out = false, g.C_scale = (uint8_t*)C_scale, g.fmt_c = fmt_c;
-    if (force == 23 || force == 24) g.tile_rows = force == 23 ? 3 : 6;
-    hipError_t e;
-    if (block) e = mxfp6::launch_gemm_block(g, s);
-    else if (split || force != 0 || !relayout_then_tiled(g, s, e)) e = mxfp6::launch_gemm_tiled(g, s);
-    return e == hipSuccess ? MXFP6_OK : (int)e;
+  // Runs the call as chosen, C quantised where it is summed; false: that choice has no fp6 form, or its workspace is not to be had
+  auto run = [&](const mxfp6::KernelChoice& ch, hipError_t& e) {
+    const bool block = ch.cand == mxfp6::kCandBlock || ch.cand == mxfp6::kCandBlockWide || ch.cand == mxfp6::kCandBlockSplit;
+    const bool split = ch.cand == mxfp6::kCandTiledSplit256 || ch.cand == mxfp6::kCandTiledSplit128;
+    // (the unsplit tiled kernel: C on 16 bytes, as ever; the others store fp6 8 bytes at a time)
+    const bool tiled = (ch.cand == mxfp6::kCandTiled256 || ch.cand == mxfp6::kCandTiled128x256) && ((uintptr_t)C_packed & 15) == 0;
+    mxfp6::GemmArgs t = g;
+    if (!(block || split || tiled) || !apply_choice(t, ch, s)) return false;
+    t.C = C_packed, t.f32out = false, t.C_scale = (uint8_t*)C_scale, t.fmt_c = fmt_c;
+    if (force == 23 || force == 24) t.tile_rows = force == 23 ? 3 : 6;
+    if (block) e = mxfp6::launch_gemm_block(t, s);
+    else if (split || force != 0 || !relayout_then_tiled(t, s, e)) e = mxfp6::launch_gemm_tiled(t, s);
+    return true;
+  };
+  hipError_t e = hipSuccess;
+  if (run(c, e)) return e == hipSuccess ? MXFP6_OK : (int)e;
+  // a split without its workspace (a stream under capture that has none): what the shape gets otherwise, as for the other outputs
+  if (c.cand == mxfp6::kCandTiledSplit256 || c.cand == mxfp6::kCandTiledSplit128 || c.cand == mxfp6::kCandBlockSplit) {
+    c = force == 0 ? choose(false) : mxfp6::choose_kernel(g, 1, false, 1u << mxfp6::kCandBlock);
+    if (run(c, e)) return e == hipSuccess ? MXFP6_OK : (int)e;
   }
   float* tmp = reinterpret_cast<float*>(stream_workspace(s, 1, (size_t)M * N * 4));
+  // ... and where the fp32 workspace is not to be had either, a kernel that needs none
+  if (!tmp && K > 0 && force == 0 && run(mxfp6::choose_kernel(g, 1, false, auto_mask(g, 0) & same_order), e)) return e == hipSuccess ? MXFP6_OK : (int)e;
   if (!tmp) return stream_is_capturing(s) ? (int)hipErrorStreamCaptureUnsupported : MXFP6_EWORKSPACE;
   rc = gemm_common(A, B, As, Bs, tmp, M, N, K, fmt_a, fmt_b, true, layout_a, layout_b, stream, ep);
   if (rc == MXFP6_OK) {

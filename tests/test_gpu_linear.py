@@ -245,3 +245,28 @@ def test_decode_rows_are_captured_in_one_launch(hk, M):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(C, steps(hk, layer, x))
+
+
+@pytest.mark.parametrize("M,N,K,act", [(512, 11008, 8192, "gelu"), (1024, 5120, 8192, "none"), (256, 8192, 28672, "relu"), (64, 8192, 28672, "none")])
+def test_fp6_output_is_captured_on_a_stream_without_workspace(hk, M, N, K, act):
+    """A K split needs its workspace and the decode kernels the fp32 one; a capture on a stream that has neither records a kernel
+    that needs none.  Its fp32 sums may differ from the eager call's in their last place (2^-24), which moves a code only next
+    to a rounding boundary of its 2^-4 steps: at most one byte in 10 000 differs."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    a, asc = hk.quantize(torch.randn(M, K, device="cuda", generator=g))
+    b, bsc = hk.quantize(torch.randn(N, K, device="cuda", generator=g) * 0.02, 2, hk.LAYOUT_TILE)
+    mk = lambda: (torch.zeros(M, N // 4 * 3, dtype=torch.uint8, device="cuda"), torch.zeros(M, N // 32, dtype=torch.uint8, device="cuda"))
+    want, got = mk(), mk()
+    call = lambda out: hk.dispatch_micro(a, b, asc, bsc, out[0], 2, 2, hk.LAYOUT_ROW, hk.LAYOUT_TILE, C_scale=out[1], activation=act)
+    call(want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        call(got)
+    for _ in range(3):
+        for t in got:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all((x != y).float().mean().item() <= 1e-4 for x, y in zip(got, want))
+        call(want)
