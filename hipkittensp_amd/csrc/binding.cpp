@@ -17,6 +17,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
@@ -47,6 +48,12 @@ int64_t scale_width(int64_t K, int layout) { return layout == MXFP6_LAYOUT_ROW ?
 bool rows_fit(int64_t rows, int64_t K, int layout) { return layout == MXFP6_LAYOUT_ROW || (rows % 32 == 0 && K % 128 == 0); }
 bool known(int fmt, int layout) { return (fmt == 2 || fmt == 3) && (layout == 0 || layout == 1); }
 hipStream_t stream_of(int dev) { return c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream(); }
+
+// The GIL released for a scope.  What may throw (data_ptr() of a tensor without memory, sizes of a nested one) is read before.
+struct NoGil {
+  PyThreadState* const state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
 
 PyObject* done(int rc, const char* what) {
   if (rc) {
@@ -88,25 +95,27 @@ PyObject* gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const void *bias, *row, *col;
   int bias_bf16 = 0, none = 0;
   if (!vector(a[9], dev, N, true, &bias, &bias_bf16) || !vector(a[10], dev, M, false, &row, &none) || !vector(a[11], dev, N, false, &col, &none)) Py_RETURN_NONE;
+  const void *const pa = A->data_ptr(), *const pb = B->data_ptr(), *const pas = As->data_ptr(), *const pbs = Bs->data_ptr();
+  void* const pc = C->data_ptr();
+  const hipStream_t s = stream_of(dev);
   int rc;
   if (a[13] != Py_None) {
     const at::Tensor* Cs = tensor(a[13]);
     const int fc = small_int(a[14]);
     if (!Cs || !known(fc, 0) || N % 32 || !plain2d(*C, at::kByte, dev, M, N / 4 * 3) || !plain2d(*Cs, at::kByte, dev, M, N / 32)) Py_RETURN_NONE;
-    const hipStream_t s = stream_of(dev);
-    Py_BEGIN_ALLOW_THREADS;
-    rc = mxfp6_gemm_fused_fp6(A->data_ptr(), B->data_ptr(), As->data_ptr(), Bs->data_ptr(), C->data_ptr(), Cs->data_ptr(), (int)M, (int)N, (int)K,
-                              fa, fb, la, lb, fc, bias, bias_bf16, (const float*)row, (const float*)col, act, s);
-    Py_END_ALLOW_THREADS;
+    void* const scales = Cs->data_ptr();
+    {
+      NoGil released;
+      rc = mxfp6_gemm_fused_fp6(pa, pb, pas, pbs, pc, scales, (int)M, (int)N, (int)K, fa, fb, la, lb, fc, bias, bias_bf16, (const float*)row, (const float*)col, act, s);
+    }
     return done(rc, "dispatch_micro");
   }
   const bool f32 = C->scalar_type() == at::kFloat;
   if (!plain2d(*C, f32 ? at::kFloat : at::kBFloat16, dev, M, N)) Py_RETURN_NONE;
-  const hipStream_t s = stream_of(dev);
-  Py_BEGIN_ALLOW_THREADS;
-  rc = mxfp6_gemm_fused(A->data_ptr(), B->data_ptr(), As->data_ptr(), Bs->data_ptr(), C->data_ptr(), (int)M, (int)N, (int)K, fa, fb, la, lb, f32, bias,
-                        bias_bf16, (const float*)row, (const float*)col, act, s);
-  Py_END_ALLOW_THREADS;
+  {
+    NoGil released;
+    rc = mxfp6_gemm_fused(pa, pb, pas, pbs, pc, (int)M, (int)N, (int)K, fa, fb, la, lb, f32, bias, bias_bf16, (const float*)row, (const float*)col, act, s);
+  }
   return done(rc, "dispatch_micro");
 }
 
@@ -120,24 +129,22 @@ PyObject* quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!known(fmt, layout) || dev != c10::hip::current_device() || !plain(*X, bf16 ? at::kBFloat16 : at::kFloat, dev) || K % 32 || rows > kMaxDim ||
       K > kMaxDim || !rows_fit(rows, K, layout))
     Py_RETURN_NONE;
-  try {
-    const auto opt = X->options().dtype(at::kByte).requires_grad(false);
-    at::Tensor packed = at::empty({rows, K / 4 * 3}, opt), scales = at::empty({rows, scale_width(K, layout)}, opt);
-    const hipStream_t s = stream_of(dev);
-    int rc;
-    Py_BEGIN_ALLOW_THREADS;
-    rc = bf16 ? mxfp6_quantize_bf16(X->data_ptr(), packed.data_ptr(), scales.data_ptr(), (int)rows, (int)K, fmt, layout, s)
-              : mxfp6_quantize_ex((const float*)X->data_ptr(), packed.data_ptr(), scales.data_ptr(), (int)rows, (int)K, fmt, layout, s);
-    Py_END_ALLOW_THREADS;
-    if (rc) return done(rc, "quantize");
-    PyObject* p = THPVariable_Wrap(std::move(packed));
-    PyObject* q = p ? THPVariable_Wrap(std::move(scales)) : nullptr;
-    PyObject* r = q ? PyTuple_Pack(2, p, q) : nullptr;
-    Py_XDECREF(p), Py_XDECREF(q);
-    return r;
-  } catch (const std::exception&) {  // an allocation that failed: the Python path raises torch's error
-    Py_RETURN_NONE;
+  const auto opt = X->options().dtype(at::kByte).requires_grad(false);
+  at::Tensor packed = at::empty({rows, K / 4 * 3}, opt), scales = at::empty({rows, scale_width(K, layout)}, opt);
+  const void* const px = X->data_ptr();
+  void *const pp = packed.data_ptr(), *const ps = scales.data_ptr();
+  const hipStream_t s = stream_of(dev);
+  int rc;
+  {
+    NoGil released;
+    rc = bf16 ? mxfp6_quantize_bf16(px, pp, ps, (int)rows, (int)K, fmt, layout, s) : mxfp6_quantize_ex((const float*)px, pp, ps, (int)rows, (int)K, fmt, layout, s);
   }
+  if (rc) return done(rc, "quantize");
+  PyObject* p = THPVariable_Wrap(std::move(packed));
+  PyObject* q = p ? THPVariable_Wrap(std::move(scales)) : nullptr;
+  PyObject* r = q ? PyTuple_Pack(2, p, q) : nullptr;
+  Py_XDECREF(p), Py_XDECREF(q);
+  return r;
 }
 
 // linear(x, weight, weight_scale, bias, fmt_x, fmt_w, layout_w, act) -> y
@@ -156,33 +163,46 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const void* bias;
   int bias_bf16 = 0;
   if (!vector(a[3], dev, N, true, &bias, &bias_bf16)) Py_RETURN_NONE;
+  const auto opt = X->options().dtype(at::kBFloat16).requires_grad(false);
+  at::Tensor C;
+  if (X->dim() == 2) {
+    C = at::empty({rows, N}, opt);
+  } else {
+    auto shape = X->sizes().vec();
+    shape.back() = N;
+    C = at::empty(shape, opt);
+  }
+  const void *const px = X->data_ptr(), *const pw = W->data_ptr(), *const pws = Ws->data_ptr();
+  void* const pc = C.data_ptr();
+  const hipStream_t s = stream_of(dev);
+  int rc;
+  {
+    NoGil released;
+    rc = mxfp6_linear(px, bf16, pw, pws, pc, (int)rows, (int)N, (int)K, fx, fw, lw, bias, bias_bf16, act, s);
+  }
+  // no workspace (a stream under capture, whose graph owns its activations; the allocator's refusal): the two steps with tensors of the caller's allocator
+  if (rc == MXFP6_EWORKSPACE) Py_RETURN_NONE;
+  if (rc) return done(rc, "linear");
+  return THPVariable_Wrap(std::move(C));
+}
+
+// What throws in torch's code (a nested tensor's sizes, a tensor without memory, a HIP error, an allocation) is not the usual call:
+// the Python code takes it and raises its error.  THPVariable_Wrap reports its own failures as python_error.
+template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
+PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   try {
-    const auto opt = X->options().dtype(at::kBFloat16).requires_grad(false);
-    at::Tensor C;
-    if (X->dim() == 2) {
-      C = at::empty({rows, N}, opt);
-    } else {
-      auto shape = X->sizes().vec();
-      shape.back() = N;
-      C = at::empty(shape, opt);
-    }
-    const hipStream_t s = stream_of(dev);
-    int rc;
-    Py_BEGIN_ALLOW_THREADS;
-    rc = mxfp6_linear(X->data_ptr(), bf16, W->data_ptr(), Ws->data_ptr(), C.data_ptr(), (int)rows, (int)N, (int)K, fx, fw, lw, bias, bias_bf16, act, s);
-    Py_END_ALLOW_THREADS;
-    // no workspace (a stream under capture, whose graph owns its activations; the allocator's refusal): the two steps with tensors of the caller's allocator
-    if (rc == MXFP6_EWORKSPACE) Py_RETURN_NONE;
-    if (rc) return done(rc, "linear");
-    return THPVariable_Wrap(std::move(C));
+    return F(self, a, n);
+  } catch (python_error& e) {
+    e.restore();
+    return nullptr;
   } catch (const std::exception&) {
     Py_RETURN_NONE;
   }
 }
 
-PyMethodDef methods[] = {{"gemm", (PyCFunction)(void (*)(void))gemm, METH_FASTCALL, nullptr},
-                         {"quantize", (PyCFunction)(void (*)(void))quantize, METH_FASTCALL, nullptr},
-                         {"linear", (PyCFunction)(void (*)(void))linear, METH_FASTCALL, nullptr},
+PyMethodDef methods[] = {{"gemm", (PyCFunction)(void (*)(void))guarded<gemm>, METH_FASTCALL, nullptr},
+                         {"quantize", (PyCFunction)(void (*)(void))guarded<quantize>, METH_FASTCALL, nullptr},
+                         {"linear", (PyCFunction)(void (*)(void))guarded<linear>, METH_FASTCALL, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

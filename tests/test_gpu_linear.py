@@ -270,3 +270,26 @@ def test_fp6_output_is_captured_on_a_stream_without_workspace(hk, M, N, K, act):
         torch.cuda.synchronize()
         assert all((x != y).float().mean().item() <= 1e-4 for x, y in zip(got, want))
         call(want)
+
+
+def test_exceptions_in_the_binding_are_python_errors(hk):
+    """Tensors whose sizes or memory cannot be read (nested ones, those a fake-tensor mode makes) end in a Python error, and the
+    calls after them work."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from hipkittensp_amd.torch_op import MXFP6Linear
+
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(8, 512, device="cuda", generator=g)
+    layer = MXFP6Linear(torch.randn(64, 512, device="cuda", generator=g) * 0.02)
+    want, (p, s) = steps(hk, layer, x), hk.quantize(x)
+    nested = torch.nested.nested_tensor([torch.zeros(24, dtype=torch.uint8), torch.zeros(48, dtype=torch.uint8)]).cuda()
+    C = torch.empty(8, 64, dtype=torch.bfloat16, device="cuda")
+    for args in ((nested, p, s, s, C), (p, nested, s, s, C), (p, p, nested, s, C), (p, p, s, s, nested)):
+        with pytest.raises(RuntimeError):
+            hk.dispatch_micro(*args)
+    with pytest.raises(RuntimeError):
+        hk.quantize(torch.nested.nested_tensor([torch.zeros(32), torch.zeros(64)]).cuda())
+    with FakeTensorMode(allow_non_fake_inputs=True), pytest.raises(RuntimeError):
+        hk.quantize(x)
+    assert torch.equal(layer(x), want) and torch.equal(hk.quantize(x)[0], p)
