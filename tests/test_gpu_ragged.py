@@ -86,3 +86,15 @@ def test_choice_is_per_alignment(hk, N, first_is_odd_c):
     for ops, off_c in (odd_c, odd_scales) if first_is_odd_c else (odd_scales, odd_c):
         got = call(hk, *ops, M, N, 2, 2, torch.float32, off_c=off_c).cpu().numpy()
         assert o.rel_err(got, ref) <= 1e-5
+
+
+@pytest.mark.parametrize("M,N,K,generic", [(200, 257, 288, True), (800, 511, 320, True), (100, 1003, 320, True), (200, 511, 480, True), (800, 257, 416, True),
+                                           (64, 1003, 320, False), (16, 257, 288, False), (200, 3001, 288, False), (200, 101, 352, False), (200, 257, 512 + 32, False), (16, 5003, 288, False)])
+def test_short_ragged_products_start_on_the_generic_kernel(hk, M, N, K, generic):
+    """Both sides of the line between the one-wave-per-tile kernel and the block kernel, on the automatic path."""
+    choice = hk.tk_kernel.kernel_choice(M, N, K)
+    assert (choice == hk.tk_kernel.KERNEL_GENERIC) == generic and choice in (hk.tk_kernel.KERNEL_GENERIC, hk.tk_kernel.KERNEL_BLOCK)
+    ap, asc = co.quantise(o.make_source("normal", (M, K), np.random.default_rng(M + K)), 2)
+    bp, bsc = co.quantise(o.make_source("weights", (N, K), np.random.default_rng(N + K)), 2)
+    got = call(hk, *(at(x, 0) for x in (ap, bp, asc, bsc)), M, N, 2, 2, torch.float32).cpu().numpy()
+    assert o.rel_err(got, o.gemm_ref(ap, bp, asc, bsc, acc=np.float64)) <= 1e-5
