@@ -472,10 +472,11 @@ int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const voi
   // The tiled and the block kernel and the reduction of a K split quantise their sums themselves (us, block kernel through the fp32
   // workspace and the quantiser / here: 256 x 2560 x 2304 16.7 / 13.0, 500 x 8192 x 8192 38.3 / 30.6, 2048 x 4096 x 4096 41.4 / 32.0,
   // 3000 x 2048 x 1024 24.9 / 11.6).  Skinny, ring, ragged and generic products, and a split without its workspace, go through the
-  // workspace.  The choice is that of the same call with fp32 output, whose bits these are; where that is the tiled kernel's 128 x
-  // 128 tile, which has no fp6 form, the best of the kernels that add up in the same order.
+  // workspace.  The choice is that of the same call with fp32 output, whose bits these are (only an activation may count otherwise,
+  // between kernels that add up in the same order); where that is the tiled kernel's 128 x 128 tile, which has no fp6 form, the
+  // best of the kernels that add up in the same order.
   mxfp6::GemmArgs g{(const uint8_t*)A, (const uint8_t*)B, (const uint8_t*)As, (const uint8_t*)Bs, nullptr, M, N, K, fmt_a, fmt_b, true, layout_a, layout_b};
-  g.ep = ep;
+  g.ep = ep, g.out_fp6 = 1;
   const int force = g_force;
   std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
   constexpr unsigned same_order = 1u << mxfp6::kCandTiled256 | 1u << mxfp6::kCandTiled128x256 | 1u << mxfp6::kCandBlock | 1u << mxfp6::kCandBlockWide;

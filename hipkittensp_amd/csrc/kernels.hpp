@@ -17,8 +17,9 @@ struct GemmArgs {
   int tile_cols = 0;               // ... and rows of B: 128 (with 128 rows of A only) or 256; 0 with tile_rows set = 256
   int skinny_geometry = 0;         // skinny kernel: 1 = 32 rows of B and all waves, 2 = 16 rows of B, 3 = half the waves, 4 - 9 = 1 or 2 with the K range split between 2 / 4 / 8 workgroups, 10 = two waves; 0 = by shape
   Epilogue ep;                     // fused bias / scales / activation (all optional)
-  uint8_t* C_scale = nullptr;      // fp6 output (tiled kernel): C is the packed operand [M, 3N/4], this its E8M0 bytes [M, N/32]
+  uint8_t* C_scale = nullptr;      // fp6 output (tiled and block kernels, reduction of a K split): C is the packed operand [M, 3N/4], this its E8M0 bytes [M, N/32]
   int fmt_c = 0;                   // 2 / 3: format of the fp6 output; 0: bf16 / fp32 output
+  int out_fp6 = 0;                 // kernel choice only: the fp32 sums (f32out) leave as MXFP6
   const void* X = nullptr;         // skinny kernel: bf16 activations [M, K] that it quantises to fmt_a itself, in place of A and As (gemm_skinny_takes_x)
   int raster_group_m = 0, raster_no_xcd_remap = 0;  // tiled kernel, measurement only: tile rows per raster group (0 = the default, 4), XCD remap off (1), or on with a K split's workgroups in tile-by-tile order (2)
   int ablation = 0;  // tiled kernel, measurement only: leave out LDS reads (1), loads (2), MFMAs (4); results are then meaningless

@@ -293,3 +293,20 @@ def test_exceptions_in_the_binding_are_python_errors(hk):
     with FakeTensorMode(allow_non_fake_inputs=True), pytest.raises(RuntimeError):
         hk.quantize(x)
     assert torch.equal(layer(x), want) and torch.equal(hk.quantize(x)[0], p)
+
+
+@pytest.mark.parametrize("M,N,K,act", [(8192, 8192, 256, "gelu"), (4096, 16384, 384, "silu"), (8192, 9216, 128, "gelu")])
+def test_activations_on_outputs_past_the_last_level_cache(hk, M, N, K, act):
+    """From 256 MB of fp32 output on the choice counts an activation for bf16 and MXFP6 output only: other tiles, the same sums, so
+    the bf16 result is the rounded fp32 one and the MXFP6 one its quantisation, bit for bit."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, asc = hk.quantize(torch.randn(M, K, device="cuda", generator=g))
+    b, bsc = hk.quantize(torch.randn(N, K, device="cuda", generator=g) * 0.1, 2, hk.LAYOUT_TILE)
+    bias = torch.randn(N, device="cuda", generator=g)
+    C = torch.empty(M, N, dtype=torch.float32, device="cuda")
+    C16 = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    P, S = torch.empty(M, N // 4 * 3, dtype=torch.uint8, device="cuda"), torch.empty(M, N // 32, dtype=torch.uint8, device="cuda")
+    for out, kw in ((C, {}), (C16, {}), (P, dict(C_scale=S))):
+        hk.dispatch_micro(a, b, asc, bsc, out, 2, 2, hk.LAYOUT_ROW, hk.LAYOUT_TILE, bias=bias, activation=act, **kw)
+    want, want_s = hk.quantize(C)
+    assert torch.equal(C16, C.to(torch.bfloat16)) and torch.equal(P, want) and torch.equal(S, want_s)
