@@ -537,7 +537,7 @@ def dispatch_sweep(hk, torch, grid):
 def calibration_sweep(hk, torch):
     """The sweep behind the kernel choice's calibration table (hipkittensp_amd/csrc/dispatch_table.inc): every candidate of the
     choice, forced, on a grid of shapes x four layout pairs, timed on the GPU's side with weights rotating through 400 MB
-    (probe_time_us), twice (the better counts).  `python -m hipkittensp_amd.calibrate` turns the JSON this prints into the
+    (probe_time_us), twice (the better counts), near ties with a K split once more (retime_k_split_ties).  `python -m hipkittensp_amd.calibrate` turns the JSON this prints into the
     table: per shape and candidate, measured time / the time model's figure."""
     import ctypes
 
@@ -590,8 +590,54 @@ def calibration_sweep(hk, torch):
                 points.append(point)
         del row, tile
         torch.cuda.empty_cache()
-    return {"what": "calibration sweep of the kernel choice: measured microseconds per candidate (GPU-side timing, weights rotating through 400 MB)", "candidates": [c[0] for c in CANDIDATES],
+    retime_k_split_ties(hk, torch, points)
+    return {"what": "calibration sweep of the kernel choice: measured microseconds per candidate (GPU-side timing, weights rotating through 400 MB; near ties with a K split, from 30 us on, with the activations rotating too)", "candidates": [c[0] for c in CANDIDATES],
             "device": torch.cuda.get_device_name(0), "cus": torch.cuda.get_device_properties(0).multi_processor_count, "points": points}
+
+
+def retime_k_split_ties(hk, torch, points):
+    """Where a K split (the tiled kernel's or the block kernel's) is the best candidate of a calibration point or within 10 % of
+    it and the call takes 30 us or more, every candidate within 10 % is timed again as a program's calls: runs of 100 on
+    three sets of activations and outputs in turn.  probe_time_us has one A, which the L2s keep from launch to launch; a
+    program's next call has new activations, and the block kernel's K split pays more for them than the tiled kernel's (256 x 8192 x
+    28672, tile-major weights, one A / three: block 67.6 / 71.3 us, tiled 256-row 69.1 / 69.2)."""
+    tk = hk.tk_kernel
+    splits = {i for i, c in enumerate(CANDIDATES) if "k_split" in c[0]}
+    ties = []
+    for p in points:
+        known = {i: t for i, t in enumerate(p["measured_us"]) if t is not None}
+        best = min(known.values())
+        near = [i for i, t in known.items() if t <= 1.1 * best]
+        if best >= 30 and len(near) > 1 and splits & set(near):
+            ties.append((p, near))
+    g = torch.Generator(device="cuda")
+    g.manual_seed(1)
+    last, weights, sets = None, None, 0
+    for p, near in sorted(ties, key=lambda t: (t[0]["N"], t[0]["K"])):
+        M, N, K, la, lb = p["M"], p["N"], p["K"], p["layouts"] & 1, p["layouts"] >> 1
+        if last != (N, K):
+            weights = None
+            torch.cuda.empty_cache()
+            sets, row, tile = weight_sets(hk, torch, N, K, g)
+            weights, last = (row, tile), (N, K)
+        B, Bs = weights[lb]
+        acts = [hk.quantize(torch.randn(M, K, device="cuda", generator=g), 2, la) for _ in range(3)]
+        outs = [torch.empty(M, N, dtype=torch.bfloat16, device="cuda") for _ in range(3)]
+
+        def us(cand):
+            prev = tk.set_kernel(CANDIDATES[cand][1]), tk.set_k_split(CANDIDATES[cand][2])
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            for i in range(110):
+                if i == 10:
+                    start.record()
+                tk.dispatch_micro(acts[i % 3][0], B[i % sets], acts[i % 3][1], Bs[i % sets], outs[i % 3], 2, 2, la, lb)
+            end.record()
+            end.synchronize()
+            tk.set_kernel(prev[0]), tk.set_k_split(prev[1])
+            return start.elapsed_time(end) * 10
+        times = [[us(cand) for cand in near] for _ in range(3)]
+        for j, cand in enumerate(near):
+            p["measured_us"][cand] = round(sorted(t[j] for t in times)[1], 2)
 
 
 def source_hash(kernel):

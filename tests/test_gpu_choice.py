@@ -1,0 +1,50 @@
+"""The kernel choice between K splits and their neighbours, timed as a program's calls: new activations and another layer's weights every
+time."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hk():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import hipkittensp_amd as m
+
+    return m
+
+
+@pytest.mark.parametrize("M,N,K,la,lb", [(256, 8192, 28672, 0, 1), (320, 4096, 24576, 0, 1), (192, 7168, 20480, 0, 1), (768, 3072, 12288, 1, 0), (2048, 4096, 8192, 1, 0)])
+def test_choice_with_new_activations_per_call(hk, M, N, K, la, lb):
+    """Within 4 % of the best forced kernel (runs of one form differ by up to 2 %; a calibration with one set of activations for
+    all its launches chose a kernel 5 to 10 % behind at the second shape and 3 % at the first)."""
+    tk = hk.tk_kernel
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    acts = [hk.quantize(torch.randn(M, K, device="cuda", generator=g), 2, la) for _ in range(3)]
+    b = hk.quantize(torch.randn(N, K, device="cuda", generator=g) * 0.02, 2, lb)
+    weights = [b] + [(b[0].clone(), b[1].clone()) for _ in range(min(15, 400_000_000 // b[0].numel()))]
+    outs = [torch.empty(M, N, dtype=torch.bfloat16, device="cuda") for _ in range(3)]
+
+    def us(kernel, k_split):
+        prev = tk.set_kernel(kernel), tk.set_k_split(k_split)
+        try:
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            for i in range(110):
+                if i == 10:
+                    start.record()
+                (a, asc), (w, ws) = acts[i % 3], weights[i % len(weights)]
+                tk.dispatch_micro(a, w, asc, ws, outs[i % 3], 2, 2, la, lb)
+            end.record()
+            end.synchronize()
+        finally:
+            tk.set_kernel(prev[0]), tk.set_k_split(prev[1])
+        return start.elapsed_time(end) * 10
+
+    forced = [(k, s) for k in (tk.KERNEL_TILED_256, tk.KERNEL_TILED_128, tk.KERNEL_BLOCK) for s in (1, -1)] + [(tk.KERNEL_BLOCK_WIDE, 0)]
+    ratios = []
+    for _ in range(3):
+        ratios.append(us(tk.KERNEL_AUTO, 0) / min(us(*f) for f in forced))
+        if ratios[-1] <= 1.04:
+            break
+    assert min(ratios) <= 1.04, ratios
