@@ -54,7 +54,6 @@ class MXFP6Linear(torch.nn.Module):
                  activation: str | None = None):
         super().__init__()
         self.activation = activation or "none"
-        self._act = tk_kernel._ACTS.get(self.activation, -1)
         if bias is not None and (bias.dim() != 1 or bias.shape[0] != weight.shape[0]):
             raise RuntimeError("bias: expected [out_features]")
         self.register_buffer("bias", None if bias is None else bias.detach().to(torch.float32 if bias.dtype != torch.bfloat16 else torch.bfloat16).contiguous())
@@ -69,7 +68,8 @@ class MXFP6Linear(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not torch.compiler.is_compiling():  # one native call; None: not the usual case
-            y = tk_kernel._native().linear(x, self.weight_packed, self.weight_scale, self.bias, self.fmt_x, self.fmt_w, self.layout_w, self._act)
+            act = tk_kernel._ACTS.get(self.activation, -1) if type(self.activation) is str else -1
+            y = tk_kernel._native().linear(x, self.weight_packed, self.weight_scale, self.bias, self.fmt_x, self.fmt_w, self.layout_w, act)
             if y is not None:
                 return y
         # the input tile-major too from 64 rows on (a whole number of 32-row tiles): the tiled and block kernels then need

@@ -310,3 +310,21 @@ def test_activations_on_outputs_past_the_last_level_cache(hk, M, N, K, act):
         hk.dispatch_micro(a, b, asc, bsc, out, 2, 2, hk.LAYOUT_ROW, hk.LAYOUT_TILE, bias=bias, activation=act, **kw)
     want, want_s = hk.quantize(C)
     assert torch.equal(C16, C.to(torch.bfloat16)) and torch.equal(P, want) and torch.equal(S, want_s)
+
+
+def test_activation_is_read_per_call(hk):
+    """A layer's activation may be set after it was made (or come from a module saved without any other state of it); what is no name
+    of one is refused."""
+    from hipkittensp_amd.torch_op import MXFP6Linear
+
+    g = torch.Generator(device="cuda").manual_seed(6)
+    layer = MXFP6Linear(torch.randn(64, 512, device="cuda", generator=g) * 0.02)
+    for M in (3, 8):
+        x = torch.randn(M, 512, device="cuda", generator=g).to(torch.bfloat16)
+        for act in ("none", "relu", "gelu", "silu"):
+            layer.activation = act
+            assert torch.equal(layer(x), steps(hk, layer, x))
+        for act in (None, 1, "tanh"):
+            layer.activation = act
+            with pytest.raises((RuntimeError, TypeError, KeyError, ValueError)):
+                layer(x)
