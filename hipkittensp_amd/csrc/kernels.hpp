@@ -37,12 +37,13 @@ inline bool operands_aligned16(const GemmArgs& g) {
   return (((uintptr_t)g.A | (uintptr_t)g.B | (uintptr_t)g.As | (uintptr_t)g.Bs) & 15) == 0;
 }
 
-// Streams of this many bytes and more are read with the non-temporal bit: half of the 256 MB last-level cache, so that little of
-// the stream would be found there by the next read.  us, plain / non-temporal, weights of 184 MB: ring kernel at 16 x 8192 x 28672
-// 36.5 / 33.6 (tile-major 35.0 / 31.7), 64 rows 41.8 / 39.7 (40.0 / 38.1); skinny kernel at 16 rows 36.7 / 34.3 (33.9 / 31.1);
-// quantiser, 8192 x 28672 fp32 in and packed out: 214 / 185.  A smaller stream may stay in that cache from one call to the next, where the bit
-// costs more than it gives: skinny kernel, 32 x 4096 x 14336 (46 MB), weights found in the cache 11.8 / 14.5, from memory
-// 15.5 / 15.1.
+// Weights (and the quantiser's output) of this many bytes and more are read (written) with the non-temporal bit: half of the 256 MB
+// last-level cache, so that with the activations and the outputs little of them would be found there by the next read.  us, plain /
+// non-temporal, N = 8192, tile-major weights, in turn from 640 MB of them (a program's layers): skinny kernel, 16 rows, 60 MB
+// 15.3 / 14.3, 120 MB 25.7 / 23.8, 144 MB 30.2 / 27.5, 168 MB 33.8 / 31.0; ring kernel, 64 rows, 20.9 / 21.2, 33.1 / 30.5, 37.9 / 34.2, 42.3 /
+// 38.2.  The same weights again in every call, which stay in that cache in part or, below the line, as a whole: skinny 13.2 / 12.0, 21.8 /
+// 22.4, 25.2 / 26.2, 28.7 / 30.0; ring 19.0 / 19.6, 28.0 / 30.0, 31.8 / 33.6, 34.9 / 37.6.  (A first pass over weights not read before, 64 rows, is the same
+// either way.)
 constexpr size_t kStreamBytes = (size_t)128 << 20;
 
 // ---- kernel choice (dispatch.hip): candidates of the automatic path, a time model per candidate, a calibration table

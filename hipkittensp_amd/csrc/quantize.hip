@@ -25,6 +25,10 @@ namespace mxfp6 {
 // read-only stream 6.05) with five workgroups per CU that each took many chunks in turn, the next one's loads under the
 // stores; one chunk per wave and as many workgroups as that takes, so that the CUs' scheduler fills every gap: 214; past the last-level
 // cache the input read and the output written with the non-temporal bit: 185 (6.1 TB/s; each alone 196 and 205).
+// The input only from the size of that cache on: below it the bit gains nothing on an input from memory and loses where the program has
+// just written it (us, plain / non-temporal, an input from memory: 128 MB of fp32 28.1 / 28.1, 192 MB 40.4 / 40.4, 256 MB 55.1 / 52.5, 128 MB of
+// bf16 30.2 / 31.9; one in the cache 24.3 / 27.0, 35.1 / 40.4, 54.6 / 52.5, 28.9 / 31.9).
+constexpr size_t kCacheBytes = (size_t)256 << 20;  // last-level cache
 constexpr int kQWaves = 4;  // waves per workgroup; a wave fetches 64 blocks at a time (8 KB of fp32, 4 KB of bf16)
 
 
@@ -143,7 +147,7 @@ hipError_t launch_quantize(const void* X, int x_bf16, uint8_t* packed, uint8_t* 
   if (nblocks == 0) return hipSuccess;
   const long nchunks = layout ? (long)((rows + 15) / 16) * (K / 128) : (nblocks + 63) / 64, want = (nchunks + kQWaves - 1) / kQWaves;
   const unsigned grid = (unsigned)(want < (1L << 30) ? want : 1L << 30);
-  const int stream_in = (size_t)rows * K * (x_bf16 ? 2 : 4) >= kStreamBytes, stream_out = (size_t)rows * (K / 4 * 3) >= kStreamBytes;
+  const int stream_in = (size_t)rows * K * (x_bf16 ? 2 : 4) >= kCacheBytes, stream_out = (size_t)rows * (K / 4 * 3) >= kStreamBytes;
 #define MXFP6_Q(FMT, T) quantize_kernel<FMT, T><<<grid, kQWaves * 64, 0, s>>>((const T*)X, packed, scales, nblocks, K / 32, layout, rows, stream_in, stream_out)
   if (fmt == 2) { if (x_bf16) MXFP6_Q(2, uint16_t); else MXFP6_Q(2, float); }
   else { if (x_bf16) MXFP6_Q(3, uint16_t); else MXFP6_Q(3, float); }

@@ -371,3 +371,17 @@ def test_a_layer_that_asks_twice_for_its_kernel_remembers_both_answers(hk):
     x = torch.randn(4, 512, device="cuda", generator=g).to(torch.bfloat16)
     one, two = us_per_call(lambda: layer(x)), us_per_call(lambda: steps(hk, layer, x))
     assert one <= 1.2 * two + 0.5
+
+
+@pytest.mark.parametrize("rows,dtype,bound", [(6144, torch.float32, 2.0), (8192, torch.bfloat16, 1.97)])
+def test_quantiser_reads_an_input_that_is_in_the_cache_from_there(hk, rows, dtype, bound):
+    """An input below the size of the last-level cache, quantised again and again, against one of half its rows: 35.1 us against 18.9 for 192
+    MB of fp32 and 28.9 against 15.5 for 128 MB of bf16 (a ratio of 1.86 each), 40.4 and 31.9 (2.14 and 2.06) when it is read past that cache."""
+    x = torch.randn(rows, 8192, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1)).to(dtype)
+    half = x[:rows // 2].contiguous()
+    ratios = []
+    for _ in range(3):
+        ratios.append(us_per_call(lambda: hk.quantize(x, 2, hk.LAYOUT_TILE), 60) / us_per_call(lambda: hk.quantize(half, 2, hk.LAYOUT_TILE), 60))
+        if ratios[-1] <= bound:
+            break
+    assert min(ratios) <= bound, ratios
