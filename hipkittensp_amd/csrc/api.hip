@@ -63,13 +63,15 @@ bool stream_is_capturing(hipStream_t s) {
 
 // kind 0: pre-pass copies, kind 1: fp32 result of mxfp6_gemm_fused_fp6, kind 2: partial sums of a K split, kind 3: arrival
 // counters of the ring kernel's K split (zeroed when allocated; the kernels leave them zero), kind 4: packed activations of
-// mxfp6_linear.
+// mxfp6_linear (never under capture: a graph's activations live in its own memory plan, since graphs captured on one stream may be
+// replayed side by side on others).
 // nullptr: no workspace (capture without one, table full of pinned entries, out of memory).
 uint8_t* stream_workspace(hipStream_t s, int kind, size_t bytes, bool zeroed = false) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
   std::lock_guard<std::mutex> lock(g_sws_mutex);
   const bool capturing = stream_is_capturing(s);
+  if (capturing && kind == 4) return nullptr;
   auto it = g_sws.find({dev, s, kind});
   if (it != g_sws.end() && it->second.bytes >= bytes) {
     it->second.used = ++g_sws_clock;
@@ -443,8 +445,6 @@ int mxfp6_linear(const void* X, int x_bf16, const void* W, const void* Ws, void*
   const int layout_x = M >= 64 && K % 128 == 0 && (M % 32 == 0 || !forced_row) ? MXFP6_LAYOUT_TILE : MXFP6_LAYOUT_ROW;
   const size_t rows = ((size_t)M + 31) & ~(size_t)31;
   const size_t nx = (rows * (K / 32) * 24 + 255) & ~(size_t)255, ns = rows * ((K + 511) / 512) * 16;
-  // A graph's activations live in its own memory plan: graphs captured on one stream may be replayed side by side on others
-  if (K > 0 && stream_is_capturing(s)) return MXFP6_EWORKSPACE;
   std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
   uint8_t* xp = K > 0 ? stream_workspace(s, 4, nx + ns) : nullptr;
   if (K > 0) {
