@@ -146,7 +146,8 @@ hipError_t launch_quantize(const void* X, int x_bf16, uint8_t* packed, uint8_t* 
   const long nblocks = (long)rows * (K / 32);
   if (nblocks == 0) return hipSuccess;
   const long nchunks = layout ? (long)((rows + 15) / 16) * (K / 128) : (nblocks + 63) / 64, want = (nchunks + kQWaves - 1) / kQWaves;
-  const unsigned grid = (unsigned)(want < (1L << 30) ? want : 1L << 30);
+  const long most = 0xffffffffL / (kQWaves * 64);  // a launch has less than 2^32 work-items; the chunks past them are the grid's next round
+  const unsigned grid = (unsigned)(want < most ? want : most);
   const int stream_in = (size_t)rows * K * (x_bf16 ? 2 : 4) >= kCacheBytes, stream_out = (size_t)rows * (K / 4 * 3) >= kStreamBytes;
 #define MXFP6_Q(FMT, T) quantize_kernel<FMT, T><<<grid, kQWaves * 64, 0, s>>>((const T*)X, packed, scales, nblocks, K / 32, layout, rows, stream_in, stream_out)
   if (fmt == 2) { if (x_bf16) MXFP6_Q(2, uint16_t); else MXFP6_Q(2, float); }
