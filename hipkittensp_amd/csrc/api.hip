@@ -2,8 +2,9 @@
 // kernel selection.  Nothing here synchronises the device.  Allocations, all from the stream-ordered allocator on the
 // caller's stream and all kept per (device, stream) until mxfp6_release_workspaces(): the workspace of the re-layout
 // pre-pass (relayout_then_tiled; mxfp6_set_relayout(0) switches it off), the fp32 workspace of mxfp6_gemm_fused_fp6
-// on shapes the tiled kernel does not run, the partial sums of the tiled and the block kernel's K split (plan_ksplit,
-// plan_block_ksplit: one workspace, shared), and the K-split workspace of the skinny kernel (gemm_skinny.hip).  mxfp6_gemm_noalloc allocates nothing.
+// on shapes that the skinny, ring, ragged and generic kernels run, the packed activations of mxfp6_linear (not under capture), the
+// partial sums of the tiled, block and ring kernels' K splits (apply_choice, apply_ragged: one workspace, shared) with the ring
+// kernel's arrival counters, and the K-split workspace of the skinny kernel (gemm_skinny.hip).  mxfp6_gemm_noalloc allocates nothing.
 #include "../../include/mxfp6_gemm.h"
 #ifdef MXFP6_PROBES
 #include "../../include/mxfp6_probes.h"

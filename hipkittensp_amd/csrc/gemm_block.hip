@@ -8,12 +8,14 @@
 // K-tile: 8 MFMAs per K-tile) and keeps two sets of fragment registers: while the MFMAs of K-tile k run on one set, the
 // LDS reads of K-tile k+1 fill the other and the direct loads of K-tile k+3 go out; one barrier per K-tile.  48 KB of LDS
 // reads per K-tile and workgroup (the 8-wave kernel's 128 x 128 shape: 72 KB).  80 KB of LDS: two workgroups per CU,
-// one's waits are the other's work.
+// one's waits are the other's work.  That is the ring of three slots of one K-tile, described below; where a CU gets one
+// workgroup anyway, or both operands are row-major, the ring is three slots of two K-tiles each (PAIR below, block_stages), and
+// tiles of 128 x 256 with eight waves have four slots of one.
 //
 // Same operand formats, LDS image, lane mapping and raster as the tiled kernel (common.hpp, gemm_tiled.hip): row-major
 // or tile-major operands and scales, any M and N (edge tiles: rows past M or N lie beyond the end of their buffer
 // resource and read as zeros, stores are predicated), K % 128 == 0, bf16 or fp32 output, fused scales / bias / activation
-// (separate instantiations).
+// (separate instantiations); fp6 output; any size and alignment in instantiations of their own (RAGGED below).
 //   ring: three slots of 24 KB (A's 128 rows x 96 bytes, then B's); K-tile k lives in slot k % 3
 //   scales: the 16 bytes a row has for four K-tiles, two buffers of (128 + 128) rows x 16 bytes, group g in buffer g % 2
 //   step k: loads of K-tile k+3 into the slot K-tile k has left (its fragments are in registers since step k-1), LDS
@@ -608,7 +610,7 @@ int cu_count_of_device() {
 // 16.8).  Beyond: PAIR where its fewer line requests outweigh the second workgroup, with both operands row-major from K = 4096 on
 // (2048 x 4096 x 4096 49.5 / 43.8, 1536 x 4096 x 4096 41.2 / 41.1, 640 x 8192 x 2048 23.6 / 25.1), with one from 8192 on (1024 x 8192 x 8192
 // 70.1 / 64.9, 256 x 28672 x 8192 81.0 / 73.0, 2048 x 4096 x 4096 39.2 / 40.3), with none never (31.5 / 36.4).
-// stages = 3 or 6 forces one (measurement).
+// (launch's and launch_fp6's `stages` = 3 or 6 forces one, for measurement.)
 int block_stages(const GemmArgs& g, int grid, int cus) {
   const int row_major = !g.layout_a + !g.layout_b;
   const int min_k = grid <= cus ? (row_major ? 1025 : 2049) : row_major == 2 ? 4096 : row_major == 1 ? 8192 : 0x7fffffff;

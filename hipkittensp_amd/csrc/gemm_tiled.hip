@@ -742,8 +742,8 @@ int tiled_grid_size(const GemmArgs& g, int tiles, int per_cu) {
   return tiles < cus ? tiles : cus;
 }
 
-// Sum of a K split's partial sums (partial_offset), in share order, with the epilogue: a wave adds one 32 x 32 tile of C, all
-// loads of up to eight shares in flight at once, and stores it as the GEMM kernels do (bf16: lanes l and l + 32 trade halves,
+// Sum of a K split's partial sums (partial_offset), in share order, with the epilogue: a wave adds one 32 x 32 tile of C, the
+// loads of up to four shares (the first five) in flight at once, and stores it as the GEMM kernels do (bf16: lanes l and l + 32 trade halves,
 // 16 bytes per lane).
 // T = uint8_t: C re-quantised to MXFP6 along N (N % 32 == 0).  Lanes l and l + 32 hold a block's halves; both get all of it, and one stores the 24
 // bytes, the other the scale.

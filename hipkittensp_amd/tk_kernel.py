@@ -46,7 +46,7 @@ KERNEL_TILED_128x128 = 17  # tiled kernel with output tiles of 128 x 128
 KERNEL_SKINNY_64 = 19  # skinny kernel with 64 rows of B per workgroup (two tiles of B against every fragment of A), K unsplit
 KERNEL_SKINNY_64_SPLIT = (20, 21)  # the same with the K range split between 2 / 4 workgroups
 KERNEL_BLOCK = 22  # 128 x 128 tiles, four waves in step: one barrier per K-tile, fragments double-buffered in registers
-KERNEL_BLOCK_3SLOTS, KERNEL_BLOCK_6SLOTS = 23, 24  # the same with its operand ring forced to three / six slots
+KERNEL_BLOCK_3SLOTS, KERNEL_BLOCK_6SLOTS = 23, 24  # the same with its operand ring forced to three K-tiles / six K-tiles (three slots of two)
 KERNEL_BLOCK_WIDE = 26  # the block kernel with tiles of 128 x 256 and eight waves
 KERNEL_RING = 28  # batched decode: a private stream of B per wave, A through a flag-guarded ring, no barrier per K-tile
 KERNEL_TILED_4WAVE = 18  # the 4-wave interleaved schedule of the tiled kernel (measurement: never chosen automatically)

@@ -33,8 +33,8 @@
  *     shares * 4 M N bytes of partial sums (tiles times shares never exceed the CUs: at most 64 MB, 256 tiles of
  *     256 x 256 fp32), one workspace for the three kernels, and for the ring kernel one counter per output tile.
  * While `hip_stream` is being captured nothing is allocated: the pre-pass and the K splits are left out
- * (same results up to the order of fp32 sums, other kernels) unless their workspace exists already, and mxfp6_gemm_fused_fp6 returns
- * hipErrorStreamCaptureUnsupported where it would need a new one.  mxfp6_linear records no packed activations
+ * (same results up to the order of fp32 sums, other kernels) unless their workspace exists already, and mxfp6_gemm_fused_fp6 runs
+ * a kernel that needs none or, on shapes and alignments that no such kernel takes, returns hipErrorStreamCaptureUnsupported.  mxfp6_linear records no packed activations
  * of its own in a graph: where it needs a workspace for them it returns MXFP6_EWORKSPACE under capture (quantise into the
  * graph's own memory and call the GEMM).  A workspace that a capture did use is recorded in the
  * graph: the library never frees such a block again (when a later call needs a larger one, or at
@@ -264,8 +264,9 @@ int mxfp6_gemm_fused(const void *A_packed, const void *B_packed, const void *A_s
  * exactly mxfp6_quantize(fmt_c) applied to the fp32 result of mxfp6_gemm_fused(out_f32 = 1), without that result
  * ever reaching memory (0.78 instead of 2 or 4 bytes per output element).  N % 32 == 0; C_packed 8-byte aligned.
  * The LDS-tiled kernel, the block kernel and the reduction of their K splits quantise their sums themselves; shapes that run
- * on another kernel (few rows of A, where C is small; ragged K) go through an fp32 workspace taken from and returned to the stream-ordered allocator on
- * hip_stream, and are refused under stream capture (hipErrorStreamCaptureUnsupported).
+ * on another kernel (few rows of A, where C is small; ragged K) go through the stream's fp32 workspace.  Under capture without it
+ * they run on the tiled or the block kernel, and those that neither takes (ragged K, operands off 16 bytes) are refused
+ * (hipErrorStreamCaptureUnsupported).
  * No counterpart in the reference.
  */
 int mxfp6_gemm_fused_fp6(const void *A_packed, const void *B_packed, const void *A_scale, const void *B_scale,
@@ -335,9 +336,10 @@ int mxfp6_allow_e3m2_pair(int allow);
 int mxfp6_set_k_split(int shares);
 
 /* The kernel the automatic path takes for a problem of this shape on the current device (e2m3 x e2m3, bf16 output, no fused
- * epilogue, 16-byte aligned tensors): a code of mxfp6_set_kernel, or 25 / 27 for the tiled / the block kernel with its
- * K split between workgroups; negative = error code.  layouts: bit 0 set = A tile-major, bit 1 set = B tile-major.
- * Reads the thread's mxfp6_set_k_split setting; launches nothing. */
+ * epilogue, 16-byte aligned tensors): a code of mxfp6_set_kernel, or 25 / 27 for the tiled / the block kernel with its K split
+ * between workgroups; negative = error code.  An activation's time counts in the choice, so that a fused call with one may run on
+ * another kernel than is named here, and so may one with MXFP6 output, which the 128 x 128 tiles of the tiled kernel do not have.
+ * layouts: bit 0 set = A tile-major, bit 1 set = B tile-major.  Reads the thread's mxfp6_set_k_split setting; launches nothing. */
 int mxfp6_kernel_choice(int M, int N, int K, int layouts);
 
 /* Human-readable text for a return code of this library (never NULL). */

@@ -1191,9 +1191,9 @@ def test_gpu_quantiser_bit_exact(hk, fmt, kind):
 
 
 @pytest.mark.parametrize("M,N,K", [(256, 256, 512), (16, 64, 1024), (64, 96, 1024)])
-def test_operands_not_16_byte_aligned_run_on_the_generic_kernel(hk, M, N, K):
+def test_operands_not_16_byte_aligned_give_the_generic_kernels_result(hk, M, N, K):
     """The fast kernels fetch 16 bytes per lane and need 16-byte aligned operands and scales; pointers that are only
-    4-byte aligned are accepted and served by the generic kernel with the same result, and a forced fast kernel refuses
+    4-byte aligned are accepted and served by the block kernel's instantiations for any alignment, with the generic kernel's result, and a forced fast kernel refuses
     them instead of issuing misaligned loads."""
     ap, asc, bp, bsc = operands(M, N, K, 2, 2, seed=M + N)
     ref = gemm(hk, ap, bp, asc, bsc, kernel=1)
