@@ -503,6 +503,7 @@ def dispatch_sweep(hk, torch, grid):
     g = torch.Generator(device="cuda")
     g.manual_seed(1)
     for N, K in shapes:
+        print(f"N = {N}, K = {K}", file=sys.stderr, flush=True)
         sets, row, tile = weight_sets(hk, torch, N, K, g)
         for M in rows_of_a:
             a, asc = hk.quantize(torch.randn(M, K, device="cuda", generator=g), 2)
