@@ -482,13 +482,13 @@ def dispatch_sweep(hk, torch, grid):
     from hipkittensp_amd import _lib
 
     tk, P = hk.tk_kernel, _lib.probes()
-    if grid == "offgrid":  # none of these (N, K) pairs and none of these row counts is in the calibration table
-        shapes = [(7168, 7168), (3584, 18944), (18944, 3584), (9216, 4608), (27648, 5120), (1792, 14336), (22016, 4096), (5632, 22528),
-                  (13312, 6656), (36864, 3072), (2304, 24576), (15360, 10240)]
+    if grid == "offgrid":  # none of these (N, K) pairs is in the calibration table
+        shapes = [(7680, 7680), (3584, 18944), (17920, 3584), (9216, 4608), (26624, 5632), (1792, 16384), (22016, 4096), (5632, 22528),
+                  (13312, 6656), (35840, 3072), (2304, 24576), (15360, 10240)]
         rows_of_a = [20, 56, 72, 144, 208, 288, 416, 576, 832, 1152, 1792, 2560]
     elif grid == "offgrid2":  # a second held-out set, never used to tune anything
-        shapes = [(5120, 5120), (9216, 9216), (14336, 7168), (3328, 16640), (25600, 5632), (2816, 11264), (45056, 3584), (6656, 13312),
-                  (19456, 6144), (1280, 28160), (10752, 10752), (30720, 2560)]
+        shapes = [(5120, 5120), (9728, 9728), (14336, 7168), (3584, 15360), (25600, 5632), (2816, 11264), (43008, 3584), (6656, 13312),
+                  (19456, 6144), (1280, 28160), (10752, 10752), (29696, 2560)]
         rows_of_a = [28, 36, 88, 104, 176, 240, 352, 480, 704, 960, 1280, 2304]
     elif grid == "full":
         shapes = [(8192, 8192), (4096, 14336), (28672, 8192), (28672, 4096), (24576, 8192), (40960, 8192), (57344, 8192), (128256, 4096),
@@ -535,6 +535,20 @@ def dispatch_sweep(hk, torch, grid):
             "behind_by_more_than_8_percent": behind, "per_shape": per_shape}
 
 
+# (N, K) pairs and row counts of the calibration sweep.  The second set, with row counts between the first one's: widths at which
+# the first alone let the choice slip by 5 to 34 % (28 x 9216 x 9216 23.5 us instead of 17.6, 2304 x 9216 x 9216 208 instead of 163)
+CALIBRATION_ROWS = [1, 8, 12, 16, 24, 32, 40, 48, 64, 80, 96, 112, 128, 160, 192, 224, 256, 320, 384, 448, 512, 640, 768, 896, 1024, 1536, 2048, 3072, 4096, 8192]
+CALIBRATION = [
+    ([(8192, 8192), (4096, 14336), (28672, 8192), (28672, 4096), (24576, 8192), (40960, 8192), (57344, 8192), (128256, 4096), (8192, 28672), (2048, 8192), (5120, 16384),
+      (10240, 8192), (1024, 16384), (14336, 4096), (32000, 4096), (4096, 4096), (16384, 16384), (2048, 28672), (11008, 4096), (4096, 11008), (2048, 2048), (512, 8192), (8192, 1024),
+      (1024, 32768), (2048, 16384), (4096, 8192), (4096, 24576), (8192, 4096), (8192, 14336), (16384, 4096), (16384, 8192), (65536, 2048), (3072, 3072), (6144, 4096), (1024, 4096),
+      (12288, 12288), (2048, 5120), (24576, 2048), (73728, 4096),
+      (6144, 6144), (12288, 6144), (3072, 12288), (20480, 5120), (18432, 9216), (7168, 20480), (49152, 4096), (2560, 10240), (13824, 5120), (5120, 13824), (100352, 2048), (1536, 32768)], CALIBRATION_ROWS),
+    ([(9216, 9216), (7168, 7168), (3328, 16640), (36864, 3072), (45056, 3584), (1792, 14336), (18944, 3584), (30720, 2560), (27648, 5120)],
+     sorted(CALIBRATION_ROWS + [28, 56, 104, 176, 208, 288, 576, 832, 1280, 2304])),
+]
+
+
 def calibration_sweep(hk, torch):
     """The sweep behind the kernel choice's calibration table (hipkittensp_amd/csrc/dispatch_table.inc): every candidate of the
     choice, forced, on a grid of shapes x four layout pairs, timed on the GPU's side with weights rotating through 400 MB
@@ -545,17 +559,10 @@ def calibration_sweep(hk, torch):
     from hipkittensp_amd import _lib
 
     tk, P = hk.tk_kernel, _lib.probes()
-    shapes = [(8192, 8192), (4096, 14336), (28672, 8192), (28672, 4096), (24576, 8192), (40960, 8192), (57344, 8192), (128256, 4096), (8192, 28672), (2048, 8192), (5120, 16384),
-              (10240, 8192), (1024, 16384), (14336, 4096), (32000, 4096), (4096, 4096), (16384, 16384), (2048, 28672), (11008, 4096), (4096, 11008), (2048, 2048), (512, 8192), (8192, 1024),
-              (1024, 32768), (2048, 16384), (4096, 8192), (4096, 24576), (8192, 4096), (8192, 14336), (16384, 4096), (16384, 8192), (65536, 2048), (3072, 3072), (6144, 4096), (1024, 4096),
-              (12288, 12288), (2048, 5120), (24576, 2048), (73728, 4096),
-              (6144, 6144), (12288, 6144), (3072, 12288), (20480, 5120), (18432, 9216), (7168, 20480), (49152, 4096), (2560, 10240), (13824, 5120), (5120, 13824), (100352, 2048), (1536, 32768)]
-    rows_of_a = [1, 8, 12, 16, 24, 32, 40, 48, 64, 80, 96, 112, 128, 160, 192, 224, 256, 320, 384, 448, 512, 640, 768, 896, 1024, 1536, 2048, 3072, 4096, 8192]
-
     points = []
     g = torch.Generator(device="cuda")
     g.manual_seed(1)
-    for N, K in shapes:
+    for N, K, rows_of_a in [(*nk, rows) for shapes, rows in CALIBRATION for nk in shapes]:
         print(f"N = {N}, K = {K}", file=sys.stderr, flush=True)
         sets, row, tile = weight_sets(hk, torch, N, K, g)
         for M in rows_of_a:

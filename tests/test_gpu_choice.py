@@ -15,10 +15,8 @@ def hk():
     return m
 
 
-@pytest.mark.parametrize("M,N,K,la,lb", [(256, 8192, 28672, 0, 1), (320, 4096, 24576, 0, 1), (192, 7168, 20480, 0, 1), (768, 3072, 12288, 1, 0), (2048, 4096, 8192, 1, 0)])
-def test_choice_with_new_activations_per_call(hk, M, N, K, la, lb):
-    """Within 4 % of the best forced kernel (runs of one form differ by up to 2 %; a calibration with one set of activations for
-    all its launches chose a kernel 5 to 10 % behind at the second shape and 3 % at the first)."""
+def ratios_to_the_best_forced_kernel(hk, M, N, K, la, lb, bound):
+    """Up to three measurements, until one is within the bound."""
     tk = hk.tk_kernel
     g = torch.Generator(device="cuda").manual_seed(M + N)
     acts = [hk.quantize(torch.randn(M, K, device="cuda", generator=g), 2, la) for _ in range(3)]
@@ -42,9 +40,26 @@ def test_choice_with_new_activations_per_call(hk, M, N, K, la, lb):
         return start.elapsed_time(end) * 10
 
     forced = [(k, s) for k in (tk.KERNEL_TILED_256, tk.KERNEL_TILED_128, tk.KERNEL_BLOCK) for s in (1, -1)] + [(tk.KERNEL_BLOCK_WIDE, 0)]
+    if M <= 128:
+        forced += [(tk.KERNEL_SKINNY, 0), (tk.KERNEL_RING, 0)]
     ratios = []
     for _ in range(3):
         ratios.append(us(tk.KERNEL_AUTO, 0) / min(us(*f) for f in forced))
-        if ratios[-1] <= 1.04:
+        if ratios[-1] <= bound:
             break
+    return ratios
+
+
+@pytest.mark.parametrize("M,N,K,la,lb", [(256, 8192, 28672, 0, 1), (320, 4096, 24576, 0, 1), (192, 7168, 20480, 0, 1), (768, 3072, 12288, 1, 0), (2048, 4096, 8192, 1, 0)])
+def test_choice_with_new_activations_per_call(hk, M, N, K, la, lb):
+    """Within 4 % of the best forced kernel (runs of one form differ by up to 2 %; a calibration with one set of activations for
+    all its launches chose a kernel 5 to 10 % behind at the second shape and 3 % at the first)."""
+    ratios = ratios_to_the_best_forced_kernel(hk, M, N, K, la, lb, 1.04)
     assert min(ratios) <= 1.04, ratios
+
+
+@pytest.mark.parametrize("M,N,K,la,lb", [(28, 9216, 9216, 0, 1), (2304, 9216, 9216, 0, 0), (1280, 3328, 16640, 0, 1), (104, 45056, 3584, 0, 0)])
+def test_choice_at_widths_of_the_second_calibration_set(hk, M, N, K, la, lb):
+    """Within 8 %; from the first set alone the choice was 14 to 34 % behind here."""
+    ratios = ratios_to_the_best_forced_kernel(hk, M, N, K, la, lb, 1.08)
+    assert min(ratios) <= 1.08, ratios
