@@ -3,8 +3,8 @@
 // caller's stream and all kept per (device, stream) until mxfp6_release_workspaces(): the workspace of the re-layout
 // pre-pass (relayout_then_tiled; mxfp6_set_relayout(0) switches it off), the fp32 workspace of mxfp6_gemm_fused_fp6
 // on shapes that the skinny, ring, ragged and generic kernels run, the packed activations of mxfp6_linear (not under capture), the
-// partial sums of the tiled, block and ring kernels' K splits (apply_choice, apply_ragged: one workspace, shared) with the ring
-// kernel's arrival counters, and the K-split workspace of the skinny kernel (gemm_skinny.hip).  mxfp6_gemm_noalloc allocates nothing.
+// partial sums of the tiled, block, ring and slice kernels' K splits (apply_choice, apply_ragged: one workspace, shared) with the ring
+// and slice kernels' arrival counters, and the K-split workspace of the skinny kernel (gemm_skinny.hip).  mxfp6_gemm_noalloc allocates nothing.
 #include "../../include/mxfp6_gemm.h"
 #ifdef MXFP6_PROBES
 #include "../../include/mxfp6_probes.h"
@@ -29,9 +29,10 @@ thread_local int g_ksplit = 0;  // mxfp6_set_k_split: 0 = where it pays, -1 = wh
 thread_local uint32_t* g_clock_stamps = nullptr;  // mxfp6_probe_tiled_clock
 thread_local int g_raster_group_m = 0, g_raster_no_xcd = 0;  // mxfp6_probe_raster
 thread_local int g_ablation = 0;                              // mxfp6_probe_tiled_ablation
+thread_local int g_slice = 0;                                 // mxfp6_probe_slice: -1 = never, a plan = always
 thread_local int g_block = 1;                                 // mxfp6_probe_block: 0 keeps the block kernel out of the automatic choice
 #else
-constexpr int g_block = 1;
+constexpr int g_slice = 0, g_block = 1;
 #endif
 
 // Workspaces kept per (device, stream, kind): launches on one stream are ordered, so they can share one; it grows on
@@ -63,7 +64,7 @@ bool stream_is_capturing(hipStream_t s) {
 }
 
 // kind 0: pre-pass copies, kind 1: fp32 result of mxfp6_gemm_fused_fp6, kind 2: partial sums of a K split, kind 3: arrival
-// counters of the ring kernel's K split (zeroed when allocated; the kernels leave them zero), kind 4: packed activations of
+// counters of the ring and slice kernels' K splits (zeroed when allocated; the kernels leave them zero), kind 4: packed activations of
 // mxfp6_linear (never under capture: a graph's activations live in its own memory plan, since graphs captured on one stream may be
 // replayed side by side on others).
 // nullptr: no workspace (capture without one, table full of pinned entries, out of memory).
@@ -131,6 +132,7 @@ int choice_code(const mxfp6::KernelChoice& c) {
     case mxfp6::kCandTiledSplit256: case mxfp6::kCandTiledSplit128: return kChoiceTiledKsplit;
     case mxfp6::kCandBlockSplit: return kChoiceBlockKsplit;
     case mxfp6::kCandRing: return kChoiceRing;
+    case mxfp6::kCandSlice: return c.shares > 1 ? kChoiceBlockKsplit : kChoiceBlock;
     default: return kChoiceGeneric;
   }
 }
@@ -139,7 +141,8 @@ int choice_code(const mxfp6::KernelChoice& c) {
 // kernel's split (1 = never split): no kernel that needs a workspace, and the skinny kernel whenever a split is asked for.
 unsigned auto_mask(const mxfp6::GemmArgs& g, int force_split) {
   unsigned mask = ~0u;
-  if (!g_block || force_split) mask &= ~kBlockAll;
+  if (!g_block || force_split) mask &= ~(kBlockAll | 1u << mxfp6::kCandSlice);
+  if (g_slice < 0) mask &= ~(1u << mxfp6::kCandSlice);
   if (force_split || g.no_alloc) mask &= ~(kNeedsWorkspace | 1u << mxfp6::kCandRing);
   if (force_split > 1 && mxfp6::gemm_skinny_supports(g)) mask = 1u << mxfp6::kCandSkinny;
   return mask;
@@ -148,6 +151,7 @@ unsigned auto_mask(const mxfp6::GemmArgs& g, int force_split) {
 // The choice for a call: by the time model and the calibration table (dispatch.hip).  allow_split = false: what it is when a
 // K split's workspace is not to be had (a stream that is being captured, the allocator's refusal).
 mxfp6::KernelChoice auto_choice(const mxfp6::GemmArgs& g, int force_split, bool allow_split) {
+  if (g_slice > 0 && !force_split && mxfp6::gemm_slice_supports(g)) return {mxfp6::kCandSlice, g_slice >> 12, 0, 0.0, {g_slice & 15, g_slice >> 4 & 15, g_slice >> 8 & 15, g_slice >> 12}};
   if (g.K == 0) return {-1, 1, 0, 0.0};  // act(bias) everywhere: the generic kernel's K loop runs zero times
   return mxfp6::choose_kernel(g, g_ksplit, allow_split, auto_mask(g, force_split));
 }
@@ -174,6 +178,16 @@ bool apply_choice(mxfp6::GemmArgs& g, const mxfp6::KernelChoice& c, hipStream_t 
       uint8_t* pc = pp ? stream_workspace(s, 3, counters * sizeof(int), true) : nullptr;
       if (!pc) return false;
       g.ksplit = c.shares, g.ks_part = reinterpret_cast<float*>(pp), g.ks_counters = reinterpret_cast<int*>(pc);
+      return true;
+    }
+    case mxfp6::kCandSlice: {
+      if (c.shares <= 1) return true;
+      size_t part = 0, counters = 0;
+      mxfp6::slice_workspace(g, c.slice, &part, &counters);
+      uint8_t* pp = stream_workspace(s, 2, part);
+      uint8_t* pc = pp ? stream_workspace(s, 3, counters * sizeof(int), true) : nullptr;
+      if (!pc) return false;
+      g.ks_part = reinterpret_cast<float*>(pp), g.ks_counters = reinterpret_cast<int*>(pc);
       return true;
     }
     default: return true;
@@ -384,6 +398,7 @@ int gemm_common(const void* A, const void* B, const void* As, const void* Bs, vo
       case mxfp6::kCandBlock: case mxfp6::kCandBlockWide: case mxfp6::kCandBlockSplit: e = mxfp6::launch_gemm_block(g, s); break;
       case mxfp6::kCandSkinny: e = mxfp6::launch_gemm_skinny(g, s); break;
       case mxfp6::kCandRing: e = mxfp6::launch_gemm_ring(g, s); break;
+      case mxfp6::kCandSlice: e = mxfp6::launch_gemm_slice(g, c.slice, s); break;
       default: e = K != 0 && apply_ragged(g, s) ? mxfp6::launch_gemm_block(g, s) : mxfp6::launch_gemm_generic(g, s); break;
     }
   }
@@ -433,7 +448,8 @@ int mxfp6_linear(const void* X, int x_bf16, const void* W, const void* Ws, void*
   if (x_bf16 && K > 0 && g_force == 0) {
     mxfp6::GemmArgs g{(const uint8_t*)X, (const uint8_t*)W, (const uint8_t*)X, (const uint8_t*)Ws, C, M, N, K, fmt_x, fmt_w, false, 0, layout_w};
     g.X = X;
-    if (mxfp6::gemm_skinny_takes_x(g) && auto_choice(g, 0, true).cand == mxfp6::kCandSkinny) {
+    // (against the kernels that would need the quantiser's launch in front of them as well: the slice kernel does not count here)
+    if (mxfp6::gemm_skinny_takes_x(g) && mxfp6::choose_kernel(g, g_ksplit, true, auto_mask(g, 0) & ~(1u << mxfp6::kCandSlice)).cand == mxfp6::kCandSkinny) {
       g.ep = ep;
       const hipError_t e = mxfp6::launch_gemm_skinny(g, s);
       return e == hipSuccess ? MXFP6_OK : (int)e;
@@ -502,17 +518,19 @@ int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const voi
     // (the unsplit tiled kernel: C on 16 bytes, as ever; the others store fp6 8 bytes at a time)
     const bool tiled = (ch.cand == mxfp6::kCandTiled256 || ch.cand == mxfp6::kCandTiled128x256) && ((uintptr_t)C_packed & 15) == 0;
     mxfp6::GemmArgs t = g;
-    if (!(block || split || tiled) || !apply_choice(t, ch, s)) return false;
+    const bool slice = ch.cand == mxfp6::kCandSlice;
+    if (!(block || split || tiled || slice) || !apply_choice(t, ch, s)) return false;
     t.C = C_packed, t.f32out = false, t.C_scale = (uint8_t*)C_scale, t.fmt_c = fmt_c;
     if (force == 23 || force == 24) t.tile_rows = force == 23 ? 3 : 6;
-    if (block) e = mxfp6::launch_gemm_block(t, s);
+    if (slice) e = mxfp6::launch_gemm_slice(t, ch.slice, s);
+    else if (block) e = mxfp6::launch_gemm_block(t, s);
     else if (split || force != 0 || !relayout_then_tiled(t, s, e)) e = mxfp6::launch_gemm_tiled(t, s);
     return true;
   };
   hipError_t e = hipSuccess;
   if (run(c, e)) return e == hipSuccess ? MXFP6_OK : (int)e;
   // a split without its workspace (a stream under capture that has none): what the shape gets otherwise, as for the other outputs
-  if (c.cand == mxfp6::kCandTiledSplit256 || c.cand == mxfp6::kCandTiledSplit128 || c.cand == mxfp6::kCandBlockSplit) {
+  if (c.cand == mxfp6::kCandTiledSplit256 || c.cand == mxfp6::kCandTiledSplit128 || c.cand == mxfp6::kCandBlockSplit || c.cand == mxfp6::kCandSlice) {
     c = force == 0 ? choose(false) : mxfp6::choose_kernel(g, 1, false, 1u << mxfp6::kCandBlock);
     if (run(c, e)) return e == hipSuccess ? MXFP6_OK : (int)e;
   }
@@ -747,6 +765,12 @@ int mxfp6_probe_block(int enable) {
   return prev;
 }
 
+
+int mxfp6_probe_slice(int plan) {
+  const int prev = g_slice;
+  g_slice = plan;
+  return prev;
+}
 
 int mxfp6_probe_raster(int group_m, int xcd_remap) {
   if (group_m < 0 || group_m > 4096) return MXFP6_EINVAL_SHAPE;

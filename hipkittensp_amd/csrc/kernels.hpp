@@ -47,12 +47,17 @@ inline bool operands_aligned16(const GemmArgs& g) {
 constexpr size_t kStreamBytes = (size_t)128 << 20;
 
 // ---- kernel choice (dispatch.hip): candidates of the automatic path, a time model per candidate, a calibration table
-enum Candidate : int { kCandTiled256 = 0, kCandTiled128x256, kCandTiled128x128, kCandBlock, kCandBlockWide, kCandSkinny, kCandTiledSplit256, kCandTiledSplit128, kCandBlockSplit, kCandRing, kNumCandidates };
+enum Candidate : int { kCandTiled256 = 0, kCandTiled128x256, kCandTiled128x128, kCandBlock, kCandBlockWide, kCandSkinny, kCandTiledSplit256, kCandTiledSplit128, kCandBlockSplit, kCandRing, kNumCandidates,
+  kCandSlice = kNumCandidates };  // not calibrated: its own model against the best of the others (slice_plan)
+struct SlicePlan {  // small problems: tiles of 32 ta x 32 tb outputs, K dealt to `waves` waves and to `shares` workgroups (gemm_slice.hip)
+  int ta, tb, waves, shares;
+};
 struct KernelChoice {
   int cand;    // a Candidate, or -1: none of them takes the shape (ragged_shares says what does)
   int shares;  // K split: workgroups per output tile (1 = none)
   int rows;    // tiled kernel's split: rows of A per tile
   double us;   // modelled time x calibration factor
+  SlicePlan slice = {};
 };
 int device_cus();
 double candidate_model_us(const GemmArgs& g, int cand, int want_split, int cus, int* shares, int* rows);  // modelled microseconds; < 0: the candidate does not take the shape
@@ -73,6 +78,9 @@ hipError_t launch_ksplit_reduce(const GemmArgs& g, hipStream_t s);  // sums g.ks
 bool gemm_ring_supports(const GemmArgs& g);  // batched decode: private streams of B per wave, A through a flag-guarded ring (no barrier per K-tile)
 int ring_ksplit_plan(const GemmArgs& g, int want, size_t* part_bytes, size_t* counters);  // its K split for this problem (want: 0 = by shape, 1 = none, n = n shares): shares (1 = none), bytes of partial tiles, arrival counters
 hipError_t launch_gemm_ring(const GemmArgs& g, hipStream_t s);
+bool gemm_slice_supports(const GemmArgs& g);
+void slice_workspace(const GemmArgs& g, const SlicePlan& p, size_t* part_bytes, size_t* counters);  // of its K split (shares > 1): g.ks_part, g.ks_counters
+hipError_t launch_gemm_slice(const GemmArgs& g, const SlicePlan& p, hipStream_t s);  // without the workspace: unsplit
 bool gemm_mid_supports(const GemmArgs& g);
 hipError_t launch_gemm_mid(const GemmArgs& g, hipStream_t s);
 bool gemm_skinny_supports(const GemmArgs& g);

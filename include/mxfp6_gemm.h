@@ -327,7 +327,7 @@ int mxfp6_allow_e3m2_pair(int allow);
  * K split between workgroups (per calling thread; returns the previous setting).  Problems of few output tiles and long K
  * (up to a few hundred rows of A against a wide weight matrix) run with several workgroups per output tile, each over a
  * part of K.  The LDS-tiled and the block kernel's shares leave fp32 partial matrices in this stream's workspace and a
- * second small kernel adds them in share order and applies the epilogue; the ring kernel's shares leave partial tiles
+ * second small kernel adds them in share order and applies the epilogue; the ring and the slice kernel's shares leave partial tiles
  * there and the workgroup that arrives last at a tile adds them in share order.  Either way the result does not depend
  * on timing.  0 = where it pays (default), 1 = never, -1 = wherever the shape allows it, n > 1 = n workgroups per output
  * tile where the shape allows it, else unsplit.  No counterpart in the reference (its GEMMs are one workgroup per
@@ -337,7 +337,9 @@ int mxfp6_set_k_split(int shares);
 
 /* The kernel the automatic path takes for a problem of this shape on the current device (e2m3 x e2m3, bf16 output, no fused
  * epilogue, 16-byte aligned tensors): a code of mxfp6_set_kernel, or 25 / 27 for the tiled / the block kernel with its K split
- * between workgroups; negative = error code.  An activation's time counts in the choice, so that a fused call with one may run on
+ * between workgroups; negative = error code.  22 and 27 also stand for the slice kernel, unsplit and split, which small problems of any
+ * size and alignment get (tiles of 32 or 64 rows and columns, K dealt to the waves of a workgroup) and no mxfp6_set_kernel code forces.
+ * An activation's time counts in the choice, so that a fused call with one may run on
  * another kernel than is named here, and so may one with MXFP6 output, which the 128 x 128 tiles of the tiled kernel do not have.
  * layouts: bit 0 set = A tile-major, bit 1 set = B tile-major.  Reads the thread's mxfp6_set_k_split setting; launches nothing. */
 int mxfp6_kernel_choice(int M, int N, int K, int layouts);

@@ -92,6 +92,11 @@ int mxfp6_probe_candidate(int M, int N, int K, int layouts, int candidate, int c
  * so that the same call can be timed with and without it; returns the previous setting.  Default 1. */
 int mxfp6_probe_block(int enable);
 
+/* Measurement switch, per calling thread: -1 keeps the slice kernel out of the automatic choice, a plan
+ * (rows of A / 32) | (rows of B / 32) << 4 | waves << 8 | shares of K << 12 takes it for every call of the automatic path, 0 (the
+ * default) leaves it to the choice; returns the previous setting.  Plans that are not built fail with hipErrorInvalidValue. */
+int mxfp6_probe_slice(int plan);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,130 @@
+"""The slice kernel (tiles of 32 or 64 rows and columns, K dealt to waves and workgroups): every tile shape at the edges of its
+tiles and chunks against the CPU oracle, and the routes that lead to it.  Bound as for the other kernels: products and partial
+sums of these inputs are exact in fp32 up to the sum's own rounding, 1e-5 in the oracle's metric."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from hipkittensp_amd import _lib
+from oracle import c_oracle as co
+from oracle import mxfp6_oracle as o
+
+pytestmark = pytest.mark.gpu
+
+PLANS = [(1, 1, 4), (1, 1, 8), (1, 2, 4), (1, 2, 8), (2, 2, 6)]
+
+
+@pytest.fixture(scope="module")
+def hk():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import hipkittensp_amd as m
+
+    return m
+
+
+def at(a, off=0):
+    """`a` on the GPU at a pointer `off` bytes past 256-byte alignment, NaN bit patterns (0xff) around it."""
+    raw = np.ascontiguousarray(a).view(np.uint8).reshape(-1)
+    buf = torch.full((raw.size + 1024,), 255, dtype=torch.uint8, device="cuda")
+    buf[256 + off:256 + off + raw.size] = torch.from_numpy(raw).cuda()
+    return buf[256 + off:256 + off + raw.size]
+
+
+def forced(plan, shares, ops, M, N, K, fa=2, fb=2, la=0, lb=0, f32=1, off_c=0):
+    """One call with the plan forced (the measurement build); C between guard values."""
+    P = _lib.probes()
+    P.mxfp6_probe_slice.argtypes, P.mxfp6_probe_slice.restype = [ctypes.c_int], ctypes.c_int
+    guard = torch.full((M * N + 64,), 7.0, dtype=torch.float32 if f32 else torch.bfloat16, device="cuda")
+    C = guard[16 + off_c:16 + off_c + M * N]
+    ta, tb, waves = plan
+    prev = P.mxfp6_probe_slice(ta | tb << 4 | waves << 8 | shares << 12)
+    try:
+        rc = P.mxfp6_gemm_ex(*(ctypes.c_void_p(t.data_ptr()) for t in (*ops, C)), M, N, K, fa, fb, la, lb, f32, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    finally:
+        P.mxfp6_probe_slice(prev)
+    torch.cuda.synchronize()
+    assert rc == 0 and bool((guard[:16 + off_c] == 7.0).all()) and bool((guard[16 + off_c + M * N:] == 7.0).all())
+    return C.view(M, N)
+
+
+@pytest.mark.parametrize("plan", PLANS)
+@pytest.mark.parametrize("M,N,K,la,lb,shares", [(1, 1, 32, 0, 0, 1), (33, 65, 96, 0, 0, 1), (31, 33, 7904, 0, 0, 16), (64, 64, 256, 1, 1, 1), (96, 160, 1152, 1, 0, 2), (128, 96, 2176, 0, 1, 3),
+                                                (257, 255, 1056, 0, 0, 2), (17, 260, 384, 0, 0, 1), (32, 32, 6272, 1, 1, 7), (65, 8, 2080, 0, 0, 5)])
+def test_plans_vs_oracle(hk, plan, M, N, K, la, lb, shares):
+    fa, fb = ((2, 2), (3, 2), (2, 3))[(M + N) % 3]
+    ap, asc = co.quantise(o.make_source("normal", (M, K), np.random.default_rng(M + K)), fa)
+    bp, bsc = co.quantise(o.make_source("weights_outliers", (N, K), np.random.default_rng(N + K)), fb)
+    ref = o.gemm_ref(ap, bp, asc, bsc, fa, fb, acc=np.float64)
+    a, b = (o.tile_operand(ap), o.tile_scales(asc)) if la else (ap, asc), (o.tile_operand(bp), o.tile_scales(bsc)) if lb else (bp, bsc)
+    ops = [at(a[0]), at(b[0]), at(a[1]), at(b[1])]
+    got = forced(plan, shares, ops, M, N, K, fa, fb, la, lb).cpu().numpy()
+    assert np.isfinite(got).all() and o.rel_err(got, ref) <= 1e-5
+    again = forced(plan, shares, ops, M, N, K, fa, fb, la, lb).cpu().numpy()
+    assert np.array_equal(got, again)  # added in share order whoever adds; the counters are back at zero
+    c16 = forced(plan, shares, ops, M, N, K, fa, fb, la, lb, f32=0)
+    assert np.array_equal(c16.view(torch.int16).cpu().numpy().view(np.uint16), o.f32_to_bf16_bits(got))
+
+
+@pytest.mark.parametrize("plan", PLANS)
+@pytest.mark.parametrize("oa,ob,osa,osb,oc", [(4, 12, 1, 2, 3), (8, 4, 3, 1, 1), (0, 0, 2, 3, 2)])
+def test_alignments(hk, plan, oa, ob, osa, osb, oc):
+    M, N, K = 70, 136, 608
+    ap, asc = co.quantise(o.make_source("normal", (M, K), np.random.default_rng(1)), 2)
+    bp, bsc = co.quantise(o.make_source("weights", (N, K), np.random.default_rng(2)), 2)
+    got = forced(plan, 1, [at(ap, oa), at(bp, ob), at(asc, osa), at(bsc, osb)], M, N, K, off_c=oc).cpu().numpy()
+    assert o.rel_err(got, o.gemm_ref(ap, bp, asc, bsc, acc=np.float64)) <= 1e-5
+
+
+@pytest.mark.parametrize("M,N,K,lb", [(256, 1024, 1024, 1), (128, 512, 2560, 0), (3, 3072, 2688, 0), (48, 704, 928, 0), (90, 390, 3424, 0), (200, 1056, 5120, 1)])
+def test_automatic_route(hk, M, N, K, lb):
+    """Shapes the choice gives to this kernel: fp32, bf16, fused and MXFP6 output on the automatic path, the last one bit for bit
+    the quantiser's of the fp32 output."""
+    tk = hk.tk_kernel
+    assert tk.kernel_choice(M, N, K, 0, lb) in (tk.KERNEL_BLOCK, tk.CHOICE_BLOCK_K_SPLIT)
+    ap, asc = co.quantise(o.make_source("normal", (M, K), np.random.default_rng(M)), 2)
+    bp, bsc = co.quantise(o.make_source("weights", (N, K), np.random.default_rng(N)), 3)
+    a, asd, b, bsd = (torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in (ap, asc, o.tile_operand(bp) if lb else bp, o.tile_scales(bsc) if lb else bsc))
+    got = torch.empty(M, N, device="cuda")
+    hk.dispatch_micro(a, b, asd, bsd, got, 2, 3, layout_b=lb)
+    assert o.rel_err(got.cpu().numpy(), o.gemm_ref(ap, bp, asc, bsc, 2, 3, acc=np.float64)) <= 1e-5
+    bias = torch.randn(N, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
+    fused = torch.empty(M, N, device="cuda")
+    hk.dispatch_micro(a, b, asd, bsd, fused, 2, 3, layout_b=lb, bias=bias, activation="relu")
+    assert torch.equal(fused, (got + bias).clamp_min(0))  # one fp32 addition: exact to its rounding
+    if N % 32 == 0:
+        cp, cs = torch.empty(M, N // 4 * 3, dtype=torch.uint8, device="cuda"), torch.empty(M, N // 32, dtype=torch.uint8, device="cuda")
+        hk.dispatch_micro(a, b, asd, bsd, cp, 2, 3, layout_b=lb, C_scale=cs)
+        qp, qs = hk.quantize(got, 2)
+        assert torch.equal(cp, qp) and torch.equal(cs, qs)
+
+
+def test_capture_and_streams(hk):
+    """A K split of this kernel: under capture on a stream without a workspace it runs unsplit, on one that has it split; replays
+    equal the eager call."""
+    M, N, K = 64, 512, 12288 + 128
+    tk = hk.tk_kernel
+    assert tk.kernel_choice(M, N, K) == tk.CHOICE_BLOCK_K_SPLIT
+    g = torch.Generator(device="cuda").manual_seed(4)
+    (a, asc), (b, bsc) = hk.quantize(torch.randn(M, K, device="cuda", generator=g)), hk.quantize(torch.randn(N, K, device="cuda", generator=g) * 0.02)
+    eager = torch.empty(M, N, device="cuda")
+    hk.dispatch_micro(a, b, asc, bsc, eager)
+    torch.cuda.synchronize()
+    for warm in (False, True):
+        side, C, graph = torch.cuda.Stream(), torch.zeros(M, N, device="cuda"), torch.cuda.CUDAGraph()
+        side.wait_stream(torch.cuda.current_stream())
+        if warm:
+            with torch.cuda.stream(side):
+                hk.dispatch_micro(a, b, asc, bsc, C)
+            side.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            hk.dispatch_micro(a, b, asc, bsc, C)
+        for _ in range(3):
+            C.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(C, eager) if warm else o.rel_err(C.cpu().numpy(), eager.cpu().numpy()) <= 1e-5
+            hk.dispatch_micro(a, b, asc, bsc, torch.empty_like(C))
+            torch.cuda.synchronize()
