@@ -142,7 +142,7 @@ int choice_code(const mxfp6::KernelChoice& c) {
 unsigned auto_mask(const mxfp6::GemmArgs& g, int force_split) {
   unsigned mask = ~0u;
   if (!g_block || force_split) mask &= ~(kBlockAll | 1u << mxfp6::kCandSlice);
-  if (g_slice < 0) mask &= ~(1u << mxfp6::kCandSlice);
+  if (g_slice < 0) mask &= ~((g_slice == -1 ? 1u << mxfp6::kCandSlice : 0u) | 1u << mxfp6::kCandSliceX);
   if (force_split || g.no_alloc) mask &= ~(kNeedsWorkspace | 1u << mxfp6::kCandRing);
   if (force_split > 1 && mxfp6::gemm_skinny_supports(g)) mask = 1u << mxfp6::kCandSkinny;
   return mask;
@@ -151,7 +151,7 @@ unsigned auto_mask(const mxfp6::GemmArgs& g, int force_split) {
 // The choice for a call: by the time model and the calibration table (dispatch.hip).  allow_split = false: what it is when a
 // K split's workspace is not to be had (a stream that is being captured, the allocator's refusal).
 mxfp6::KernelChoice auto_choice(const mxfp6::GemmArgs& g, int force_split, bool allow_split) {
-  if (g_slice > 0 && !force_split && mxfp6::gemm_slice_supports(g)) return {mxfp6::kCandSlice, g_slice >> 12, 0, 0.0, {g_slice & 15, g_slice >> 4 & 15, g_slice >> 8 & 15, g_slice >> 12}};
+  if (g_slice > 0 && g_slice >> 20 == 0 && !force_split && mxfp6::gemm_slice_supports(g)) return {mxfp6::kCandSlice, g_slice >> 12, 0, 0.0, {g_slice & 15, g_slice >> 4 & 15, g_slice >> 8 & 15, g_slice >> 12}};
   if (g.K == 0) return {-1, 1, 0, 0.0};  // act(bias) everywhere: the generic kernel's K loop runs zero times
   return mxfp6::choose_kernel(g, g_ksplit, allow_split, auto_mask(g, force_split));
 }
@@ -444,12 +444,21 @@ int mxfp6_linear(const void* X, int x_bf16, const void* W, const void* Ws, void*
   rc = check_device();
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  // Up to four rows of bf16 the skinny kernel quantises itself where it is the choice: one launch instead of two, nothing in the workspace
-  if (x_bf16 && K > 0 && g_force == 0) {
+  // Few rows: the slice and (up to four of bf16) the skinny kernel quantise the activations themselves where they are the choice: one
+  // launch instead of two, no activations in the workspace
+  if (K > 0 && g_force == 0) {
     mxfp6::GemmArgs g{(const uint8_t*)X, (const uint8_t*)W, (const uint8_t*)X, (const uint8_t*)Ws, C, M, N, K, fmt_x, fmt_w, false, 0, layout_w};
-    g.X = X;
-    // (against the kernels that would need the quantiser's launch in front of them as well: the slice kernel does not count here)
-    if (mxfp6::gemm_skinny_takes_x(g) && mxfp6::choose_kernel(g, g_ksplit, true, auto_mask(g, 0) & ~(1u << mxfp6::kCandSlice)).cand == mxfp6::kCandSkinny) {
+    g.X = X, g.x_bf16 = x_bf16 != 0;
+    mxfp6::KernelChoice c = mxfp6::choose_linear_kernel(g, g_ksplit, auto_mask(g, 0));
+    if (g_slice >> 20 > 0) c = {mxfp6::kCandSlice, g_slice >> 12 & 255, 0, 0.0, {g_slice & 15, g_slice >> 4 & 15, g_slice >> 8 & 15, g_slice >> 12 & 255, g_slice >> 20}};
+    if (c.cand == mxfp6::kCandSlice) {
+      std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
+      if (!apply_choice(g, c, s)) c.slice.shares = 1;  // without a workspace: unsplit
+      g.ep = ep;
+      const hipError_t e = mxfp6::launch_gemm_slice(g, c.slice, s);
+      return e == hipSuccess ? MXFP6_OK : (int)e;
+    }
+    if (c.cand == mxfp6::kCandSkinny) {
       g.ep = ep;
       const hipError_t e = mxfp6::launch_gemm_skinny(g, s);
       return e == hipSuccess ? MXFP6_OK : (int)e;

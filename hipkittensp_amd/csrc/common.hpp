@@ -57,6 +57,23 @@ __device__ __forceinline__ u32x6 quantise_block_bf16(const v4i (&x)[4], int& sb)
   else return __builtin_amdgcn_cvt_scalef32_pk32_bf6_bf16(xb, scale);
 }
 
+// The same for a 32-block of fp32 (128 bytes)
+template <int FMT>
+__device__ __forceinline__ u32x6 quantise_block_f32(const v4i (&x)[8], int& sb) {
+  float amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) amax = fmaxf(amax, fabsf(__int_as_float(x[i][j])));
+  sb = e8m0_of_amax(amax, FMT == 2 ? 2 : 4);
+  const float scale = __uint_as_float((uint32_t)sb << 23);  // 2^(sb - 127); the instruction uses the exponent field
+  v16f ev, od;
+#pragma unroll
+  for (int i = 0; i < 16; i++) ev[i] = __int_as_float(x[i / 2][(2 * i) & 3]), od[i] = __int_as_float(x[i / 2][(2 * i + 1) & 3]);
+  if constexpr (FMT == 2) return __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ev, od, scale);
+  else return __builtin_amdgcn_cvt_scalef32_2xpk16_bf6_f32(ev, od, scale);
+}
+
 // The same for a 32-block of fp32 as two lanes of an MFMA tile hold it: column 8 (k / 4) + k % 4 of the block in p0[k], that + 4 in
 // p1[k].  fmt (2 or 3) is uniform.
 __device__ __forceinline__ u32x6 quantise_block_acc(const float (&p0)[16], const float (&p1)[16], int fmt, int& sb) {

@@ -324,7 +324,7 @@ bool gemm_skinny_supports(const GemmArgs& g) {
 }
 
 bool gemm_skinny_takes_x(const GemmArgs& g) {
-  return g.M >= 1 && g.M <= kXqRows && g.K >= 512 && g.K % 512 == 0 && ((uintptr_t)g.X & 15) == 0 && !g.no_alloc && !g.f32out;
+  return g.M >= 1 && g.M <= kXqRows && g.K >= 512 && g.K % 512 == 0 && ((uintptr_t)g.X & 15) == 0 && !g.no_alloc && !g.f32out && g.x_bf16;
 }
 
 // Workspace of the K split: 4 KB of partial tile per (tile, split) and a counter per tile that is zero between

@@ -19,6 +19,15 @@
 // LDS image of a chunk (a wave's buffer): 32-row tiles of 6 KB.  Row-major: rows of 192 bytes, 16-byte piece p of row r at
 // r * 192 + (p ^ ((r >> 2) & 3)) * 16 (the 16 rows of a ds_read_b128 phase fall into different banks); tile-major: the two
 // K-tiles' 3 KB as they are stored.  MFMA operand map as in the other kernels (common.hpp).
+//
+// Activations (XT = uint16_t for bf16, float): A is not packed yet, and every wave quantises the part of it that its chunk
+// needs: XR rows x 256 elements come into LDS in front of the chunk's B, and while B is on its way every lane turns 32-blocks
+// into A's image (the quantiser's own conversion, so the operand has the same bits).  A linear layer of few rows is then one
+// launch: the quantiser's is 2.5 us and more of GPU time, of 6 to 9 in all (8 x 4096 x 4096 8.2 -> 6.1 us, 61 x 512 x 2048 7.4 -> 4.8).
+// What it costs: every column tile reads and quantises the activations anew, about 300 clocks of a SIMD per 64 blocks, so that it
+// pays for few rows (choose_linear_kernel).
+#include <type_traits>
+
 #include "kernels.hpp"
 #include "loader.hpp"
 
@@ -29,7 +38,7 @@ constexpr int kSliceTile = 6144;      // bytes of 32 rows of a chunk (two K-tile
 constexpr int kSliceMaxShares = 16;   // workgroups that share an output tile at most
 
 struct SliceArgs {
-  const uint8_t *A, *B, *As, *Bs;
+  const uint8_t *A, *B, *As, *Bs;  // XT: A are the activations, As is not used
   void* C;
   uint8_t* C_scale;  // fp6 output only
   float* part;       // nsplit > 1: the shares' sums, [tile][share][TA TB tiles of 4 KB]
@@ -41,13 +50,18 @@ struct SliceArgs {
   Epilogue ep;
 };
 
-template <int FA, int FB, typename Out, int TA, int TB, int NW>
+struct PackedA {};  // XT of a packed A
+template <int FA, int FB, typename Out, int TA, int TB, int NW, typename XT = PackedA, int XR = 32>
 __global__ __launch_bounds__(NW * 64) void gemm_slice_kernel(const SliceArgs args) {
   typedef typename Out::type OutT;
   static_assert((TA == 1 || TA == 2) && (TB == 1 || TB == 2) && NW % 2 == 0, "tile, waves (the chunks of a wave keep their place in a group of four K-tiles)");
-  constexpr int TT = TA * TB;
-  constexpr int kA = TA * kSliceTile, kB = TB * kSliceTile, kScA = kA + kB, kScB = kScA + 1024, kBuf = kScB + 1024;
-  constexpr int NAL = kA / 1024, NBL = kB / 1024;
+  constexpr bool XQ = !std::is_same_v<XT, PackedA>;
+  static_assert(XQ ? TA == 1 && XR % 8 == 0 && XR >= 8 && XR <= 32 : XR == 32, "rows of activations");
+  constexpr int TT = TA * TB, kRowsA = TA * XR;
+  constexpr int kA = TA * XR * 192, kB = TB * kSliceTile, kScA = kA + kB, kScB = kScA + (XQ ? 512 : 1024), kX = kScB + 1024;
+  constexpr int kXBlock = XQ ? 32 * (int)sizeof(XT) : 0, kXRow = 8 * kXBlock;  // bytes of activations: of a block, of a row's chunk
+  constexpr int kBuf = kX + XR * kXRow;
+  constexpr int NAL = XQ ? 1 : kA / 1024, NBL = kB / 1024, NXL = XR * kXRow / 1024;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[NW * kBuf];
   static_assert(NW * kBuf <= 163840 && NW * kBuf >= NW * TT * 4096 + 64, "LDS budget (the buffers double as the reduction buffer)");
 
@@ -64,11 +78,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_slice_kernel(const SliceArgs arg
   const int order = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + (blockIdx.x >> 3);
   const int share = order / tiles, tile = order - share * tiles;
   const int ct = tile / args.m_blocks, mb = tile - ct * args.m_blocks;
-  const int m0 = mb * (32 * TA), n0 = ct * (32 * TB);
-  const int rows_a = min(32 * TA, args.M - m0), rows_b = min(32 * TB, args.N - n0);
+  const int m0 = mb * kRowsA, n0 = ct * (32 * TB);
+  const int rows_a = min(kRowsA, args.M - m0), rows_b = min(32 * TB, args.N - n0);
 
   // (a tile-major operand may end in a partial row-tile: its rows past the end are there, of no meaning)
-  const __amdgpu_buffer_rsrc_t rA = make_rsrc(args.A + (size_t)m0 * rowbytes, (uint32_t)(layout_a ? (rows_a + 31) & ~31 : rows_a) * rowbytes);
+  const __amdgpu_buffer_rsrc_t rA = XQ ? make_rsrc(args.A + (size_t)m0 * sbytes * kXBlock, (uint32_t)rows_a * sbytes * kXBlock)
+                                       : make_rsrc(args.A + (size_t)m0 * rowbytes, (uint32_t)(layout_a ? (rows_a + 31) & ~31 : rows_a) * rowbytes);
   const __amdgpu_buffer_rsrc_t rB = make_rsrc(args.B + (size_t)n0 * rowbytes, (uint32_t)(layout_b ? (rows_b + 31) & ~31 : rows_b) * rowbytes);
   // scales: the resource starts and ends at aligned dwords (which hold at least one byte of the tensor each)
   const uint8_t* const sa0 = args.As + (layout_a ? (size_t)(m0 >> 5) * nk4 * 512 : (size_t)m0 * sbytes);
@@ -88,8 +103,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_slice_kernel(const SliceArgs arg
     const int o = i * 64 + lane, r = o / 12, p = (o - r * 12) ^ ((r >> 2) & 3);
     return layout ? (o / 384) * (nkt * 3072) + (o % 384) * 16 + first * 6144 : r * rowbytes + p * 16 + first * 192;
   };
+  if constexpr (!XQ) {
 #pragma unroll
-  for (int i = 0; i < NAL; i++) voff_a[i] = load_offset(i, layout_a);
+    for (int i = 0; i < NAL; i++) voff_a[i] = load_offset(i, layout_a);
+  }
 #pragma unroll
   for (int i = 0; i < NBL; i++) voff_b[i] = load_offset(i, layout_b);
   const int kstep_a = layout_a ? NW * 6144 : NW * 192, kstep_b = layout_b ? NW * 6144 : NW * 192;
@@ -98,15 +115,33 @@ __global__ __launch_bounds__(NW * 64) void gemm_slice_kernel(const SliceArgs arg
     return layout ? (row >> 5) * (nk4 * 512) + (row & 31) * 16 + (first >> 1) * 512 + (first & 1) * 8 : ((row * sbytes + (int)mis) & ~3) + first * 8;
   };
   int voff_sa = scale_offset(TA == 2 ? lane : r32, layout_a, mis_a), voff_sb = scale_offset(TB == 2 ? lane : r32, layout_b, mis_b);
+  // activations: load i fills LDS bytes [i * 1024, + 1024); the 16-byte pieces of a block are rotated by its place among the 16
+  // blocks of two rows, so that the 16 lanes of a ds_read_b128 phase, each on a block of its own, fall into different banks
+  constexpr int kXPieces = XQ ? kXBlock / 16 : 1, kXSame = XQ ? 16 / kXPieces : 1;  // blocks next to each other that cover all banks
+  auto x_rotate = [](int block) __attribute__((always_inline)) { return (block & 15) / kXSame; };
+  [[maybe_unused]] int voff_x[XQ ? NXL : 1];
+  if constexpr (XQ) {
+#pragma unroll
+    for (int i = 0; i < NXL; i++) {
+      const int o = i * 64 + lane, b = o / kXPieces, c = (o ^ x_rotate(b)) & (kXPieces - 1);
+      voff_x[i] = (b >> 3) * sbytes * kXBlock + (b & 7) * kXBlock + c * 16 + first * kXRow;
+    }
+  }
   const int sstep_a = layout_a ? NW / 2 * 512 : NW * 8, sstep_b = layout_b ? NW / 2 * 512 : NW * 8;
   // how many bytes a row's scales start behind the aligned dwords fetched for it (taken modulo 4; rows 32 apart share it)
-  const uint32_t shift_a = mis_a + (layout_a ? 0 : r32 * sbytes), shift_b = mis_b + (layout_b ? 0 : r32 * sbytes);
+  const uint32_t shift_a = XQ ? 0 : mis_a + (layout_a ? 0 : r32 * sbytes), shift_b = mis_b + (layout_b ? 0 : r32 * sbytes);
 
   const uint32_t buf = lds_address(smem) + wave * kBuf;
   const uint8_t* const bufp = smem + wave * kBuf;
+  [[maybe_unused]] auto issue_x = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < (XQ ? NXL : 0); i++) dma16(rA, buf + kX + i * 1024, voff_x[i], 0);
+#pragma unroll
+    for (int i = 0; i < (XQ ? NXL : 0); i++) voff_x[i] += NW * kXRow;
+  };
   auto issue = [&]() __attribute__((always_inline)) {
     dma16(rBs, buf + kScB, voff_sb, 0);
-    dma16(rAs, buf + kScA, voff_sa, 0);
+    if constexpr (!XQ) dma16(rAs, buf + kScA, voff_sa, 0);
     voff_sa += sstep_a, voff_sb += sstep_b;
     if (args.stream) {
 #pragma unroll
@@ -115,14 +150,53 @@ __global__ __launch_bounds__(NW * 64) void gemm_slice_kernel(const SliceArgs arg
 #pragma unroll
       for (int i = 0; i < NBL; i++) dma16(rB, buf + kA + i * 1024, voff_b[i], 0);
     }
+    if constexpr (!XQ) {
 #pragma unroll
-    for (int i = 0; i < NAL; i++) dma16(rA, buf + i * 1024, voff_a[i], 0);
+      for (int i = 0; i < NAL; i++) dma16(rA, buf + i * 1024, voff_a[i], 0);
+#pragma unroll
+      for (int i = 0; i < NAL; i++) voff_a[i] += kstep_a;
+    }
 #pragma unroll
     for (int i = 0; i < NBL; i++) voff_b[i] += kstep_b;
-#pragma unroll
-    for (int i = 0; i < NAL; i++) voff_a[i] += kstep_a;
   };
-  if (first < c1) issue();
+  // Lane l of pass p quantises block (64 p + l) % 8 of row (64 p + l) / 8 of the chunk's activations.  All of them go into registers
+  // first, so that the next chunk's are on their way while this one's are quantised and multiplied.
+  [[maybe_unused]] auto quantise = [&](bool more) __attribute__((always_inline)) {
+    uint8_t* const own = smem + wave * kBuf;
+    v4i x[XR / 8][kXPieces];
+#pragma unroll
+    for (int p = 0; p < XR / 8; p++)
+#pragma unroll
+      for (int c = 0; c < kXPieces; c++) {
+        const int b = p * 64 + lane;
+        x[p][c] = *reinterpret_cast<const v4i*>(own + kX + b * kXBlock + ((c ^ x_rotate(b)) & (kXPieces - 1)) * 16);
+      }
+    wait_lds_reads();
+#pragma unroll
+    for (int p = 0; p < XR / 8; p++)
+#pragma unroll
+      for (int c = 0; c < kXPieces; c++) asm volatile("" : "+v"(x[p][c]));
+    if (more) issue_x();
+#pragma unroll
+    for (int p = 0; p < XR / 8; p++) {
+      const int b = p * 64 + lane, row = b >> 3, blk = b & 7;
+      int sb;
+      u32x6 w;
+      if constexpr (kXBlock == 64) w = quantise_block_bf16<FA>(x[p], sb);
+      else if constexpr (XQ) w = quantise_block_f32<FA>(x[p], sb);
+#pragma unroll
+      for (int i = 0; i < 3; i++) {
+        const int byte = blk * 24 + 8 * i;
+        *reinterpret_cast<u32x2*>(own + row * 192 + ((byte >> 4) ^ ((row >> 2) & 3)) * 16 + (byte & 15)) = u32x2{w[2 * i], w[2 * i + 1]};
+      }
+      own[kScA + row * 16 + blk] = (uint8_t)sb;
+    }
+    wait_lds_reads();  // (writes too)
+  };
+  if (first < c1) {
+    if constexpr (XQ) issue_x();  // in front of B: quantised while B is on its way
+    issue();
+  }
 
   int a_rd[2][3], b_rd[2][3];  // K-tile u of a chunk, piece 3h + c of the row's 96 bytes
 #pragma unroll
@@ -130,7 +204,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_slice_kernel(const SliceArgs arg
 #pragma unroll
     for (int c = 0; c < 3; c++) {
       const int row = r32 * 192 + ((6 * u + 3 * h + c) ^ ((r32 >> 2) & 3)) * 16, til = u * 3072 + r32 * 96 + ((3 * h + c) ^ ((r32 >> 3) & 1)) * 16;
-      a_rd[u][c] = layout_a ? til : row;
+      const int ra = XQ ? r32 % XR : r32, rowx = ra * 192 + ((6 * u + 3 * h + c) ^ ((ra >> 2) & 3)) * 16;
+      a_rd[u][c] = XQ ? rowx : layout_a ? til : row;  // rows past the XR that are staged mirror those; their outputs are not stored
       b_rd[u][c] = kA + (layout_b ? til : row);
     }
 
@@ -143,7 +218,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_slice_kernel(const SliceArgs arg
       for (int e = 0; e < 16; e++) acc[t][s][e] = 0.f;
 
   for (int c = first; c < c1; c += NW) {
-    wait_vmcnt<0>();
+    if constexpr (XQ) {
+      wait_vmcnt<NBL + 1>();
+      quantise(c + NW < c1);
+      if (c + NW < c1) wait_vmcnt<NXL>();
+      else wait_vmcnt<0>();
+    } else {
+      wait_vmcnt<0>();
+    }
     v4i fa[TA][2][3], fb[TB][2][3], raw_a[TA], raw_b[TB];
 #pragma unroll
     for (int s = 0; s < TB; s++) {
@@ -155,7 +237,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_slice_kernel(const SliceArgs arg
     }
 #pragma unroll
     for (int t = 0; t < TA; t++) {
-      raw_a[t] = *reinterpret_cast<const v4i*>(bufp + kScA + (t * 32 + r32) * 16);
+      raw_a[t] = *reinterpret_cast<const v4i*>(bufp + kScA + (t * 32 + (XQ ? r32 % XR : r32)) * 16);
 #pragma unroll
       for (int u = 0; u < 2; u++)
 #pragma unroll
@@ -267,7 +349,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_slice_kernel(const SliceArgs arg
   for (int k = 0; k < kItems; k++) {
     const int item = tid + k * (NW * 64), t = item >> 8, row = (item >> 3) & 31, quad = item & 7;
     const long m = (long)m0 + (t / TB) * 32 + row, n = (long)n0 + (t % TB) * 32 + quad * 4;
-    if (item >= TT * 256) continue;
+    if (item >= TT * 256 || (XR < 32 && row >= XR)) continue;
     if (has_ep && m < M) {
 #pragma unroll
       for (int e = 0; e < 4; e++)
@@ -318,19 +400,38 @@ bool gemm_slice_supports(const GemmArgs& g) {
 
 // Workspace of the K split: bytes of partial tiles and arrival counters
 void slice_workspace(const GemmArgs& g, const SlicePlan& p, size_t* part_bytes, size_t* counters) {
-  *counters = (size_t)((g.M + 32 * p.ta - 1) / (32 * p.ta)) * ((g.N + 32 * p.tb - 1) / (32 * p.tb));
+  const int rows = p.xrows ? p.xrows : 32 * p.ta;
+  *counters = (size_t)((g.M + rows - 1) / rows) * ((g.N + 32 * p.tb - 1) / (32 * p.tb));
   *part_bytes = *counters * p.shares * p.ta * p.tb * 4096;
 }
 
 template <int FA, int FB, typename Out>
 static hipError_t launch(const GemmArgs& g, const SlicePlan& p, hipStream_t s) {
-  const int col_tiles = (g.N + 32 * p.tb - 1) / (32 * p.tb), m_blocks = (g.M + 32 * p.ta - 1) / (32 * p.ta);
+  const int rows = p.xrows ? p.xrows : 32 * p.ta, col_tiles = (g.N + 32 * p.tb - 1) / (32 * p.tb), m_blocks = (g.M + rows - 1) / rows;
   const int nchunks = ((g.K + 127) / 128 + 1) / 2, shares = p.shares > 1 && g.ks_part && g.ks_counters ? p.shares : 1;
   if (shares > kSliceMaxShares || (shares - 1) * ((nchunks + shares - 1) / shares) >= nchunks) return hipErrorInvalidValue;  // no empty share
-  const size_t out = sizeof(typename Out::type);
+  constexpr size_t out = sizeof(typename Out::type);
   const SliceArgs a{g.A, g.B, g.As, g.Bs, g.C, g.C_scale, g.ks_part, reinterpret_cast<unsigned*>(g.ks_counters), g.M, g.N, g.K, g.layout_a, g.layout_b, col_tiles, m_blocks, shares,
                     m_blocks == 1 && (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes, g.N % 4 == 0 && ((uintptr_t)g.C & (4 * out - 1)) == 0, g.fmt_c, g.ep};
   const unsigned grid = (unsigned)col_tiles * m_blocks * shares;
+  if (p.xrows) {
+    if constexpr (out == 2) {
+      SliceArgs x = a;
+      x.A = static_cast<const uint8_t*>(g.X), x.As = g.Bs, x.layout_a = 0;
+#define MXFP6_SLICE_X(T, BF16, XR, TB, NW) \
+  if (g.x_bf16 == BF16 && p.xrows == XR && p.tb == TB && p.waves == NW) { \
+    gemm_slice_kernel<FA, FB, Out, 1, TB, NW, T, XR><<<grid, NW * 64, 0, s>>>(x); \
+    return hipGetLastError(); \
+  }
+      MXFP6_SLICE_X(uint16_t, 1, 8, 1, 4) MXFP6_SLICE_X(uint16_t, 1, 8, 1, 8) MXFP6_SLICE_X(uint16_t, 1, 8, 2, 4) MXFP6_SLICE_X(uint16_t, 1, 8, 2, 8)
+      MXFP6_SLICE_X(uint16_t, 1, 16, 1, 4) MXFP6_SLICE_X(uint16_t, 1, 16, 1, 8) MXFP6_SLICE_X(uint16_t, 1, 16, 2, 4) MXFP6_SLICE_X(uint16_t, 1, 16, 2, 6)
+      MXFP6_SLICE_X(uint16_t, 1, 32, 1, 4) MXFP6_SLICE_X(uint16_t, 1, 32, 2, 4)
+      MXFP6_SLICE_X(float, 0, 8, 1, 4) MXFP6_SLICE_X(float, 0, 8, 1, 8) MXFP6_SLICE_X(float, 0, 8, 2, 4) MXFP6_SLICE_X(float, 0, 8, 2, 6)
+      MXFP6_SLICE_X(float, 0, 16, 1, 4) MXFP6_SLICE_X(float, 0, 16, 2, 4) MXFP6_SLICE_X(float, 0, 24, 1, 4)
+#undef MXFP6_SLICE_X
+    }
+    return hipErrorInvalidValue;
+  }
 #define MXFP6_SLICE(TA, TB, NW) \
   if (p.ta == TA && p.tb == TB && p.waves == NW) { \
     gemm_slice_kernel<FA, FB, Out, TA, TB, NW><<<grid, NW * 64, 0, s>>>(a); \

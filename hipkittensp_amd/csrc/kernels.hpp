@@ -20,7 +20,8 @@ struct GemmArgs {
   uint8_t* C_scale = nullptr;      // fp6 output (tiled and block kernels, reduction of a K split): C is the packed operand [M, 3N/4], this its E8M0 bytes [M, N/32]
   int fmt_c = 0;                   // 2 / 3: format of the fp6 output; 0: bf16 / fp32 output
   int out_fp6 = 0;                 // kernel choice only: the fp32 sums (f32out) leave as MXFP6
-  const void* X = nullptr;         // skinny kernel: bf16 activations [M, K] that it quantises to fmt_a itself, in place of A and As (gemm_skinny_takes_x)
+  const void* X = nullptr;         // skinny and slice kernel: activations [M, K] that they quantise to fmt_a themselves, in place of A and As (gemm_skinny_takes_x, choose_linear_kernel)
+  int x_bf16 = 0;                  // ... in bf16 (the skinny kernel takes no others), else fp32
   int raster_group_m = 0, raster_no_xcd_remap = 0;  // tiled kernel, measurement only: tile rows per raster group (0 = the default, 4), XCD remap off (1), or on with a K split's workgroups in tile-by-tile order (2)
   int ablation = 0;  // tiled kernel, measurement only: leave out LDS reads (1), loads (2), MFMAs (4); results are then meaningless
   uint32_t* clock_stamps = nullptr;  // tiled kernel, measurement only: four words for workgroup 0's clock / real-time counters at start and end
@@ -48,9 +49,11 @@ constexpr size_t kStreamBytes = (size_t)128 << 20;
 
 // ---- kernel choice (dispatch.hip): candidates of the automatic path, a time model per candidate, a calibration table
 enum Candidate : int { kCandTiled256 = 0, kCandTiled128x256, kCandTiled128x128, kCandBlock, kCandBlockWide, kCandSkinny, kCandTiledSplit256, kCandTiledSplit128, kCandBlockSplit, kCandRing, kNumCandidates,
-  kCandSlice = kNumCandidates };  // not calibrated: its own model against the best of the others (slice_plan)
+  kCandSlice = kNumCandidates,  // not calibrated: its own model against the best of the others (slice_plan)
+  kCandSliceX };  // in candidate sets only: the slice kernel on a linear layer's activations (choose_linear_kernel)
 struct SlicePlan {  // small problems: tiles of 32 ta x 32 tb outputs, K dealt to `waves` waves and to `shares` workgroups (gemm_slice.hip)
   int ta, tb, waves, shares;
+  int xrows = 0;  // rows of activations a workgroup quantises itself (8, 16, 24, 32); 0: A is packed
 };
 struct KernelChoice {
   int cand;    // a Candidate, or -1: none of them takes the shape (ragged_shares says what does)
@@ -62,6 +65,7 @@ struct KernelChoice {
 int device_cus();
 double candidate_model_us(const GemmArgs& g, int cand, int want_split, int cus, int* shares, int* rows);  // modelled microseconds; < 0: the candidate does not take the shape
 KernelChoice choose_kernel(const GemmArgs& g, int want_split, bool allow_split, unsigned mask = ~0u);  // mask: bit per Candidate that may be chosen; want_split: 0 = by the model, 1 = never, n = n shares where a candidate splits; allow_split: a workspace is to be had
+KernelChoice choose_linear_kernel(const GemmArgs& g, int want_split, unsigned mask);  // g.X, g.x_bf16: the activations
 int tiled_split_shares(const GemmArgs& g, int want, int cus, int bm);  // the tiled kernel's K split with tiles of bm (256 or 128) rows when it is to split: shares (1 = the shape has none)
 int ragged_shares(const GemmArgs& g, int want, bool allow_split);  // shapes no candidate takes: shares of the block kernel's K split (1 = unsplit), 0 = the generic kernel
 int block_split_shares(const GemmArgs& g, int want, int cus);             // ... the block kernel's

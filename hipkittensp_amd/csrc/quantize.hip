@@ -88,22 +88,8 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
 
     int sb;
     u32x6 w;
-    if constexpr (sizeof(In) == 4) {
-      float amax = 0.f;
-#pragma unroll
-      for (int i = 0; i < P; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) amax = fmaxf(amax, fabsf(__int_as_float(x[i][j])));
-      sb = e8m0_of_amax(amax, FMT == 2 ? 2 : 4);
-      const float scale = __uint_as_float((uint32_t)sb << 23);  // 2^(sb - 127); the instruction uses the exponent field
-      v16f ev, od;
-#pragma unroll
-      for (int i = 0; i < 16; i++) ev[i] = __int_as_float(x[i / 2][(2 * i) & 3]), od[i] = __int_as_float(x[i / 2][(2 * i + 1) & 3]);
-      if constexpr (FMT == 2) w = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ev, od, scale);
-      else w = __builtin_amdgcn_cvt_scalef32_2xpk16_bf6_f32(ev, od, scale);
-    } else {
-      w = quantise_block_bf16<FMT>(x, sb);
-    }
+    if constexpr (sizeof(In) == 4) w = quantise_block_f32<FMT>(x, sb);
+    else w = quantise_block_bf16<FMT>(x, sb);
     // the chunk's 1536 output bytes in order, in the buffer its input has left
     uint8_t* const image = smem + wave * kChunk;
     const long g16 = layout ? chunk / nkt : 0;

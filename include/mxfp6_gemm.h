@@ -25,7 +25,7 @@
  *   - the gemm entry points on large row-major problems (re-layout pre-pass, see mxfp6_set_relayout):
  *     up to 0.78 (M + N) K bytes;
  *   - mxfp6_gemm_fused_fp6 on shapes that the decode, ragged and generic kernels run: 4 M N bytes;
- *   - mxfp6_linear: 0.79 M K bytes, M rounded up to 32;
+ *   - mxfp6_linear: 0.79 M K bytes, M rounded up to 32 (none for calls of few rows that quantise inside the GEMM kernel);
  *   - the gemm entry points on decode shapes whose K range is split between workgroups (M <= 32, N <= 2048,
  *     K >= 24576): 2 MB;
  *   - the gemm entry points on problems of few output tiles and long K (up to a few hundred rows of A; see
@@ -281,8 +281,8 @@ int mxfp6_gemm_fused_fp6(const void *A_packed, const void *B_packed, const void 
  * as mxfp6_gemm_fused would compute it from that operand.  W_packed [N, 3K/4], W_scale: the weights in layout_w; bias as in
  * mxfp6_gemm_fused (NULL = none).  The packed activations live in a workspace of this stream (0.79 bytes per element of X,
  * rows rounded up to 32), in the layout the GEMM prefers.  MXFP6_EWORKSPACE, and nothing launched, where it cannot be had,
- * and while the stream is being captured (two graphs captured on one stream would share it).  Up to four bf16 rows on the
- * decode kernel need none and are captured.  No counterpart in the reference.
+ * and while the stream is being captured (two graphs captured on one stream would share it).  Calls of few rows (up to 128, by
+ * size) quantise inside the slice or the decode kernel: they need none and are captured.  No counterpart in the reference.
  */
 int mxfp6_linear(const void *X, int x_bf16, const void *W_packed, const void *W_scale, void *C_bf16, int M, int N, int K,
                  int fmt_x, int fmt_w, int layout_w, const void *bias, int bias_bf16, int activation, void *hip_stream);

@@ -93,7 +93,8 @@ int mxfp6_probe_candidate(int M, int N, int K, int layouts, int candidate, int c
 int mxfp6_probe_block(int enable);
 
 /* Measurement switch, per calling thread: -1 keeps the slice kernel out of the automatic choice, a plan
- * (rows of A / 32) | (rows of B / 32) << 4 | waves << 8 | shares of K << 12 takes it for every call of the automatic path, 0 (the
+ * (rows of A / 32) | (rows of B / 32) << 4 | waves << 8 | shares of K << 12 takes it for every call of the automatic path, that with
+ * rows of activations << 20 for every mxfp6_linear (which quantises them in the kernel), -2 keeps it from the latter only, 0 (the
  * default) leaves it to the choice; returns the previous setting.  Plans that are not built fail with hipErrorInvalidValue. */
 int mxfp6_probe_slice(int plan);
 

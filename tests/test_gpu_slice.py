@@ -128,3 +128,69 @@ def test_capture_and_streams(hk):
             assert torch.equal(C, eager) if warm else o.rel_err(C.cpu().numpy(), eager.cpu().numpy()) <= 1e-5
             hk.dispatch_micro(a, b, asc, bsc, torch.empty_like(C))
             torch.cuda.synchronize()
+
+
+# (rows of activations, rows of B / 32, waves) of the instantiations that quantise the activations themselves
+X_PLANS = {1: [(8, 1, 4), (8, 1, 8), (8, 2, 4), (8, 2, 8), (16, 1, 4), (16, 1, 8), (16, 2, 4), (16, 2, 6), (32, 1, 4), (32, 2, 4)],
+           0: [(8, 1, 4), (8, 1, 8), (8, 2, 4), (8, 2, 6), (16, 1, 4), (16, 2, 4), (24, 1, 4)]}
+
+
+@pytest.mark.parametrize("bf16,plan", [(b, p) for b in X_PLANS for p in X_PLANS[b]])
+@pytest.mark.parametrize("M,N,K,lb,shares", [(1, 1, 32, 0, 1), (7, 65, 96, 0, 1), (33, 33, 7904, 0, 8), (24, 64, 256, 1, 1), (25, 160, 1152, 1, 2), (50, 260, 416, 0, 1), (65, 32, 6272, 1, 5)])
+def test_quantising_plans_vs_oracle(hk, bf16, plan, M, N, K, lb, shares):
+    """The activations quantised in the kernel: quantiser and product of the oracle.  The output is bf16: half a last place, 2^-8 of
+    the value, and the fp32 sums' own bound."""
+    P = _lib.probes()
+    P.mxfp6_probe_slice.argtypes, P.mxfp6_probe_slice.restype = [ctypes.c_int], ctypes.c_int
+    fa, fb = ((2, 2), (3, 2), (2, 3))[(M + N) % 3]
+    xs = torch.from_numpy(o.make_source("normal", (M, K), np.random.default_rng(M + K)).astype(np.float32))
+    xs[M // 2, :32] = 0  # a block of zeros
+    x = xs.to(torch.bfloat16) if bf16 else xs
+    ap, asc = co.quantise(x.float().numpy(), fa)
+    bp, bsc = co.quantise(o.make_source("weights_outliers", (N, K), np.random.default_rng(N + K)), fb)
+    ref = o.gemm_ref(ap, bp, asc, bsc, fa, fb, acc=np.float64)
+    ops = [at((x.view(torch.int16) if bf16 else x).numpy()), at(o.tile_operand(bp) if lb else bp), at(o.tile_scales(bsc) if lb else bsc)]
+    guard = torch.full((M * N + 64,), 7.0, dtype=torch.bfloat16, device="cuda")
+    C = guard[16:16 + M * N]
+    prev = P.mxfp6_probe_slice(1 | plan[1] << 4 | plan[2] << 8 | shares << 12 | plan[0] << 20)
+    try:
+        rc = P.mxfp6_linear(ops[0].data_ptr(), bf16, ops[1].data_ptr(), ops[2].data_ptr(), C.data_ptr(), M, N, K, fa, fb, lb, None, 0, 0,
+                            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    finally:
+        P.mxfp6_probe_slice(prev)
+    torch.cuda.synchronize()
+    assert rc == 0 and bool((guard[:16] == 7.0).all()) and bool((guard[16 + M * N:] == 7.0).all())
+    got = C.view(M, N).float().cpu().numpy()
+    bound = np.abs(ref) * 2.0**-8 + 1e-5 * np.maximum(np.abs(ref), 0.01 * np.sqrt((ref**2).mean()))
+    assert np.isfinite(got).all() and (np.abs(got - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("M,N,K,bf16", [(5, 512, 1024, 1), (23, 1056, 2080, 1), (64, 512, 1536, 1), (17, 768, 640, 0), (100, 512, 768, 0), (8, 512, 18176, 1)])
+def test_quantising_route(hk, M, N, K, bf16):
+    """MXFP6Linear's calls of few rows: the bits of quantise, then GEMM (these sums are exact or rounded far below bf16), eager and
+    captured on a stream that has no workspace, odd values in the activations among them."""
+    from hipkittensp_amd.torch_op import MXFP6Linear
+
+    g = torch.Generator(device="cuda").manual_seed(M)
+    layer = MXFP6Linear(torch.randn(N, K, device="cuda", generator=g) * 0.02, bias=torch.randn(N, device="cuda", generator=g), activation="relu")
+    x = torch.randn(M, K, device="cuda", generator=g)
+    x[0, :6] = torch.tensor([float("nan"), float("inf"), -float("inf"), 1e-42, 3e38, -0.0], device="cuda")
+    x[M - 1, 64:96] = 1e-41
+    x = x.to(torch.bfloat16) if bf16 else x
+
+    def steps():
+        xp, xs = hk.quantize(x, 2)
+        want = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+        hk.dispatch_micro(xp, layer.weight_packed, xs, layer.weight_scale, want, layout_b=layer.layout_w, bias=layer.bias, activation="relu")
+        return want
+
+    assert torch.equal(layer(x).view(torch.int16), steps().view(torch.int16))
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        y = layer(x)
+    for _ in range(3):
+        x.copy_(torch.randn(M, K, device="cuda", generator=g))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, steps()) and torch.equal(layer(x), steps())
