@@ -34,6 +34,9 @@ __device__ __forceinline__ int e8m0_of_amax(float amax, int emax) {
 
 // A 32-block of bf16 (64 bytes) quantised to FMT: six dwords and its E8M0 byte.  The instruction divides by the power of two and
 // rounds (nearest even, saturating).
+// The conversions read their sources over several passes and write the result meanwhile: registers that the two share come out
+// wrong (v[0:5] from v[18:33], v[2:17]: the third dword on).  The compiler does not know, so every source is kept in use until
+// behind the instruction.
 typedef uint32_t u32x6 __attribute__((ext_vector_type(6)));
 template <int FMT>
 __device__ __forceinline__ u32x6 quantise_block_bf16(const v4i (&x)[4], int& sb) {
@@ -53,8 +56,11 @@ __device__ __forceinline__ u32x6 quantise_block_bf16(const v4i (&x)[4], int& sb)
 #pragma unroll
   for (int i = 0; i < 16; i++) raw[i] = x[i / 4][i & 3];
   const v32bf xb = __builtin_bit_cast(v32bf, raw);
-  if constexpr (FMT == 2) return __builtin_amdgcn_cvt_scalef32_pk32_fp6_bf16(xb, scale);
-  else return __builtin_amdgcn_cvt_scalef32_pk32_bf6_bf16(xb, scale);
+  u32x6 w;
+  if constexpr (FMT == 2) w = __builtin_amdgcn_cvt_scalef32_pk32_fp6_bf16(xb, scale);
+  else w = __builtin_amdgcn_cvt_scalef32_pk32_bf6_bf16(xb, scale);
+  asm volatile("" : "+v"(w) : "v"(raw), "v"(scale));
+  return w;
 }
 
 // The same for a 32-block of fp32 (128 bytes)
@@ -70,8 +76,11 @@ __device__ __forceinline__ u32x6 quantise_block_f32(const v4i (&x)[8], int& sb) 
   v16f ev, od;
 #pragma unroll
   for (int i = 0; i < 16; i++) ev[i] = __int_as_float(x[i / 2][(2 * i) & 3]), od[i] = __int_as_float(x[i / 2][(2 * i + 1) & 3]);
-  if constexpr (FMT == 2) return __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ev, od, scale);
-  else return __builtin_amdgcn_cvt_scalef32_2xpk16_bf6_f32(ev, od, scale);
+  u32x6 w;
+  if constexpr (FMT == 2) w = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ev, od, scale);
+  else w = __builtin_amdgcn_cvt_scalef32_2xpk16_bf6_f32(ev, od, scale);
+  asm volatile("" : "+v"(w) : "v"(ev), "v"(od), "v"(scale));
+  return w;
 }
 
 // The same for a 32-block of fp32 as two lanes of an MFMA tile hold it: column 8 (k / 4) + k % 4 of the block in p0[k], that + 4 in
@@ -89,15 +98,13 @@ __device__ __forceinline__ u32x6 quantise_block_acc(const float (&p0)[16], const
     ev[t] = (ne & 4) ? p1[4 * (ne >> 3) + (ne & 3)] : p0[4 * (ne >> 3) + (ne & 3)];
     od[t] = (no & 4) ? p1[4 * (no >> 3) + (no & 3)] : p0[4 * (no >> 3) + (no & 3)];
   }
-  // a real branch (the empty asm keeps it one): with both conversions issued on the same sources and a select
-  // behind them, the second one's result came out wrong from the third dword on
   u32x6 w;
   if (fmt == 2) {
     w = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ev, od, scale);
-    asm volatile("" : "+v"(w));
+    asm volatile("" : "+v"(w) : "v"(ev), "v"(od), "v"(scale));
   } else {
     w = __builtin_amdgcn_cvt_scalef32_2xpk16_bf6_f32(ev, od, scale);
-    asm volatile("" : "+v"(w));
+    asm volatile("" : "+v"(w) : "v"(ev), "v"(od), "v"(scale));
   }
   return w;
 }
