@@ -30,9 +30,10 @@ thread_local uint32_t* g_clock_stamps = nullptr;  // mxfp6_probe_tiled_clock
 thread_local int g_raster_group_m = 0, g_raster_no_xcd = 0;  // mxfp6_probe_raster
 thread_local int g_ablation = 0;                              // mxfp6_probe_tiled_ablation
 thread_local int g_slice = 0;                                 // mxfp6_probe_slice: -1 = never, a plan = always
+thread_local int g_padded = 0;                                // mxfp6_probe_padded: 1 = always, -1 = never
 thread_local int g_block = 1;                                 // mxfp6_probe_block: 0 keeps the block kernel out of the automatic choice
 #else
-constexpr int g_slice = 0, g_block = 1;
+constexpr int g_slice = 0, g_padded = 0, g_block = 1;
 #endif
 
 // Workspaces kept per (device, stream, kind): launches on one stream are ordered, so they can share one; it grows on
@@ -301,6 +302,42 @@ bool relayout_then_tiled(const mxfp6::GemmArgs& g, hipStream_t s, hipError_t& e)
   return true;
 }
 
+// Bytes of a padded tile-major copy: packed bytes, then its scales
+size_t padded_bytes(int rows, int K) {
+  const size_t r = ((size_t)rows + 31) & ~(size_t)31, nkt = ((size_t)K + 127) / 128;
+  return ((r * nkt * 96 + 255) & ~(size_t)255) + ((r * ((nkt + 3) / 4) * 16 + 255) & ~(size_t)255);
+}
+uint8_t* padded_scales(uint8_t* p, int rows, int K) { return p + (((((size_t)rows + 31) & ~(size_t)31) * (((size_t)K + 127) / 128) * 96 + 255) & ~(size_t)255); }
+
+// A ragged product on padded tile-major copies of its operands where those pay (padded_pays; `c`: the choice otherwise).  a_pad:
+// A's copy is there already.  Returns false, nothing launched, where they don't or no workspace is to be had.
+bool padded_then_gemm(const mxfp6::GemmArgs& g, const mxfp6::KernelChoice& c, uint8_t* a_pad, hipStream_t s, hipError_t& e) {
+  if (!g_relayout || g_padded < 0) return false;
+  mxfp6::GemmArgs t = g;
+  mxfp6::KernelChoice tc{-1, 1, 0, 0.0};
+  const mxfp6::KernelChoice never{mxfp6::kCandSlice, 1, 0, 1e30};
+  if (!mxfp6::padded_pays(g, g_ksplit, auto_mask(g, 0), g_padded > 0 ? never : c, a_pad != nullptr, &t, &tc)) return false;
+  const size_t na = a_pad ? 0 : padded_bytes(g.M, g.K), nb = g.layout_b ? 0 : padded_bytes(g.N, g.K);
+  uint8_t* const ws = na + nb ? stream_workspace(s, 0, na + nb) : nullptr;
+  if (na + nb && !ws) return false;
+  uint8_t *const pa = a_pad ? a_pad : ws, *const pb = ws + na;
+  uint8_t *const sa = padded_scales(pa, g.M, g.K), *const sb = padded_scales(pb, g.N, g.K);
+  t.A = pa, t.As = sa;
+  if (nb) t.B = pb, t.Bs = sb;
+  else t.B = g.B, t.Bs = g.Bs;
+  if (tc.cand >= 0 && !apply_choice(t, tc, s)) {  // a split without its workspace
+    tc = mxfp6::choose_kernel(t, g_ksplit, false, auto_mask(t, 0) & (kTiledUnsplit | 1u << mxfp6::kCandBlock | 1u << mxfp6::kCandBlockWide));
+    (void)apply_choice(t, tc, s);
+  }
+  if (tc.cand < 0 && !apply_ragged(t, s)) return false;
+  e = hipSuccess;
+  if (na && nb) e = mxfp6::launch_pad_both(g.A, pa, g.As, sa, g.M, g.B, pb, g.Bs, sb, g.N, g.K, s);
+  else if (na) e = mxfp6::launch_pad_both(g.A, pa, g.As, sa, g.M, nullptr, nullptr, nullptr, nullptr, 0, g.K, s);
+  else if (nb) e = mxfp6::launch_pad_both(g.B, pb, g.Bs, sb, g.N, nullptr, nullptr, nullptr, nullptr, 0, g.K, s);
+  if (e == hipSuccess) e = tc.cand >= mxfp6::kCandTiled256 && (kTiledFamily >> tc.cand & 1) ? mxfp6::launch_gemm_tiled(t, s) : mxfp6::launch_gemm_block(t, s);
+  return true;
+}
+
 // The argument checks shared by the gemm entry points (c_align: alignment mask of C).  *empty: nothing to compute.
 int check_gemm_args(const void* A, const void* B, const void* As, const void* Bs, const void* C, int M, int N, int K, int fmt_a, int fmt_b,
                     uintptr_t c_align, int layout_a, int layout_b, const mxfp6::Epilogue& ep, bool* empty) {
@@ -385,6 +422,7 @@ int gemm_common(const void* A, const void* B, const void* As, const void* Bs, vo
     e = mxfp6::launch_gemm_block(g, s);
   } else {
     mxfp6::KernelChoice c = auto_choice(g, force_split, true);
+    if (K != 0 && (c.cand < 0 || c.cand == mxfp6::kCandSlice) && !mxfp6::gemm_block_supports(g) && padded_then_gemm(g, c, nullptr, s, e)) return e == hipSuccess ? MXFP6_OK : (int)e;
     // a split needs this stream's workspace: without it, what the shape gets otherwise
     if (!apply_choice(g, c, s)) {
       c = auto_choice(g, force_split, false);
@@ -469,9 +507,24 @@ int mxfp6_linear(const void* X, int x_bf16, const void* W, const void* Ws, void*
   // skinny kernel, and so does a partial last tile for a forced kernel that takes a row-major A only (skinny, mid).
   const bool forced_row = g_force == 3 || g_force == 4 || (g_force >= 7 && g_force <= 16) || (g_force >= 19 && g_force <= 21);
   const int layout_x = M >= 64 && K % 128 == 0 && (M % 32 == 0 || !forced_row) ? MXFP6_LAYOUT_TILE : MXFP6_LAYOUT_ROW;
+  std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
+  // Sizes that no kernel takes as they are: the activations quantised straight into a padded tile-major operand, a copy of the weights
+  if (K > 0 && g_force == 0 && (K % 128 || N % 8)) {
+    mxfp6::GemmArgs g{(const uint8_t*)X, (const uint8_t*)W, (const uint8_t*)X, (const uint8_t*)Ws, C, M, N, K, fmt_x, fmt_w, false, layout_x, layout_w};
+    const mxfp6::KernelChoice other = auto_choice(g, 0, true);
+    mxfp6::GemmArgs t = g;
+    mxfp6::KernelChoice tc{-1, 1, 0, 0.0};
+    g.layout_a = 1, g.ep = ep;
+    if (g_relayout && g_padded >= 0 && mxfp6::padded_pays(g, g_ksplit, auto_mask(g, 0), g_padded > 0 ? mxfp6::KernelChoice{mxfp6::kCandSlice, 1, 0, 1e30} : other, true, &t, &tc)) {
+      uint8_t* const xp = stream_workspace(s, 4, padded_bytes(M, K));
+      if (!xp) return MXFP6_EWORKSPACE;
+      hipError_t e = mxfp6::launch_quantize(X, x_bf16 != 0, xp, padded_scales(xp, M, K), M, K, fmt_x, 1, s);
+      if (e != hipSuccess) return (int)e;
+      if (padded_then_gemm(g, other, xp, s, e)) return e == hipSuccess ? MXFP6_OK : (int)e;
+    }
+  }
   const size_t rows = ((size_t)M + 31) & ~(size_t)31;
   const size_t nx = (rows * (K / 32) * 24 + 255) & ~(size_t)255, ns = rows * ((K + 511) / 512) * 16;
-  std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
   uint8_t* xp = K > 0 ? stream_workspace(s, 4, nx + ns) : nullptr;
   if (K > 0) {
     if (!xp) return MXFP6_EWORKSPACE;
@@ -774,6 +827,12 @@ int mxfp6_probe_block(int enable) {
   return prev;
 }
 
+
+int mxfp6_probe_padded(int mode) {
+  const int prev = g_padded;
+  g_padded = mode;
+  return prev;
+}
 
 int mxfp6_probe_slice(int plan) {
   const int prev = g_slice;

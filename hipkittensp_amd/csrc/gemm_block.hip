@@ -113,9 +113,9 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   // (a share's resources start at its first K-tile, 96 or 3072 bytes times kt0 into a row or row-tile, and end that much
   // earlier, so that rows past the tile's last still lie beyond the end)
   const uint32_t oa = (uint32_t)kt0 * (layout_a ? 3072 : 96), ob = (uint32_t)kt0 * (layout_b ? 3072 : 96);
-  // (a tile-major A may end in a partial row-tile: its rows past M are there, of no meaning)
+  // (a tile-major operand may end in a partial row-tile: its rows past the end are there, of no meaning)
   const __amdgpu_buffer_rsrc_t rA = make_rsrc(args.A + (size_t)pm * kBM * rowbytes + oa, (uint32_t)(layout_a ? (rows_a + 31) & ~31 : rows_a) * rowbytes - oa);
-  const __amdgpu_buffer_rsrc_t rB = make_rsrc(args.B + (size_t)pn * kBN * rowbytes + ob, (uint32_t)rows_b * rowbytes - ob);
+  const __amdgpu_buffer_rsrc_t rB = make_rsrc(args.B + (size_t)pn * kBN * rowbytes + ob, (uint32_t)(layout_b ? (rows_b + 31) & ~31 : rows_b) * rowbytes - ob);
   const __amdgpu_buffer_rsrc_t rZ = make_rsrc(args.A, 0);
   // scales: the first half of the waves fetch A's (rows 0-63, 64-127 of the tile; with eight waves, waves 2, 3 fetch what
   // waves 0, 1 fetch, into the same place, so that every wave issues one scale load per group), the second half B's, 64

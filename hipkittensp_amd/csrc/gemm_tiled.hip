@@ -198,8 +198,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
   auto operand_rsrc = [&](int tile, int kt0) __attribute__((always_inline)) {
     const auto g = fresh_args();
     const int pm = tile < 0 ? 0 : tile & 0xffff, pn = tile < 0 ? 0 : tile >> 16;
-    const int valid_a = tile < 0 ? 0 : min(kBM, g->M - pm * kBM), rows_b = tile < 0 ? 0 : min(kBN, g->N - pn * kBN);
-    const int rows_a = layout_a ? (valid_a + 31) & ~31 : valid_a;  // a tile-major A may end in a partial row-tile: its rows past M are there, of no meaning
+    const int valid_a = tile < 0 ? 0 : min(kBM, g->M - pm * kBM), valid_b = tile < 0 ? 0 : min(kBN, g->N - pn * kBN);
+    // a tile-major operand may end in a partial row-tile: its rows past the end are there, of no meaning
+    const int rows_a = layout_a ? (valid_a + 31) & ~31 : valid_a, rows_b = layout_b ? (valid_b + 31) & ~31 : valid_b;
     if constexpr (SPLIT) {  // a wave loads one operand only: rA is that operand's resource (no branch at the loads)
       rA = sc_a ? make_rsrc(g->A + (size_t)pm * kBM * rowbytes, (uint32_t)rows_a * rowbytes)
                 : make_rsrc(g->B + (size_t)pn * kBN * rowbytes, (uint32_t)rows_b * rowbytes);

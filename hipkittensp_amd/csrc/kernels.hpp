@@ -65,6 +65,7 @@ struct KernelChoice {
 int device_cus();
 double candidate_model_us(const GemmArgs& g, int cand, int want_split, int cus, int* shares, int* rows);  // modelled microseconds; < 0: the candidate does not take the shape
 KernelChoice choose_kernel(const GemmArgs& g, int want_split, bool allow_split, unsigned mask = ~0u);  // mask: bit per Candidate that may be chosen; want_split: 0 = by the model, 1 = never, n = n shares where a candidate splits; allow_split: a workspace is to be had
+bool padded_pays(const GemmArgs& g, int want_split, unsigned mask, const KernelChoice& other, bool a_done, GemmArgs* t, KernelChoice* c);  // a ragged product on padded tile-major copies
 KernelChoice choose_linear_kernel(const GemmArgs& g, int want_split, unsigned mask);  // g.X, g.x_bf16: the activations
 int tiled_split_shares(const GemmArgs& g, int want, int cus, int bm);  // the tiled kernel's K split with tiles of bm (256 or 128) rows when it is to split: shares (1 = the shape has none)
 int ragged_shares(const GemmArgs& g, int want, bool allow_split);  // shapes no candidate takes: shares of the block kernel's K split (1 = unsplit), 0 = the generic kernel
@@ -95,6 +96,8 @@ hipError_t release_split_workspaces();             // returns every K-split work
 hipError_t launch_quantize(const void* X, int x_bf16, uint8_t* packed, uint8_t* scales, int rows, int K, int fmt, int layout, hipStream_t s);
 hipError_t launch_tile_operand(const uint8_t* src, uint8_t* dst, int rows, int K, int tile, hipStream_t s);
 hipError_t launch_tile_scales(const uint8_t* src, uint8_t* dst, int rows, int K, int tile, hipStream_t s);
+hipError_t launch_pad_both(const uint8_t* src0, uint8_t* dst0, const uint8_t* ssrc0, uint8_t* sdst0, int rows0, const uint8_t* src1, uint8_t* dst1, const uint8_t* ssrc1,
+                           uint8_t* sdst1, int rows1, int K, hipStream_t s);  // any size and alignment -> padded tile-major; rows1 == 0: one operand
 hipError_t launch_tile_both(const uint8_t* src0, uint8_t* dst0, const uint8_t* ssrc0, uint8_t* sdst0, int rows0, const uint8_t* src1,
                             uint8_t* dst1, const uint8_t* ssrc1, uint8_t* sdst1, int rows1, int K, hipStream_t s);
 hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t s);

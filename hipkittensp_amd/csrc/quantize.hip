@@ -43,7 +43,7 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t buf = (uint32_t)(uintptr_t)(MXFP6_LDS uint8_t*)smem + wave * kChunk;
-  const int nkt = nkb / 4;  // tile-major only: K-tiles per row
+  const int nkt = (nkb + 3) / 4;  // tile-major only: K-tiles per row (the last one padded with zeros)
   const long nchunks = layout ? (long)((rows + 15) / 16) * nkt : (nblocks + 63) / 64;
   const long stride = (long)gridDim.x * kQWaves;
   long chunk = (long)blockIdx.x * kQWaves + wave;
@@ -63,7 +63,7 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
     if (layout) {
       const long g16 = ch / nkt, kt = ch - g16 * nkt;
       base = reinterpret_cast<const uint8_t*>(X) + (g16 * 16 * nkb + kt * 4) * BB;
-      len = (uint32_t)((min(16, rows - (int)g16 * 16) - 1) * nkb * BB + 4 * BB);  // rows past the last read as zeros
+      len = (uint32_t)((min(16, rows - (int)g16 * 16) - 1) * nkb * BB + min(4, nkb - (int)kt * 4) * BB);  // rows past the last read as zeros
     } else {
       const long left = nblocks * BB - ch * kChunk;
       base = reinterpret_cast<const uint8_t*>(X) + ch * kChunk;
@@ -85,6 +85,10 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
 #pragma unroll
     for (int c = 0; c < P; c++) x[c] = *reinterpret_cast<const v4i*>(smem + wave * kChunk + lane * BB + ((c ^ (lane % P)) * 16));
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (layout && (nkb & 3) && (int)(chunk % nkt) * 4 + (lane & 3) >= nkb) {  // K-blocks past K
+#pragma unroll
+      for (int c = 0; c < P; c++) x[c] = v4i{0, 0, 0, 0};
+    }
 
     int sb;
     u32x6 w;
@@ -120,10 +124,10 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
     if (layout == 0) {
       if (chunk * 64 + lane < nblocks) scales[chunk * 64 + lane] = (uint8_t)sb;
     } else {
-      uint8_t* const sp = scales + tile_major_scale_offset(row, kt * 4 + (lane & 3), (nkb + 15) / 16);
+      uint8_t* const sp = scales + tile_major_scale_offset(row, kt * 4 + (lane & 3), (nkt + 3) / 4);
       *sp = (uint8_t)sb;
       if (kt == nkt - 1)  // the bytes of K-blocks past K (K % 512 != 0) are zeros
-        for (int b = 4; b < 16 - ((nkb - 4) & 15); b += 4) sp[b] = 0;
+        for (int b = 4; b < 16 - ((nkt * 4 - 4) & 15); b += 4) sp[b] = 0;
     }
   }
 }
@@ -131,7 +135,7 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
 hipError_t launch_quantize(const void* X, int x_bf16, uint8_t* packed, uint8_t* scales, int rows, int K, int fmt, int layout, hipStream_t s) {
   const long nblocks = (long)rows * (K / 32);
   if (nblocks == 0) return hipSuccess;
-  const long nchunks = layout ? (long)((rows + 15) / 16) * (K / 128) : (nblocks + 63) / 64, want = (nchunks + kQWaves - 1) / kQWaves;
+  const long nchunks = layout ? (long)((rows + 15) / 16) * ((K + 127) / 128) : (nblocks + 63) / 64, want = (nchunks + kQWaves - 1) / kQWaves;
   const long most = 0xffffffffL / (kQWaves * 64);  // a launch has less than 2^32 work-items; the chunks past them are the grid's next round
   const unsigned grid = (unsigned)(want < most ? want : most);
   const int stream_in = (size_t)rows * K * (x_bf16 ? 2 : 4) >= kCacheBytes, stream_out = (size_t)rows * (K / 4 * 3) >= kStreamBytes;
@@ -254,6 +258,76 @@ hipError_t launch_tile_both(const uint8_t* src0, uint8_t* dst0, const uint8_t* s
   const unsigned blocks = j0.pblocks + j0.sblocks + j1.pblocks + j1.sblocks;
   if (blocks == 0) return hipSuccess;
   tile_both_kernel<<<blocks, 256, 0, s>>>(j0, j1, nkt, nkb, nk4);
+  return hipGetLastError();
+}
+
+// The same for operands of any size and alignment: row-major -> tile-major with K padded to whole K-tiles and the rows to whole
+// row-tiles, zeros in both.  A row's scales start at any byte: five aligned dwords (the resource ends at the dword that holds the
+// tensor's last byte) are shifted into place.
+struct PadJob {
+  const uint8_t *src, *ssrc;
+  uint8_t *dst, *sdst;
+  int rows;
+  unsigned pblocks, sblocks;
+};
+__global__ __launch_bounds__(256) void pad_both_kernel(PadJob j0, PadJob j1, int nkb, int nkt, int nk4) {
+  unsigned bid = blockIdx.x;
+  const bool second = bid >= j0.pblocks + j0.sblocks;
+  if (second) bid -= j0.pblocks + j0.sblocks;
+  const PadJob& j = second ? j1 : j0;
+  const int rowbytes = nkb * 24;
+  if (bid < j.pblocks) {
+    const int rt = bid / nk4, g = bid - rt * nk4, ntile = min(4, nkt - 4 * g);
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(j.src + (size_t)rt * 32 * rowbytes, (uint32_t)min(32, j.rows - rt * 32) * rowbytes);
+    uint8_t* const dst = j.dst + ((size_t)rt * nkt + 4 * g) * 3072;
+    v4i v[3];
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const int p = threadIdx.x + 256 * i, row = p / 24, q = p - row * 24, at = g * 384 + q * 16;
+      v[i] = at < rowbytes ? __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, row * rowbytes + at, 0, 0)) : v4i{0, 0, 0, 0};
+      if (at + 16 > rowbytes) v[i][2] = v[i][3] = 0;  // rows are whole runs of 8 bytes
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const int p = threadIdx.x + 256 * i, row = p / 24, q = p - row * 24, tg = q / 6, c = q - tg * 6;
+      if (tg < ntile) *reinterpret_cast<v4i*>(dst + tg * 3072 + (row * 6 + (c ^ ((row >> 3) & 1))) * 16) = v[i];
+    }
+  } else {
+    const long s = (long)(bid - j.pblocks) * 256 + threadIdx.x;
+    const long row = s / nk4;
+    const int g = (int)(s - row * nk4);
+    if (row >= ((j.rows + 31) & ~31)) return;
+    v4i out = {0, 0, 0, 0};
+    if (row < j.rows) {
+      const size_t at = (size_t)row * nkb + g * 16, end = ((uintptr_t)j.ssrc + (size_t)j.rows * nkb + 3) & ~(uintptr_t)3;
+      const uintptr_t from = (uintptr_t)j.ssrc + at;
+      const uint32_t* const d = reinterpret_cast<const uint32_t*>(from & ~(uintptr_t)3);
+      uint32_t w[5];
+#pragma unroll
+      for (int i = 0; i < 5; i++) w[i] = (uintptr_t)(d + i) < end ? d[i] : 0u;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int valid = nkb - g * 16 - 4 * i;
+        const uint32_t keep = valid >= 4 ? ~0u : valid <= 0 ? 0u : (1u << (8 * valid)) - 1;
+        out[i] = (int)(__builtin_amdgcn_alignbyte(w[i + 1], w[i], (uint32_t)from) & keep);
+      }
+    }
+    *reinterpret_cast<v4i*>(j.sdst + tile_major_scale_offset((int)row, g * 16, nk4)) = out;
+  }
+}
+
+// rows1 == 0: only the first operand
+hipError_t launch_pad_both(const uint8_t* src0, uint8_t* dst0, const uint8_t* ssrc0, uint8_t* sdst0, int rows0, const uint8_t* src1, uint8_t* dst1, const uint8_t* ssrc1,
+                           uint8_t* sdst1, int rows1, int K, hipStream_t s) {
+  const int nkb = K / 32, nkt = (nkb + 3) / 4, nk4 = (nkt + 3) / 4;
+  auto job = [&](const uint8_t* src, uint8_t* dst, const uint8_t* ssrc, uint8_t* sdst, int rows) {
+    const long tiles = ((long)rows + 31) / 32;
+    return PadJob{src, ssrc, dst, sdst, rows, (unsigned)(tiles * nk4), (unsigned)((tiles * 32 * nk4 + 255) / 256)};
+  };
+  const PadJob j0 = job(src0, dst0, ssrc0, sdst0, rows0), j1 = job(src1, dst1, ssrc1, sdst1, rows1);
+  const unsigned blocks = j0.pblocks + j0.sblocks + j1.pblocks + j1.sblocks;
+  if (blocks == 0) return hipSuccess;
+  pad_both_kernel<<<blocks, 256, 0, s>>>(j0, j1, nkb, nkt, nk4);
   return hipGetLastError();
 }
 

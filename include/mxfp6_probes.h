@@ -98,6 +98,10 @@ int mxfp6_probe_block(int enable);
  * default) leaves it to the choice; returns the previous setting.  Plans that are not built fail with hipErrorInvalidValue. */
 int mxfp6_probe_slice(int plan);
 
+/* Measurement switch, per calling thread: 1 = every ragged product of the automatic path on padded tile-major copies of its operands, -1 =
+ * none, 0 (the default) = where that pays; returns the previous setting. */
+int mxfp6_probe_padded(int mode);
+
 #ifdef __cplusplus
 }
 #endif

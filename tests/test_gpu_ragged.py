@@ -98,3 +98,86 @@ def test_short_ragged_products_start_on_the_generic_kernel(hk, M, N, K, generic)
     bp, bsc = co.quantise(o.make_source("weights", (N, K), np.random.default_rng(N + K)), 2)
     got = call(hk, *(at(x, 0) for x in (ap, bp, asc, bsc)), M, N, 2, 2, torch.float32).cpu().numpy()
     assert o.rel_err(got, o.gemm_ref(ap, bp, asc, bsc, acc=np.float64)) <= 1e-5
+
+
+@pytest.fixture
+def padded():
+    """Every ragged call of the measurement build on padded tile-major copies of its operands."""
+    import ctypes
+
+    from hipkittensp_amd import _lib
+
+    P = _lib.probes()
+    P.mxfp6_probe_padded.argtypes, P.mxfp6_probe_padded.restype = [ctypes.c_int], ctypes.c_int
+    prev = P.mxfp6_probe_padded(1)
+    yield P
+    P.mxfp6_probe_padded(prev)
+
+
+@pytest.mark.parametrize("M,N,K,offs,fa,fb", [(1, 1, 32, (0, 0, 0, 0, 0), 2, 2), (33, 65, 160, (4, 12, 1, 3, 1), 2, 3), (31, 264, 480, (8, 4, 2, 1, 0), 3, 2), (256, 256, 2080, (0, 0, 0, 0, 0), 2, 2),
+                                              (129, 2048, 1056, (4, 8, 3, 2, 0), 2, 2), (100, 1003, 672, (0, 0, 0, 0, 3), 2, 2), (300, 40, 640, (4, 0, 0, 0, 0), 2, 2), (64, 8, 8224, (0, 0, 1, 1, 0), 2, 2)])
+@pytest.mark.parametrize("f32", [0, 1])
+def test_padded_copies_vs_oracle(hk, padded, M, N, K, offs, fa, fb, f32):
+    ap, asc = co.quantise(o.make_source("normal", (M, K), np.random.default_rng(M + K)), fa)
+    bp, bsc = co.quantise(o.make_source("weights_outliers", (N, K), np.random.default_rng(N + K)), fb)
+    ref = o.gemm_ref(ap, bp, asc, bsc, fa, fb, acc=np.float64)
+    ops = [at(x, off) for x, off in zip((ap, bp, asc, bsc), offs)]
+    guard = torch.full((M * N + 64,), 7.0, dtype=torch.float32 if f32 else torch.bfloat16, device="cuda")
+    C = guard[16 + offs[4]:16 + offs[4] + M * N]
+    rc = padded.mxfp6_gemm_ex(*(t.data_ptr() for t in (*ops, C)), M, N, K, fa, fb, 0, 0, f32, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert rc == 0 and bool((guard[:16 + offs[4]] == 7.0).all()) and bool((guard[16 + offs[4] + M * N:] == 7.0).all())
+    got = C.view(M, N).float().cpu().numpy()
+    # fp32: the sums' own bound; bf16: half a last place on top, 2^-8 of the value
+    bound = 1e-5 * np.maximum(np.abs(ref), 0.01 * np.sqrt((ref**2).mean())) + (0 if f32 else np.abs(ref) * 2.0**-8)
+    assert np.isfinite(got).all() and (np.abs(got - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("M,N,K,bf16", [(64, 96, 160, 1), (129, 1056, 672, 0), (200, 264, 2080, 1), (333, 515, 640, 1), (70, 8, 96, 0)])
+def test_padded_linear_vs_oracle(hk, padded, M, N, K, bf16):
+    """The quantiser writes the padded operand itself; NaN bit patterns in the workspace before the call reach nothing."""
+    x = torch.from_numpy(o.make_source("normal", (M, K), np.random.default_rng(M)).astype(np.float32))
+    x = x.to(torch.bfloat16) if bf16 else x
+    ap, asc = co.quantise(x.float().numpy(), 2)
+    bp, bsc = co.quantise(o.make_source("weights", (N, K), np.random.default_rng(N)), 2)
+    ref = o.gemm_ref(ap, bp, asc, bsc, acc=np.float64)
+    b, bs = at(bp, 0), at(bsc, 1)
+    C = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    for fill in (float("nan"), 0.0):
+        big, junk = torch.full((2 * M, K + 128), fill, device="cuda"), torch.empty(2 * M, N, dtype=torch.bfloat16, device="cuda")
+        prev = padded.mxfp6_probe_slice(-1)
+        try:
+            assert padded.mxfp6_linear(big.data_ptr(), 0, b.data_ptr(), bs.data_ptr(), junk.data_ptr(), M, N, K, 2, 2, 0, None, 0, 0, stream) == 0
+            xc = at((x.view(torch.int16) if bf16 else x).numpy().view(np.uint8), 0)
+            assert padded.mxfp6_linear(xc.data_ptr(), bf16, b.data_ptr(), bs.data_ptr(), C.data_ptr(), M, N, K, 2, 2, 0, None, 0, 0, stream) == 0
+        finally:
+            padded.mxfp6_probe_slice(prev)
+        torch.cuda.synchronize()
+        got = C.float().cpu().numpy()
+        bound = 1e-5 * np.maximum(np.abs(ref), 0.01 * np.sqrt((ref**2).mean())) + np.abs(ref) * 2.0**-8
+        assert np.isfinite(got).all() and (np.abs(got - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(2604, 704, 5664), (2048, 3784, 3680)])
+def test_padded_route_and_capture(hk, M, N, K):
+    """Products the choice gives to padded copies: the bits of the block kernel's ragged instantiations (sums in the same order), and
+    under capture on a stream without a workspace, where those run."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    (a, asc), (b, bsc) = hk.quantize(torch.randn(M, K, device="cuda", generator=g)), hk.quantize(torch.randn(N, K, device="cuda", generator=g) * 0.02)
+    prev, want, got = hk.tk_kernel.set_relayout(0), torch.empty(M, N, device="cuda"), torch.empty(M, N, device="cuda")
+    try:
+        hk.dispatch_micro(a, b, asc, bsc, want)
+    finally:
+        hk.tk_kernel.set_relayout(prev)
+    hk.dispatch_micro(a, b, asc, bsc, got)
+    assert torch.equal(got, want)
+    graph, C = torch.cuda.CUDAGraph(), torch.zeros(M, N, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        hk.dispatch_micro(a, b, asc, bsc, C)
+    for _ in range(3):
+        C.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C, want)
