@@ -2,7 +2,7 @@
 // kernel selection.  Nothing here synchronises the device.  Allocations, all from the stream-ordered allocator on the
 // caller's stream and all kept per (device, stream) until mxfp6_release_workspaces(): the workspace of the re-layout
 // pre-pass (relayout_then_tiled; mxfp6_set_relayout(0) switches it off), the fp32 workspace of mxfp6_gemm_fused_fp6
-// on shapes that the skinny, ring, ragged and generic kernels run, the packed activations of mxfp6_linear (not under capture), the
+// on shapes that the ragged and generic kernels and the skinny kernel's narrow workgroups run, the packed activations of mxfp6_linear (not under capture), the
 // partial sums of the tiled, block, ring and slice kernels' K splits (apply_choice, apply_ragged: one workspace, shared) with the ring
 // and slice kernels' arrival counters, and the K-split workspace of the skinny kernel (gemm_skinny.hip).  mxfp6_gemm_noalloc allocates nothing.
 #include "../../include/mxfp6_gemm.h"
@@ -550,8 +550,8 @@ int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const voi
   hipStream_t s = (hipStream_t)stream;
   // The tiled and the block kernel and the reduction of a K split quantise their sums themselves (us, block kernel through the fp32
   // workspace and the quantiser / here: 256 x 2560 x 2304 16.7 / 13.0, 500 x 8192 x 8192 38.3 / 30.6, 2048 x 4096 x 4096 41.4 / 32.0,
-  // 3000 x 2048 x 1024 24.9 / 11.6).  Skinny, ring, ragged and generic products, and a split without its workspace, go through the
-  // workspace.  The choice is that of the same call with fp32 output, whose bits these are (only an activation may count otherwise,
+  // 3000 x 2048 x 1024 24.9 / 11.6), and so do the slice, ring and skinny kernels.  The skinny kernel's workgroups of 16 rows of B,
+  // ragged and generic products, and a split without its workspace, go through the workspace.  The choice is that of the same call with fp32 output, whose bits these are (only an activation may count otherwise,
   // between kernels that add up in the same order); where that is the tiled kernel's 128 x 128 tile, which has no fp6 form, the
   // best of the kernels that add up in the same order.
   mxfp6::GemmArgs g{(const uint8_t*)A, (const uint8_t*)B, (const uint8_t*)As, (const uint8_t*)Bs, nullptr, M, N, K, fmt_a, fmt_b, true, layout_a, layout_b};
@@ -572,6 +572,10 @@ int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const voi
     c = mxfp6::choose_kernel(g, 1, false, 1u << mxfp6::kCandBlockWide);
   } else if (K > 0 && force >= 22 && force <= 24) {
     c = family_choice(g, 1u << mxfp6::kCandBlock, 1u << mxfp6::kCandBlockSplit);
+  } else if (K > 0 && force == 28) {
+    c = mxfp6::choose_kernel(g, g_ksplit, true, 1u << mxfp6::kCandRing);
+  } else if (K > 0 && (force == 3 || (force >= 7 && force <= 16) || (force >= 19 && force <= 21))) {
+    c.cand = mxfp6::kCandSkinny;
   }
   // Runs the call as chosen, C quantised where it is summed; false: that choice has no fp6 form, or its workspace is not to be had
   auto run = [&](const mxfp6::KernelChoice& ch, hipError_t& e) {
@@ -580,11 +584,14 @@ int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const voi
     // (the unsplit tiled kernel: C on 16 bytes, as ever; the others store fp6 8 bytes at a time)
     const bool tiled = (ch.cand == mxfp6::kCandTiled256 || ch.cand == mxfp6::kCandTiled128x256) && ((uintptr_t)C_packed & 15) == 0;
     mxfp6::GemmArgs t = g;
-    const bool slice = ch.cand == mxfp6::kCandSlice;
-    if (!(block || split || tiled || slice) || !apply_choice(t, ch, s)) return false;
+    const bool slice = ch.cand == mxfp6::kCandSlice, ring = ch.cand == mxfp6::kCandRing, skinny = ch.cand == mxfp6::kCandSkinny;
+    if (force == 3 || (force >= 7 && force <= 16) || (force >= 19 && force <= 21)) t.skinny_geometry = force == 3 ? 0 : force >= 19 ? force - 8 : force - 6;
+    if (!(block || split || tiled || slice || ring || (skinny && mxfp6::gemm_skinny_stores_fp6(t))) || !apply_choice(t, ch, s)) return false;
     t.C = C_packed, t.f32out = false, t.C_scale = (uint8_t*)C_scale, t.fmt_c = fmt_c;
     if (force == 23 || force == 24) t.tile_rows = force == 23 ? 3 : 6;
     if (slice) e = mxfp6::launch_gemm_slice(t, ch.slice, s);
+    else if (ring) e = mxfp6::launch_gemm_ring(t, s);
+    else if (skinny) e = mxfp6::launch_gemm_skinny(t, s);
     else if (block) e = mxfp6::launch_gemm_block(t, s);
     else if (split || force != 0 || !relayout_then_tiled(t, s, e)) e = mxfp6::launch_gemm_tiled(t, s);
     return true;

@@ -20,7 +20,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // unrounded accumulators, used to state the accuracy contract before the bf16 rounding).
 struct OutBf16 { typedef uint16_t type; };
 struct OutF32 { typedef float type; };
-struct OutFp6 { typedef uint8_t type; };  // C re-quantised to MXFP6: packed [M, 3N/4] + E8M0 [M, N/32] (tiled and block kernels, reduction of a K split)
+struct OutFp6 { typedef uint8_t type; };  // C re-quantised to MXFP6: packed [M, 3N/4] + E8M0 [M, N/32]
 
 // E8M0 byte of a 32-block with largest magnitude amax (floor(log2(amax)) - emax, clamped; 0 for an all-zero block)
 __device__ __forceinline__ int e8m0_of_amax(float amax, int emax) {

@@ -46,6 +46,8 @@ struct RingArgs {
   int M, N, K, layout_a, layout_b, col_tiles, m_blocks, nsplit;
   int stream;  // B is read with the non-temporal bit (kStreamBytes)
   Epilogue ep;
+  uint8_t* C_scale;  // fp6 output only
+  int fmt_c;
 };
 
 template <typename F>
@@ -298,6 +300,23 @@ __global__ __launch_bounds__((kRingNC + 1) * 64) void gemm_ring_kernel(const Rin
     return;
   }
   const bool has_ep = epilogue_any(args.ep);
+  if constexpr (sizeof(OutT) == 1) {
+    // MXFP6 output (N % 32 == 0): a wave's 32 columns are one 32-block of every row, which lanes l and l + 32 hold half each; the
+    // lower lanes quantise and store it.  A row-tile at a time: two side by side, one for either half of the wave, spilled registers
+    // by the thousand (40 x 24576 x 6144 went from 30 to 470 us).
+    if (n0 >= N) return;
+#pragma unroll
+    for (int t = 0; t < TA; t++) {
+      const long m = (long)m0 + 32 * t + r32;
+      v16f c = acc[t];
+      if (has_ep && m < M) {
+#pragma unroll
+        for (int e = 0; e < 16; e++) c[e] = epilogue_apply(args.ep, c[e], m, (long)n0 + 8 * (e >> 2) + 4 * h + (e & 3));
+      }
+      store_fp6_band(c, c, args.fmt_c, reinterpret_cast<uint8_t*>(args.C), args.C_scale, h ? (long)M : m, M, n0 / 32 - h, N / 32);
+    }
+    return;
+  } else {
 #pragma unroll
   for (int t = 0; t < TA; t++) {
     const long m = (long)m0 + 32 * t + r32;
@@ -312,6 +331,7 @@ __global__ __launch_bounds__((kRingNC + 1) * 64) void gemm_ring_kernel(const Rin
       }
       store4(reinterpret_cast<OutT*>(args.C) + (size_t)m * N + n, v[0], v[1], v[2], v[3]);
     }
+  }
   }
 }
 
@@ -377,7 +397,7 @@ static hipError_t launch(const GemmArgs& g, hipStream_t s) {
   RingPlan p = ring_plan(g, split ? g.ksplit : 1);
   if (split && p.nsplit != g.ksplit) return hipErrorInvalidValue;
   RingArgs ra = {g.A, g.B, g.As, g.Bs, g.C, g.ks_part, g.ks_counters, g.M, g.N, g.K, g.layout_a, g.layout_b, p.col_tiles, p.m_blocks, p.nsplit,
-                 p.m_blocks == 1 && (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes, g.ep};
+                 p.m_blocks == 1 && (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes, g.ep, g.C_scale, g.fmt_c};
   const unsigned grid = (unsigned)p.col_tiles * p.m_blocks * p.nsplit;
   constexpr int threads = (kRingNC + 1) * 64;
   if (p.ta == 1) gemm_ring_kernel<FA, FB, Out, 1><<<grid, threads, 0, s>>>(ra);
@@ -388,7 +408,7 @@ static hipError_t launch(const GemmArgs& g, hipStream_t s) {
 
 hipError_t launch_gemm_ring(const GemmArgs& g, hipStream_t s) {
 #define MXFP6_CASE(FA, FB) \
-  if (g.fmt_a == FA && g.fmt_b == FB) return g.f32out ? launch<FA, FB, OutF32>(g, s) : launch<FA, FB, OutBf16>(g, s);
+  if (g.fmt_a == FA && g.fmt_b == FB) return g.fmt_c ? launch<FA, FB, OutFp6>(g, s) : g.f32out ? launch<FA, FB, OutF32>(g, s) : launch<FA, FB, OutBf16>(g, s);
   MXFP6_CASE(2, 2) MXFP6_CASE(2, 3) MXFP6_CASE(3, 2) MXFP6_CASE(3, 3)
 #undef MXFP6_CASE
   return hipErrorInvalidValue;

@@ -56,7 +56,8 @@ template <int FA, int FB, typename Out, int AR, int NW, int BR, int DB, bool XQ 
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                                                               const uint8_t* __restrict__ As, const uint8_t* __restrict__ Bs,
                                                               typename Out::type* __restrict__ C, int M, int N, int K, int layout_b,
-                                                              const Epilogue ep, int nsplit, float* ws_part, int* ws_cnt, int stream) {
+                                                              const Epilogue ep, int nsplit, float* ws_part, int* ws_cnt, int stream,
+                                                              uint8_t* __restrict__ C_scale, int fmt_c) {
   static_assert(BR == 64 || BR == 32 || BR == 16, "rows of B per workgroup");
   static_assert(AR == 16 || AR == 32 || AR == 64 || AR == 128, "rows of A");
   constexpr int TA = AR > 32 ? AR / 32 : 1;   // 32-row tiles of A per wave
@@ -273,6 +274,37 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
     for (int e = 0; e < 16; e++) part[((wave * TT + t) * 16 + e) * 64 + lane] = acc[t][e];
   __syncthreads();
   const bool has_ep = epilogue_any(ep);
+  // MXFP6 output (N % 32 == 0, BR >= 32): the finished values go back to LDS, over partial sums that only their own thread reads, and a
+  // thread quantises each 32-block of a row.  What it saves is the fp32 matrix' way through memory and the quantiser's launch.
+  auto finish = [&](int idx, float v) __attribute__((always_inline)) {
+    const int tt = idx >> 10, e = (idx >> 6) & 15, l = idx & 63;
+    const int m = (tt / TB) * 32 + (l & 31), nl = (tt % TB) * 32 + 8 * (e >> 2) + 4 * (l >> 5) + (e & 3);
+    const long nn = (long)n0 + nl;
+    const bool inside = m < M && nl < BR && nn < N;
+    if (inside && has_ep) v = epilogue_apply(ep, v, m, nn);
+    if constexpr (sizeof(*C) == 1) part[idx] = v;
+    else if (inside) store1(C + (long)m * N + nn, v);
+  };
+  auto store_fp6 = [&]() __attribute__((always_inline)) {
+    if constexpr (sizeof(*C) == 1) {
+      static_assert(BR >= 32, "a workgroup holds whole 32-blocks");
+      __syncthreads();
+      const int nkb = N / 32;
+      for (int u = tid; u < TT * 32; u += NW * 64) {
+        const int tt = u >> 5, row = u & 31, m = (tt / TB) * 32 + row, blk = n0 / 32 + tt % TB;
+        if (m >= M || blk >= nkb) continue;
+        float p0[16], p1[16];
+#pragma unroll
+        for (int e = 0; e < 16; e++) p0[e] = part[(tt * 16 + e) * 64 + row], p1[e] = part[(tt * 16 + e) * 64 + 32 + row];
+        int sb;
+        const u32x6 w = quantise_block_acc(p0, p1, fmt_c, sb);
+        u32x2* const dst = reinterpret_cast<u32x2*>(C + ((size_t)m * nkb + blk) * 24);
+#pragma unroll
+        for (int i = 0; i < 3; i++) dst[i] = u32x2{w[2 * i], w[2 * i + 1]};
+        C_scale[(size_t)m * nkb + blk] = (uint8_t)sb;
+      }
+    }
+  };
   if (nsplit > 1) {
     // K split between workgroups: every workgroup leaves its partial tile in the workspace; the one that arrives last
     // (a counter per tile) adds them up in split order, so the result does not depend on who that is.  The other
@@ -295,27 +327,21 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
     if (!*flag) return;
     const float* all = ws_part + (size_t)tile * nsplit * (TT * 1024);
     for (int idx = tid; idx < TT * 1024; idx += NW * 64) {
-      const int tt = idx >> 10, e = (idx >> 6) & 15, l = idx & 63;
       float t = 0.f;
       for (int q = 0; q < nsplit; q++) t += __hip_atomic_load(all + q * (TT * 1024) + idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const int m = (tt / TB) * 32 + (l & 31);
-      const int nl = (tt % TB) * 32 + 8 * (e >> 2) + 4 * (l >> 5) + (e & 3);
-      const long nn = (long)n0 + nl;
-      if (m < M && nl < BR && nn < N) store1(C + (long)m * N + nn, has_ep ? epilogue_apply(ep, t, m, nn) : t);
+      finish(idx, t);
     }
+    store_fp6();
     if (tid == 0) __hip_atomic_store(ws_cnt + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
     return;
   }
   for (int idx = tid; idx < TT * 1024; idx += NW * 64) {
-    const int tt = idx >> 10, e = (idx >> 6) & 15, l = idx & 63;
     float s = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; w++) s += part[w * (TT * 1024) + idx];
-    const int m = (tt / TB) * 32 + (l & 31);
-    const int nl = (tt % TB) * 32 + 8 * (e >> 2) + 4 * (l >> 5) + (e & 3);
-    const long nn = (long)n0 + nl;
-    if (m < M && nl < BR && nn < N) store1(C + (long)m * N + nn, has_ep ? epilogue_apply(ep, s, m, nn) : s);
+    finish(idx, s);
   }
+  store_fp6();
 }
 
 bool gemm_skinny_supports(const GemmArgs& g) {
@@ -479,11 +505,15 @@ bool gemm_skinny_scratch_fits(const GemmArgs& g) {
   return p.want <= 1 || (p.tiles <= (unsigned)kScratchTiles && p.slots <= (unsigned)kScratchSlots);
 }
 
+// MXFP6 output straight from the kernel: workgroups of 16 rows of B hold halves of 32-blocks and have no such form
+bool gemm_skinny_stores_fp6(const GemmArgs& g) { return gemm_skinny_supports(g) && g.N % 32 == 0 && skinny_plan(g).geo != 2; }
+
 template <int FA, int FB, typename Out>
 static hipError_t launch(const GemmArgs& g, hipStream_t s) {
   typedef typename Out::type T;
   const SkinnyPlan plan = skinny_plan(g);
   const int geo = plan.geo, want = plan.want;
+  if (sizeof(T) == 1 && (geo == 2 || !g.C_scale || g.N % 32)) return hipErrorInvalidValue;
   int nsplit = 1;
   SplitWs ws;
   const unsigned tiles = plan.tiles;
@@ -509,12 +539,12 @@ static hipError_t launch(const GemmArgs& g, hipStream_t s) {
 #define MXFP6_SK(AR, NW, BR) MXFP6_SKD(AR, NW, BR, 1)
 #define MXFP6_SKD(AR, NW, BR, DB) \
   gemm_skinny_kernel<FA, FB, Out, AR, NW, BR, DB><<<(g.N + BR - 1) / BR * nsplit, NW * 64, 0, s>>>( \
-      g.A, g.B, g.As, g.Bs, (T*)g.C, g.M, g.N, g.K, g.layout_b, g.ep, nsplit, ws.part, ws.cnt, (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes)
+      g.A, g.B, g.As, g.Bs, (T*)g.C, g.M, g.N, g.K, g.layout_b, g.ep, nsplit, ws.part, ws.cnt, (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes, g.C_scale, g.fmt_c)
   if (g.X) {
     if constexpr (sizeof(T) == 2) {
 #define MXFP6_SKX(NW, BR)                                                                                                       \
   gemm_skinny_kernel<FA, FB, Out, 16, NW, BR, 1, true><<<(g.N + BR - 1) / BR * nsplit, NW * 64, 0, s>>>(                          \
-      (const uint8_t*)g.X, g.B, nullptr, g.Bs, (T*)g.C, g.M, g.N, g.K, g.layout_b, g.ep, nsplit, ws.part, ws.cnt, (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes)
+      (const uint8_t*)g.X, g.B, nullptr, g.Bs, (T*)g.C, g.M, g.N, g.K, g.layout_b, g.ep, nsplit, ws.part, ws.cnt, (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes, g.C_scale, g.fmt_c)
       if (geo == 2) MXFP6_SKX(8, 16); else if (geo == 3) MXFP6_SKX(4, 32); else if (geo == 5) MXFP6_SKX(2, 32); else MXFP6_SKX(8, 32);
 #undef MXFP6_SKX
       return hipGetLastError();
@@ -530,9 +560,9 @@ static hipError_t launch(const GemmArgs& g, hipStream_t s) {
   } else if (g.M > 32) {
     if (geo == 3) MXFP6_SK(64, 2, 32); else MXFP6_SK(64, 4, 32);  // two chunks of B and three waves: measured level with this
   } else if (g.M <= 16) {
-    if (geo == 2) MXFP6_SK(16, 8, 16); else if (geo == 3) MXFP6_SK(16, 4, 32); else if (geo == 5) MXFP6_SK(16, 2, 32); else MXFP6_SK(16, 8, 32);
+    if (geo == 2) { if constexpr (sizeof(T) != 1) MXFP6_SK(16, 8, 16); } else if (geo == 3) MXFP6_SK(16, 4, 32); else if (geo == 5) MXFP6_SK(16, 2, 32); else MXFP6_SK(16, 8, 32);
   } else {
-    if (geo == 2) MXFP6_SK(32, 6, 16); else if (geo == 3) MXFP6_SK(32, 3, 32); else if (db && geo == 1) MXFP6_SKD(32, 4, 32, 2); else MXFP6_SK(32, 6, 32);
+    if (geo == 2) { if constexpr (sizeof(T) != 1) MXFP6_SK(32, 6, 16); } else if (geo == 3) MXFP6_SK(32, 3, 32); else if (db && geo == 1) MXFP6_SKD(32, 4, 32, 2); else MXFP6_SK(32, 6, 32);
   }
 #undef MXFP6_SKD
 #undef MXFP6_SK
@@ -541,7 +571,7 @@ static hipError_t launch(const GemmArgs& g, hipStream_t s) {
 
 hipError_t launch_gemm_skinny(const GemmArgs& g, hipStream_t s) {
 #define MXFP6_CASE(FA, FB) \
-  if (g.fmt_a == FA && g.fmt_b == FB) return g.f32out ? launch<FA, FB, OutF32>(g, s) : launch<FA, FB, OutBf16>(g, s);
+  if (g.fmt_a == FA && g.fmt_b == FB) return g.fmt_c ? launch<FA, FB, OutFp6>(g, s) : g.f32out ? launch<FA, FB, OutF32>(g, s) : launch<FA, FB, OutBf16>(g, s);
   MXFP6_CASE(2, 2) MXFP6_CASE(2, 3) MXFP6_CASE(3, 2) MXFP6_CASE(3, 3)
 #undef MXFP6_CASE
   return hipErrorInvalidValue;

@@ -17,7 +17,7 @@ struct GemmArgs {
   int tile_cols = 0;               // ... and rows of B: 128 (with 128 rows of A only) or 256; 0 with tile_rows set = 256
   int skinny_geometry = 0;         // skinny kernel: 1 = 32 rows of B and all waves, 2 = 16 rows of B, 3 = half the waves, 4 - 9 = 1 or 2 with the K range split between 2 / 4 / 8 workgroups, 10 = two waves; 0 = by shape
   Epilogue ep;                     // fused bias / scales / activation (all optional)
-  uint8_t* C_scale = nullptr;      // fp6 output (tiled and block kernels, reduction of a K split): C is the packed operand [M, 3N/4], this its E8M0 bytes [M, N/32]
+  uint8_t* C_scale = nullptr;      // fp6 output (every kernel but the ragged and generic ones; skinny: gemm_skinny_stores_fp6): C is the packed operand [M, 3N/4], this its E8M0 bytes [M, N/32]
   int fmt_c = 0;                   // 2 / 3: format of the fp6 output; 0: bf16 / fp32 output
   int out_fp6 = 0;                 // kernel choice only: the fp32 sums (f32out) leave as MXFP6
   const void* X = nullptr;         // skinny and slice kernel: activations [M, K] that they quantise to fmt_a themselves, in place of A and As (gemm_skinny_takes_x, choose_linear_kernel)
@@ -89,6 +89,7 @@ hipError_t launch_gemm_slice(const GemmArgs& g, const SlicePlan& p, hipStream_t 
 bool gemm_mid_supports(const GemmArgs& g);
 hipError_t launch_gemm_mid(const GemmArgs& g, hipStream_t s);
 bool gemm_skinny_supports(const GemmArgs& g);
+bool gemm_skinny_stores_fp6(const GemmArgs& g);  // MXFP6 output without a workspace (N % 32, the workgroup's shape)
 bool gemm_skinny_takes_x(const GemmArgs& g);  // M and K of a call whose activations the kernel can quantise itself
 hipError_t launch_gemm_skinny(const GemmArgs& g, hipStream_t s);
 bool gemm_skinny_scratch_fits(const GemmArgs& g);  // no_alloc: the K split this call would use fits the static scratch array

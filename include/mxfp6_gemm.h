@@ -24,7 +24,8 @@
  * needs more), and keep it until mxfp6_release_workspaces():
  *   - the gemm entry points on large row-major problems (re-layout pre-pass, see mxfp6_set_relayout):
  *     up to 0.78 (M + N) K bytes;
- *   - mxfp6_gemm_fused_fp6 on shapes that the decode, ragged and generic kernels run: 4 M N bytes;
+ *   - mxfp6_gemm_fused_fp6 on shapes that the ragged and generic kernels run, or the decode kernel with narrow workgroups (M <= 32, N <= 4096):
+ *     4 M N bytes;
  *   - mxfp6_linear: 0.79 M K bytes, M rounded up to 32 (none for calls of few rows that quantise inside the GEMM kernel);
  *   - the gemm entry points on decode shapes whose K range is split between workgroups (M <= 32, N <= 2048,
  *     K >= 24576): 2 MB;
@@ -263,8 +264,8 @@ int mxfp6_gemm_fused(const void *A_packed, const void *B_packed, const void *A_s
  * C_packed [M, 3N/4] and its E8M0 scales C_scale [M, N/32] (row-major) that the next layer's GEMM takes as A:
  * exactly mxfp6_quantize(fmt_c) applied to the fp32 result of mxfp6_gemm_fused(out_f32 = 1), without that result
  * ever reaching memory (0.78 instead of 2 or 4 bytes per output element).  N % 32 == 0; C_packed 8-byte aligned.
- * The LDS-tiled kernel, the block kernel and the reduction of their K splits quantise their sums themselves; shapes that run
- * on another kernel (few rows of A, where C is small; ragged K) go through the stream's fp32 workspace.  Under capture without it
+ * All kernels but three quantise their sums themselves: shapes that run on the ragged and generic kernels (ragged K) or on the
+ * decode kernel with 16 rows of B a workgroup (M <= 32, N <= 4096) go through the stream's fp32 workspace.  Under capture without it
  * they run on the tiled or the block kernel, and those that neither takes (ragged K, operands off 16 bytes) are refused
  * (hipErrorStreamCaptureUnsupported).
  * No counterpart in the reference.
