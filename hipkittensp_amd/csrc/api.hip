@@ -249,12 +249,21 @@ int check_device() {
   return cached;
 }
 
+// Bytes of a padded tile-major copy: packed bytes, then its scales
+size_t padded_bytes(int rows, int K) {
+  const size_t r = ((size_t)rows + 31) & ~(size_t)31, nkt = ((size_t)K + 127) / 128;
+  return ((r * nkt * 96 + 255) & ~(size_t)255) + ((r * ((nkt + 3) / 4) * 16 + 255) & ~(size_t)255);
+}
+uint8_t* padded_scales(uint8_t* p, int rows, int K) { return p + (((((size_t)rows + 31) & ~(size_t)31) * (((size_t)K + 127) / 128) * 96 + 255) & ~(size_t)255); }
+
 // Large row-major problems on the tiled kernel are bound by L2 request throughput: a 96-byte row piece straddles
 // 128-byte lines and every row's scales are a request of their own (896 requests per K-tile and workgroup against
 // 648 with one operand tile-major and 400 with both).  Re-laying an operand out tile-major first costs two passes
 // over it at HBM speed (measured 23 us for 8192 x 8192) and shortens the GEMM by about 15 % (first operand) and
 // 11 % (second): from about 8192^3 on that pays for both, for a tall or wide problem only for the operand with
-// fewer rows.  The workspace is this stream's (stream_workspace: allocated once, kept).  Returns false when no
+// fewer rows.  Rows need not fill the last row-tile: the copy has it whole (us, row-major / on copies: 5393 x 8192 x 8192 270 / 239, 1777 x
+// 14336 x 8192 190 / 168, with A's copy alone 6007 x 6144 x 8192 216 / 207, MLP of 4095 rows, 8192 -> 8192 -> 8192, 354 / 327).
+// The workspace is this stream's (stream_workspace: allocated once, kept).  Returns false when no
 // pre-pass pays or it cannot run (then the caller launches the row-major path).
 bool relayout_then_tiled(const mxfp6::GemmArgs& g, hipStream_t s, hipError_t& e) {
   if (!g_relayout || g.no_alloc || (g.layout_a && g.layout_b) || g.K % 128) return false;
@@ -270,44 +279,29 @@ bool relayout_then_tiled(const mxfp6::GemmArgs& g, hipStream_t s, hipError_t& e)
     // worth about 11 % of the row-major GEMM, for one launch in front of it
     const bool first_is_row = a_first ? !g.layout_a : !g.layout_b;
     const int rows = first_is_row ? rows1 : rows2;
-    const bool conv = rows % 32 == 0 && 0.11 * t_gemm_us > 6 + cost_us(rows);
+    const bool conv = 0.11 * t_gemm_us > 6 + cost_us(rows);
     conv1 = first_is_row && conv, conv2 = !first_is_row && conv;
   } else {
     // fixed costs: the dependent launch in front of the GEMM (about 10 us measured on a 33 us GEMM), a second operand about 3 us
-    conv1 = rows1 % 32 == 0 && 0.15 * t_gemm_us > 10 + 1.5 * cost_us(rows1);
-    conv2 = rows2 % 32 == 0 && (conv1 ? 0.11 * t_gemm_us > 3 + 1.5 * cost_us(rows2) : 0.15 * t_gemm_us > 10 + 1.5 * cost_us(rows2));
+    conv1 = 0.15 * t_gemm_us > 10 + 1.5 * cost_us(rows1);
+    conv2 = conv1 ? 0.11 * t_gemm_us > 3 + 1.5 * cost_us(rows2) : 0.15 * t_gemm_us > 10 + 1.5 * cost_us(rows2);
   }
   if (!conv1 && !conv2) return false;
   const bool conv_a = a_first ? conv1 : conv2, conv_b = a_first ? conv2 : conv1;
-  auto bytes_of = [&](int rows) { return (((size_t)rows * (g.K / 4 * 3) + 255) & ~(size_t)255) + (((size_t)rows * ((g.K + 511) / 512) * 16 + 255) & ~(size_t)255); };
-  const size_t bytes_a = conv_a ? bytes_of(g.M) : 0, bytes_b = conv_b ? bytes_of(g.N) : 0;
+  const size_t bytes_a = conv_a ? padded_bytes(g.M, g.K) : 0, bytes_b = conv_b ? padded_bytes(g.N, g.K) : 0;
   std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
   uint8_t* ws = stream_workspace(s, 0, bytes_a + bytes_b);
   if (!ws) return false;
   mxfp6::GemmArgs t = g;
-  uint8_t* pa = ws;
-  uint8_t* sa = pa + (((size_t)g.M * (g.K / 4 * 3) + 255) & ~(size_t)255);
-  uint8_t* pb = ws + bytes_a;
-  uint8_t* sb = pb + (((size_t)g.N * (g.K / 4 * 3) + 255) & ~(size_t)255);
-  if (conv_a && conv_b) {
-    e = mxfp6::launch_tile_both(g.A, pa, g.As, sa, g.M, g.B, pb, g.Bs, sb, g.N, g.K, s);
-  } else if (conv_a) {
-    e = mxfp6::launch_tile_both(g.A, pa, g.As, sa, g.M, nullptr, nullptr, nullptr, nullptr, 0, g.K, s);
-  } else {
-    e = mxfp6::launch_tile_both(g.B, pb, g.Bs, sb, g.N, nullptr, nullptr, nullptr, nullptr, 0, g.K, s);
-  }
+  uint8_t *const pa = ws, *const pb = ws + bytes_a, *const sa = padded_scales(pa, g.M, g.K), *const sb = padded_scales(pb, g.N, g.K);
+  if (conv_a && conv_b) e = mxfp6::launch_pad_both(g.A, pa, g.As, sa, g.M, g.B, pb, g.Bs, sb, g.N, g.K, s);
+  else if (conv_a) e = mxfp6::launch_pad_both(g.A, pa, g.As, sa, g.M, nullptr, nullptr, nullptr, nullptr, 0, g.K, s);
+  else e = mxfp6::launch_pad_both(g.B, pb, g.Bs, sb, g.N, nullptr, nullptr, nullptr, nullptr, 0, g.K, s);
   if (conv_a) { t.A = pa; t.As = sa; t.layout_a = 1; }
   if (conv_b) { t.B = pb; t.Bs = sb; t.layout_b = 1; }
   if (e == hipSuccess) e = mxfp6::launch_gemm_tiled(t, s);
   return true;
 }
-
-// Bytes of a padded tile-major copy: packed bytes, then its scales
-size_t padded_bytes(int rows, int K) {
-  const size_t r = ((size_t)rows + 31) & ~(size_t)31, nkt = ((size_t)K + 127) / 128;
-  return ((r * nkt * 96 + 255) & ~(size_t)255) + ((r * ((nkt + 3) / 4) * 16 + 255) & ~(size_t)255);
-}
-uint8_t* padded_scales(uint8_t* p, int rows, int K) { return p + (((((size_t)rows + 31) & ~(size_t)31) * (((size_t)K + 127) / 128) * 96 + 255) & ~(size_t)255); }
 
 // A ragged product on padded tile-major copies of its operands where those pay (padded_pays; `c`: the choice otherwise).  a_pad:
 // A's copy is there already.  Returns false, nothing launched, where they don't or no workspace is to be had.

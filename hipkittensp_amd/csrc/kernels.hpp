@@ -99,8 +99,6 @@ hipError_t launch_tile_operand(const uint8_t* src, uint8_t* dst, int rows, int K
 hipError_t launch_tile_scales(const uint8_t* src, uint8_t* dst, int rows, int K, int tile, hipStream_t s);
 hipError_t launch_pad_both(const uint8_t* src0, uint8_t* dst0, const uint8_t* ssrc0, uint8_t* sdst0, int rows0, const uint8_t* src1, uint8_t* dst1, const uint8_t* ssrc1,
                            uint8_t* sdst1, int rows1, int K, hipStream_t s);  // any size and alignment -> padded tile-major; rows1 == 0: one operand
-hipError_t launch_tile_both(const uint8_t* src0, uint8_t* dst0, const uint8_t* ssrc0, uint8_t* sdst0, int rows0, const uint8_t* src1,
-                            uint8_t* dst1, const uint8_t* ssrc1, uint8_t* sdst1, int rows1, int K, hipStream_t s);
 hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t s);
 hipError_t launch_mfma_probe(const uint8_t* A, const uint8_t* B, const uint8_t* As, const uint8_t* Bs, int rows_a, int rows_b, int K, int fmt_a,
                              int fmt_b, int iters, int workgroups, float* sink, uint32_t* stats, hipStream_t s);

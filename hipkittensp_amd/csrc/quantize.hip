@@ -199,71 +199,14 @@ hipError_t launch_tile_scales(const uint8_t* src, uint8_t* dst, int rows, int K,
   return hipGetLastError();
 }
 
-// Row-major -> tile-major for up to two operands (packed bytes and scales) in one launch: the re-layout pre-pass of
-// the gemm entry points, where every extra launch would cost as much as part of the copy.  A workgroup copies 32
-// rows x four K-tiles (384 source bytes per row = three whole cache lines; a single K-tile's 96 bytes straddle
-// lines, and lines shared between workgroups on different XCDs were fetched twice: 1.64x read traffic) in source
-// order: consecutive lanes read consecutive 16-byte pieces of a row and write runs of 96 bytes into the four 3 KB
-// tiles.  Other workgroups move the 16 scale bytes one row has for four K-tiles, one row per lane.
-struct TileJob {
-  const uint8_t* src;
-  uint8_t* dst;
-  const uint8_t* ssrc;
-  uint8_t* sdst;
-  long ngroups, nchunks;  // groups of 32 rows x four K-tiles; (row, four K-tiles) scale chunks
-  unsigned pblocks, sblocks;
-};
-
-__global__ __launch_bounds__(256) void tile_both_kernel(TileJob j0, TileJob j1, int nkt, int nkb, int nk4) {
-  unsigned bid = blockIdx.x;
-  const bool second = bid >= j0.pblocks + j0.sblocks;
-  if (second) bid -= j0.pblocks + j0.sblocks;
-  const TileJob& j = second ? j1 : j0;
-  if (bid < j.pblocks) {
-    const int rt = bid / nk4, g = bid - rt * nk4;  // row-tile, group of four K-tiles
-    const int ntile = min(4, nkt - 4 * g);
-    const uint8_t* src = j.src + ((size_t)rt * 32 * nkt + 4 * g) * 96;
-    uint8_t* dst = j.dst + ((size_t)rt * nkt + 4 * g) * 3072;
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-      const int p = threadIdx.x + 256 * i, r = p / 24, q = p - r * 24;  // piece q of the row's 384 bytes
-      const int tg = q / 6, c = q - tg * 6;
-      if (tg < ntile)
-        *reinterpret_cast<v4i*>(dst + tg * 3072 + (r * 6 + (c ^ ((r >> 3) & 1))) * 16) =
-            *reinterpret_cast<const v4i*>(src + (size_t)r * nkt * 96 + q * 16);
-    }
-  } else {
-    const long s = (long)(bid - j.pblocks) * 256 + threadIdx.x;
-    if (s >= j.nchunks) return;
-    const int row = (int)(s / nk4), g = (int)(s - (long)row * nk4);
-    const int nvalid = min(16, nkb - g * 16);
-    const size_t rm = (size_t)row * nkb + (size_t)g * 16, tm = tile_major_scale_offset(row, g * 16, nk4);
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-      *reinterpret_cast<uint32_t*>(j.sdst + tm + 4 * i) = 4 * i < nvalid ? *reinterpret_cast<const uint32_t*>(j.ssrc + rm + 4 * i) : 0u;
-  }
-}
-
-// rows1 == 0: only the first operand
-hipError_t launch_tile_both(const uint8_t* src0, uint8_t* dst0, const uint8_t* ssrc0, uint8_t* sdst0, int rows0, const uint8_t* src1,
-                            uint8_t* dst1, const uint8_t* ssrc1, uint8_t* sdst1, int rows1, int K, hipStream_t s) {
-  const int nkt = K / 128, nkb = K / 32, nk4 = (nkb + 15) / 16;
-  auto job = [&](const uint8_t* src, uint8_t* dst, const uint8_t* ssrc, uint8_t* sdst, int rows) {
-    TileJob j{src, dst, ssrc, sdst, (long)(rows / 32) * nk4, (long)rows * nk4, 0, 0};
-    j.pblocks = (unsigned)j.ngroups;
-    j.sblocks = (unsigned)((j.nchunks + 255) / 256);
-    return j;
-  };
-  const TileJob j0 = job(src0, dst0, ssrc0, sdst0, rows0), j1 = job(src1, dst1, ssrc1, sdst1, rows1);
-  const unsigned blocks = j0.pblocks + j0.sblocks + j1.pblocks + j1.sblocks;
-  if (blocks == 0) return hipSuccess;
-  tile_both_kernel<<<blocks, 256, 0, s>>>(j0, j1, nkt, nkb, nk4);
-  return hipGetLastError();
-}
-
-// The same for operands of any size and alignment: row-major -> tile-major with K padded to whole K-tiles and the rows to whole
-// row-tiles, zeros in both.  A row's scales start at any byte: five aligned dwords (the resource ends at the dword that holds the
-// tensor's last byte) are shifted into place.
+// Row-major -> tile-major for up to two operands (packed bytes and scales) of any size and alignment in one launch, K padded to
+// whole K-tiles and the rows to whole row-tiles, zeros in both: the pre-pass of large and of ragged products, where every extra launch
+// would cost as much as part of the copy.  A workgroup copies 32 rows x four K-tiles (384 source bytes per row = three whole cache
+// lines; a single K-tile's 96 bytes straddle lines, and lines shared between workgroups on different XCDs were fetched twice: 1.64x
+// read traffic) in source order, all three loads of a lane in flight: consecutive lanes read consecutive 16-byte pieces of a row and
+// write runs of 96 bytes into the four 3 KB tiles.  Other workgroups move the 16 scale bytes one row has for four K-tiles, one row per lane; a
+// row's scales start at any byte: five aligned dwords (the last one that is read holds the tensor's last byte) are shifted into
+// place.  Bound by memory: both operands of 8192^3, 200 MB moved, about 30 us; level there with a form for whole row- and K-tiles only.
 struct PadJob {
   const uint8_t *src, *ssrc;
   uint8_t *dst, *sdst;

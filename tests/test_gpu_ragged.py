@@ -181,3 +181,39 @@ def test_padded_route_and_capture(hk, M, N, K):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(C, want)
+
+
+@pytest.mark.parametrize("M,N,K", [(1001, 2056, 8192), (31, 4104, 8192), (2049, 1000, 16384), (1793, 14336, 8192)])
+@pytest.mark.parametrize("tile_b", [0, 1])
+def test_relayout_of_rows_that_fill_no_row_tile(hk, M, N, K, tile_b):
+    """The tiled kernel's pre-pass on operands whose rows end inside a row-tile: the bits of the row-major path, whose sums are in the
+    same order, for every output type, with NaN patterns around the operands and in the workspace before the call."""
+    if tile_b and N % 32:
+        N -= N % 32
+    g = torch.Generator(device="cuda").manual_seed(M)
+    qa, qb = hk.quantize(torch.randn(M, K, device="cuda", generator=g)), hk.quantize(torch.randn(N, K, device="cuda", generator=g) * 0.02, 2, tile_b)
+    (a, asc), (b, bsc) = [[at(x.cpu().numpy(), 0).view(x.shape) for x in q] for q in (qa, qb)]
+    T = hk.tk_kernel
+    prev_k = T.set_kernel(2 if M * N < 10**7 else 0)
+    try:
+        for dtype in (torch.float32, torch.bfloat16, torch.uint8):
+            outs = []
+            for on in (0, 1, 1):
+                if on and not outs[1:]:  # the stream's workspace full of NaN patterns
+                    full = [torch.full((M, K // 4 * 3), 255, dtype=torch.uint8, device="cuda"), torch.full((M, K // 32), 255, dtype=torch.uint8, device="cuda")]
+                    hk.dispatch_micro(*full[:1], b, *full[1:], bsc, torch.empty(M, N, device="cuda"), layout_b=tile_b)
+                prev = T.set_relayout(on)
+                try:
+                    if dtype == torch.uint8 and N % 32 == 0:
+                        C, S = torch.zeros(M, N // 4 * 3, dtype=dtype, device="cuda"), torch.zeros(M, N // 32, dtype=dtype, device="cuda")
+                        hk.dispatch_micro(a, b, asc, bsc, C, layout_b=tile_b, C_scale=S)
+                        outs.append(torch.cat([C, S], 1))
+                    elif dtype != torch.uint8:
+                        C = torch.empty(M, N, dtype=dtype, device="cuda")
+                        hk.dispatch_micro(a, b, asc, bsc, C, layout_b=tile_b)
+                        outs.append(C)
+                finally:
+                    T.set_relayout(prev)
+            assert all(torch.equal(x, outs[0]) for x in outs[1:])
+    finally:
+        T.set_kernel(prev_k)
