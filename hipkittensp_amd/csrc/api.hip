@@ -66,15 +66,15 @@ bool stream_is_capturing(hipStream_t s) {
 
 // kind 0: pre-pass copies, kind 1: fp32 result of mxfp6_gemm_fused_fp6, kind 2: partial sums of a K split, kind 3: arrival
 // counters of the ring and slice kernels' K splits (zeroed when allocated; the kernels leave them zero), kind 4: packed activations of
-// mxfp6_linear (never under capture: a graph's activations live in its own memory plan, since graphs captured on one stream may be
-// replayed side by side on others).
+// mxfp6_linear.  recorded = false: never under capture, since graphs captured on one stream may be replayed side by side on others
+// (a graph's packed activations live in its own memory plan, its slice kernels run unsplit).
 // nullptr: no workspace (capture without one, table full of pinned entries, out of memory).
-uint8_t* stream_workspace(hipStream_t s, int kind, size_t bytes, bool zeroed = false) {
+uint8_t* stream_workspace(hipStream_t s, int kind, size_t bytes, bool zeroed = false, bool recorded = true) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
   std::lock_guard<std::mutex> lock(g_sws_mutex);
   const bool capturing = stream_is_capturing(s);
-  if (capturing && kind == 4) return nullptr;
+  if (capturing && !recorded) return nullptr;
   auto it = g_sws.find({dev, s, kind});
   if (it != g_sws.end() && it->second.bytes >= bytes) {
     it->second.used = ++g_sws_clock;
@@ -182,11 +182,13 @@ bool apply_choice(mxfp6::GemmArgs& g, const mxfp6::KernelChoice& c, hipStream_t 
       return true;
     }
     case mxfp6::kCandSlice: {
+      // Never recorded in a graph: small calls, linear layers of few rows among them, are captured by the dozen, and of two graphs of one
+      // stream replayed at once each would write the other's partial tiles and count in its counters.
       if (c.shares <= 1) return true;
       size_t part = 0, counters = 0;
       mxfp6::slice_workspace(g, c.slice, &part, &counters);
-      uint8_t* pp = stream_workspace(s, 2, part);
-      uint8_t* pc = pp ? stream_workspace(s, 3, counters * sizeof(int), true) : nullptr;
+      uint8_t* pp = stream_workspace(s, 2, part, false, false);
+      uint8_t* pc = pp ? stream_workspace(s, 3, counters * sizeof(int), true, false) : nullptr;
       if (!pc) return false;
       g.ks_part = reinterpret_cast<float*>(pp), g.ks_counters = reinterpret_cast<int*>(pc);
       return true;
@@ -485,7 +487,7 @@ int mxfp6_linear(const void* X, int x_bf16, const void* W, const void* Ws, void*
     if (g_slice >> 20 > 0) c = {mxfp6::kCandSlice, g_slice >> 12 & 255, 0, 0.0, {g_slice & 15, g_slice >> 4 & 15, g_slice >> 8 & 15, g_slice >> 12 & 255, g_slice >> 20}};
     if (c.cand == mxfp6::kCandSlice) {
       std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
-      if (!apply_choice(g, c, s)) c.slice.shares = 1;  // without a workspace: unsplit
+      if (!apply_choice(g, c, s)) c.slice.shares = 1;  // without a workspace, and under capture: unsplit
       g.ep = ep;
       const hipError_t e = mxfp6::launch_gemm_slice(g, c.slice, s);
       return e == hipSuccess ? MXFP6_OK : (int)e;
@@ -510,7 +512,7 @@ int mxfp6_linear(const void* X, int x_bf16, const void* W, const void* Ws, void*
     mxfp6::KernelChoice tc{-1, 1, 0, 0.0};
     g.layout_a = 1, g.ep = ep;
     if (g_relayout && g_padded >= 0 && mxfp6::padded_pays(g, g_ksplit, auto_mask(g, 0), g_padded > 0 ? mxfp6::KernelChoice{mxfp6::kCandSlice, 1, 0, 1e30} : other, true, &t, &tc)) {
-      uint8_t* const xp = stream_workspace(s, 4, padded_bytes(M, K));
+      uint8_t* const xp = stream_workspace(s, 4, padded_bytes(M, K), false, false);
       if (!xp) return MXFP6_EWORKSPACE;
       hipError_t e = mxfp6::launch_quantize(X, x_bf16 != 0, xp, padded_scales(xp, M, K), M, K, fmt_x, 1, s);
       if (e != hipSuccess) return (int)e;
@@ -519,7 +521,7 @@ int mxfp6_linear(const void* X, int x_bf16, const void* W, const void* Ws, void*
   }
   const size_t rows = ((size_t)M + 31) & ~(size_t)31;
   const size_t nx = (rows * (K / 32) * 24 + 255) & ~(size_t)255, ns = rows * ((K + 511) / 512) * 16;
-  uint8_t* xp = K > 0 ? stream_workspace(s, 4, nx + ns) : nullptr;
+  uint8_t* xp = K > 0 ? stream_workspace(s, 4, nx + ns, false, false) : nullptr;
   if (K > 0) {
     if (!xp) return MXFP6_EWORKSPACE;
     const hipError_t e = mxfp6::launch_quantize(X, x_bf16 != 0, xp, xp + nx, M, K, fmt_x, layout_x, s);
@@ -592,7 +594,8 @@ int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const voi
   };
   hipError_t e = hipSuccess;
   if (run(c, e)) return e == hipSuccess ? MXFP6_OK : (int)e;
-  // a split without its workspace (a stream under capture that has none): what the shape gets otherwise, as for the other outputs
+  // a split without its workspace (a stream under capture that has none, the slice kernel's on any): what the shape gets otherwise, as
+  // for the other outputs
   if (c.cand == mxfp6::kCandTiledSplit256 || c.cand == mxfp6::kCandTiledSplit128 || c.cand == mxfp6::kCandBlockSplit || c.cand == mxfp6::kCandSlice) {
     c = force == 0 ? choose(false) : mxfp6::choose_kernel(g, 1, false, 1u << mxfp6::kCandBlock);
     if (run(c, e)) return e == hipSuccess ? MXFP6_OK : (int)e;

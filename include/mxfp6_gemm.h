@@ -34,7 +34,8 @@
  *     shares * 4 M N bytes of partial sums (tiles times shares never exceed the CUs: at most 64 MB, 256 tiles of
  *     256 x 256 fp32), one workspace for the three kernels, and for the ring kernel one counter per output tile.
  * While `hip_stream` is being captured nothing is allocated: the pre-pass and the K splits are left out
- * (same results up to the order of fp32 sums, other kernels) unless their workspace exists already, and mxfp6_gemm_fused_fp6 runs
+ * (same results up to the order of fp32 sums, other kernels) unless their workspace exists already, the slice kernel's K split in any
+ * case (so that graphs of small calls share nothing), and mxfp6_gemm_fused_fp6 runs
  * a kernel that needs none or, on shapes and alignments that no such kernel takes, returns hipErrorStreamCaptureUnsupported.  mxfp6_linear records no packed activations
  * of its own in a graph: where it needs a workspace for them it returns MXFP6_EWORKSPACE under capture (quantise into the
  * graph's own memory and call the GEMM).  A workspace that a capture did use is recorded in the
@@ -283,7 +284,7 @@ int mxfp6_gemm_fused_fp6(const void *A_packed, const void *B_packed, const void 
  * mxfp6_gemm_fused (NULL = none).  The packed activations live in a workspace of this stream (0.79 bytes per element of X,
  * rows rounded up to 32), in the layout the GEMM prefers.  MXFP6_EWORKSPACE, and nothing launched, where it cannot be had,
  * and while the stream is being captured (two graphs captured on one stream would share it).  Calls of few rows (up to 128, by
- * size) quantise inside the slice or the decode kernel: they need none and are captured.  No counterpart in the reference.
+ * size) quantise inside the slice or the decode kernel: they need no workspace for them and are captured.  No counterpart in the reference.
  */
 int mxfp6_linear(const void *X, int x_bf16, const void *W_packed, const void *W_scale, void *C_bf16, int M, int N, int K,
                  int fmt_x, int fmt_w, int layout_w, const void *bias, int bias_bf16, int activation, void *hip_stream);

@@ -130,6 +130,77 @@ def test_capture_and_streams(hk):
             torch.cuda.synchronize()
 
 
+def order_shows(g, rows, K, scale, sign):
+    """Rows whose products with those of the other sign cancel in every other K-block of the first half, 2^18 times the rest: what the
+    fp32 sums keep of the rest depends on their order."""
+    x = (torch.randn(rows, K, device="cuda", generator=g) * scale).view(rows, K // 32, 32)
+    q = K // 128
+    x[:, :q:2] *= 2.0**18 if sign < 0 else 1.0
+    x[:, q:2 * q:2] = sign * x[:, :q:2]
+    return x.reshape(rows, K)
+
+
+@pytest.mark.parametrize("kind,M,N,K,lb", [("linear", 16, 512, 7680, 1), ("linear", 8, 1024, 8192, 1), ("gemm", 64, 1024, 8192, 0), ("gemm", 16, 512, 15872, 1), ("fp6", 64, 1024, 8192, 0)])
+def test_graphs_of_one_stream_share_no_partial_sums(hk, kind, M, N, K, lb):
+    """Calls whose eager form splits K, captured twice on a stream that has run them: a graph has the bits of one captured on a stream
+    that has no workspace (which runs unsplit), not those of the split, alone and replayed beside the other graph and the eager call."""
+    from hipkittensp_amd.torch_op import MXFP6Linear
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    w = order_shows(g, N, K, 0.02, 1.0)
+    xs = [order_shows(g, M, K, 1.0, -1.0) for _ in range(2)]
+    if kind == "linear":
+        layer = MXFP6Linear(w)
+        xs = [x.to(torch.bfloat16) for x in xs]
+        call = lambda x: (layer(x),)
+    else:
+        b, bsc = hk.quantize(w, 2, lb)
+        xs = [hk.quantize(x, 2) for x in xs]
+
+        def call(x):
+            if kind == "gemm":
+                C = torch.empty(M, N, device="cuda")
+                hk.dispatch_micro(x[0], b, x[1], bsc, C, layout_b=lb)
+                return (C,)
+            C, S = torch.empty(M, N // 4 * 3, dtype=torch.uint8, device="cuda"), torch.empty(M, N // 32, dtype=torch.uint8, device="cuda")
+            hk.dispatch_micro(x[0], b, x[1], bsc, C, layout_b=lb, C_scale=S)
+            return C, S
+
+    def captured(x, stream):
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            y = call(x)
+        return graph, y
+
+    def copies(stream):
+        out = []
+        for graph, y in (captured(x, stream) for x in xs):
+            graph.replay()
+            torch.cuda.synchronize()
+            out.append((graph, y, [t.clone() for t in y]))
+        return out
+
+    same = lambda y, z: all(torch.equal(a.view(torch.uint8), b.view(torch.uint8)) for a, b in zip(y, z))
+    unsplit = [want for _, _, want in copies(torch.cuda.Stream())]
+    capture, streams = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(capture):
+        eager = [call(x) for x in xs]
+    torch.cuda.synchronize()
+    assert not any(same(y, z) for y, z in zip(eager, unsplit))  # these sums show their order
+    graphs = copies(capture)
+    assert all(same(want, z) for (_, _, want), z in zip(graphs, unsplit))
+    for _ in range(20):
+        for s, (graph, _, _) in zip(streams, graphs):
+            with torch.cuda.stream(s):
+                graph.replay()
+        with torch.cuda.stream(capture):
+            again = call(xs[0])
+        torch.cuda.synchronize()
+        assert same(again, eager[0]) and all(same(y, want) for _, y, want in graphs)
+
+
 # (rows of activations, rows of B / 32, waves) of the instantiations that quantise the activations themselves
 X_PLANS = {1: [(8, 1, 4), (8, 1, 8), (8, 2, 4), (8, 2, 8), (16, 1, 4), (16, 1, 8), (16, 2, 4), (16, 2, 6), (32, 1, 4), (32, 2, 4)],
            0: [(8, 1, 4), (8, 1, 8), (8, 2, 4), (8, 2, 6), (16, 1, 4), (16, 2, 4), (24, 1, 4)]}
