@@ -418,7 +418,8 @@ int gemm_common(const void* A, const void* B, const void* As, const void* Bs, vo
     e = mxfp6::launch_gemm_block(g, s);
   } else {
     mxfp6::KernelChoice c = auto_choice(g, force_split, true);
-    if (K != 0 && (c.cand < 0 || c.cand == mxfp6::kCandSlice) && !mxfp6::gemm_block_supports(g) && padded_then_gemm(g, c, nullptr, s, e)) return e == hipSuccess ? MXFP6_OK : (int)e;
+    // (products that no candidate takes only: what the slice kernel takes it takes for MXFP6 output as well, whose bits are those of this call's)
+    if (K != 0 && (c.cand < 0 || g_padded > 0) && !mxfp6::gemm_block_supports(g) && padded_then_gemm(g, c, nullptr, s, e)) return e == hipSuccess ? MXFP6_OK : (int)e;
     // a split needs this stream's workspace: without it, what the shape gets otherwise
     if (!apply_choice(g, c, s)) {
       c = auto_choice(g, force_split, false);

@@ -47,6 +47,31 @@ def test_decode_kernels_store_mxfp6(hk, kernel, M, N, K):
         hk.tk_kernel.set_kernel(prev)
 
 
+@pytest.mark.parametrize("M,N,K,off", [(793, 1024, 640, (4, 0)), (400, 1536, 1024, (0, 1)), (130, 2560, 512, (8, 2)), (96, 768, 6144, (4, 0))])
+def test_mxfp6_output_beside_fp32_output_off_16_bytes(hk, M, N, K, off):
+    """A (its packed bytes, its scales) off 16 bytes against prepared weights: MXFP6 output has the bits of the quantised fp32 output here
+    too, on sums that show their order (every other K-block of the first half is 2^18 times the rest and cancels)."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x, w = ((torch.randn(r, K, device="cuda", generator=g) * c).view(r, K // 32, 32) for r, c in ((M, 1.0), (N, 0.02)))
+    q = K // 128
+    x[:, :q:2] *= 2.0**18
+    x[:, q:2 * q:2], w[:, q:2 * q:2] = -x[:, :q:2], w[:, :q:2]
+    b, bsc = hk.quantize(w.reshape(N, K), 2, 1)
+
+    def moved(t, by):
+        buf = torch.empty(t.numel() + 256, dtype=torch.uint8, device="cuda")
+        out = buf[by:by + t.numel()].view(t.shape)
+        return out.copy_(t)
+
+    a, asc = (moved(t, by) for t, by in zip(hk.quantize(x.reshape(M, K), 2), off))
+    C = torch.empty(M, N, device="cuda")
+    p, s = torch.empty(M, N // 4 * 3, dtype=torch.uint8, device="cuda"), torch.empty(M, N // 32, dtype=torch.uint8, device="cuda")
+    hk.dispatch_micro(a, b, asc, bsc, C, layout_b=1)
+    hk.dispatch_micro(a, b, asc, bsc, p, layout_b=1, C_scale=s)
+    want_p, want_s = hk.quantize(C, 2)
+    assert torch.equal(p, want_p) and torch.equal(s, want_s)
+
+
 def test_decode_output_under_capture_without_a_workspace(hk):
     M, N, K = 24, 8192, 4096
     g = torch.Generator(device="cuda").manual_seed(3)
