@@ -24,10 +24,11 @@ NATIVE = os.path.join(HERE, "_native.so")
 PROBES_LIB = os.path.join(HERE, "libmxfp6_probes.so")
 SOURCES = ["api.hip", "dispatch.hip", "gemm_generic.hip", "gemm_tiled.hip", "gemm_tiled4.hip", "gemm_block.hip", "gemm_mid.hip", "gemm_skinny.hip", "gemm_ring.hip", "gemm_slice.hip", "quantize.hip"]
 # (source, object name, extra flags).  gemm_tiled.hip gives five objects: its host-side part, and the kernel
-# instantiations of each pair of operand formats (the bulk of the build time; they compile side by side).
+# instantiations of each pair of operand formats (the bulk of the build time; they compile side by side).  gemm_skinny.hip gives two:
+# on packed operands, and on a linear layer's activations.
 UNITS = [(src, src.replace(".hip", ""), []) for src in SOURCES] + [
     ("gemm_tiled.hip", f"gemm_tiled_fmt{fmt}", [f"-DMXFP6_TILED_FMT={fmt}"]) for fmt in (22, 23, 32, 33)
-]
+] + [("gemm_skinny.hip", "gemm_skinny_x", ["-DMXFP6_SKINNY_X"])]
 # what the measurement build compiles again (or in addition), with -DMXFP6_PROBES
 PROBE_UNITS = [("api.hip", "api_probes", ["-DMXFP6_PROBES"]), ("gemm_tiled.hip", "gemm_tiled_fmt22_probes", ["-DMXFP6_TILED_FMT=22", "-DMXFP6_PROBES"]),
                ("probes.hip", "probes", ["-DMXFP6_PROBES"])]

@@ -27,6 +27,9 @@
 // The reference has no kernel for this shape (its GEMMs need M, N multiples of the 256 tile,
 // analysis/bf16_gemm/mi325x/kernel_8192.cpp:24-32).  Algorithmic bytes per launch:
 // 0.75*K*(M+N) + (K/32)*(M+N) + 2*M*N.
+//
+// Compiled twice: as it is, and with -DMXFP6_SKINNY_X for the instantiations on a linear layer's activations, which take their
+// arguments otherwise (SkinnyXArgs).
 #include <map>
 #include <mutex>
 #include <utility>
@@ -34,13 +37,31 @@
 #include "kernels.hpp"
 #include "loader.hpp"
 
+#ifndef MXFP6_SKINNY_X
 // Scratch memory of mxfp6_gemm_noalloc: kScratchSlots partial tiles of 4 KB (one per (tile, split) pair of a K split) followed by
 // kScratchTiles arrival counters.  In host code this name is only a handle for hipGetSymbolAddress; kernels get the device
 // address that call returns.
 constexpr int kScratchSlots = 256, kScratchTiles = 256;
 static __device__ __align__(256) unsigned char scratch[kScratchSlots * 4096 + kScratchTiles * 4];
+#endif
 
 namespace mxfp6 {
+
+// Arguments on activations.  One argument: a call of one token is bound by its host side, where the runtime handles the arguments one by
+// one; it holds how many runs of BR rows of B there are, so that without a split no division stands in front of the first load (GPU time
+// with the twenty arguments of the other instantiations / with this one: 1 x 4096 x 4096 5.41 / 5.08 us, 3 x 8192 x 2048 5.70 / 5.41, 1 x 14336 x
+// 4096 11.65 / 11.37; the Python call, mostly host, 6.8 / 6.35).  Packed operands keep theirs: as one struct 4 x 1024 x 8192 took 5.0 / 4.8, 100 x
+// 6144 x 4096 11.9 / 11.8, but 23 x 4096 x 14336 11.0 / 11.2 and 16 x 4096 x 4096 5.4 / 5.5.
+struct SkinnyXArgs {
+  const uint8_t *X, *B, *Bs;
+  uint16_t* C;
+  int M, N, K, layout_b, nsplit, ntiles;
+  Epilogue ep;
+  float* ws_part;
+  int* ws_cnt;
+  int stream;  // B is read with the non-temporal bit (kStreamBytes)
+};
+hipError_t launch_gemm_skinny_x(const GemmArgs& g, int geo, SkinnyXArgs x, hipStream_t s);
 
 // AR = rows of A staged (16, 32 or 64: one or two 32-row accumulator tiles per wave); NW = waves per workgroup;
 // BR = rows of B per workgroup (32; 16 so that a narrow N still gives every CU a workgroup: the MFMA's other 16
@@ -52,12 +73,22 @@ namespace mxfp6 {
 // token the quantiser's 2.2 us and the gap behind it, of 10 us in all; every workgroup reads the activations anew, 1 KB per row
 // against the 6 or 12 KB of B a wave reads per chunk.
 constexpr int kXqRows = 4;
+#ifdef MXFP6_SKINNY_X
+// (place: which tile and share of K a workgroup has; split_ws: where a split's partial tiles and counters are, asked for in the branch that needs them)
+struct SkinnyPlace { int tile, split; };
+struct SkinnyWs { float* part; int* cnt; };
+template <int FA, int FB, typename Out, int AR, int NW, int BR, int DB, bool XQ, typename P, typename W>
+__device__ __forceinline__ void skinny(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, const uint8_t* __restrict__ As, const uint8_t* __restrict__ Bs,
+                                       typename Out::type* __restrict__ C, int M, int N, int K, int layout_b, const Epilogue& ep, int nsplit, W split_ws, int stream,
+                                       uint8_t* __restrict__ C_scale, int fmt_c, P place) {
+#else
 template <int FA, int FB, typename Out, int AR, int NW, int BR, int DB, bool XQ = false>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                                                               const uint8_t* __restrict__ As, const uint8_t* __restrict__ Bs,
                                                               typename Out::type* __restrict__ C, int M, int N, int K, int layout_b,
                                                               const Epilogue ep, int nsplit, float* ws_part, int* ws_cnt, int stream,
                                                               uint8_t* __restrict__ C_scale, int fmt_c) {
+#endif
   static_assert(BR == 64 || BR == 32 || BR == 16, "rows of B per workgroup");
   static_assert(AR == 16 || AR == 32 || AR == 64 || AR == 128, "rows of A");
   constexpr int TA = AR > 32 ? AR / 32 : 1;   // 32-row tiles of A per wave
@@ -84,8 +115,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
   const int h = lane >> 5, r32 = lane & 31;
   const int nkt = K / 128, sbytes = K / 32, rowbytes = K / 4 * 3;
   // nsplit > 1: the K range is split between nsplit workgroups per BR rows of B (workgroup = split * ntiles + tile)
+#ifdef MXFP6_SKINNY_X
+  const auto [tile, split] = place();
+#else
   const int ntiles = gridDim.x / nsplit;
   const int tile = blockIdx.x % ntiles, split = blockIdx.x / ntiles;
+#endif
   const int n0 = tile * BR;
   const int nrows = min(BR, N - n0);
   // tile-major B: first row-tile of this workgroup, how many it has, and (BR = 16) which 16 rows of it
@@ -312,6 +347,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
     // device-scope atomic accesses, which go past those caches, instead of device-scope fences, which write back and
     // invalidate a whole L2 per wave (measured: 0.2 us per workgroup, one after the other).
     // (a workgroup's partial result is TT tiles of 4 KB: idx = (tile of the wave * 16 + register) * 64 + lane)
+#ifdef MXFP6_SKINNY_X
+    const auto [ws_part, ws_cnt] = split_ws();
+#endif
     float* mine_ws = ws_part + ((size_t)tile * nsplit + split) * (TT * 1024);
     for (int idx = tid; idx < TT * 1024; idx += NW * 64) {
       float t = 0.f;
@@ -344,6 +382,39 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const uint8_t* __r
   store_fp6();
 }
 
+#ifdef MXFP6_SKINNY_X
+// (the body as a function of its own: inside the kernel the compiler puts 120 more instructions in front of the first load)
+template <int FA, int FB, int NW, int BR>
+__global__ __launch_bounds__(NW * 64) void gemm_skinny_x_kernel(const SkinnyXArgs args) {
+  auto place = [&] {
+    const int split = args.nsplit > 1 ? blockIdx.x / args.ntiles : 0;
+    return SkinnyPlace{(int)blockIdx.x - split * args.ntiles, split};
+  };
+  // (through a pointer that hides them from the compiler, which would load them in front of the branch, in every call's way)
+  auto split_ws = [] {
+    auto p = (const __attribute__((address_space(4))) SkinnyXArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return SkinnyWs{p->ws_part, p->ws_cnt};
+  };
+  skinny<FA, FB, OutBf16, 16, NW, BR, 1, true>(args.X, args.B, nullptr, args.Bs, args.C, args.M, args.N, args.K, args.layout_b, args.ep, args.nsplit, split_ws,
+                                               args.stream, nullptr, 0, place);
+}
+
+template <int FA, int FB>
+static hipError_t launch_x(int geo, SkinnyXArgs x, hipStream_t s) {
+#define MXFP6_SKX(NW, BR) (x.ntiles = (x.N + BR - 1) / BR, gemm_skinny_x_kernel<FA, FB, NW, BR><<<x.ntiles * x.nsplit, NW * 64, 0, s>>>(x))
+  if (geo == 2) MXFP6_SKX(8, 16); else if (geo == 3) MXFP6_SKX(4, 32); else if (geo == 5) MXFP6_SKX(2, 32); else MXFP6_SKX(8, 32);
+#undef MXFP6_SKX
+  return hipGetLastError();
+}
+
+hipError_t launch_gemm_skinny_x(const GemmArgs& g, int geo, SkinnyXArgs x, hipStream_t s) {
+#define MXFP6_CASE(FA, FB) if (g.fmt_a == FA && g.fmt_b == FB) return launch_x<FA, FB>(geo, x, s);
+  MXFP6_CASE(2, 2) MXFP6_CASE(2, 3) MXFP6_CASE(3, 2) MXFP6_CASE(3, 3)
+#undef MXFP6_CASE
+  return hipErrorInvalidValue;
+}
+#else
 bool gemm_skinny_supports(const GemmArgs& g) {
   // K % 512: chunks of four K-tiles are whole (three 128-byte lines per row, 16 scale bytes per row)
   return g.layout_a == 0 && g.M >= 1 && g.M <= 128 && g.N >= 1 && g.K >= 512 && g.K % 512 == 0 && (long)128 * (g.K / 4 * 3) < (1L << 31) && operands_aligned16(g);
@@ -541,15 +612,8 @@ static hipError_t launch(const GemmArgs& g, hipStream_t s) {
   gemm_skinny_kernel<FA, FB, Out, AR, NW, BR, DB><<<(g.N + BR - 1) / BR * nsplit, NW * 64, 0, s>>>( \
       g.A, g.B, g.As, g.Bs, (T*)g.C, g.M, g.N, g.K, g.layout_b, g.ep, nsplit, ws.part, ws.cnt, (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes, g.C_scale, g.fmt_c)
   if (g.X) {
-    if constexpr (sizeof(T) == 2) {
-#define MXFP6_SKX(NW, BR)                                                                                                       \
-  gemm_skinny_kernel<FA, FB, Out, 16, NW, BR, 1, true><<<(g.N + BR - 1) / BR * nsplit, NW * 64, 0, s>>>(                          \
-      (const uint8_t*)g.X, g.B, nullptr, g.Bs, (T*)g.C, g.M, g.N, g.K, g.layout_b, g.ep, nsplit, ws.part, ws.cnt, (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes, g.C_scale, g.fmt_c)
-      if (geo == 2) MXFP6_SKX(8, 16); else if (geo == 3) MXFP6_SKX(4, 32); else if (geo == 5) MXFP6_SKX(2, 32); else MXFP6_SKX(8, 32);
-#undef MXFP6_SKX
-      return hipGetLastError();
-    }
-    return hipErrorInvalidValue;
+    const SkinnyXArgs x = {static_cast<const uint8_t*>(g.X), g.B, g.Bs, (uint16_t*)g.C, g.M, g.N, g.K, g.layout_b, nsplit, 0, g.ep, ws.part, ws.cnt, (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes};
+    return sizeof(T) == 2 ? launch_gemm_skinny_x(g, geo, x, s) : hipErrorInvalidValue;
   }
   // two chunks of B per wave (17 - 32 and 65 - 128 rows of A: measured 3 - 15 % and 3 - 6 %); forced geometry 1: one
   const bool db = g.skinny_geometry != 1;
@@ -576,5 +640,7 @@ hipError_t launch_gemm_skinny(const GemmArgs& g, hipStream_t s) {
 #undef MXFP6_CASE
   return hipErrorInvalidValue;
 }
+
+#endif  // MXFP6_SKINNY_X
 
 }  // namespace mxfp6
