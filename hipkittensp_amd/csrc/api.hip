@@ -32,9 +32,14 @@ thread_local int g_ablation = 0;                              // mxfp6_probe_til
 thread_local int g_slice = 0;                                 // mxfp6_probe_slice: -1 = never, a plan = always
 thread_local int g_padded = 0;                                // mxfp6_probe_padded: 1 = always, -1 = never
 thread_local int g_block = 1;                                 // mxfp6_probe_block: 0 keeps the block kernel out of the automatic choice
+thread_local int g_route = 0;                                 // mxfp6_probe_route
+void note_route(int route) { g_route = route; }
 #else
 constexpr int g_slice = 0, g_padded = 0, g_block = 1;
+inline void note_route(int) {}
 #endif
+// What mxfp6_probe_route reports beside a kernel's code: the slice kernel's code, copies in front of the GEMM, quantised inside
+constexpr int kRouteSlice = 29, kRouteCopyA = 0x100, kRouteCopyB = 0x200, kRouteSplit = 0x400, kRouteX = 0x800;
 
 // Workspaces kept per (device, stream, kind): launches on one stream are ordered, so they can share one; it grows on
 // demand (old one returned to the allocator in stream order) and lives until mxfp6_release_workspaces().
@@ -136,6 +141,10 @@ int choice_code(const mxfp6::KernelChoice& c) {
     case mxfp6::kCandSlice: return c.shares > 1 ? kChoiceBlockKsplit : kChoiceBlock;
     default: return kChoiceGeneric;
   }
+}
+
+int route_of(const mxfp6::GemmArgs& g, const mxfp6::KernelChoice& c, bool split) {
+  return (c.cand == mxfp6::kCandSlice ? kRouteSlice : c.cand < 0 ? (g.ragged ? kChoiceBlock : kChoiceGeneric) : c.cand == mxfp6::kCandTiledSplit256 || c.cand == mxfp6::kCandTiledSplit128 ? kChoiceTiled : c.cand == mxfp6::kCandBlockSplit ? kChoiceBlock : choice_code(c)) | (split ? kRouteSplit : 0);
 }
 
 // What the automatic path may choose from for a call.  force_split: the entry point that allocates nothing fixes the skinny
@@ -301,6 +310,7 @@ bool relayout_then_tiled(const mxfp6::GemmArgs& g, hipStream_t s, hipError_t& e)
   else e = mxfp6::launch_pad_both(g.B, pb, g.Bs, sb, g.N, nullptr, nullptr, nullptr, nullptr, 0, g.K, s);
   if (conv_a) { t.A = pa; t.As = sa; t.layout_a = 1; }
   if (conv_b) { t.B = pb; t.Bs = sb; t.layout_b = 1; }
+  note_route(kChoiceTiled | (conv_a ? kRouteCopyA : 0) | (conv_b ? kRouteCopyB : 0));
   if (e == hipSuccess) e = mxfp6::launch_gemm_tiled(t, s);
   return true;
 }
@@ -326,6 +336,7 @@ bool padded_then_gemm(const mxfp6::GemmArgs& g, const mxfp6::KernelChoice& c, ui
     (void)apply_choice(t, tc, s);
   }
   if (tc.cand < 0 && !apply_ragged(t, s)) return false;
+  note_route(route_of(t, tc, t.ksplit > 1) | kRouteCopyA | (nb ? kRouteCopyB : 0));
   e = hipSuccess;
   if (na && nb) e = mxfp6::launch_pad_both(g.A, pa, g.As, sa, g.M, g.B, pb, g.Bs, sb, g.N, g.K, s);
   else if (na) e = mxfp6::launch_pad_both(g.A, pa, g.As, sa, g.M, nullptr, nullptr, nullptr, nullptr, 0, g.K, s);
@@ -388,6 +399,7 @@ int gemm_common(const void* A, const void* B, const void* As, const void* Bs, vo
   if (no_alloc && force_split > 1 && !(M <= 32 && mxfp6::gemm_skinny_supports(g))) return MXFP6_EINVAL_SHAPE;
   if (no_alloc && mxfp6::gemm_skinny_supports(g) && (force_split || auto_choice(g, force_split, false).cand == mxfp6::kCandSkinny) && !mxfp6::gemm_skinny_scratch_fits(g)) return MXFP6_ESCRATCH;
   std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);  // a K split writes and then reads this stream's workspace
+  note_route(force ? force : kChoiceGeneric);
   if (K != 0 && force == 1) {
     e = mxfp6::launch_gemm_generic(g, s);
   } else if (K != 0 && (force == 2 || force == 5 || force == 6 || force == 17)) {
@@ -425,6 +437,7 @@ int gemm_common(const void* A, const void* B, const void* As, const void* Bs, vo
       c = auto_choice(g, force_split, false);
       (void)apply_choice(g, c, s);
     }
+    note_route(route_of(g, c, g.ksplit > 1 || (c.cand == mxfp6::kCandSlice && g.ks_part)));
     switch (c.cand) {
       case mxfp6::kCandTiled256: case mxfp6::kCandTiled128x256: case mxfp6::kCandTiled128x128:
         if (!relayout_then_tiled(g, s, e)) e = mxfp6::launch_gemm_tiled(g, s);
@@ -434,7 +447,14 @@ int gemm_common(const void* A, const void* B, const void* As, const void* Bs, vo
       case mxfp6::kCandSkinny: e = mxfp6::launch_gemm_skinny(g, s); break;
       case mxfp6::kCandRing: e = mxfp6::launch_gemm_ring(g, s); break;
       case mxfp6::kCandSlice: e = mxfp6::launch_gemm_slice(g, c.slice, s); break;
-      default: e = K != 0 && apply_ragged(g, s) ? mxfp6::launch_gemm_block(g, s) : mxfp6::launch_gemm_generic(g, s); break;
+      default:
+        if (K != 0 && apply_ragged(g, s)) {
+          note_route(route_of(g, c, g.ksplit > 1));
+          e = mxfp6::launch_gemm_block(g, s);
+        } else {
+          e = mxfp6::launch_gemm_generic(g, s);
+        }
+        break;
     }
   }
   return e == hipSuccess ? MXFP6_OK : (int)e;
@@ -490,11 +510,13 @@ int mxfp6_linear(const void* X, int x_bf16, const void* W, const void* Ws, void*
       std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
       if (!apply_choice(g, c, s)) c.slice.shares = 1;  // without a workspace, and under capture: unsplit
       g.ep = ep;
+      note_route(kRouteSlice | kRouteX | (c.slice.shares > 1 ? kRouteSplit : 0));
       const hipError_t e = mxfp6::launch_gemm_slice(g, c.slice, s);
       return e == hipSuccess ? MXFP6_OK : (int)e;
     }
     if (c.cand == mxfp6::kCandSkinny) {
       g.ep = ep;
+      note_route(kChoiceSkinny | kRouteX);
       const hipError_t e = mxfp6::launch_gemm_skinny(g, s);
       return e == hipSuccess ? MXFP6_OK : (int)e;
     }
@@ -586,6 +608,7 @@ int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const voi
     if (!(block || split || tiled || slice || ring || (skinny && mxfp6::gemm_skinny_stores_fp6(t))) || !apply_choice(t, ch, s)) return false;
     t.C = C_packed, t.f32out = false, t.C_scale = (uint8_t*)C_scale, t.fmt_c = fmt_c;
     if (force == 23 || force == 24) t.tile_rows = force == 23 ? 3 : 6;
+    note_route(route_of(t, ch, t.ksplit > 1 || (slice && t.ks_part)));
     if (slice) e = mxfp6::launch_gemm_slice(t, ch.slice, s);
     else if (ring) e = mxfp6::launch_gemm_ring(t, s);
     else if (skinny) e = mxfp6::launch_gemm_skinny(t, s);
@@ -838,6 +861,8 @@ int mxfp6_probe_padded(int mode) {
   g_padded = mode;
   return prev;
 }
+
+int mxfp6_probe_route(void) { return g_route; }
 
 int mxfp6_probe_slice(int plan) {
   const int prev = g_slice;

@@ -159,9 +159,9 @@ def test_padded_linear_vs_oracle(hk, padded, M, N, K, bf16):
         assert np.isfinite(got).all() and (np.abs(got - ref) <= bound).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(2604, 704, 5664), (2048, 3784, 3680)])
-def test_padded_route_and_capture(hk, M, N, K):
-    """Products the choice gives to padded copies: the bits of the block kernel's ragged instantiations (sums in the same order), and
+@pytest.mark.parametrize("M,N,K,pays", [(2604, 704, 5664, False), (2048, 3784, 3680, True), (4096, 1504, 3680, True), (2100, 5000, 4000, True)])
+def test_padded_route_and_capture(hk, route, M, N, K, pays):
+    """Products the choice gives to padded copies (and one that it does not): the bits of the block kernel's ragged instantiations (sums in the same order), and
     under capture on a stream without a workspace, where those run."""
     g = torch.Generator(device="cuda").manual_seed(M)
     (a, asc), (b, bsc) = hk.quantize(torch.randn(M, K, device="cuda", generator=g)), hk.quantize(torch.randn(N, K, device="cuda", generator=g) * 0.02)
@@ -170,6 +170,8 @@ def test_padded_route_and_capture(hk, M, N, K):
         hk.dispatch_micro(a, b, asc, bsc, want)
     finally:
         hk.tk_kernel.set_relayout(prev)
+    copies = route.COPY_A | route.COPY_B
+    assert route.gemm(a, b, asc, bsc, got, M, N, K) & copies == (copies if pays else 0)
     hk.dispatch_micro(a, b, asc, bsc, got)
     assert torch.equal(got, want)
     graph, C = torch.cuda.CUDAGraph(), torch.zeros(M, N, device="cuda")
@@ -183,9 +185,10 @@ def test_padded_route_and_capture(hk, M, N, K):
         assert torch.equal(C, want)
 
 
-@pytest.mark.parametrize("M,N,K", [(1001, 2056, 8192), (31, 4104, 8192), (2049, 1000, 16384), (1793, 14336, 8192)])
+# kernel 2 is forced (unsplit: a K split takes no copies) where the choice would be another; MXFP6 output takes copies unforced only
+@pytest.mark.parametrize("M,N,K,kernel", [(1001, 2056, 8192, 2), (31, 4104, 8192, 2), (2049, 1000, 16384, 2), (1793, 14336, 8192, 0), (4999, 2048, 16384, 0), (777, 6152, 16384, 2)])
 @pytest.mark.parametrize("tile_b", [0, 1])
-def test_relayout_of_rows_that_fill_no_row_tile(hk, M, N, K, tile_b):
+def test_relayout_of_rows_that_fill_no_row_tile(hk, route, M, N, K, kernel, tile_b):
     """The tiled kernel's pre-pass on operands whose rows end inside a row-tile: the bits of the row-major path, whose sums are in the
     same order, for every output type, with NaN patterns around the operands and in the workspace before the call."""
     if tile_b and N % 32:
@@ -194,7 +197,9 @@ def test_relayout_of_rows_that_fill_no_row_tile(hk, M, N, K, tile_b):
     qa, qb = hk.quantize(torch.randn(M, K, device="cuda", generator=g)), hk.quantize(torch.randn(N, K, device="cuda", generator=g) * 0.02, 2, tile_b)
     (a, asc), (b, bsc) = [[at(x.cpu().numpy(), 0).view(x.shape) for x in q] for q in (qa, qb)]
     T = hk.tk_kernel
-    prev_k = T.set_kernel(2 if M * N < 10**7 else 0)
+    # which operands are copied: the one with fewer rows, and where that pays twice the other one
+    copied = {(1001, 0): 1, (31, 0): 1, (2049, 0): 3, (1793, 0): 1, (4999, 0): 2, (777, 0): 1}.get((M, tile_b))
+    prev_k, prev_split = T.set_kernel(kernel), T.set_k_split(1)
     try:
         for dtype in (torch.float32, torch.bfloat16, torch.uint8):
             outs = []
@@ -206,14 +211,19 @@ def test_relayout_of_rows_that_fill_no_row_tile(hk, M, N, K, tile_b):
                 try:
                     if dtype == torch.uint8 and N % 32 == 0:
                         C, S = torch.zeros(M, N // 4 * 3, dtype=dtype, device="cuda"), torch.zeros(M, N // 32, dtype=dtype, device="cuda")
+                        if on and copied and not kernel:
+                            assert route.gemm(a, b, asc, bsc, C, M, N, K, lb=tile_b, C_scale=S, k_split=1) == route.TILED | copied << 8
                         hk.dispatch_micro(a, b, asc, bsc, C, layout_b=tile_b, C_scale=S)
                         outs.append(torch.cat([C, S], 1))
                     elif dtype != torch.uint8:
                         C = torch.empty(M, N, dtype=dtype, device="cuda")
+                        if on:
+                            taken = route.gemm(a, b, asc, bsc, C, M, N, K, lb=tile_b, kernel=kernel, k_split=1)
+                            assert taken & 0xff == route.TILED and (taken >> 8 == copied if copied else not taken & route.COPY_B)
                         hk.dispatch_micro(a, b, asc, bsc, C, layout_b=tile_b)
                         outs.append(C)
                 finally:
                     T.set_relayout(prev)
             assert all(torch.equal(x, outs[0]) for x in outs[1:])
     finally:
-        T.set_kernel(prev_k)
+        T.set_kernel(prev_k), T.set_k_split(prev_split)

@@ -79,7 +79,7 @@ def test_alignments(hk, plan, oa, ob, osa, osb, oc):
 
 
 @pytest.mark.parametrize("M,N,K,lb", [(256, 1024, 1024, 1), (128, 512, 2560, 0), (3, 3072, 2688, 0), (48, 704, 928, 0), (90, 390, 3424, 0), (200, 1056, 5120, 1)])
-def test_automatic_route(hk, M, N, K, lb):
+def test_automatic_route(hk, route, M, N, K, lb):
     """Shapes the choice gives to this kernel: fp32, bf16, fused and MXFP6 output on the automatic path, the last one bit for bit
     the quantiser's of the fp32 output."""
     tk = hk.tk_kernel
@@ -88,6 +88,7 @@ def test_automatic_route(hk, M, N, K, lb):
     bp, bsc = co.quantise(o.make_source("weights", (N, K), np.random.default_rng(N)), 3)
     a, asd, b, bsd = (torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in (ap, asc, o.tile_operand(bp) if lb else bp, o.tile_scales(bsc) if lb else bsc))
     got = torch.empty(M, N, device="cuda")
+    assert route.gemm(a, b, asd, bsd, got, M, N, K, 2, 3, 0, lb) & 0xff == route.SLICE
     hk.dispatch_micro(a, b, asd, bsd, got, 2, 3, layout_b=lb)
     assert o.rel_err(got.cpu().numpy(), o.gemm_ref(ap, bp, asc, bsc, 2, 3, acc=np.float64)) <= 1e-5
     bias = torch.randn(N, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
@@ -96,20 +97,22 @@ def test_automatic_route(hk, M, N, K, lb):
     assert torch.equal(fused, (got + bias).clamp_min(0))  # one fp32 addition: exact to its rounding
     if N % 32 == 0:
         cp, cs = torch.empty(M, N // 4 * 3, dtype=torch.uint8, device="cuda"), torch.empty(M, N // 32, dtype=torch.uint8, device="cuda")
+        assert route.gemm(a, b, asd, bsd, cp, M, N, K, 2, 3, 0, lb, C_scale=cs) & 0xff == route.SLICE
         hk.dispatch_micro(a, b, asd, bsd, cp, 2, 3, layout_b=lb, C_scale=cs)
         qp, qs = hk.quantize(got, 2)
         assert torch.equal(cp, qp) and torch.equal(cs, qs)
 
 
-def test_capture_and_streams(hk):
-    """A K split of this kernel: under capture on a stream without a workspace it runs unsplit, on one that has it split; replays
-    equal the eager call."""
+def test_capture_and_streams(hk, route):
+    """A K split of this kernel: under capture it runs unsplit, on a stream that has a workspace too; replays equal the eager call (these
+    sums are exact)."""
     M, N, K = 64, 512, 12288 + 128
     tk = hk.tk_kernel
     assert tk.kernel_choice(M, N, K) == tk.CHOICE_BLOCK_K_SPLIT
     g = torch.Generator(device="cuda").manual_seed(4)
     (a, asc), (b, bsc) = hk.quantize(torch.randn(M, K, device="cuda", generator=g)), hk.quantize(torch.randn(N, K, device="cuda", generator=g) * 0.02)
     eager = torch.empty(M, N, device="cuda")
+    assert route.gemm(a, b, asc, bsc, eager, M, N, K) == route.SLICE | route.SPLIT
     hk.dispatch_micro(a, b, asc, bsc, eager)
     torch.cuda.synchronize()
     for warm in (False, True):
@@ -141,7 +144,7 @@ def order_shows(g, rows, K, scale, sign):
 
 
 @pytest.mark.parametrize("kind,M,N,K,lb", [("linear", 16, 512, 7680, 1), ("linear", 8, 1024, 8192, 1), ("gemm", 64, 1024, 8192, 0), ("gemm", 16, 512, 15872, 1), ("fp6", 64, 1024, 8192, 0)])
-def test_graphs_of_one_stream_share_no_partial_sums(hk, kind, M, N, K, lb):
+def test_graphs_of_one_stream_share_no_partial_sums(hk, route, kind, M, N, K, lb):
     """Calls whose eager form splits K, captured twice on a stream that has run them: a graph has the bits of one captured on a stream
     that has no workspace (which runs unsplit), not those of the split, alone and replayed beside the other graph and the eager call."""
     from hipkittensp_amd.torch_op import MXFP6Linear
@@ -153,9 +156,11 @@ def test_graphs_of_one_stream_share_no_partial_sums(hk, kind, M, N, K, lb):
         layer = MXFP6Linear(w)
         xs = [x.to(torch.bfloat16) for x in xs]
         call = lambda x: (layer(x),)
+        assert route.linear(xs[0], layer, torch.empty(M, N, dtype=torch.bfloat16, device="cuda")) == route.SLICE | route.X | route.SPLIT
     else:
         b, bsc = hk.quantize(w, 2, lb)
         xs = [hk.quantize(x, 2) for x in xs]
+        assert route.gemm(xs[0][0], b, xs[0][1], bsc, torch.empty(M, N, device="cuda"), M, N, K, lb=lb) == route.SLICE | route.SPLIT
 
         def call(x):
             if kind == "gemm":
@@ -236,10 +241,11 @@ def test_quantising_plans_vs_oracle(hk, bf16, plan, M, N, K, lb, shares):
     assert np.isfinite(got).all() and (np.abs(got - ref) <= bound).all()
 
 
-@pytest.mark.parametrize("M,N,K,bf16", [(5, 512, 1024, 1), (23, 1056, 2080, 1), (64, 512, 1536, 1), (17, 768, 640, 0), (100, 512, 768, 0), (8, 512, 18176, 1)])
-def test_quantising_route(hk, M, N, K, bf16):
+@pytest.mark.parametrize("M,N,K,bf16", [(5, 512, 1024, 1), (23, 1056, 2080, 1), (64, 512, 1536, 1), (17, 768, 640, 0), (100, 512, 768, 0), (8, 512, 18176, 1), (12, 1024, 1024, 1)])
+def test_quantising_route(hk, route, M, N, K, bf16):
     """MXFP6Linear's calls of few rows: the bits of quantise, then GEMM (these sums are exact or rounded far below bf16), eager and
-    captured on a stream that has no workspace, odd values in the activations among them."""
+    captured on a stream that has no workspace, odd values in the activations among them.  All but five bf16 rows with K % 512 == 0, which
+    stay with the quantiser, run on the slice kernel."""
     from hipkittensp_amd.torch_op import MXFP6Linear
 
     g = torch.Generator(device="cuda").manual_seed(M)
@@ -255,6 +261,8 @@ def test_quantising_route(hk, M, N, K, bf16):
         hk.dispatch_micro(xp, layer.weight_packed, xs, layer.weight_scale, want, layout_b=layer.layout_w, bias=layer.bias, activation="relu")
         return want
 
+    taken = route.linear(x, layer, torch.empty(M, N, dtype=torch.bfloat16, device="cuda"))
+    assert (taken & ~route.SPLIT == route.SLICE | route.X) == ((M, bf16) != (5, 1)) and bool(taken & route.X) == ((M, bf16) != (5, 1))
     assert torch.equal(layer(x).view(torch.int16), steps().view(torch.int16))
     graph = torch.cuda.CUDAGraph()
     torch.cuda.synchronize()
