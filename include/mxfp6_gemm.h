@@ -280,8 +280,10 @@ int mxfp6_gemm_fused_fp6(const void *A_packed, const void *B_packed, const void 
  * A linear layer on unquantised activations: X [M, K] (fp32, or bf16 with x_bf16 != 0; 16-byte aligned) is quantised to
  * MXFP6 (fmt_x) as mxfp6_quantize_ex / mxfp6_quantize_bf16 would, and
  *   C[m][n] = act((dq(X) . dq(W)^T)[m][n] + bias[n])         bf16
- * as mxfp6_gemm_fused would compute it from that operand.  W_packed [N, 3K/4], W_scale: the weights in layout_w; bias as in
- * mxfp6_gemm_fused (NULL = none).  The packed activations live in a workspace of this stream (0.79 bytes per element of X,
+ * in fp32 sums of the products that mxfp6_gemm_fused forms from that operand.  Where the activations are quantised inside the GEMM kernel
+ * or the operands copied first, another kernel may run than in the two calls and add in another order: equal where the sums are exact, else
+ * within their rounding, K / 32 + 32 last places of fp32 (2^-24 each) of sum_k |x_mk| |w_nk|, which shows where large products cancel.
+ * W_packed [N, 3K/4], W_scale: the weights in layout_w; bias as in mxfp6_gemm_fused (NULL = none).  The packed activations live in a workspace of this stream (0.79 bytes per element of X,
  * rows rounded up to 32), in the layout the GEMM prefers.  MXFP6_EWORKSPACE, and nothing launched, where it cannot be had,
  * and while the stream is being captured (two graphs captured on one stream would share it).  Calls of few rows (up to 128, by
  * size) quantise inside the slice or the decode kernel: they need no workspace for them and are captured.  No counterpart in the reference.

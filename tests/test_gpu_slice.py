@@ -273,3 +273,26 @@ def test_quantising_route(hk, route, M, N, K, bf16):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, steps()) and torch.equal(layer(x), steps())
+
+
+@pytest.mark.parametrize("M,N,K,bf16", [(8, 512, 4096, 1), (16, 512, 7680, 1), (33, 96, 2080, 1), (100, 512, 768, 0), (7, 1024, 2048, 0), (128, 544, 1056, 1)])
+def test_layers_whose_products_cancel(hk, route, M, N, K, bf16):
+    """Quantised inside the kernel the sums run in another order than in the two calls: both lie within the fp32 sums' rounding of
+    the exact product, half a last place (2^-24 of the largest partial sum, sum |x||w| at most) for each of the K / 32 products of a block
+    and the up to 32 partial sums of waves and shares, then half a last place of bf16, 2^-9 of the value (2^-8 with the value's own error)."""
+    from hipkittensp_amd.torch_op import MXFP6Linear
+
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    w, x = order_shows(g, N, K, 0.02, 1.0), order_shows(g, M, K, 1.0, -1.0)
+    x = x.to(torch.bfloat16) if bf16 else x
+    layer = MXFP6Linear(w)
+    assert route.linear(x, layer, torch.empty(M, N, dtype=torch.bfloat16, device="cuda")) & ~route.SPLIT == route.SLICE | route.X
+    xp, xs = hk.quantize(x, 2)
+    two = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    hk.dispatch_micro(xp, layer.weight_packed, xs, layer.weight_scale, two, layout_b=layer.layout_w)
+    wp, ws = co.quantise(w.cpu().numpy(), 2)
+    xd, wd = o.dequantise(xp.cpu().numpy(), xs.cpu().numpy(), 2, np.float64), o.dequantise(wp, ws, 2, np.float64)
+    ref = xd @ wd.T
+    bound = (K / 32 + 32) * 2.0**-24 * (np.abs(xd) @ np.abs(wd).T) + np.abs(ref) * 2.0**-8
+    for y in (layer(x), two):
+        assert (np.abs(y.float().cpu().numpy() - ref) <= bound).all()
