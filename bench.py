@@ -49,8 +49,8 @@ TRAFFIC_JSON = os.path.join(ROOT, "profiles", "traffic.json")
 # the sources whose text decides what the two profiled kernels move; profiles/traffic.json records their hash
 TRAFFIC_SOURCES = {"gemm_tiled_kernel": ("gemm_tiled.hip", "common.hpp", "loader.hpp"), "gemm_skinny_kernel": ("gemm_skinny.hip", "common.hpp", "loader.hpp"),
                    "gemm_ring_kernel_m16": ("gemm_ring.hip", "common.hpp", "loader.hpp"), "gemm_ring_kernel_m64": ("gemm_ring.hip", "common.hpp", "loader.hpp")}
-# kernel behind a code of tk_kernel.kernel_choice, for the decode shapes
-DECODE_KERNELS = {3: "gemm_skinny_kernel", 28: "gemm_ring_kernel", 22: "gemm_block_kernel", 26: "gemm_block_kernel", 27: "gemm_block_kernel", 2: "gemm_tiled_kernel", 25: "gemm_tiled_kernel", 1: "gemm_generic_kernel"}
+# kernel behind a code of tk_kernel.kernel_choice, for the decode shapes (22 and 27 also stand for the slice kernel of small problems)
+DECODE_KERNELS = {3: "gemm_skinny_kernel", 28: "gemm_ring_kernel", 22: "gemm_block_kernel or gemm_slice_kernel", 26: "gemm_block_kernel", 27: "gemm_block_kernel or gemm_slice_kernel", 2: "gemm_tiled_kernel", 25: "gemm_tiled_kernel", 1: "gemm_generic_kernel"}
 
 # shape, formats, source distributions (A, B), seed
 CONFIGS = {

@@ -508,7 +508,11 @@ int mxfp6_linear(const void* X, int x_bf16, const void* W, const void* Ws, void*
     if (g_slice >> 20 > 0) c = {mxfp6::kCandSlice, g_slice >> 12 & 255, 0, 0.0, {g_slice & 15, g_slice >> 4 & 15, g_slice >> 8 & 15, g_slice >> 12 & 255, g_slice >> 20}};
     if (c.cand == mxfp6::kCandSlice) {
       std::lock_guard<std::recursive_mutex> launch_lock(g_sws_launch_mutex);
-      if (!apply_choice(g, c, s)) c.slice.shares = 1;  // without a workspace, and under capture: unsplit
+      if (!apply_choice(g, c, s)) {  // without a workspace, and under capture: unsplit, by the plan for that where there is one
+        const mxfp6::KernelChoice u = mxfp6::choose_linear_kernel(g, 1, auto_mask(g, 0));
+        if (u.cand == mxfp6::kCandSlice) c = u;
+        else c.slice.shares = 1;
+      }
       g.ep = ep;
       note_route(kRouteSlice | kRouteX | (c.slice.shares > 1 ? kRouteSplit : 0));
       const hipError_t e = mxfp6::launch_gemm_slice(g, c.slice, s);

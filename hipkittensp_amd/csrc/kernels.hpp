@@ -29,8 +29,8 @@ struct GemmArgs {
   int no_alloc = 0;                // skinny kernel: the K split keeps its partial tiles in the library's static scratch array instead of an allocated workspace
   int force_split = 0;             // skinny kernel, M <= 32: split K between this many workgroups (1, 2, 4, 8); 0 = by shape
   int ksplit = 0;                  // tiled, block and ring kernels: workgroups that share an output tile (KernelChoice::shares, ragged_shares); needs ks_part
-  float* ks_part = nullptr;        // ... their partial sums: ksplit sets of 32 x 32 tiles (partial_offset), ragged: matrices [M, ragged_pitch(N)] of floats (ring kernel: partial tiles)
-  int* ks_counters = nullptr;      // ring kernel's K split: one arrival counter per tile of C, zero between launches
+  float* ks_part = nullptr;        // ... their partial sums: ksplit sets of 32 x 32 tiles (partial_offset), ragged: matrices [M, ragged_pitch(N)] of floats (ring and slice kernels: partial tiles)
+  int* ks_counters = nullptr;      // K split of the ring and slice kernels: one arrival counter per tile of C, zero between launches
 };
 
 // the LDS-staged kernels fetch operands and scales 16 bytes per lane: all four tensors must be 16-byte aligned

@@ -22,17 +22,19 @@
  * Device memory.  Five uses take a workspace from the stream-ordered allocator
  * (hipMallocAsync on `hip_stream`), at most once per (device, stream) and use (regrown when a later call
  * needs more), and keep it until mxfp6_release_workspaces():
- *   - the gemm entry points on large row-major problems (re-layout pre-pass, see mxfp6_set_relayout):
- *     up to 0.78 (M + N) K bytes;
+ *   - the gemm entry points on large row-major problems and on ragged ones (K % 128, N % 8, operands off 16 bytes) that pay for it
+ *     (copies of the operands, see mxfp6_set_relayout): up to 0.79 (M + N) K bytes with M and N rounded up to 32 and K to 128; mxfp6_linear on ragged
+ *     layers: the same for the weights;
  *   - mxfp6_gemm_fused_fp6 on shapes that the ragged and generic kernels run, or the decode kernel with narrow workgroups (M <= 32, N <= 4096):
  *     4 M N bytes;
- *   - mxfp6_linear: 0.79 M K bytes, M rounded up to 32 (none for calls of few rows that quantise inside the GEMM kernel);
+ *   - mxfp6_linear: 0.79 M K bytes, M rounded up to 32, K to 128 (none for calls of few rows that quantise inside the GEMM kernel);
  *   - the gemm entry points on decode shapes whose K range is split between workgroups (M <= 32, N <= 2048,
  *     K >= 24576): 2 MB;
  *   - the gemm entry points on problems of few output tiles and long K (up to a few hundred rows of A; see
- *     mxfp6_set_k_split), where the LDS-tiled kernel, the block kernel or the ring kernel splits K between workgroups:
+ *     mxfp6_set_k_split), where the LDS-tiled, the block, the ring or the slice kernel splits K between workgroups:
  *     shares * 4 M N bytes of partial sums (tiles times shares never exceed the CUs: at most 64 MB, 256 tiles of
- *     256 x 256 fp32), one workspace for the three kernels, and for the ring kernel one counter per output tile.
+ *     256 x 256 fp32; the slice kernel: at most 640 tiles of 64 x 64, 10.5 MB), one workspace for the four kernels, and for the ring and the slice
+ *     kernel one counter per output tile.
  * While `hip_stream` is being captured nothing is allocated: the pre-pass and the K splits are left out
  * (same results up to the order of fp32 sums, other kernels) unless their workspace exists already, the slice kernel's K split in any
  * case (so that graphs of small calls share nothing), and mxfp6_gemm_fused_fp6 runs
@@ -48,8 +50,9 @@
  *
  * Alignment.  Pointers are accepted from 4-byte alignment on (C: its element size).  The fast kernels
  * fetch 16 bytes per lane: they run when A_packed, B_packed, both scale tensors and C are 16-byte aligned
- * (any tensor PyTorch allocates is); otherwise the call is served by the block kernel's instantiations for any size and
- * alignment (or, where it is small, by the generic kernel), with the same results.
+ * (any tensor PyTorch allocates is); otherwise the call is served by the slice kernel where it is small, by the block kernel's
+ * instantiations for any size and alignment, by kernels on aligned copies of the operands, or, where it is short, by the generic kernel, with the same
+ * results up to the order of fp32 sums.
  *
  * Accuracy.  Products of dequantised values are exact in fp32; with an e2m3 operand on either side the
  * accumulators agree with an fp64 dequantise-and-matmul to fp32 rounding (relative error < 1e-6 of the
@@ -153,7 +156,9 @@ int mxfp6_set_kernel(int which);
  * For large row-major problems the gemm calls first copy one operand or both (with their scales) into
  * tile-major order in this stream's workspace (hipMallocAsync on the caller's stream the first time, kept
  * until mxfp6_release_workspaces()), because the tiled kernel is bound by L2 requests on row-major operands;
- * results are bit-identical.  On a stream that is being captured it runs only if the workspace exists already.
+ * results are bit-identical.  Ragged products (K % 128, N % 8, operands off 16 bytes) and linear layers take such copies too, padded with zeros,
+ * where they pay, and are switched by the same setting; a K split on the copies may add up in another order than without them.
+ * On a stream that is being captured it runs only if the workspace exists already.
  * Switch it off to measure the row-major kernel itself.  No counterpart in the reference.
  */
 int mxfp6_set_relayout(int on);
