@@ -49,7 +49,7 @@ namespace mxfp6 {
 
 // Arguments on activations.  One argument: a call of one token is bound by its host side, where the runtime handles the arguments one by
 // one; it holds how many runs of BR rows of B there are, so that without a split no division stands in front of the first load (GPU time
-// with the twenty arguments of the other instantiations / with this one: 1 x 4096 x 4096 5.41 / 5.08 us, 3 x 8192 x 2048 5.70 / 5.41, 1 x 14336 x
+// with the sixteen arguments of the other instantiations / with this one: 1 x 4096 x 4096 5.41 / 5.08 us, 3 x 8192 x 2048 5.70 / 5.41, 1 x 14336 x
 // 4096 11.65 / 11.37; the Python call, mostly host, 6.8 / 6.35).  Packed operands keep theirs: as one struct 4 x 1024 x 8192 took 5.0 / 4.8, 100 x
 // 6144 x 4096 11.9 / 11.8, but 23 x 4096 x 14336 11.0 / 11.2 and 16 x 4096 x 4096 5.4 / 5.5.
 struct SkinnyXArgs {

@@ -328,7 +328,8 @@ CHOICE_BLOCK_K_SPLIT = 27  # kernel_choice(): the block kernel with its K split 
 
 
 def kernel_choice(M: int, N: int, K: int, layout_a: int = LAYOUT_ROW, layout_b: int = LAYOUT_ROW) -> int:
-    """The kernel (KERNEL_* code, or CHOICE_TILED_K_SPLIT / CHOICE_BLOCK_K_SPLIT) the automatic path takes for this shape; launches nothing."""
+    """The kernel (KERNEL_* code, or CHOICE_TILED_K_SPLIT / CHOICE_BLOCK_K_SPLIT) the automatic path takes for this shape; launches nothing.
+    KERNEL_BLOCK and CHOICE_BLOCK_K_SPLIT also stand for the slice kernel of small problems, which no KERNEL_* code forces."""
     n = _lib.lib().mxfp6_kernel_choice(int(M), int(N), int(K), int(bool(layout_a)) | int(bool(layout_b)) << 1)
     if n < 0:
         _lib.check(n, "kernel_choice")
