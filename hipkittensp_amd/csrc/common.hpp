@@ -152,6 +152,52 @@ __device__ __forceinline__ void store4(float* p, float a, float b, float c, floa
 __device__ __forceinline__ void store1(uint16_t* p, float a) { *p = (uint16_t)(pack_bf16x2(a, 0.f) & 0xffffu); }
 __device__ __forceinline__ void store1(float* p, float a) { *p = a; }
 
+// Whole lines for the stores of an MFMA tile.  A lane holds 16 bytes of row l % 32 in each register, the upper half of the wave the 16
+// bytes behind the lower half's: a store of them touches 32 rows, 32 bytes each, and a line is whole after four stores.  The L2s put that
+// together, but keep all of it until the write-back at the end of the kernel, which nothing runs beside; sent out early, in parts, it
+// takes longer still.  With whole lines, sent out at once (store_streamed), C leaves under the rest of the kernel: us, before / after, tiled 256 x 256
+// and block kernel, tile-major operands: 8192 x 2048 x 512 17.1 / 12.2, 19.6 / 13.7; 1024 x 23552 x 512 26.2 / 22.2, 27.6 / 22.5; 6255 x 1920 x 1536
+// 24.3 / 21.5, 28.0 / 24.9; 4530 x 7936 x 2048 71.7 / 67.3, 78.5 / 75.0; 8192^3 287 / 280 (tiled).  (The same non-temporal in parts of 32 bytes: 19.7, 36.2;
+// 34.7, 56.6; 27.2, 35.7; 91, 95; 307; in parts of 64: 16.0, 16.1; 25.8, 26.2; 21.4, 25.1; 70, 78; 297.  Whole lines without it: 16.6, 19.0; 25.8, 27.2; 24.3,
+// 27.1; 71.1, 76.3; 284.)  A program that reads C in its next kernel keeps the gain or is level (2048 x 14336 x 1024 on the block kernel and the
+// quantiser 57.7 / 51.6, 512 x 2048 x 2048 12.4 / 12.6).
+// pair_rows: y holds what lies 32 bytes behind x's.  Afterwards x holds 64 contiguous bytes of rows 0 - 15 and y those of rows 16 - 31:
+// row l % 16, 16-byte piece 2 (l / 16 % 2) + l / 32 of the four.
+__device__ __forceinline__ void pair_rows(v4i& x, v4i& y) {
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const auto sw = __builtin_amdgcn_permlane16_swap(x[c], y[c], false, false);
+    x[c] = sw[0], y[c] = sw[1];
+  }
+}
+// join_lines: x and y as pair_rows leaves them (the same 16 rows), y's bytes 64 behind x's.  Afterwards x holds 128 contiguous bytes of rows 0
+// - 7 and y those of rows 8 - 15: row l % 8, half l / 8 % 2, piece as before.
+__device__ __forceinline__ void join_lines(v4i& x, v4i& y) {
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    constexpr int kRowRor8 = 0x128;
+    const int lower = __builtin_amdgcn_update_dpp(x[c], y[c], kRowRor8, 0xf, 0xc, false);
+    y[c] = __builtin_amdgcn_update_dpp(y[c], x[c], kRowRor8, 0xf, 0x3, false);
+    x[c] = lower;
+  }
+}
+// A lane's place in what pair_rows leaves (LINE 0) or join_lines (LINE 1): its row, and the 16-byte pieces in front of its own in the row
+template <int LINE>
+__device__ __forceinline__ int line_row(int lane) { return lane & (LINE ? 7 : 15); }
+template <int LINE>
+__device__ __forceinline__ int line_piece(int lane) { return (LINE ? lane >> 1 & 4 : 0) + (lane >> 3 & 2) + (lane >> 5); }
+
+// Stores 16 bytes per lane, non-temporal: lines that are whole go out to memory at once, under the rest of the kernel, and do not wait in the
+// L2s for the write-back at its end.
+// The registers stay as they are for four more cycles: a buffer store of 16 bytes reads its data a little after it has been issued.  The
+// compiler leaves two cycles where the store has no scalar offset and none where it has one, which is not enough (a v_mov of the first
+// dword right behind the store: the last four of every sixteen lanes stored the new value now and then).
+__device__ __forceinline__ void store_streamed(v4i v, const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff) {
+  constexpr int kNonTemporal = 2;
+  __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, voff, soff, kNonTemporal);
+  asm volatile("s_nop 3" ::"v"(v) : "memory");
+}
+
 // Optional work fused into every kernel's epilogue, in fp32 before the output rounding:
 //   y = act(acc * row_scale[m] * col_scale[n] + bias[n])        (each factor / term only if its pointer is set)
 // act: 0 none, 1 relu, 2 gelu (erf form), 3 silu.  bias is float or bf16 (bias_bf16).

@@ -67,7 +67,8 @@ struct BlockArgs {
 //     one of 4) and the reader shifts them into place (v_alignbyte_b32, once per four K-tiles).  With three slots one scale
 //     buffer serves (a group's scales are in registers, and a barrier passed, before the next group's are fetched): 77 KB
 //   * C's rows start at any element: 16-byte stores at element alignment, and single elements where a run of eight (bf16) or
-//     four (fp32) outputs crosses N
+//     four (fp32) outputs crosses N.  Eight lanes' runs are 128 bytes of a row as in the aligned instantiations, if not one line, and leave
+//     non-temporal too (us, before / after: 4000 x 3001 x 1056 32.2 / 28.8, 7490 x 1056 x 672 17.1 / 15.3, 300 x 6001 x 1056 12.4 / 11.4)
 // 500 x 5003 x 2880: 17.0 us against 148.5 on the one-wave-per-tile kernel, which fetches every operand row again for each of
 // its 32 x 32 tiles, 4 bytes per lane.
 template <int FA, int FB, typename Out, int STAGES, int WN, bool FUSED, bool RAGGED = false>
@@ -444,7 +445,7 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
 
   // ---- epilogue, straight from the accumulators.  Register v of lane l is C[m][n] with m = l % 32 and
   // n = 8 (v / 4) + 4 (l / 32) + v % 4 inside a 32 x 32 tile.  bf16: after the conversion lanes l and l + 32 trade halves
-  // (v_permlane32_swap), so that every lane owns 8 consecutive outputs and stores them as 16 bytes.
+  // (v_permlane32_swap), so that every lane owns 8 consecutive outputs, 16 bytes; then lanes trade for whole lines (pair_rows, join_lines).
   const int N = args.N, N2 = N * (int)sizeof(OutT);
   const bool edge = rows_a != kBM || rows_b != kBN;
   if constexpr (FUSED) {
@@ -513,14 +514,15 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   [[maybe_unused]] const size_t ldc = RAGGED && args.nsplit > 1 ? ragged_pitch(N) : N;
   const __amdgpu_buffer_rsrc_t rC = make_rsrc((OutT*)args.C + (size_t)share * args.M * N + (size_t)pm * kBM * N + (size_t)pn * kBN,
                                               (uint32_t)((rows_a - 1) * N + rows_b) * (uint32_t)sizeof(OutT));
-  const int row_l = wm * 64 + r32;
+  const int row_l = wm * 64 + line_row<1>(lane), col_l = wn * 64 + line_piece<1>(lane) * (16 / (int)sizeof(OutT)), voff = row_l * N2 + col_l * (int)sizeof(OutT);
   // RAGGED: `n` consecutive outputs of a row, 16 bytes of them at C's element alignment or, across N, one by one
   [[maybe_unused]] auto store_run = [&](v4i v, int row, int col) __attribute__((always_inline)) {
     constexpr int kRun = 16 / (int)sizeof(OutT);
     if (row >= rows_a || col >= rows_b) return;
     OutT* const p = (OutT*)args.C + ((size_t)share * args.M + (size_t)pm * kBM + row) * ldc + (size_t)pn * kBN + col;
     if (col + kRun <= rows_b) {
-      __builtin_memcpy(p, &v, 16);
+      typedef int v4i_element __attribute__((ext_vector_type(4), aligned(2)));
+      __builtin_nontemporal_store((v4i_element)v, reinterpret_cast<v4i_element*>(p));
     } else {
       OutT o[kRun];
       __builtin_memcpy(o, &v, 16);
@@ -529,9 +531,18 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
         if (col + e < rows_b) p[e] = o[e];
     }
   };
+  // x, y: as pair_rows leaves them, rows `row` on; `col` columns on
+  auto store_rows = [&](v4i x, v4i y, int row, int col) __attribute__((always_inline)) {
+    join_lines(x, y);
+    if constexpr (RAGGED) {
+      store_run(x, row_l + row, col_l + col);
+      store_run(y, row_l + row + 8, col_l + col);
+    } else {
+      if (!edge || (row_l + row < rows_a && col_l + col < rows_b)) store_streamed(x, rC, voff + col * (int)sizeof(OutT), row * N2);
+      if (!edge || (row_l + row + 8 < rows_a && col_l + col < rows_b)) store_streamed(y, rC, voff + col * (int)sizeof(OutT), (row + 8) * N2);
+    }
+  };
   if constexpr (sizeof(OutT) == 2) {
-    const int col_l = wn * 64 + 8 * h;
-    const int voff = row_l * N2 + col_l * 2;
 #pragma unroll
     for (int i = 0; i < 2; i++) {
       uint32_t pk[2][8];
@@ -549,15 +560,15 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
             const auto x = __builtin_amdgcn_permlane32_swap(pk[j][4 * t + c], pk[j][4 * t + 2 + c], false, false);
             pk[j][4 * t + c] = x[0], pk[j][4 * t + 2 + c] = x[1];
           }
+      v4i v[2][2];
 #pragma unroll
-      for (int j = 0; j < 2; j++)
+      for (int j = 0; j < 2; j++) {
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-          const v4i v = {(int)pk[j][4 * t], (int)pk[j][4 * t + 1], (int)pk[j][4 * t + 2], (int)pk[j][4 * t + 3]};
-          if constexpr (RAGGED) store_run(v, row_l + i * 32, col_l + j * 32 + t * 16);
-          else if (!edge || (row_l + i * 32 < rows_a && col_l + j * 32 + t * 16 < rows_b))
-            __builtin_amdgcn_raw_buffer_store_b128(v, rC, voff + j * 64 + t * 32, i * 32 * N2, 0);
-        }
+        for (int t = 0; t < 2; t++) v[j][t] = v4i{(int)pk[j][4 * t], (int)pk[j][4 * t + 1], (int)pk[j][4 * t + 2], (int)pk[j][4 * t + 3]};
+        pair_rows(v[j][0], v[j][1]);
+      }
+#pragma unroll
+      for (int t = 0; t < 2; t++) store_rows(v[0][t], v[1][t], i * 32 + t * 16, 0);
     }
   } else if (!RAGGED && args.nsplit > 1) {
     // this share's partial sums, in the accumulators' order (partial_offset)
@@ -574,19 +585,20 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
             *reinterpret_cast<v4f*>(base + i * band_stride + j * 1024 + gq * 256) = v4f{acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]};
         }
   } else {
-    const int col_l = wn * 64 + 4 * h;
-    const int voff = row_l * N2 + col_l * 4;
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-      for (int j = 0; j < 2; j++)
+      for (int j = 0; j < 2; j++) {
+        v4i v[2][2];
 #pragma unroll
-        for (int gq = 0; gq < 4; gq++) {
-          const v4f f = {acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]};
-          if constexpr (RAGGED) store_run(__builtin_bit_cast(v4i, f), row_l + i * 32, col_l + j * 32 + gq * 8);
-          else if (!edge || (row_l + i * 32 < rows_a && col_l + j * 32 + gq * 8 < rows_b))
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, f), rC, voff + j * 128 + gq * 32, i * 32 * N2, 0);
-        }
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) v[q >> 1][q & 1][e] = __float_as_int(acc[i][j][4 * q + e]);
+#pragma unroll
+        for (int p = 0; p < 2; p++) pair_rows(v[p][0], v[p][1]);
+#pragma unroll
+        for (int t = 0; t < 2; t++) store_rows(v[0][t], v[1][t], i * 32 + t * 16, j * 32);
+      }
   }
 }
 

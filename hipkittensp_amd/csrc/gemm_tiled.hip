@@ -3,7 +3,7 @@
 // Data path (no operand byte ever passes through a VGPR on its way to LDS):
 //   global --buffer_load_dwordx4 ... lds--> LDS (3-stage ring) --ds_read_b128--> MFMA source VGPRs
 //   v_mfma_scale_f32_32x32x64_f8f6f4 (fp32 accumulate, E8M0 block scales applied by the instruction)
-//   accumulators --v_cvt_pk_bf16_f32, v_permlane32_swap--> 16 bytes per lane to global
+//   accumulators --v_cvt_pk_bf16_f32, v_permlane{32,16}_swap, v_mov_dpp--> whole lines to global, non-temporal (common.hpp)
 // When there are more output tiles than compute units, one workgroup per CU walks through several tiles:
 // the K-tiles of all its output tiles form one stream through the ring, so the loads of the next tile
 // run under the last K-tiles of the current one and the stores of a finished tile under the first
@@ -601,10 +601,17 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
     OutT* cbase = (OutT*)g->C;
     const __amdgpu_buffer_rsrc_t rC = make_rsrc(cbase + (size_t)(tile_cur & 0xffff) * kBM * N + (size_t)(tile_cur >> 16) * kBN,
                                                 (uint32_t)((rows_a - 1) * N + rows_b) * (uint32_t)sizeof(OutT));
-    const int row_l = wm * (TM * 32) + r32;
+    constexpr int LINE = sizeof(OutT) == 4 || TN == 2;  // a wave's part of a row is at least a line
+    const int row_l = wm * (TM * 32) + line_row<LINE>(lane), col_l = wn * (TN * 32) + line_piece<LINE>(lane) * (16 / (int)sizeof(OutT));
+    const int voff = row_l * N2 + col_l * (int)sizeof(OutT);
+    // x, y: as pair_rows leaves them, rows `row` on; `col` columns on
+    auto store_rows = [&](v4i x, v4i y, int row, int col) __attribute__((always_inline)) {
+      if constexpr (LINE) join_lines(x, y);
+      constexpr int kNext = LINE ? 8 : 16;
+      if (!EDGE || (row_l + row < rows_a && col_l + col < rows_b)) store_streamed(x, rC, voff + col * (int)sizeof(OutT), row * N2);
+      if (!EDGE || (row_l + row + kNext < rows_a && col_l + col < rows_b)) store_streamed(y, rC, voff + col * (int)sizeof(OutT), (row + kNext) * N2);
+    };
     if constexpr (sizeof(OutT) == 2) {
-      const int col_l = wn * (TN * 32) + 8 * h;
-      const int voff = row_l * N2 + col_l * 2;
 #pragma unroll
       for (int i = 0; i < TM; i++) {
         // each phase for the whole 32-row band before the next one, so that no dword waits for its predecessor
@@ -625,29 +632,36 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
               pk[j][4 * t + c] = sw[0], pk[j][4 * t + 2 + c] = sw[1];
             }
         __builtin_amdgcn_sched_barrier(0);
+        v4i v[TN][2];
 #pragma unroll
-        for (int j = 0; j < TN; j++)
+        for (int j = 0; j < TN; j++) {
 #pragma unroll
-          for (int t = 0; t < 2; t++) {
-            const v4i v = {(int)pk[j][4 * t], (int)pk[j][4 * t + 1], (int)pk[j][4 * t + 2], (int)pk[j][4 * t + 3]};
-            if (!EDGE || (row_l + i * 32 < rows_a && col_l + j * 32 + t * 16 < rows_b))
-              __builtin_amdgcn_raw_buffer_store_b128(v, rC, voff + j * 64 + t * 32, i * 32 * N2, 0);
-          }
+          for (int t = 0; t < 2; t++) v[j][t] = v4i{(int)pk[j][4 * t], (int)pk[j][4 * t + 1], (int)pk[j][4 * t + 2], (int)pk[j][4 * t + 3]};
+          pair_rows(v[j][0], v[j][1]);
+        }
+        if constexpr (LINE) {
+#pragma unroll
+          for (int t = 0; t < 2; t++) store_rows(v[0][t], v[TN - 1][t], i * 32 + t * 16, 0);
+        } else {
+          store_rows(v[0][0], v[0][1], i * 32, 0);
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {
-      const int col_l = wn * (TN * 32) + 4 * h;
-      const int voff = row_l * N2 + col_l * 4;
 #pragma unroll
       for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < TN; j++)
+        for (int j = 0; j < TN; j++) {
+          v4i v[2][2];
 #pragma unroll
-          for (int gq = 0; gq < 4; gq++) {
-            const v4f f = {acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]};
-            if (!EDGE || (row_l + i * 32 < rows_a && col_l + j * 32 + gq * 8 < rows_b))
-              __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, f), rC, voff + j * 128 + gq * 32, i * 32 * N2, 0);
-          }
+          for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[q >> 1][q & 1][e] = __float_as_int(acc[i][j][4 * q + e]);
+#pragma unroll
+          for (int p = 0; p < 2; p++) pair_rows(v[p][0], v[p][1]);
+#pragma unroll
+          for (int t = 0; t < 2; t++) store_rows(v[0][t], v[1][t], i * 32 + t * 16, j * 32);
+        }
     }
   };
 
