@@ -29,24 +29,28 @@ namespace mxfp6 {
 // just written it (us, plain / non-temporal, an input from memory: 128 MB of fp32 28.1 / 28.1, 192 MB 40.4 / 40.4, 256 MB 55.1 / 52.5, 128 MB of
 // bf16 30.2 / 31.9; one in the cache 24.3 / 27.0, 35.1 / 40.4, 54.6 / 52.5, 28.9 / 31.9).
 constexpr size_t kCacheBytes = (size_t)256 << 20;  // last-level cache
+// Up to so many chunks, workgroups of one wave: four on one compute unit share its way to memory while other units have none.  us, four
+// waves / one, replayed back to back: 23 x 14336 of bf16 (161 chunks) 2.56 / 2.40, 64 x 4096 2.51 / 2.39, 512 x 4096 (1024) 2.81 / 2.69, 64 x 4096 of
+// fp32 2.80 / 2.52; at twice as many chunks level (1024 x 4096 3.30 / 3.31).
+constexpr long kQFewChunks = 1024;
 constexpr int kQWaves = 4;  // waves per workgroup; a wave fetches 64 blocks at a time (8 KB of fp32, 4 KB of bf16)
 
 
 // In: float, or uint16_t for bf16 (the same values after the exact widening: the bf16 instruction
 // v_cvt_scalef32_pk32_{fp6,bf6}_bf16 was checked against the fp32 one on 1 M values per format, no difference).
-template <int FMT, typename In>
-__global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __restrict__ X, uint8_t* __restrict__ packed,
+template <int FMT, typename In, int W>
+__global__ __launch_bounds__(W * 64) void quantize_kernel(const In* __restrict__ X, uint8_t* __restrict__ packed,
                                                               uint8_t* __restrict__ scales, long nblocks, int nkb, int layout, int rows, int stream_in, int stream_out) {
   constexpr int BB = 32 * (int)sizeof(In), P = BB / 16;  // bytes and 16-byte pieces of a block
   constexpr int kChunk = 64 * BB, NLD = kChunk / 1024;   // bytes and direct loads of a chunk
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[kQWaves * kChunk];
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[W * kChunk];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t buf = (uint32_t)(uintptr_t)(MXFP6_LDS uint8_t*)smem + wave * kChunk;
   const int nkt = (nkb + 3) / 4;  // tile-major only: K-tiles per row (the last one padded with zeros)
   const long nchunks = layout ? (long)((rows + 15) / 16) * nkt : (nblocks + 63) / 64;
-  const long stride = (long)gridDim.x * kQWaves;
-  long chunk = (long)blockIdx.x * kQWaves + wave;
+  const long stride = (long)gridDim.x * W;
+  long chunk = (long)blockIdx.x * W + wave;
 
   // slot s = q * 64 + lane of load q holds piece (s % P) ^ (b % P) of the chunk's block b = s / P; tile-major:
   // block b is K-block b % 4 of row b / 4 of the chunk
@@ -135,14 +139,17 @@ __global__ __launch_bounds__(kQWaves * 64) void quantize_kernel(const In* __rest
 hipError_t launch_quantize(const void* X, int x_bf16, uint8_t* packed, uint8_t* scales, int rows, int K, int fmt, int layout, hipStream_t s) {
   const long nblocks = (long)rows * (K / 32);
   if (nblocks == 0) return hipSuccess;
-  const long nchunks = layout ? (long)((rows + 15) / 16) * ((K + 127) / 128) : (nblocks + 63) / 64, want = (nchunks + kQWaves - 1) / kQWaves;
-  const long most = 0xffffffffL / (kQWaves * 64);  // a launch has less than 2^32 work-items; the chunks past them are the grid's next round
+  const long nchunks = layout ? (long)((rows + 15) / 16) * ((K + 127) / 128) : (nblocks + 63) / 64;
+  const int waves = nchunks <= kQFewChunks ? 1 : kQWaves;
+  const long want = (nchunks + waves - 1) / waves, most = 0xffffffffL / (waves * 64);  // a launch has less than 2^32 work-items; the chunks past them are the grid's next round
   const unsigned grid = (unsigned)(want < most ? want : most);
   const int stream_in = (size_t)rows * K * (x_bf16 ? 2 : 4) >= kCacheBytes, stream_out = (size_t)rows * (K / 4 * 3) >= kStreamBytes;
-#define MXFP6_Q(FMT, T) quantize_kernel<FMT, T><<<grid, kQWaves * 64, 0, s>>>((const T*)X, packed, scales, nblocks, K / 32, layout, rows, stream_in, stream_out)
+#define MXFP6_QW(FMT, T, W) quantize_kernel<FMT, T, W><<<grid, W * 64, 0, s>>>((const T*)X, packed, scales, nblocks, K / 32, layout, rows, stream_in, stream_out)
+#define MXFP6_Q(FMT, T) do { if (waves == 1) MXFP6_QW(FMT, T, 1); else MXFP6_QW(FMT, T, kQWaves); } while (0)
   if (fmt == 2) { if (x_bf16) MXFP6_Q(2, uint16_t); else MXFP6_Q(2, float); }
   else { if (x_bf16) MXFP6_Q(3, uint16_t); else MXFP6_Q(3, float); }
 #undef MXFP6_Q
+#undef MXFP6_QW
   return hipGetLastError();
 }
 
