@@ -69,15 +69,19 @@ struct BlockArgs {
 //   * C's rows start at any element: 16-byte stores at element alignment, and single elements where a run of eight (bf16) or
 //     four (fp32) outputs crosses N.  Eight lanes' runs are 128 bytes of a row as in the aligned instantiations, if not one line, and leave
 //     non-temporal too (us, before / after: 4000 x 3001 x 1056 32.2 / 28.8, 7490 x 1056 x 672 17.1 / 15.3, 300 x 6001 x 1056 12.4 / 11.4)
+// STREAM: B is read with the non-temporal bit: weights larger than the last-level cache holds (kStreamBytes) against one tile row, which
+// nothing reads again.  us, plain / non-temporal, K split: 128 x 8192 x 28672 50.6 / 44.8, row-major 54.0 / 51.9, 96 rows 45.6 / 42.1; unsplit:
+// 128 x 28672 x 8192 41.0 / 38.1.  (An instantiation of its own: picked as the kernel runs, 1024 x 4096 x 14336 paid 58.6 / 59.5 for it.)
 // 500 x 5003 x 2880: 17.0 us against 148.5 on the one-wave-per-tile kernel, which fetches every operand row again for each of
 // its 32 x 32 tiles, 4 bytes per lane.
-template <int FA, int FB, typename Out, int STAGES, int WN, bool FUSED, bool RAGGED = false>
+template <int FA, int FB, typename Out, int STAGES, int WN, bool FUSED, bool RAGGED = false, bool STREAM = false>
 __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_block_kernel(const BlockArgs args) {
   typedef typename Out::type OutT;
   static_assert((STAGES == 3 || STAGES == 4 || STAGES == 6) && (WN == 2 || WN == 4), "ring depth, tile width");
   constexpr bool PAIR = STAGES == 6;
   static_assert(!RAGGED || (WN == 2 && FUSED), "one tile width, one epilogue");
   static_assert(!PAIR || WN == 2, "three slots of two K-tiles");
+  static_assert(!STREAM || PAIR, "three slots of two K-tiles");
   static_assert(sizeof(OutT) != 1 || (FUSED && !RAGGED), "fp6 output: one epilogue, whole 32-blocks");
   constexpr int NW = 2 * WN, kBN = WN * 64, kSlot = kATile + kBN * 96, kScRows = kScA + kBN * 16;
   constexpr int kScBuf = kScRows + (RAGGED ? (kBM + kBN) * 4 : 0);  // RAGGED: 4 more bytes per row behind the rows' 16
@@ -221,6 +225,7 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   auto load_pair = [&]<bool OF_A>(int c, int slot, int n) __attribute__((always_inline)) {
     const uint32_t dst = lds0 + slot * (2 * kSlot) + (OF_A ? 0 : 2 * kATile) + (wave * 6 + n) * 1024;
     if constexpr (OF_A) dma16(c < nchunks ? rA : rZ, dst, voff_a[PAIR ? n : 0] + c * (2 * kstep_a), 0);
+    else if constexpr (STREAM) dma16_nt(c < nchunks ? rB : rZ, dst, voff_b[PAIR ? n : 0] + c * (2 * kstep_b), 0);
     else dma16(c < nchunks ? rB : rZ, dst, voff_b[PAIR ? n : 0] + c * (2 * kstep_b), 0);
   };
   auto load_tile = [&]<bool LA>(int t, int slot) __attribute__((always_inline)) {
@@ -639,7 +644,10 @@ hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, 
     return hipGetLastError();
   }
   if (stages == 0) stages = block_stages(g, grid, cus);
-  if (stages == 6) {
+  if (stages == 6 && a.tiles_m == 1 && (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes && (!f32 || !FUSED)) {
+    if (!f32) gemm_block_kernel<FA, FB, OutBf16, 6, 2, FUSED, false, true><<<grid, 256, 0, s>>>(a);
+    else if constexpr (!FUSED) gemm_block_kernel<FA, FB, OutF32, 6, 2, false, false, true><<<grid, 256, 0, s>>>(a);
+  } else if (stages == 6) {
     if (f32) gemm_block_kernel<FA, FB, OutF32, 6, 2, FUSED><<<grid, 256, 0, s>>>(a);
     else gemm_block_kernel<FA, FB, OutBf16, 6, 2, FUSED><<<grid, 256, 0, s>>>(a);
   } else {

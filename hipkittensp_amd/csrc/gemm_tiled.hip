@@ -137,7 +137,11 @@ struct TiledArgs {
 // then a workspace (partial_offset); ksplit_reduce_kernel adds them in share order and applies
 // the epilogue.  (Summed inside this kernel instead -- partial tiles and arrival counters at device scope, the last
 // wave to arrive adds -- the few waves that end up adding read nsplit tiles each past the L2s: 30 us for 32 MB.)
-template <int FA, int FB, typename Out, int TM, int TN, bool FUSED, int ABL = 0, bool KSPLIT = false>
+// KSPLIT 2: B is read with the non-temporal bit: tile-major weights larger than the last-level cache holds (kStreamBytes) that no second
+// tile row reads again.  us, plain / non-temporal, N = 8192, K = 28672: 256 rows on tiles of 256 70.3 / 66.6, 128 rows on tiles of 128 52.4 / 47.1; not with
+// two tile rows (192 rows on tiles of 128 61.4 / 70.2), nor below that size (256 x 4096 x 14336 36.5 / 37.5), nor row-major, where a line is read
+// twice (128 rows 60.4 / 67.8).  (A kernel that picks the bit as it runs: 256 x 4096 x 14336 39.4 / 41.2 in the same call.)
+template <int FA, int FB, typename Out, int TM, int TN, bool FUSED, int ABL = 0, int KSPLIT = 0>
 __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs args) {
   typedef Shape<TM, TN> S;
   constexpr int kBM = S::BM, kBN = S::BN, OPA = S::OPA, OPA1 = S::OPA1, OPB = S::OPB, kLoadsInCompute = S::kLoadsInCompute;
@@ -315,6 +319,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
       dma16(rA, dst + split_base + n * 1024, voff_a[n], t * kstep_a);
     } else {
       if (n < OPAg) dma16(rA, dst + (qa0 + n) * 1024, voff_a[n], t * kstep_a);
+      else if constexpr (KSPLIT == 2) dma16_nt(rB, dst + kAStage + (wave * OPB + n - OPAg) * 1024, voff_b[n - OPAg], t * kstep_b);
       else dma16(rB, dst + kAStage + (wave * OPB + n - OPAg) * 1024, voff_b[n - OPAg], t * kstep_b);
     }
   };
@@ -501,9 +506,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
   // m = l % 32 and n = 8 (v / 4) + 4 (l / 32) + v % 4 inside every 32x32 tile: lanes l and l + 32 hold the two
   // halves of each run of 8 consecutive n of one row.  bf16: after the conversion the two lanes trade halves
   // (v_permlane32_swap: the upper lanes' first run for the lower lanes' second), so that every lane owns 8
-  // consecutive outputs and stores them as 16 bytes; two stores complete a row's 64-byte sector and four its
-  // 128-byte line, back to back.  (8 bytes per lane and row, the accumulators as they are, measured 1.4x the
-  // output in HBM write traffic; 4 bytes per lane with rows down the lanes, 64 stores per wave, measured
+  // consecutive outputs, 16 bytes; further trades (pair_rows, join_lines) make a store eight whole lines.  (8 bytes per lane and row, the
+  // accumulators as they are, measured 1.4x the output in HBM write traffic; 4 bytes per lane with rows down the lanes, 64 stores per wave, measured
   // ~47 clocks per store instruction.)  Nothing here touches LDS, so the ring keeps streaming the next output
   // tile meanwhile.  The stores count in vmcnt like the loads and retire in order with them, so the waits of
   // the K loop ("all but the newest batch") stay valid.
@@ -922,8 +926,11 @@ static hipError_t launch(const GemmArgs& g, hipStream_t s) {
       TiledArgs tp = ta;  // the shares write fp32 partial matrices into the workspace, without the epilogue
       tp.C = g.ks_part, tp.ep = Epilogue{};
       const int grid = tiled_grid_size(g, tm * tn * g.ksplit, 1);
-      if (bm == 128) gemm_tiled_kernel<FA, FB, OutF32, 2, 2, false, 0, true><<<grid, NW * 64, 0, s>>>(tp);
-      else gemm_tiled_kernel<FA, FB, OutF32, 4, 2, false, 0, true><<<grid, NW * 64, 0, s>>>(tp);
+      if (tm == 1 && g.layout_b && (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes) {
+        if (bm == 128) gemm_tiled_kernel<FA, FB, OutF32, 2, 2, false, 0, 2><<<grid, NW * 64, 0, s>>>(tp);
+        else gemm_tiled_kernel<FA, FB, OutF32, 4, 2, false, 0, 2><<<grid, NW * 64, 0, s>>>(tp);
+      } else if (bm == 128) gemm_tiled_kernel<FA, FB, OutF32, 2, 2, false, 0, 1><<<grid, NW * 64, 0, s>>>(tp);
+      else gemm_tiled_kernel<FA, FB, OutF32, 4, 2, false, 0, 1><<<grid, NW * 64, 0, s>>>(tp);
       const hipError_t e = hipGetLastError();
       return e != hipSuccess ? e : launch_ksplit_reduce(g, s);
     } else {
