@@ -669,10 +669,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
     }
   };
 
-  // ---- all output tiles of this workgroup
-  auto run = [&]<int GRP>() __attribute__((always_inline)) {
+  // ---- all output tiles of this workgroup.  The two groups have K loops of their own but one epilogue: code that runs once per output tile
+  // comes through the instruction cache line by line, and what the first group has fetched the second finds there (us, an epilogue
+  // for each group / one: 2048 x 14336 x 4096 with silu 92.7 / 86.9, gelu 99.6 / 93.8; 4530 x 7936 x 2048 with silu 85.2 / 78.4; 1024 x 14336 x 4096 with silu and
+  // MXFP6 output 47.9 / 45.8; without an activation level).
+  auto run = [&]() __attribute__((always_inline)) {
     for (;;) {
-      k_loop.template operator()<GRP>();
+      if (wm == 0) k_loop.template operator()<0>();
+      else k_loop.template operator()<1>();
       if constexpr (FUSED) fuse();
       {
         const auto g = fresh_args();
@@ -727,13 +731,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
   }
   barrier();
   abl_started = true;
-  if (wm == 0) {
-    run.template operator()<0>();
-    barrier();  // every wave executes the same number of barriers
-  } else {
-    barrier();  // phase offset of group 1
-    run.template operator()<1>();
-  }
+  if (wm == 1) barrier();  // phase offset of group 1
+  run();
+  if (wm == 0) barrier();  // every wave executes the same number of barriers
   wait_vmcnt<0>();  // no direct load may still be on its way into LDS when the workgroup gives the memory back
   clock_stamp(1);
 }
