@@ -71,7 +71,7 @@ struct BlockArgs {
 //     non-temporal too (us, before / after: 4000 x 3001 x 1056 32.2 / 28.8, 7490 x 1056 x 672 17.1 / 15.3, 300 x 6001 x 1056 12.4 / 11.4)
 // STREAM: B is read with the non-temporal bit: weights larger than the last-level cache holds (kStreamBytes) against one tile row, which
 // nothing reads again.  us, plain / non-temporal, K split: 128 x 8192 x 28672 50.6 / 44.8, row-major 54.0 / 51.9, 96 rows 45.6 / 42.1; unsplit:
-// 128 x 28672 x 8192 41.0 / 38.1.  (An instantiation of its own: picked as the kernel runs, 1024 x 4096 x 14336 paid 58.6 / 59.5 for it.)
+// 128 x 28672 x 8192 41.0 / 38.1; not where row-major rows start inside a line, which is then read twice (128 x 17840 x 10880 67.7 / 70.9).  (An instantiation of its own: picked as the kernel runs, 1024 x 4096 x 14336 paid 58.6 / 59.5 for it.)
 // 500 x 5003 x 2880: 17.0 us against 148.5 on the one-wave-per-tile kernel, which fetches every operand row again for each of
 // its 32 x 32 tiles, 4 bytes per lane.
 template <int FA, int FB, typename Out, int STAGES, int WN, bool FUSED, bool RAGGED = false, bool STREAM = false>
@@ -644,7 +644,7 @@ hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, 
     return hipGetLastError();
   }
   if (stages == 0) stages = block_stages(g, grid, cus);
-  if (stages == 6 && a.tiles_m == 1 && (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes && (!f32 || !FUSED)) {
+  if (stages == 6 && a.tiles_m == 1 && (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes && (g.layout_b || g.K % 512 == 0) && (!f32 || !FUSED)) {
     if (!f32) gemm_block_kernel<FA, FB, OutBf16, 6, 2, FUSED, false, true><<<grid, 256, 0, s>>>(a);
     else if constexpr (!FUSED) gemm_block_kernel<FA, FB, OutF32, 6, 2, false, false, true><<<grid, 256, 0, s>>>(a);
   } else if (stages == 6) {
