@@ -546,6 +546,10 @@ CALIBRATION = [
       (6144, 6144), (12288, 6144), (3072, 12288), (20480, 5120), (18432, 9216), (7168, 20480), (49152, 4096), (2560, 10240), (13824, 5120), (5120, 13824), (100352, 2048), (1536, 32768)], CALIBRATION_ROWS),
     ([(9216, 9216), (7168, 7168), (3328, 16640), (36864, 3072), (45056, 3584), (1792, 14336), (18944, 3584), (30720, 2560), (27648, 5120)],
      sorted(CALIBRATION_ROWS + [28, 56, 104, 176, 208, 288, 576, 832, 1280, 2304])),
+    # short K, where a call is mostly its output: without these the longer K of the others spoke for it (8192 x 2048 x 512 13.9 us on the block kernel, 12.2 on
+    # tiles of 256 x 256; 6255 x 1920 x 1536 24.9 and 21.5)
+    ([(2048, 512), (8192, 512), (24576, 512), (1024, 1536), (2048, 1536), (5120, 1536), (14336, 1536), (4608, 768), (16384, 768), (4096, 256), (16384, 256)],
+     [1, 16, 32, 64, 96, 128, 192, 256, 384, 512, 768, 1024, 1536, 2048, 3072, 4096, 6144, 8192]),
 ]
 
 
