@@ -155,7 +155,7 @@ __device__ __forceinline__ void store1(float* p, float a) { *p = a; }
 // Whole lines for the stores of an MFMA tile.  A lane holds 16 bytes of row l % 32 in each register, the upper half of the wave the 16
 // bytes behind the lower half's: a store of them touches 32 rows, 32 bytes each, and a line is whole after four stores.  The L2s put that
 // together, but keep all of it until the write-back at the end of the kernel, which nothing runs beside; sent out early, in parts, it
-// takes longer still.  With whole lines, sent out at once (store_streamed), C leaves under the rest of the kernel: us, before / after, tiled 256 x 256
+// takes longer still.  With whole lines, sent out at once (store_c), C leaves under the rest of the kernel: us, before / after, tiled 256 x 256
 // and block kernel, tile-major operands: 8192 x 2048 x 512 17.1 / 12.2, 19.6 / 13.7; 1024 x 23552 x 512 26.2 / 22.2, 27.6 / 22.5; 6255 x 1920 x 1536
 // 24.3 / 21.5, 28.0 / 24.9; 4530 x 7936 x 2048 71.7 / 67.3, 78.5 / 75.0; 8192^3 287 / 280 (tiled).  (The same non-temporal in parts of 32 bytes: 19.7, 36.2;
 // 34.7, 56.6; 27.2, 35.7; 91, 95; 307; in parts of 64: 16.0, 16.1; 25.8, 26.2; 21.4, 25.1; 70, 78; 297.  Whole lines without it: 16.6, 19.0; 25.8, 27.2; 24.3,
@@ -192,10 +192,22 @@ __device__ __forceinline__ int line_piece(int lane) { return (LINE ? lane >> 1 &
 // The registers stay as they are for four more cycles: a buffer store of 16 bytes reads its data a little after it has been issued.  The
 // compiler leaves two cycles where the store has no scalar offset and none where it has one, which is not enough (a v_mov of the first
 // dword right behind the store: the last four of every sixteen lanes stored the new value now and then).
-__device__ __forceinline__ void store_streamed(v4i v, const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff) {
+// STREAM false: the same through the L2s.
+template <bool STREAM>
+__device__ __forceinline__ void store_c(v4i v, const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff) {
   constexpr int kNonTemporal = 2;
-  __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, voff, soff, kNonTemporal);
+  __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, voff, soff, STREAM ? kNonTemporal : 0);
   asm volatile("s_nop 3" ::"v"(v) : "memory");
+}
+// Whether C, `rows` rows of `pitch` outputs, goes out non-temporally: where its rows start on lines, and where all of it is small beside the
+// L2s (32 MB).  Rows that start inside a line leave every line to two stores, and of a large C the L2s send out the first part before the
+// second has come.  us, non-temporal / through the L2s, fp32: 2000 x 8191 x 1056 52.4 / 42.8, 4096 x 11000 x 1024 113 / 82, 1000 x 5003 x 1056 (20 MB) 18.8 /
+// 20.2; bf16: 4096 x 11000 x 1024 69.6 / 64.1, 3500 x 5000 x 1024 (35 MB) 31.9 / 29.9, 2048 x 5000 x 1024 (20 MB) 18.9 / 20.4.
+constexpr size_t kStreamedPartLines = (size_t)24 << 20;
+template <typename OutT>
+__device__ __forceinline__ bool streams_c(const void* C, int rows, size_t pitch, size_t limit = kStreamedPartLines) {
+  const size_t row = pitch * sizeof(OutT);
+  return (((uintptr_t)C | row) & 127) == 0 || rows * row <= limit;
 }
 
 // Optional work fused into every kernel's epilogue, in fp32 before the output rounding:

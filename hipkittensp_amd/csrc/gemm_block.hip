@@ -520,14 +520,17 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   const __amdgpu_buffer_rsrc_t rC = make_rsrc((OutT*)args.C + (size_t)share * args.M * N + (size_t)pm * kBM * N + (size_t)pn * kBN,
                                               (uint32_t)((rows_a - 1) * N + rows_b) * (uint32_t)sizeof(OutT));
   const int row_l = wm * 64 + line_row<1>(lane), col_l = wn * 64 + line_piece<1>(lane) * (16 / (int)sizeof(OutT)), voff = row_l * N2 + col_l * (int)sizeof(OutT);
+  // (RAGGED, bf16: up to 36 MB; us as at streams_c: 2000 x 8191 x 1056 (33 MB) 39.7 / 42.3, 2000 x 8189 x 2080 50.2 / 54.9)
+  const bool streamed = streams_c<OutT>(args.C, args.M * (RAGGED ? args.nsplit : 1), ldc, RAGGED && sizeof(OutT) == 2 ? (size_t)36 << 20 : kStreamedPartLines);
   // RAGGED: `n` consecutive outputs of a row, 16 bytes of them at C's element alignment or, across N, one by one
-  [[maybe_unused]] auto store_run = [&](v4i v, int row, int col) __attribute__((always_inline)) {
+  [[maybe_unused]] auto store_run = [&]<bool NT>(v4i v, int row, int col) __attribute__((always_inline)) {
     constexpr int kRun = 16 / (int)sizeof(OutT);
     if (row >= rows_a || col >= rows_b) return;
     OutT* const p = (OutT*)args.C + ((size_t)share * args.M + (size_t)pm * kBM + row) * ldc + (size_t)pn * kBN + col;
     if (col + kRun <= rows_b) {
       typedef int v4i_element __attribute__((ext_vector_type(4), aligned(2)));
-      __builtin_nontemporal_store((v4i_element)v, reinterpret_cast<v4i_element*>(p));
+      if constexpr (NT) __builtin_nontemporal_store((v4i_element)v, reinterpret_cast<v4i_element*>(p));
+      else *reinterpret_cast<v4i_element*>(p) = (v4i_element)v;
     } else {
       OutT o[kRun];
       __builtin_memcpy(o, &v, 16);
@@ -537,74 +540,79 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
     }
   };
   // x, y: as pair_rows leaves them, rows `row` on; `col` columns on
-  auto store_rows = [&](v4i x, v4i y, int row, int col) __attribute__((always_inline)) {
+  auto store_rows = [&]<bool NT>(v4i x, v4i y, int row, int col) __attribute__((always_inline)) {
     join_lines(x, y);
     if constexpr (RAGGED) {
-      store_run(x, row_l + row, col_l + col);
-      store_run(y, row_l + row + 8, col_l + col);
+      store_run.template operator()<NT>(x, row_l + row, col_l + col);
+      store_run.template operator()<NT>(y, row_l + row + 8, col_l + col);
     } else {
-      if (!edge || (row_l + row < rows_a && col_l + col < rows_b)) store_streamed(x, rC, voff + col * (int)sizeof(OutT), row * N2);
-      if (!edge || (row_l + row + 8 < rows_a && col_l + col < rows_b)) store_streamed(y, rC, voff + col * (int)sizeof(OutT), (row + 8) * N2);
+      if (!edge || (row_l + row < rows_a && col_l + col < rows_b)) store_c<NT>(x, rC, voff + col * (int)sizeof(OutT), row * N2);
+      if (!edge || (row_l + row + 8 < rows_a && col_l + col < rows_b)) store_c<NT>(y, rC, voff + col * (int)sizeof(OutT), (row + 8) * N2);
     }
   };
-  if constexpr (sizeof(OutT) == 2) {
+  // two copies of the rest, rather than a choice at each store: that costs up to 3 % of a short fp32 product
+  auto store_tile = [&]<bool NT>() __attribute__((always_inline)) {
+    if constexpr (sizeof(OutT) == 2) {
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-      uint32_t pk[2][8];
+      for (int i = 0; i < 2; i++) {
+        uint32_t pk[2][8];
 #pragma unroll
-      for (int j = 0; j < 2; j++)
+        for (int j = 0; j < 2; j++)
 #pragma unroll
-        for (int e = 0; e < 8; e++) pk[j][e] = pack_bf16x2(acc[i][j][2 * e], acc[i][j][2 * e + 1]);
+          for (int e = 0; e < 8; e++) pk[j][e] = pack_bf16x2(acc[i][j][2 * e], acc[i][j][2 * e + 1]);
 #pragma unroll
-      for (int j = 0; j < 2; j++)
+        for (int j = 0; j < 2; j++)
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+          for (int t = 0; t < 2; t++)
 #pragma unroll
-          for (int c = 0; c < 2; c++) {
-            // runs 2t and 2t+1 (dwords 4t+c and 4t+2+c): lower lanes keep run 2t and get the partner's, upper lanes run 2t+1
-            const auto x = __builtin_amdgcn_permlane32_swap(pk[j][4 * t + c], pk[j][4 * t + 2 + c], false, false);
-            pk[j][4 * t + c] = x[0], pk[j][4 * t + 2 + c] = x[1];
-          }
-      v4i v[2][2];
-#pragma unroll
-      for (int j = 0; j < 2; j++) {
-#pragma unroll
-        for (int t = 0; t < 2; t++) v[j][t] = v4i{(int)pk[j][4 * t], (int)pk[j][4 * t + 1], (int)pk[j][4 * t + 2], (int)pk[j][4 * t + 3]};
-        pair_rows(v[j][0], v[j][1]);
-      }
-#pragma unroll
-      for (int t = 0; t < 2; t++) store_rows(v[0][t], v[1][t], i * 32 + t * 16, 0);
-    }
-  } else if (!RAGGED && args.nsplit > 1) {
-    // this share's partial sums, in the accumulators' order (partial_offset)
-    const int band0 = pm * (kBM / 32) + wm * 2, ct0 = pn * (kBN / 32) + wn * 2;
-    float* const base = (float*)args.C + partial_offset(share, band0, ct0, args.M, N) / 4 + lane * 4;
-    const size_t band_stride = ((size_t)N + 31) / 32 * 1024;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int j = 0; j < 2; j++)
-        if ((band0 + i) * 32 + r32 < args.M && (ct0 + j) * 32 < N) {
-#pragma unroll
-          for (int gq = 0; gq < 4; gq++)
-            *reinterpret_cast<v4f*>(base + i * band_stride + j * 1024 + gq * 256) = v4f{acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]};
-        }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int j = 0; j < 2; j++) {
+            for (int c = 0; c < 2; c++) {
+              // runs 2t and 2t+1 (dwords 4t+c and 4t+2+c): lower lanes keep run 2t and get the partner's, upper lanes run 2t+1
+              const auto x = __builtin_amdgcn_permlane32_swap(pk[j][4 * t + c], pk[j][4 * t + 2 + c], false, false);
+              pk[j][4 * t + c] = x[0], pk[j][4 * t + 2 + c] = x[1];
+            }
         v4i v[2][2];
 #pragma unroll
-        for (int q = 0; q < 4; q++)
+        for (int j = 0; j < 2; j++) {
 #pragma unroll
-          for (int e = 0; e < 4; e++) v[q >> 1][q & 1][e] = __float_as_int(acc[i][j][4 * q + e]);
+          for (int t = 0; t < 2; t++) v[j][t] = v4i{(int)pk[j][4 * t], (int)pk[j][4 * t + 1], (int)pk[j][4 * t + 2], (int)pk[j][4 * t + 3]};
+          pair_rows(v[j][0], v[j][1]);
+        }
 #pragma unroll
-        for (int p = 0; p < 2; p++) pair_rows(v[p][0], v[p][1]);
-#pragma unroll
-        for (int t = 0; t < 2; t++) store_rows(v[0][t], v[1][t], i * 32 + t * 16, j * 32);
+        for (int t = 0; t < 2; t++) store_rows.template operator()<NT>(v[0][t], v[1][t], i * 32 + t * 16, 0);
       }
-  }
+    } else if (!RAGGED && args.nsplit > 1) {
+      // this share's partial sums, in the accumulators' order (partial_offset)
+      const int band0 = pm * (kBM / 32) + wm * 2, ct0 = pn * (kBN / 32) + wn * 2;
+      float* const base = (float*)args.C + partial_offset(share, band0, ct0, args.M, N) / 4 + lane * 4;
+      const size_t band_stride = ((size_t)N + 31) / 32 * 1024;
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          if ((band0 + i) * 32 + r32 < args.M && (ct0 + j) * 32 < N) {
+#pragma unroll
+            for (int gq = 0; gq < 4; gq++)
+              *reinterpret_cast<v4f*>(base + i * band_stride + j * 1024 + gq * 256) = v4f{acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]};
+          }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          v4i v[2][2];
+#pragma unroll
+          for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[q >> 1][q & 1][e] = __float_as_int(acc[i][j][4 * q + e]);
+#pragma unroll
+          for (int p = 0; p < 2; p++) pair_rows(v[p][0], v[p][1]);
+#pragma unroll
+          for (int t = 0; t < 2; t++) store_rows.template operator()<NT>(v[0][t], v[1][t], i * 32 + t * 16, j * 32);
+        }
+    }
+  };
+  if (streamed) store_tile.template operator()<true>();
+  else store_tile.template operator()<false>();
 }
 
 int cu_count_of_device() {

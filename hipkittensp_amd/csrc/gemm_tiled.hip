@@ -511,7 +511,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
   // ~47 clocks per store instruction.)  Nothing here touches LDS, so the ring keeps streaming the next output
   // tile meanwhile.  The stores count in vmcnt like the loads and retire in order with them, so the waits of
   // the K loop ("all but the newest batch") stay valid.
-  // EDGE: the tile has fewer than 256 valid rows or columns; those stores are predicated per lane.
+  // EDGE: the tile has fewer than 256 valid rows or columns; those stores are predicated per lane, and so are all of a C
+  // that goes through the L2s (streams_c; a third copy for those made the loop's code worse: 8192 x 8192 x 16384 e3m2 x e2m3 605 -> 619 us).
   typedef typename Out::type OutT;
   // Fused scales / bias / activation, on the accumulators themselves, before the epilogue proper.  Per 32x32 tile a
   // lane owns row wm * TM * 32 + 32 i + lane % 32 and columns 8 q + 4 h .. + 3 for q = 0..3; N % 8 == 0, so a run of
@@ -573,7 +574,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
       }
     }
   };
-  auto epilogue = [&]<bool EDGE>(int rows_a, int rows_b) __attribute__((always_inline)) {
+  auto c_streams = [&]() __attribute__((always_inline)) {
+    if constexpr (KSPLIT != 0 || sizeof(OutT) == 1) return true;
+    else {
+      const auto g = fresh_args();
+      return streams_c<OutT>(g->C, g->M, (size_t)g->N);
+    }
+  };
+  auto epilogue = [&]<bool EDGE>(int rows_a, int rows_b, [[maybe_unused]] bool streamed) __attribute__((always_inline)) {
     const auto g = fresh_args();
     if constexpr (sizeof(OutT) == 1) {
       // C re-quantised to MXFP6 along N (the next GEMM's K): a wave's two tiles of a band at a time
@@ -612,8 +620,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
     auto store_rows = [&](v4i x, v4i y, int row, int col) __attribute__((always_inline)) {
       if constexpr (LINE) join_lines(x, y);
       constexpr int kNext = LINE ? 8 : 16;
-      if (!EDGE || (row_l + row < rows_a && col_l + col < rows_b)) store_streamed(x, rC, voff + col * (int)sizeof(OutT), row * N2);
-      if (!EDGE || (row_l + row + kNext < rows_a && col_l + col < rows_b)) store_streamed(y, rC, voff + col * (int)sizeof(OutT), (row + kNext) * N2);
+      if (!EDGE || streamed) {
+        if (!EDGE || (row_l + row < rows_a && col_l + col < rows_b)) store_c<true>(x, rC, voff + col * (int)sizeof(OutT), row * N2);
+        if (!EDGE || (row_l + row + kNext < rows_a && col_l + col < rows_b)) store_c<true>(y, rC, voff + col * (int)sizeof(OutT), (row + kNext) * N2);
+      } else {
+        if (row_l + row < rows_a && col_l + col < rows_b) store_c<false>(x, rC, voff + col * (int)sizeof(OutT), row * N2);
+        if (row_l + row + kNext < rows_a && col_l + col < rows_b) store_c<false>(y, rC, voff + col * (int)sizeof(OutT), (row + kNext) * N2);
+      }
     };
     if constexpr (sizeof(OutT) == 2) {
 #pragma unroll
@@ -681,8 +694,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
       {
         const auto g = fresh_args();
         const int rows_a = min(kBM, g->M - (tile_cur & 0xffff) * kBM), rows_b = min(kBN, g->N - (tile_cur >> 16) * kBN);
-        if (rows_a == kBM && rows_b == kBN) epilogue.template operator()<false>(rows_a, rows_b);
-        else epilogue.template operator()<true>(rows_a, rows_b);
+        const bool streamed = c_streams();
+        if (rows_a == kBM && rows_b == kBN && streamed) epilogue.template operator()<false>(rows_a, rows_b, streamed);
+        else epilogue.template operator()<true>(rows_a, rows_b, streamed);
       }
       if (tile_next < 0) break;
       p0 = (p0 + nk4) & 1;

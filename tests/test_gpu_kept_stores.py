@@ -1,0 +1,38 @@
+"""C goes out non-temporally or through the L2s by its size, row pitch and address: both ways give the same bits, on both sides of the line."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+LIMIT = 24 << 20  # bytes of C whose rows start inside lines
+
+
+# kernel (0: the block kernel's ragged instantiation), N, K, rows past a multiple of the tile
+@pytest.mark.parametrize("kernel,N,K,rem", [(2, 4104, 256, 0), (2, 4104, 256, 9), (5, 4104, 256, 5), (6, 4168, 256, 3), (22, 4104, 256, 1), (22, 4168, 1152, 0), (24, 4104, 256, 0), (0, 4107, 1056, 0), (0, 4099, 2080, 7)])
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
+def test_large_output_matches_its_parts(kernel, N, K, rem, out):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import hipkittensp_amd as hk
+
+    tk, size = hk.tk_kernel, torch.finfo(out).bits // 8
+    limit = (36 << 20) if kernel == 0 and size == 2 else LIMIT
+    step = 512
+    M = (limit // (N * size) // step + 2) * step + rem  # past the line; its parts of `step` rows are below
+    assert (N * size) % 128 and M * N * size > limit and step * N * size < limit
+    g = torch.Generator(device="cuda").manual_seed(N)
+    A, As = hk.quantize(torch.randn(M, K, device="cuda", generator=g), 2)
+    B, Bs = hk.quantize(torch.randn(N, K, device="cuda", generator=g).mul_(0.05), 2)
+    guard = torch.full((M * N + 512,), 7.0, dtype=out, device="cuda")
+    prev, prev_split = tk.set_kernel(kernel), tk.set_k_split(1)
+    try:
+        C = guard[256 : 256 + M * N].view(M, N)
+        tk.dispatch_micro(A, B, As, Bs, C, 2, 2)
+        for m in range(0, M, step):
+            part = torch.full((min(step, M - m), N), float("nan"), dtype=out, device="cuda")
+            tk.dispatch_micro(A[m : m + step], B, As[m : m + step], Bs, part, 2, 2)
+            assert torch.equal(part, C[m : m + step]), m
+    finally:
+        tk.set_kernel(prev)
+        tk.set_k_split(prev_split)
+    assert (guard[:256] == 7).all() and (guard[256 + M * N :] == 7).all()
