@@ -205,7 +205,7 @@ __device__ __forceinline__ void store_c(v4i v, const __amdgpu_buffer_rsrc_t& rsr
 // 20.2; bf16: 4096 x 11000 x 1024 69.6 / 64.1, 3500 x 5000 x 1024 (35 MB) 31.9 / 29.9, 2048 x 5000 x 1024 (20 MB) 18.9 / 20.4.
 constexpr size_t kStreamedPartLines = (size_t)24 << 20;
 template <typename OutT>
-__device__ __forceinline__ bool streams_c(const void* C, int rows, size_t pitch, size_t limit = kStreamedPartLines) {
+__host__ __device__ inline bool streams_c(const void* C, int rows, size_t pitch, size_t limit = kStreamedPartLines) {
   const size_t row = pitch * sizeof(OutT);
   return (((uintptr_t)C | row) & 127) == 0 || rows * row <= limit;
 }

@@ -72,6 +72,7 @@ struct BlockArgs {
 // STREAM: B is read with the non-temporal bit: weights larger than the last-level cache holds (kStreamBytes) against one tile row, which
 // nothing reads again.  us, plain / non-temporal, K split: 128 x 8192 x 28672 50.6 / 44.8, row-major 54.0 / 51.9, 96 rows 45.6 / 42.1; unsplit:
 // 128 x 28672 x 8192 41.0 / 38.1; not where row-major rows start inside a line, which is then read twice (128 x 17840 x 10880 67.7 / 70.9).  (An instantiation of its own: picked as the kernel runs, 1024 x 4096 x 14336 paid 58.6 / 59.5 for it.)
+// RAGGED and STREAM: C leaves non-temporally (launch_ragged).
 // 500 x 5003 x 2880: 17.0 us against 148.5 on the one-wave-per-tile kernel, which fetches every operand row again for each of
 // its 32 x 32 tiles, 4 bytes per lane.
 template <int FA, int FB, typename Out, int STAGES, int WN, bool FUSED, bool RAGGED = false, bool STREAM = false>
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   constexpr bool PAIR = STAGES == 6;
   static_assert(!RAGGED || (WN == 2 && FUSED), "one tile width, one epilogue");
   static_assert(!PAIR || WN == 2, "three slots of two K-tiles");
-  static_assert(!STREAM || PAIR, "three slots of two K-tiles");
+  static_assert(!STREAM || PAIR || RAGGED, "three slots of two K-tiles");
   static_assert(sizeof(OutT) != 1 || (FUSED && !RAGGED), "fp6 output: one epilogue, whole 32-blocks");
   constexpr int NW = 2 * WN, kBN = WN * 64, kSlot = kATile + kBN * 96, kScRows = kScA + kBN * 16;
   constexpr int kScBuf = kScRows + (RAGGED ? (kBM + kBN) * 4 : 0);  // RAGGED: 4 more bytes per row behind the rows' 16
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   auto load_pair = [&]<bool OF_A>(int c, int slot, int n) __attribute__((always_inline)) {
     const uint32_t dst = lds0 + slot * (2 * kSlot) + (OF_A ? 0 : 2 * kATile) + (wave * 6 + n) * 1024;
     if constexpr (OF_A) dma16(c < nchunks ? rA : rZ, dst, voff_a[PAIR ? n : 0] + c * (2 * kstep_a), 0);
-    else if constexpr (STREAM) dma16_nt(c < nchunks ? rB : rZ, dst, voff_b[PAIR ? n : 0] + c * (2 * kstep_b), 0);
+    else if constexpr (STREAM && !RAGGED) dma16_nt(c < nchunks ? rB : rZ, dst, voff_b[PAIR ? n : 0] + c * (2 * kstep_b), 0);
     else dma16(c < nchunks ? rB : rZ, dst, voff_b[PAIR ? n : 0] + c * (2 * kstep_b), 0);
   };
   auto load_tile = [&]<bool LA>(int t, int slot) __attribute__((always_inline)) {
@@ -520,8 +521,6 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   const __amdgpu_buffer_rsrc_t rC = make_rsrc((OutT*)args.C + (size_t)share * args.M * N + (size_t)pm * kBM * N + (size_t)pn * kBN,
                                               (uint32_t)((rows_a - 1) * N + rows_b) * (uint32_t)sizeof(OutT));
   const int row_l = wm * 64 + line_row<1>(lane), col_l = wn * 64 + line_piece<1>(lane) * (16 / (int)sizeof(OutT)), voff = row_l * N2 + col_l * (int)sizeof(OutT);
-  // (RAGGED, bf16: up to 36 MB; us as at streams_c: 2000 x 8191 x 1056 (33 MB) 39.7 / 42.3, 2000 x 8189 x 2080 50.2 / 54.9)
-  const bool streamed = streams_c<OutT>(args.C, args.M * (RAGGED ? args.nsplit : 1), ldc, RAGGED && sizeof(OutT) == 2 ? (size_t)36 << 20 : kStreamedPartLines);
   // RAGGED: `n` consecutive outputs of a row, 16 bytes of them at C's element alignment or, across N, one by one
   [[maybe_unused]] auto store_run = [&]<bool NT>(v4i v, int row, int col) __attribute__((always_inline)) {
     constexpr int kRun = 16 / (int)sizeof(OutT);
@@ -550,7 +549,24 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
       if (!edge || (row_l + row + 8 < rows_a && col_l + col < rows_b)) store_c<NT>(y, rC, voff + col * (int)sizeof(OutT), (row + 8) * N2);
     }
   };
-  // two copies of the rest, rather than a choice at each store: that costs up to 3 % of a short fp32 product
+  if constexpr (!RAGGED && sizeof(OutT) == 4) {
+    if (args.nsplit > 1) {
+      // this share's partial sums, in the accumulators' order (partial_offset)
+      const int band0 = pm * (kBM / 32) + wm * 2, ct0 = pn * (kBN / 32) + wn * 2;
+      float* const base = (float*)args.C + partial_offset(share, band0, ct0, args.M, N) / 4 + lane * 4;
+      const size_t band_stride = ((size_t)N + 31) / 32 * 1024;
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          if ((band0 + i) * 32 + r32 < args.M && (ct0 + j) * 32 < N) {
+#pragma unroll
+            for (int gq = 0; gq < 4; gq++)
+              *reinterpret_cast<v4f*>(base + i * band_stride + j * 1024 + gq * 256) = v4f{acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]};
+          }
+      return;
+    }
+  }
   auto store_tile = [&]<bool NT>() __attribute__((always_inline)) {
     if constexpr (sizeof(OutT) == 2) {
 #pragma unroll
@@ -580,20 +596,6 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
 #pragma unroll
         for (int t = 0; t < 2; t++) store_rows.template operator()<NT>(v[0][t], v[1][t], i * 32 + t * 16, 0);
       }
-    } else if (!RAGGED && args.nsplit > 1) {
-      // this share's partial sums, in the accumulators' order (partial_offset)
-      const int band0 = pm * (kBM / 32) + wm * 2, ct0 = pn * (kBN / 32) + wn * 2;
-      float* const base = (float*)args.C + partial_offset(share, band0, ct0, args.M, N) / 4 + lane * 4;
-      const size_t band_stride = ((size_t)N + 31) / 32 * 1024;
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-          if ((band0 + i) * 32 + r32 < args.M && (ct0 + j) * 32 < N) {
-#pragma unroll
-            for (int gq = 0; gq < 4; gq++)
-              *reinterpret_cast<v4f*>(base + i * band_stride + j * 1024 + gq * 256) = v4f{acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]};
-          }
     } else {
 #pragma unroll
       for (int i = 0; i < 2; i++)
@@ -611,7 +613,9 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
         }
     }
   };
-  if (streamed) store_tile.template operator()<true>();
+  // Two copies, rather than a choice at each store, which costs a short fp32 product 3 %; of RAGGED's longer code one (STREAM, launch_ragged)
+  if constexpr (RAGGED) store_tile.template operator()<STREAM>();
+  else if (streams_c<OutT>(args.C, args.M, N)) store_tile.template operator()<true>();
   else store_tile.template operator()<false>();
 }
 
@@ -667,17 +671,25 @@ hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, 
 // RAGGED instantiations, the fused epilogue applied or not inside.  PAIR from K = 1920 on while no CU gets a second workgroup (us,
 // three slots / PAIR: 64 x 3001 x 1888 11.1 / 11.1, 500 x 5003 x 1056 13.2 / 13.6, 100 x 5003 x 2016 17.8 / 16.1), from 6144 on
 // beyond (2000 x 8191 x 4128 107.5 / 105.0, 1000 x 4097 x 4128 47.3 / 48.6, 572 x 22563 x 13760 295 / 266).
+// STREAM: C goes out non-temporally.  As streams_c says, bf16 up to 36 MB (us as there: 2000 x 8191 x 1056, 33 MB, 39.7 / 42.3, 2000 x 8189 x 2080 50.2 /
+// 54.9), from 65 rows on (fp32, 49 x 20832 x 672 7.7 / 7.4, 128 rows 8.7 / 9.7; bf16, 100 x 28001 x 1568 17.7 / 18.3); not the sums of a K split's
+// shares, which are read again at once (512 x 296 x 16960 20.0 / 18.9, a layer of 191 x 664 x 18624 26.5 / 24.5).
 template <int FA, int FB>
 hipError_t launch_ragged(const GemmArgs& g, const BlockArgs& a, int tiles, hipStream_t s) {
   const int grid = tiles * a.nsplit, cus = cu_count_of_device();
   const bool deep = g.K >= (grid <= cus ? 1920 : 6144);
-  if (g.f32out || a.nsplit > 1) {
-    if (deep) gemm_block_kernel<FA, FB, OutF32, 6, 2, true, true><<<grid, 256, 0, s>>>(a);
-    else gemm_block_kernel<FA, FB, OutF32, 3, 2, true, true><<<grid, 256, 0, s>>>(a);
-  } else {
-    if (deep) gemm_block_kernel<FA, FB, OutBf16, 6, 2, true, true><<<grid, 256, 0, s>>>(a);
-    else gemm_block_kernel<FA, FB, OutBf16, 3, 2, true, true><<<grid, 256, 0, s>>>(a);
-  }
+  auto with = [&]<bool STREAM>() {
+    if (g.f32out || a.nsplit > 1) {
+      if (deep) gemm_block_kernel<FA, FB, OutF32, 6, 2, true, true, STREAM><<<grid, 256, 0, s>>>(a);
+      else gemm_block_kernel<FA, FB, OutF32, 3, 2, true, true, STREAM><<<grid, 256, 0, s>>>(a);
+    } else {
+      if (deep) gemm_block_kernel<FA, FB, OutBf16, 6, 2, true, true, STREAM><<<grid, 256, 0, s>>>(a);
+      else gemm_block_kernel<FA, FB, OutBf16, 3, 2, true, true, STREAM><<<grid, 256, 0, s>>>(a);
+    }
+  };
+  const bool stream = a.nsplit == 1 && g.M > 64 && (g.f32out ? streams_c<float>(g.C, g.M, g.N) : streams_c<uint16_t>(g.C, g.M, g.N, (size_t)36 << 20));
+  if (stream) with.template operator()<true>();
+  else with.template operator()<false>();
   return hipGetLastError();
 }
 // fp6 output, the fused epilogue applied or not inside
