@@ -522,11 +522,14 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
                                               (uint32_t)((rows_a - 1) * N + rows_b) * (uint32_t)sizeof(OutT));
   const int row_l = wm * 64 + line_row<1>(lane), col_l = wn * 64 + line_piece<1>(lane) * (16 / (int)sizeof(OutT)), voff = row_l * N2 + col_l * (int)sizeof(OutT);
   // RAGGED: `n` consecutive outputs of a row, 16 bytes of them at C's element alignment or, across N, one by one
+  // (the lane's address once, the stores' places from it: 512 x 296 x 16960 19.6 / 19.0, 49 x 20832 x 672 fp32 7.8 / 7.5)
+  [[maybe_unused]] OutT* const lane_c = (OutT*)args.C + ((size_t)share * args.M + (size_t)pm * kBM + row_l) * ldc + (size_t)pn * kBN + col_l;
   [[maybe_unused]] auto store_run = [&]<bool NT>(v4i v, int row, int col) __attribute__((always_inline)) {
     constexpr int kRun = 16 / (int)sizeof(OutT);
-    if (row >= rows_a || col >= rows_b) return;
-    OutT* const p = (OutT*)args.C + ((size_t)share * args.M + (size_t)pm * kBM + row) * ldc + (size_t)pn * kBN + col;
-    if (col + kRun <= rows_b) {
+    const int m = row_l + row, n = col_l + col;
+    if (m >= rows_a || n >= rows_b) return;
+    OutT* const p = lane_c + row * ldc + col;
+    if (n + kRun <= rows_b) {
       typedef int v4i_element __attribute__((ext_vector_type(4), aligned(2)));
       if constexpr (NT) __builtin_nontemporal_store((v4i_element)v, reinterpret_cast<v4i_element*>(p));
       else *reinterpret_cast<v4i_element*>(p) = (v4i_element)v;
@@ -535,15 +538,15 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
       __builtin_memcpy(o, &v, 16);
 #pragma unroll
       for (int e = 0; e + 1 < kRun; e++)
-        if (col + e < rows_b) p[e] = o[e];
+        if (n + e < rows_b) p[e] = o[e];
     }
   };
   // x, y: as pair_rows leaves them, rows `row` on; `col` columns on
   auto store_rows = [&]<bool NT>(v4i x, v4i y, int row, int col) __attribute__((always_inline)) {
     join_lines(x, y);
     if constexpr (RAGGED) {
-      store_run.template operator()<NT>(x, row_l + row, col_l + col);
-      store_run.template operator()<NT>(y, row_l + row + 8, col_l + col);
+      store_run.template operator()<NT>(x, row, col);
+      store_run.template operator()<NT>(y, row + 8, col);
     } else {
       if (!edge || (row_l + row < rows_a && col_l + col < rows_b)) store_c<NT>(x, rC, voff + col * (int)sizeof(OutT), row * N2);
       if (!edge || (row_l + row + 8 < rows_a && col_l + col < rows_b)) store_c<NT>(y, rC, voff + col * (int)sizeof(OutT), (row + 8) * N2);
@@ -673,7 +676,7 @@ hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, 
 // beyond (2000 x 8191 x 4128 107.5 / 105.0, 1000 x 4097 x 4128 47.3 / 48.6, 572 x 22563 x 13760 295 / 266).
 // STREAM: C goes out non-temporally.  As streams_c says, bf16 up to 36 MB (us as there: 2000 x 8191 x 1056, 33 MB, 39.7 / 42.3, 2000 x 8189 x 2080 50.2 /
 // 54.9), from 65 rows on (fp32, 49 x 20832 x 672 7.7 / 7.4, 128 rows 8.7 / 9.7; bf16, 100 x 28001 x 1568 17.7 / 18.3); not the sums of a K split's
-// shares, which are read again at once (512 x 296 x 16960 20.0 / 18.9, a layer of 191 x 664 x 18624 26.5 / 24.5).
+// shares, which are read again at once (512 x 296 x 16960 20.0 / 19.0, a layer of 191 x 664 x 18624 26.5 / 24.9).
 template <int FA, int FB>
 hipError_t launch_ragged(const GemmArgs& g, const BlockArgs& a, int tiles, hipStream_t s) {
   const int grid = tiles * a.nsplit, cus = cu_count_of_device();
