@@ -39,7 +39,7 @@ constexpr int g_slice = 0, g_padded = 0, g_block = 1;
 inline void note_route(int) {}
 #endif
 // What mxfp6_probe_route reports beside a kernel's code: the slice kernel's code, copies in front of the GEMM, quantised inside
-constexpr int kRouteSlice = 29, kRouteCopyA = 0x100, kRouteCopyB = 0x200, kRouteSplit = 0x400, kRouteX = 0x800;
+constexpr int kRouteSlice = 29, kRouteCopyA = 0x100, kRouteCopyB = 0x200, kRouteSplit = 0x400, kRouteX = 0x800, kRouteStreamB = 0x1000;
 
 // Workspaces kept per (device, stream, kind): launches on one stream are ordered, so they can share one; it grows on
 // demand (old one returned to the allocator in stream order) and lives until mxfp6_release_workspaces().
@@ -59,6 +59,19 @@ std::recursive_mutex g_sws_launch_mutex;
 std::map<std::tuple<int, hipStream_t, int>, StreamWs> g_sws;
 uint64_t g_sws_clock = 0;
 constexpr size_t kStreamWsMax = 128;
+
+hipError_t launch_tiled(const mxfp6::GemmArgs& g, hipStream_t s) {
+#ifdef MXFP6_PROBES
+  g_route |= mxfp6::tiled_streams_weights(g) ? kRouteStreamB : 0;
+#endif
+  return mxfp6::launch_gemm_tiled(g, s);
+}
+hipError_t launch_block(const mxfp6::GemmArgs& g, hipStream_t s) {
+#ifdef MXFP6_PROBES
+  g_route |= mxfp6::block_streams_weights(g) ? kRouteStreamB : 0;
+#endif
+  return mxfp6::launch_gemm_block(g, s);
+}
 
 bool stream_is_capturing(hipStream_t s) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -311,7 +324,7 @@ bool relayout_then_tiled(const mxfp6::GemmArgs& g, hipStream_t s, hipError_t& e)
   if (conv_a) { t.A = pa; t.As = sa; t.layout_a = 1; }
   if (conv_b) { t.B = pb; t.Bs = sb; t.layout_b = 1; }
   note_route(kChoiceTiled | (conv_a ? kRouteCopyA : 0) | (conv_b ? kRouteCopyB : 0));
-  if (e == hipSuccess) e = mxfp6::launch_gemm_tiled(t, s);
+  if (e == hipSuccess) e = launch_tiled(t, s);
   return true;
 }
 
@@ -341,7 +354,7 @@ bool padded_then_gemm(const mxfp6::GemmArgs& g, const mxfp6::KernelChoice& c, ui
   if (na && nb) e = mxfp6::launch_pad_both(g.A, pa, g.As, sa, g.M, g.B, pb, g.Bs, sb, g.N, g.K, s);
   else if (na) e = mxfp6::launch_pad_both(g.A, pa, g.As, sa, g.M, nullptr, nullptr, nullptr, nullptr, 0, g.K, s);
   else if (nb) e = mxfp6::launch_pad_both(g.B, pb, g.Bs, sb, g.N, nullptr, nullptr, nullptr, nullptr, 0, g.K, s);
-  if (e == hipSuccess) e = tc.cand >= mxfp6::kCandTiled256 && (kTiledFamily >> tc.cand & 1) ? mxfp6::launch_gemm_tiled(t, s) : mxfp6::launch_gemm_block(t, s);
+  if (e == hipSuccess) e = tc.cand >= mxfp6::kCandTiled256 && (kTiledFamily >> tc.cand & 1) ? launch_tiled(t, s) : launch_block(t, s);
   return true;
 }
 
@@ -408,7 +421,7 @@ int gemm_common(const void* A, const void* B, const void* As, const void* Bs, vo
     const unsigned shapes = force == 2 ? kTiledUnsplit : 1u << (force == 6 ? mxfp6::kCandTiled256 : force == 5 ? mxfp6::kCandTiled128x256 : mxfp6::kCandTiled128x128);
     mxfp6::KernelChoice c = family_choice(g, shapes, kTiledSplits);
     if (!apply_choice(g, c, s)) apply_choice(g, mxfp6::choose_kernel(g, 1, false, shapes), s);
-    if (g.ksplit > 1 || !relayout_then_tiled(g, s, e)) e = mxfp6::launch_gemm_tiled(g, s);
+    if (g.ksplit > 1 || !relayout_then_tiled(g, s, e)) e = launch_tiled(g, s);
   } else if (K != 0 && (force == 3 || (force >= 7 && force <= 16) || (force >= 19 && force <= 21))) {
     if (!mxfp6::gemm_skinny_supports(g)) return MXFP6_EINVAL_SHAPE;
     g.skinny_geometry = force == 3 ? 0 : force >= 19 ? force - 8 : force - 6;
@@ -427,7 +440,7 @@ int gemm_common(const void* A, const void* B, const void* As, const void* Bs, vo
     if (!mxfp6::gemm_block_supports(g)) return MXFP6_EINVAL_SHAPE;
     if (force != 26) (void)apply_choice(g, family_choice(g, 1u << mxfp6::kCandBlock, 1u << mxfp6::kCandBlockSplit), s);  // without a workspace: unsplit
     g.tile_rows = force == 23 ? 3 : force == 24 ? 6 : 0, g.tile_cols = force == 26 ? 256 : 0;
-    e = mxfp6::launch_gemm_block(g, s);
+    e = launch_block(g, s);
   } else {
     mxfp6::KernelChoice c = auto_choice(g, force_split, true);
     // (products that no candidate takes only: what the slice kernel takes it takes for MXFP6 output as well, whose bits are those of this call's)
@@ -440,17 +453,17 @@ int gemm_common(const void* A, const void* B, const void* As, const void* Bs, vo
     note_route(route_of(g, c, g.ksplit > 1 || (c.cand == mxfp6::kCandSlice && g.ks_part)));
     switch (c.cand) {
       case mxfp6::kCandTiled256: case mxfp6::kCandTiled128x256: case mxfp6::kCandTiled128x128:
-        if (!relayout_then_tiled(g, s, e)) e = mxfp6::launch_gemm_tiled(g, s);
+        if (!relayout_then_tiled(g, s, e)) e = launch_tiled(g, s);
         break;
-      case mxfp6::kCandTiledSplit256: case mxfp6::kCandTiledSplit128: e = mxfp6::launch_gemm_tiled(g, s); break;
-      case mxfp6::kCandBlock: case mxfp6::kCandBlockWide: case mxfp6::kCandBlockSplit: e = mxfp6::launch_gemm_block(g, s); break;
+      case mxfp6::kCandTiledSplit256: case mxfp6::kCandTiledSplit128: e = launch_tiled(g, s); break;
+      case mxfp6::kCandBlock: case mxfp6::kCandBlockWide: case mxfp6::kCandBlockSplit: e = launch_block(g, s); break;
       case mxfp6::kCandSkinny: e = mxfp6::launch_gemm_skinny(g, s); break;
       case mxfp6::kCandRing: e = mxfp6::launch_gemm_ring(g, s); break;
       case mxfp6::kCandSlice: e = mxfp6::launch_gemm_slice(g, c.slice, s); break;
       default:
         if (K != 0 && apply_ragged(g, s)) {
           note_route(route_of(g, c, g.ksplit > 1));
-          e = mxfp6::launch_gemm_block(g, s);
+          e = launch_block(g, s);
         } else {
           e = mxfp6::launch_gemm_generic(g, s);
         }
@@ -616,8 +629,8 @@ int mxfp6_gemm_fused_fp6(const void* A, const void* B, const void* As, const voi
     if (slice) e = mxfp6::launch_gemm_slice(t, ch.slice, s);
     else if (ring) e = mxfp6::launch_gemm_ring(t, s);
     else if (skinny) e = mxfp6::launch_gemm_skinny(t, s);
-    else if (block) e = mxfp6::launch_gemm_block(t, s);
-    else if (split || force != 0 || !relayout_then_tiled(t, s, e)) e = mxfp6::launch_gemm_tiled(t, s);
+    else if (block) e = launch_block(t, s);
+    else if (split || force != 0 || !relayout_then_tiled(t, s, e)) e = launch_tiled(t, s);
     return true;
   };
   hipError_t e = hipSuccess;

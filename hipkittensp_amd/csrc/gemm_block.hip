@@ -69,9 +69,12 @@ struct BlockArgs {
 //   * C's rows start at any element: 16-byte stores at element alignment, and single elements where a run of eight (bf16) or
 //     four (fp32) outputs crosses N.  Eight lanes' runs are 128 bytes of a row as in the aligned instantiations, if not one line, and leave
 //     non-temporal too (us, before / after: 4000 x 3001 x 1056 32.2 / 28.8, 7490 x 1056 x 672 17.1 / 15.3, 300 x 6001 x 1056 12.4 / 11.4)
-// STREAM: B is read with the non-temporal bit: weights larger than the last-level cache holds (kStreamBytes) against one tile row, which
-// nothing reads again.  us, plain / non-temporal, K split: 128 x 8192 x 28672 50.6 / 44.8, row-major 54.0 / 51.9, 96 rows 45.6 / 42.1; unsplit:
-// 128 x 28672 x 8192 41.0 / 38.1; not where row-major rows start inside a line, which is then read twice (128 x 17840 x 10880 67.7 / 70.9).  (An instantiation of its own: picked as the kernel runs, 1024 x 4096 x 14336 paid 58.6 / 59.5 for it.)
+// STREAM: B is read with the non-temporal bit: tile-major weights of kStreamBytes and more against one tile row, which nothing reads again.  us,
+// plain / non-temporal, layers' weights in turn, one set of activations (and one for each layer): K split, 128 x 8192 x 28672 44.8 / 44.3 (50.3 / 44.2),
+// 96 rows (45.2 / 41.2); unsplit, 128 x 28672 x 8192 (48.8 / 40.2); 24 linear layers of these two shapes one after the other, a layer, 128 rows 47.6 / 44.4, 80
+// rows 44.1 / 40.8.  What it costs stands at kStreamBytes.  Not row-major weights: 50.6 / 51.8, 96 rows 47.7 / 49.4, 128 x 8192 x 24576 45.0 / 47.5, unsplit 49.7 / 50.5 (with
+// activations for each layer 53.8 / 51.6, but 54.0 / 55.0 over 24 layers).  (An instantiation of its own: picked as the kernel runs, 1024 x 4096 x 14336
+// paid 58.6 / 59.5 for it.)
 // RAGGED and STREAM: C leaves non-temporally (launch_ragged).
 // 500 x 5003 x 2880: 17.0 us against 148.5 on the one-wave-per-tile kernel, which fetches every operand row again for each of
 // its 32 x 32 tiles, 4 bytes per lane.
@@ -648,6 +651,7 @@ int block_stages(const GemmArgs& g, int grid, int cus) {
   const int min_k = grid <= cus ? (row_major ? 1025 : 2049) : row_major == 2 ? 4096 : row_major == 1 ? 8192 : 0x7fffffff;
   return g.K >= min_k ? 6 : 3;
 }
+int forced_stages(const GemmArgs& g) { return g.tile_rows == 3 || g.tile_rows == 6 ? g.tile_rows : 0; }
 template <int FA, int FB, bool FUSED>
 hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, hipStream_t s) {
   const int cus = cu_count_of_device();
@@ -659,7 +663,7 @@ hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, 
     return hipGetLastError();
   }
   if (stages == 0) stages = block_stages(g, grid, cus);
-  if (stages == 6 && a.tiles_m == 1 && (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes && (g.layout_b || g.K % 512 == 0) && (!f32 || !FUSED)) {
+  if (block_streams_weights(g) && (!f32 || !FUSED)) {
     if (!f32) gemm_block_kernel<FA, FB, OutBf16, 6, 2, FUSED, false, true><<<grid, 256, 0, s>>>(a);
     else if constexpr (!FUSED) gemm_block_kernel<FA, FB, OutF32, 6, 2, false, false, true><<<grid, 256, 0, s>>>(a);
   } else if (stages == 6) {
@@ -729,6 +733,13 @@ bool gemm_block_ragged_supports(const GemmArgs& g) {
          (long)((g.N + 127) / 128) <= 32767 && (long)((g.M + 127) / 128) * ((g.N + 127) / 128) < (1L << 31) && !g.fmt_c;
 }
 
+bool block_streams_weights(const GemmArgs& g) {
+  const int split = g.ksplit > 1 ? g.ksplit : 1;
+  if (g.ragged || g.tile_cols == 256 || !g.layout_b || g.M > kBM || (size_t)g.N * (g.K / 4 * 3) < kStreamBytes) return false;
+  if (split == 1 && (g.fmt_c || (g.f32out && epilogue_any(g.ep)))) return false;  // not built
+  return (forced_stages(g) ? forced_stages(g) : block_stages(g, (g.N + 127) / 128 * split, cu_count_of_device())) == 6;
+}
+
 // g.ksplit > 1 (with g.ks_part): the K range of every output tile split between that many workgroups, then
 // ksplit_reduce_kernel (gemm_tiled.hip), which also applies a fused epilogue.  The caller has checked that the last share
 // is not empty (block_split_shares, dispatch.hip).
@@ -736,7 +747,7 @@ hipError_t launch_gemm_block(const GemmArgs& g, hipStream_t s) {
   const int bn = g.tile_cols == 256 ? 256 : 128, nsplit = g.ksplit > 1 ? g.ksplit : 1;
   BlockArgs a{g.A, g.B, g.As, g.Bs, nsplit > 1 ? (void*)g.ks_part : g.C, g.M, g.N, g.K, (g.M + kBM - 1) / kBM, (g.N + bn - 1) / bn, g.layout_a, g.layout_b,
               g.raster_group_m > 0 ? g.raster_group_m : kGroupM, g.raster_no_xcd_remap == 1 ? 0 : g.raster_no_xcd_remap == 2 ? 2 : 1, nsplit, g.ep, g.C_scale, g.fmt_c};
-  const int tiles = a.tiles_m * a.tiles_n, stages = g.tile_rows == 3 || g.tile_rows == 6 ? g.tile_rows : 0;
+  const int tiles = a.tiles_m * a.tiles_n, stages = forced_stages(g);
   hipError_t e;
   if (g.ragged) {
     if (nsplit > 1) a.ep = Epilogue{};  // the reduction applies it

@@ -912,6 +912,10 @@ hipError_t launch_ksplit_reduce(const GemmArgs& g, hipStream_t s) {
   return hipGetLastError();
 }
 
+bool tiled_streams_weights(const GemmArgs& g) {
+  return g.ksplit > 1 && g.ks_part && g.M <= (g.tile_rows == 128 ? 128 : 256) && g.layout_b && (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes;
+}
+
 hipError_t launch_gemm_tiled(const GemmArgs& g, hipStream_t s) {
   if (g.fmt_a == 2 && g.fmt_b == 2) return launch_gemm_tiled_fmt22(g, s);
   if (g.fmt_a == 2 && g.fmt_b == 3) return launch_gemm_tiled_fmt23(g, s);
@@ -940,7 +944,7 @@ static hipError_t launch(const GemmArgs& g, hipStream_t s) {
       TiledArgs tp = ta;  // the shares write fp32 partial matrices into the workspace, without the epilogue
       tp.C = g.ks_part, tp.ep = Epilogue{};
       const int grid = tiled_grid_size(g, tm * tn * g.ksplit, 1);
-      if (tm == 1 && g.layout_b && (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes) {
+      if (tiled_streams_weights(g)) {
         if (bm == 128) gemm_tiled_kernel<FA, FB, OutF32, 2, 2, false, 0, 2><<<grid, NW * 64, 0, s>>>(tp);
         else gemm_tiled_kernel<FA, FB, OutF32, 4, 2, false, 0, 2><<<grid, NW * 64, 0, s>>>(tp);
       } else if (bm == 128) gemm_tiled_kernel<FA, FB, OutF32, 2, 2, false, 0, 1><<<grid, NW * 64, 0, s>>>(tp);

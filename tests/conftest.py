@@ -22,7 +22,7 @@ class Route:
     settings of the measurement build count; kernel and k_split are set for the call."""
 
     TILED, SKINNY, BLOCK, RING, SLICE = 2, 3, 22, 28, 29
-    COPY_A, COPY_B, SPLIT, X = 0x100, 0x200, 0x400, 0x800
+    COPY_A, COPY_B, SPLIT, X, STREAM_B = 0x100, 0x200, 0x400, 0x800, 0x1000
 
     def _run(self, kernel, k_split, call):
         import torch

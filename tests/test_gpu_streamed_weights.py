@@ -1,5 +1,5 @@
-"""Weights past the last-level cache, which the tiled kernel's K split and the block kernel read with the non-temporal bit where one tile
-row meets them: the same rows with a second tile row behind them, which are read without it, give the same bits."""
+"""Weights of 128 MB and more, which the tiled kernel's K split and the block kernel read with the non-temporal bit where they are tile-major and
+one tile row meets them: the same rows with a second tile row behind them, which are read without it, give the same bits."""
 import pytest
 import torch
 
@@ -30,7 +30,7 @@ def operands():
 @pytest.mark.parametrize("kernel,rows,shares,N,K", [(6, 256, 4, 8192, 22528), (5, 128, 2, 8192, 22528), (24, 128, 2, 8192, 22528), (24, 128, 3, 5120, 35200), (24, 128, 1, 24576, 7680)])
 @pytest.mark.parametrize("tile_b", [0, 1])
 @pytest.mark.parametrize("out,act", [(torch.bfloat16, None), (torch.bfloat16, "silu"), (torch.float32, None)])
-def test_one_tile_row_matches_two(operands, kernel, rows, shares, N, K, tile_b, out, act):
+def test_one_tile_row_matches_two(operands, route, kernel, rows, shares, N, K, tile_b, out, act):
     hk, (A, As), row, tile = operands(N, K)
     B, Bs = tile if tile_b else row
     tk, res = hk.tk_kernel, []
@@ -43,4 +43,7 @@ def test_one_tile_row_matches_two(operands, kernel, rows, shares, N, K, tile_b, 
             tk.set_kernel(prev)
             tk.set_k_split(prev_split)
         res.append(C)
+        if act is None:
+            taken = route.gemm(A[:M], B, As[:M], Bs, torch.empty_like(C), M, N, K, lb=tile_b, kernel=kernel, k_split=shares)
+            assert bool(taken & route.STREAM_B) == (tile_b == 1 and M <= rows), hex(taken)
     assert torch.isfinite(res[2]).all() and torch.equal(res[0], res[2][:rows]) and torch.equal(res[1], res[2][: rows - 3])
