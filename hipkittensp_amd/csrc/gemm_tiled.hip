@@ -137,10 +137,10 @@ struct TiledArgs {
 // then a workspace (partial_offset); ksplit_reduce_kernel adds them in share order and applies
 // the epilogue.  (Summed inside this kernel instead -- partial tiles and arrival counters at device scope, the last
 // wave to arrive adds -- the few waves that end up adding read nsplit tiles each past the L2s: 30 us for 32 MB.)
-// KSPLIT 2: B is read with the non-temporal bit: tile-major weights larger than the last-level cache holds (kStreamBytes) that no second
-// tile row reads again.  us, plain / non-temporal, N = 8192, K = 28672: 256 rows on tiles of 256 70.3 / 66.6, 128 rows on tiles of 128 52.4 / 47.1; not with
-// two tile rows (192 rows on tiles of 128 61.4 / 70.2), nor below that size (256 x 4096 x 14336 36.5 / 37.5), nor row-major, where a line is read
-// twice (128 rows 60.4 / 67.8).  (A kernel that picks the bit as it runs: 256 x 4096 x 14336 39.4 / 41.2 in the same call.)
+// KSPLIT 2: B is read with the non-temporal bit: tile-major weights of kStreamBytes and more (where its figures stand, gains and losses) that no
+// second tile row reads again.  Not with two tile rows (us, plain / non-temporal, N = 8192, K = 28672: 192 rows on tiles of 128 61.4 / 70.2), nor below that size
+// (256 x 4096 x 14336 36.5 / 37.5), nor row-major, where a line is read twice (128 rows 60.4 / 67.8).  (A kernel that picks the bit as it runs: 256 x 4096 x 14336
+// 39.4 / 41.2 in the same call.)
 template <int FA, int FB, typename Out, int TM, int TN, bool FUSED, int ABL = 0, int KSPLIT = 0>
 __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs args) {
   typedef Shape<TM, TN> S;

@@ -43,8 +43,18 @@ inline bool operands_aligned16(const GemmArgs& g) {
 // non-temporal, N = 8192, tile-major weights, in turn from 640 MB of them (a program's layers): skinny kernel, 16 rows, 60 MB
 // 15.3 / 14.3, 120 MB 25.7 / 23.8, 144 MB 30.2 / 27.5, 168 MB 33.8 / 31.0; ring kernel, 64 rows, 20.9 / 21.2, 33.1 / 30.5, 37.9 / 34.2, 42.3 /
 // 38.2.  The same weights again in every call, which stay in that cache in part or, below the line, as a whole: skinny 13.2 / 12.0, 21.8 /
-// 22.4, 25.2 / 26.2, 28.7 / 30.0; ring 19.0 / 19.6, 28.0 / 30.0, 31.8 / 33.6, 34.9 / 37.6.  (A first pass over weights not read before, 64 rows, is the same
-// either way.)
+// 22.4, 25.2 / 26.2, 28.7 / 30.0; ring 19.0 / 19.6, 28.0 / 30.0, 31.8 / 33.6, 34.9 / 37.6.
+// The tiled kernel's K split and the block kernel, tile-major weights of 176 MB that one tile row meets, N = 8192 (up: N = 28672, K = 8192):
+//   * layers' weights in turn, one set of activations: tiled, 256 rows 67.9 / 66.0, 224 63.3 / 62.5; block, 128 rows 44.8 / 44.3; with activations for each of 2
+//     to 8 layers 69.6 / 64.9, 50.2 / 44.1, up 48.7 / 40.0, for each of 24 69.9 / 69.8, 50.4 / 48.4, up 49.1 / 40.5.  (What B does not displace stays: activations,
+//     partial sums, C.)
+//   * 24 linear layers, up and down in turn, a layer: 128 rows 47.6 / 44.4, 80 rows 44.1 / 40.8, 160 60.7 / 60.2, 256 68.2 / 67.9; their first forward pass
+//     49.2 / 48.9, 68.7 / 68.3
+//   * the same weights in every call: 60.0 / 67.5, 39.9 / 46.2, up 36.2 / 40.2
+//   * a first pass right behind the quantiser that made the weights, from a source that is 940 MB of new fp32: 85.4 / 88.6 (host clock), 58.5 / 62.5, up 59.2 /
+//     63.1; from one that was there before: 94.2 / 88.2, 67.6 / 64.4, up 65.1 / 63.9; behind a copy of the weights 88.4 / 89.9, 59.2 / 58.8; behind 1 GB of other
+//     stores 113 / 86, 92 / 64, up 93 / 59
+// So it costs a program that runs one layer over and over, or quantises and multiplies once, up to a sixth, and gives one with layers up to a sixth.
 constexpr size_t kStreamBytes = (size_t)128 << 20;
 
 // ---- kernel choice (dispatch.hip): candidates of the automatic path, a time model per candidate, a calibration table
