@@ -39,7 +39,7 @@ constexpr int g_slice = 0, g_padded = 0, g_block = 1;
 inline void note_route(int) {}
 #endif
 // What mxfp6_probe_route reports beside a kernel's code: the slice kernel's code, copies in front of the GEMM, quantised inside
-constexpr int kRouteSlice = 29, kRouteCopyA = 0x100, kRouteCopyB = 0x200, kRouteSplit = 0x400, kRouteX = 0x800, kRouteStreamB = 0x1000;
+constexpr int kRouteSlice = 29, kRouteCopyA = 0x100, kRouteCopyB = 0x200, kRouteSplit = 0x400, kRouteX = 0x800, kRouteStreamB = 0x1000, kRouteForm = 0x2000;
 
 // Workspaces kept per (device, stream, kind): launches on one stream are ordered, so they can share one; it grows on
 // demand (old one returned to the allocator in stream order) and lives until mxfp6_release_workspaces().
@@ -68,7 +68,7 @@ hipError_t launch_tiled(const mxfp6::GemmArgs& g, hipStream_t s) {
 }
 hipError_t launch_block(const mxfp6::GemmArgs& g, hipStream_t s) {
 #ifdef MXFP6_PROBES
-  g_route |= mxfp6::block_streams_weights(g) ? kRouteStreamB : 0;
+  g_route |= (mxfp6::block_streams_weights(g) ? kRouteStreamB : 0) | mxfp6::block_c_form(g) * kRouteForm;
 #endif
   return mxfp6::launch_gemm_block(g, s);
 }

@@ -161,6 +161,8 @@ __device__ __forceinline__ void store1(float* p, float a) { *p = a; }
 // 34.7, 56.6; 27.2, 35.7; 91, 95; 307; in parts of 64: 16.0, 16.1; 25.8, 26.2; 21.4, 25.1; 70, 78; 297.  Whole lines without it: 16.6, 19.0; 25.8, 27.2; 24.3,
 // 27.1; 71.1, 76.3; 284.)  A program that reads C in its next kernel keeps the gain or is level (2048 x 14336 x 1024 on the block kernel and the
 // quantiser 57.7 / 51.6, 512 x 2048 x 2048 12.4 / 12.6).
+// How a tile kernel stores C: 16 bytes of 32 rows at a time, as the accumulators hold them; whole lines, through the L2s; whole lines, non-temporally
+enum CStore : int { kCPieces, kCKept, kCOut };
 // pair_rows: y holds what lies 32 bytes behind x's.  Afterwards x holds 64 contiguous bytes of rows 0 - 15 and y those of rows 16 - 31:
 // row l % 16, 16-byte piece 2 (l / 16 % 2) + l / 32 of the four.
 __device__ __forceinline__ void pair_rows(v4i& x, v4i& y) {

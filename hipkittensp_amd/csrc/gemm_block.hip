@@ -67,25 +67,24 @@ struct BlockArgs {
 //     one of 4) and the reader shifts them into place (v_alignbyte_b32, once per four K-tiles).  With three slots one scale
 //     buffer serves (a group's scales are in registers, and a barrier passed, before the next group's are fetched): 77 KB
 //   * C's rows start at any element: 16-byte stores at element alignment, and single elements where a run of eight (bf16) or
-//     four (fp32) outputs crosses N.  Eight lanes' runs are 128 bytes of a row as in the aligned instantiations, if not one line, and leave
-//     non-temporal too (us, before / after: 4000 x 3001 x 1056 32.2 / 28.8, 7490 x 1056 x 672 17.1 / 15.3, 300 x 6001 x 1056 12.4 / 11.4)
+//     four (fp32) outputs crosses N.  Eight lanes' runs can be 128 bytes of a row as in the aligned instantiations, if not one line
 // STREAM: B is read with the non-temporal bit: tile-major weights of kStreamBytes and more against one tile row, which nothing reads again.  us,
 // plain / non-temporal, layers' weights in turn, one set of activations (and one for each layer): K split, 128 x 8192 x 28672 44.8 / 44.3 (50.3 / 44.2),
 // 96 rows (45.2 / 41.2); unsplit, 128 x 28672 x 8192 (48.8 / 40.2); 24 linear layers of these two shapes one after the other, a layer, 128 rows 47.6 / 44.4, 80
 // rows 44.1 / 40.8.  What it costs stands at kStreamBytes.  Not row-major weights: 50.6 / 51.8, 96 rows 47.7 / 49.4, 128 x 8192 x 24576 45.0 / 47.5, unsplit 49.7 / 50.5 (with
 // activations for each layer 53.8 / 51.6, but 54.0 / 55.0 over 24 layers).  (An instantiation of its own: picked as the kernel runs, 1024 x 4096 x 14336
 // paid 58.6 / 59.5 for it.)
-// RAGGED and STREAM: C leaves non-temporally (launch_ragged).
+// CFORM: how RAGGED stores C (CStore, ragged_c_form).
 // 500 x 5003 x 2880: 17.0 us against 148.5 on the one-wave-per-tile kernel, which fetches every operand row again for each of
 // its 32 x 32 tiles, 4 bytes per lane.
-template <int FA, int FB, typename Out, int STAGES, int WN, bool FUSED, bool RAGGED = false, bool STREAM = false>
+template <int FA, int FB, typename Out, int STAGES, int WN, bool FUSED, bool RAGGED = false, bool STREAM = false, int CFORM = kCOut>
 __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_block_kernel(const BlockArgs args) {
   typedef typename Out::type OutT;
   static_assert((STAGES == 3 || STAGES == 4 || STAGES == 6) && (WN == 2 || WN == 4), "ring depth, tile width");
   constexpr bool PAIR = STAGES == 6;
   static_assert(!RAGGED || (WN == 2 && FUSED), "one tile width, one epilogue");
   static_assert(!PAIR || WN == 2, "three slots of two K-tiles");
-  static_assert(!STREAM || PAIR || RAGGED, "three slots of two K-tiles");
+  static_assert(!STREAM || (PAIR && !RAGGED), "three slots of two K-tiles");
   static_assert(sizeof(OutT) != 1 || (FUSED && !RAGGED), "fp6 output: one epilogue, whole 32-blocks");
   constexpr int NW = 2 * WN, kBN = WN * 64, kSlot = kATile + kBN * 96, kScRows = kScA + kBN * 16;
   constexpr int kScBuf = kScRows + (RAGGED ? (kBM + kBN) * 4 : 0);  // RAGGED: 4 more bytes per row behind the rows' 16
@@ -229,7 +228,7 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   auto load_pair = [&]<bool OF_A>(int c, int slot, int n) __attribute__((always_inline)) {
     const uint32_t dst = lds0 + slot * (2 * kSlot) + (OF_A ? 0 : 2 * kATile) + (wave * 6 + n) * 1024;
     if constexpr (OF_A) dma16(c < nchunks ? rA : rZ, dst, voff_a[PAIR ? n : 0] + c * (2 * kstep_a), 0);
-    else if constexpr (STREAM && !RAGGED) dma16_nt(c < nchunks ? rB : rZ, dst, voff_b[PAIR ? n : 0] + c * (2 * kstep_b), 0);
+    else if constexpr (STREAM) dma16_nt(c < nchunks ? rB : rZ, dst, voff_b[PAIR ? n : 0] + c * (2 * kstep_b), 0);
     else dma16(c < nchunks ? rB : rZ, dst, voff_b[PAIR ? n : 0] + c * (2 * kstep_b), 0);
   };
   auto load_tile = [&]<bool LA>(int t, int slot) __attribute__((always_inline)) {
@@ -523,38 +522,6 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
   [[maybe_unused]] const size_t ldc = RAGGED && args.nsplit > 1 ? ragged_pitch(N) : N;
   const __amdgpu_buffer_rsrc_t rC = make_rsrc((OutT*)args.C + (size_t)share * args.M * N + (size_t)pm * kBM * N + (size_t)pn * kBN,
                                               (uint32_t)((rows_a - 1) * N + rows_b) * (uint32_t)sizeof(OutT));
-  const int row_l = wm * 64 + line_row<1>(lane), col_l = wn * 64 + line_piece<1>(lane) * (16 / (int)sizeof(OutT)), voff = row_l * N2 + col_l * (int)sizeof(OutT);
-  // RAGGED: `n` consecutive outputs of a row, 16 bytes of them at C's element alignment or, across N, one by one
-  // (the lane's address once, the stores' places from it: 512 x 296 x 16960 19.6 / 19.0, 49 x 20832 x 672 fp32 7.8 / 7.5)
-  [[maybe_unused]] OutT* const lane_c = (OutT*)args.C + ((size_t)share * args.M + (size_t)pm * kBM + row_l) * ldc + (size_t)pn * kBN + col_l;
-  [[maybe_unused]] auto store_run = [&]<bool NT>(v4i v, int row, int col) __attribute__((always_inline)) {
-    constexpr int kRun = 16 / (int)sizeof(OutT);
-    const int m = row_l + row, n = col_l + col;
-    if (m >= rows_a || n >= rows_b) return;
-    OutT* const p = lane_c + row * ldc + col;
-    if (n + kRun <= rows_b) {
-      typedef int v4i_element __attribute__((ext_vector_type(4), aligned(2)));
-      if constexpr (NT) __builtin_nontemporal_store((v4i_element)v, reinterpret_cast<v4i_element*>(p));
-      else *reinterpret_cast<v4i_element*>(p) = (v4i_element)v;
-    } else {
-      OutT o[kRun];
-      __builtin_memcpy(o, &v, 16);
-#pragma unroll
-      for (int e = 0; e + 1 < kRun; e++)
-        if (n + e < rows_b) p[e] = o[e];
-    }
-  };
-  // x, y: as pair_rows leaves them, rows `row` on; `col` columns on
-  auto store_rows = [&]<bool NT>(v4i x, v4i y, int row, int col) __attribute__((always_inline)) {
-    join_lines(x, y);
-    if constexpr (RAGGED) {
-      store_run.template operator()<NT>(x, row, col);
-      store_run.template operator()<NT>(y, row + 8, col);
-    } else {
-      if (!edge || (row_l + row < rows_a && col_l + col < rows_b)) store_c<NT>(x, rC, voff + col * (int)sizeof(OutT), row * N2);
-      if (!edge || (row_l + row + 8 < rows_a && col_l + col < rows_b)) store_c<NT>(y, rC, voff + col * (int)sizeof(OutT), (row + 8) * N2);
-    }
-  };
   if constexpr (!RAGGED && sizeof(OutT) == 4) {
     if (args.nsplit > 1) {
       // this share's partial sums, in the accumulators' order (partial_offset)
@@ -573,7 +540,53 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
       return;
     }
   }
-  auto store_tile = [&]<bool NT>() __attribute__((always_inline)) {
+  // C as `FORM` says (CStore)
+  auto store_tile = [&]<int FORM>() __attribute__((always_inline)) {
+    constexpr bool LINES = FORM != kCPieces, OUT = FORM == kCOut;
+    constexpr int kRun = 16 / (int)sizeof(OutT);
+    const int row_l = wm * 64 + (LINES ? line_row<1>(lane) : r32), col_l = wn * 64 + (LINES ? line_piece<1>(lane) : h) * kRun;
+    const int voff = row_l * N2 + col_l * (int)sizeof(OutT);
+    // RAGGED: `n` consecutive outputs of a row, 16 bytes of them at C's element alignment or, across N, one by one
+    // (the lane's address once, the stores' places from it: 512 x 296 x 16960 19.6 / 19.0, 49 x 20832 x 672 fp32 7.8 / 7.5)
+    [[maybe_unused]] OutT* const lane_c = (OutT*)args.C + ((size_t)share * args.M + (size_t)pm * kBM + row_l) * ldc + (size_t)pn * kBN + col_l;
+    // 16 bytes of the lane, `row` rows and `col` columns on
+    auto put = [&](v4i v, int row, int col) __attribute__((always_inline)) {
+      const int m = row_l + row, n = col_l + col;
+      if constexpr (!RAGGED) {
+        if (!edge || (m < rows_a && n < rows_b)) store_c<OUT>(v, rC, voff + col * (int)sizeof(OutT), row * N2);
+      } else {
+        if (m >= rows_a || n >= rows_b) return;
+        OutT* const p = lane_c + row * ldc + col;
+        if (n + kRun <= rows_b) {
+          typedef int v4i_element __attribute__((ext_vector_type(4), aligned(2)));
+          if constexpr (OUT) __builtin_nontemporal_store((v4i_element)v, reinterpret_cast<v4i_element*>(p));
+          else *reinterpret_cast<v4i_element*>(p) = (v4i_element)v;
+        } else {
+          OutT o[kRun];
+          __builtin_memcpy(o, &v, 16);
+#pragma unroll
+          for (int e = 0; e + 1 < kRun; e++)
+            if (n + e < rows_b) p[e] = o[e];
+        }
+      }
+    };
+    // four registers, 16 outputs (bf16) or 8 (fp32) of a row apart, of rows `row` on; `col` columns on
+    auto put4 = [&](v4i (&v)[2][2], int row, int col) __attribute__((always_inline)) {
+      constexpr int kApart = 2 * kRun;
+      if constexpr (LINES) {
+#pragma unroll
+        for (int p = 0; p < 2; p++) pair_rows(v[p][0], v[p][1]);
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+          join_lines(v[0][t], v[1][t]);
+          put(v[0][t], row + t * 16, col);
+          put(v[1][t], row + t * 16 + 8, col);
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; q++) put(v[q >> 1][q & 1], row, col + q * kApart);
+      }
+    };
     if constexpr (sizeof(OutT) == 2) {
 #pragma unroll
       for (int i = 0; i < 2; i++) {
@@ -594,13 +607,10 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
             }
         v4i v[2][2];
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
+        for (int j = 0; j < 2; j++)
 #pragma unroll
           for (int t = 0; t < 2; t++) v[j][t] = v4i{(int)pk[j][4 * t], (int)pk[j][4 * t + 1], (int)pk[j][4 * t + 2], (int)pk[j][4 * t + 3]};
-          pair_rows(v[j][0], v[j][1]);
-        }
-#pragma unroll
-        for (int t = 0; t < 2; t++) store_rows.template operator()<NT>(v[0][t], v[1][t], i * 32 + t * 16, 0);
+        put4(v, i * 32, 0);
       }
     } else {
 #pragma unroll
@@ -612,17 +622,14 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
           for (int q = 0; q < 4; q++)
 #pragma unroll
             for (int e = 0; e < 4; e++) v[q >> 1][q & 1][e] = __float_as_int(acc[i][j][4 * q + e]);
-#pragma unroll
-          for (int p = 0; p < 2; p++) pair_rows(v[p][0], v[p][1]);
-#pragma unroll
-          for (int t = 0; t < 2; t++) store_rows.template operator()<NT>(v[0][t], v[1][t], i * 32 + t * 16, j * 32);
+          put4(v, i * 32, j * 32);
         }
     }
   };
-  // Two copies, rather than a choice at each store, which costs a short fp32 product 3 %; of RAGGED's longer code one (STREAM, launch_ragged)
-  if constexpr (RAGGED) store_tile.template operator()<STREAM>();
-  else if (streams_c<OutT>(args.C, args.M, N)) store_tile.template operator()<true>();
-  else store_tile.template operator()<false>();
+  // Two copies, rather than a choice at each store, which costs a short fp32 product 3 %; of RAGGED's longer code one (FORM, launch_ragged)
+  if constexpr (RAGGED) store_tile.template operator()<CFORM>();
+  else if (streams_c<OutT>(args.C, args.M, N)) store_tile.template operator()<kCOut>();
+  else store_tile.template operator()<kCKept>();
 }
 
 int cu_count_of_device() {
@@ -675,28 +682,39 @@ hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, 
   }
   return hipGetLastError();
 }
+// How a RAGGED instantiation stores C.  As it comes where that is little: below 4 MB, up to 64 rows, and the sums of a K split's shares, which are
+// read again at once (us, as it comes / whole lines through the L2s / whole lines non-temporal, fp32: 49 x 20832 x 672 7.45 / 7.75 / 7.5, 20 x 30001 x 672 7.35 /
+// 7.65 / 7.8, 64 x 20001 x 2080 13.1 / 13.35 / 13.4; 191 x 664 x 18624 18.6 / 18.85 / 18.85, 512 x 296 x 16960 19.05 / 19.2 / 19.2).  Else non-temporally where
+// its rows start on lines.  Where they do not, a line is two stores: bf16 up to 32 MB (1000 x 5003 x 1056, 9.5 MB, 17.1 / 17.1 / 16.6; 256 x 16001 x 1056 13.2 / 13.2 /
+// 12.8; 2000 x 8191 x 1056, 31 MB, 38.5 / 38.4 / 37.2; 6000 x 3001 x 672, 34 MB, 33.6 / 33.2 / 36.2); fp32 never (256 x 16001 x 1056, 16 MB, 13.4 / 12.2 /
+// 16.3; 1000 x 5003 x 1056, 19 MB, 16.5 / 15.5 / 18.6; 2000 x 8191 x 1056 36.3 / 34.2 / 49.3).  Over 70 drawn shapes of each type, of the time as it comes: bf16
+// 4 to 32 MB 1.00 / 0.97, above 1.00 / 1.04; fp32 8 to 12 MB 0.96 / 1.00, 12 to 20 MB 0.93 / 1.09, above 0.94 / 1.28.
+int ragged_c_form(const GemmArgs& g) {
+  const size_t row = (size_t)g.N * (g.f32out ? 4 : 2), bytes = g.M * row;
+  if (g.ksplit > 1 || g.M <= 64 || bytes < (size_t)4 << 20) return kCPieces;
+  if ((((uintptr_t)g.C | row) & 127) == 0) return kCOut;
+  return g.f32out ? kCKept : bytes <= (size_t)32 << 20 ? kCOut : kCPieces;
+}
 // RAGGED instantiations, the fused epilogue applied or not inside.  PAIR from K = 1920 on while no CU gets a second workgroup (us,
 // three slots / PAIR: 64 x 3001 x 1888 11.1 / 11.1, 500 x 5003 x 1056 13.2 / 13.6, 100 x 5003 x 2016 17.8 / 16.1), from 6144 on
 // beyond (2000 x 8191 x 4128 107.5 / 105.0, 1000 x 4097 x 4128 47.3 / 48.6, 572 x 22563 x 13760 295 / 266).
-// STREAM: C goes out non-temporally.  As streams_c says, bf16 up to 36 MB (us as there: 2000 x 8191 x 1056, 33 MB, 39.7 / 42.3, 2000 x 8189 x 2080 50.2 /
-// 54.9), from 65 rows on (fp32, 49 x 20832 x 672 7.7 / 7.4, 128 rows 8.7 / 9.7; bf16, 100 x 28001 x 1568 17.7 / 18.3); not the sums of a K split's
-// shares, which are read again at once (512 x 296 x 16960 20.0 / 19.0, a layer of 191 x 664 x 18624 26.5 / 24.9).
 template <int FA, int FB>
 hipError_t launch_ragged(const GemmArgs& g, const BlockArgs& a, int tiles, hipStream_t s) {
   const int grid = tiles * a.nsplit, cus = cu_count_of_device();
   const bool deep = g.K >= (grid <= cus ? 1920 : 6144);
-  auto with = [&]<bool STREAM>() {
-    if (g.f32out || a.nsplit > 1) {
-      if (deep) gemm_block_kernel<FA, FB, OutF32, 6, 2, true, true, STREAM><<<grid, 256, 0, s>>>(a);
-      else gemm_block_kernel<FA, FB, OutF32, 3, 2, true, true, STREAM><<<grid, 256, 0, s>>>(a);
-    } else {
-      if (deep) gemm_block_kernel<FA, FB, OutBf16, 6, 2, true, true, STREAM><<<grid, 256, 0, s>>>(a);
-      else gemm_block_kernel<FA, FB, OutBf16, 3, 2, true, true, STREAM><<<grid, 256, 0, s>>>(a);
-    }
+  auto with = [&]<typename Out, int CFORM>() {
+    if (deep) gemm_block_kernel<FA, FB, Out, 6, 2, true, true, false, CFORM><<<grid, 256, 0, s>>>(a);
+    else gemm_block_kernel<FA, FB, Out, 3, 2, true, true, false, CFORM><<<grid, 256, 0, s>>>(a);
   };
-  const bool stream = a.nsplit == 1 && g.M > 64 && (g.f32out ? streams_c<float>(g.C, g.M, g.N) : streams_c<uint16_t>(g.C, g.M, g.N, (size_t)36 << 20));
-  if (stream) with.template operator()<true>();
-  else with.template operator()<false>();
+  const int form = ragged_c_form(g);
+  if (g.f32out || a.nsplit > 1) {
+    if (form == kCOut) with.template operator()<OutF32, kCOut>();
+    else if (form == kCKept) with.template operator()<OutF32, kCKept>();
+    else with.template operator()<OutF32, kCPieces>();
+  } else {
+    if (form == kCOut) with.template operator()<OutBf16, kCOut>();
+    else with.template operator()<OutBf16, kCPieces>();
+  }
   return hipGetLastError();
 }
 // fp6 output, the fused epilogue applied or not inside
@@ -738,6 +756,12 @@ bool block_streams_weights(const GemmArgs& g) {
   if (g.ragged || g.tile_cols == 256 || !g.layout_b || g.M > kBM || (size_t)g.N * (g.K / 4 * 3) < kStreamBytes) return false;
   if (split == 1 && (g.fmt_c || (g.f32out && epilogue_any(g.ep)))) return false;  // not built
   return (forced_stages(g) ? forced_stages(g) : block_stages(g, (g.N + 127) / 128 * split, cu_count_of_device())) == 6;
+}
+
+int block_c_form(const GemmArgs& g) {
+  if (g.ragged) return ragged_c_form(g);
+  if (g.ksplit > 1 || g.fmt_c) return kCPieces;
+  return (g.f32out ? streams_c<float>(g.C, g.M, g.N) : streams_c<uint16_t>(g.C, g.M, g.N)) ? kCOut : kCKept;
 }
 
 // g.ksplit > 1 (with g.ks_part): the K range of every output tile split between that many workgroups, then

@@ -91,6 +91,7 @@ bool gemm_block_supports(const GemmArgs& g);  // 128 x 128 tiles, four waves in 
 bool gemm_block_ragged_supports(const GemmArgs& g);  // with GemmArgs::ragged: any M, N, K % 32 == 0 and alignment
 hipError_t launch_gemm_block(const GemmArgs& g, hipStream_t s);
 bool block_streams_weights(const GemmArgs& g);  // whether launch_gemm_block reads B with the non-temporal bit
+int block_c_form(const GemmArgs& g);            // how it stores C or, split, its shares' sums (CStore)
 hipError_t launch_ksplit_reduce(const GemmArgs& g, hipStream_t s);  // sums g.ksplit shares' partial sums at g.ks_part into g.C, with the epilogue
 bool gemm_ring_supports(const GemmArgs& g);  // batched decode: private streams of B per wave, A through a flag-guarded ring (no barrier per K-tile)
 int ring_ksplit_plan(const GemmArgs& g, int want, size_t* part_bytes, size_t* counters);  // its K split for this problem (want: 0 = by shape, 1 = none, n = n shares): shares (1 = none), bytes of partial tiles, arrival counters

@@ -23,6 +23,7 @@ class Route:
 
     TILED, SKINNY, BLOCK, RING, SLICE = 2, 3, 22, 28, 29
     COPY_A, COPY_B, SPLIT, X, STREAM_B = 0x100, 0x200, 0x400, 0x800, 0x1000
+    FORM, PIECES, KEPT, OUT = 0x6000, 0, 0x2000, 0x4000  # how C is stored
 
     def _run(self, kernel, k_split, call):
         import torch

@@ -16,7 +16,7 @@ def test_large_output_matches_its_parts(kernel, N, K, rem, out):
     import hipkittensp_amd as hk
 
     tk, size = hk.tk_kernel, torch.finfo(out).bits // 8
-    limit = (36 << 20) if kernel == 0 and size == 2 else LIMIT
+    limit = (32 << 20) if kernel == 0 and size == 2 else LIMIT
     step = 512
     M = (limit // (N * size) // step + 2) * step + rem  # past the line; its parts of `step` rows are below
     assert (N * size) % 128 and M * N * size > limit and step * N * size < limit
@@ -36,3 +36,32 @@ def test_large_output_matches_its_parts(kernel, N, K, rem, out):
         tk.set_kernel(prev)
         tk.set_k_split(prev_split)
     assert (guard[:256] == 7).all() and (guard[256 + M * N :] == 7).all()
+
+
+# on both sides of each line of the rule: up to 64 rows; 4 MB of C; bf16 32 MB, fp32 never non-temporally, but rows and an address that start on lines
+@pytest.mark.parametrize("M,N,K,out,shift,form", [
+    (64, 20001, 1056, torch.float32, 0, "PIECES"), (65, 20001, 1056, torch.float32, 0, "KEPT"), (65, 16001, 1056, torch.float32, 0, "PIECES"),
+    (300, 6989, 1056, torch.bfloat16, 0, "PIECES"), (300, 7001, 1056, torch.bfloat16, 0, "OUT"), (2100, 7989, 1056, torch.bfloat16, 0, "OUT"),
+    (2100, 7991, 1056, torch.bfloat16, 0, "PIECES"), (1100, 1024, 1056, torch.float32, 0, "OUT"), (1100, 1024, 1056, torch.float32, 1, "KEPT"),
+    (2100, 8000, 1056, torch.bfloat16, 0, "OUT"), (2100, 8000, 1056, torch.bfloat16, 3, "PIECES")])
+def test_ragged_products_store_as_the_rule_says(route, M, N, K, out, shift, form):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import hipkittensp_amd as hk
+
+    tk, pad = hk.tk_kernel, 512
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    A, As = hk.quantize(torch.randn(M, K, device="cuda", generator=g), 2)
+    B, Bs = hk.quantize(torch.randn(N, K, device="cuda", generator=g).mul_(0.05), 2)
+    whole = torch.full((2 * pad + M * N,), 7.0, dtype=out, device="cuda")
+    C = whole[pad + shift : pad + shift + M * N].view(M, N)
+    taken = route.gemm(A, B, As, Bs, C, M, N, K, k_split=1)
+    assert taken == route.BLOCK | getattr(route, form), hex(taken)
+    assert (whole[: pad + shift] == 7).all() and (whole[pad + shift + M * N :] == 7).all()
+    want = torch.empty(M, N, dtype=out, device="cuda")
+    prev = tk.set_kernel(1)  # one wave per tile: the same sums
+    try:
+        tk.dispatch_micro(A, B, As, Bs, want, 2, 2)
+    finally:
+        tk.set_kernel(prev)
+    assert torch.equal(C, want)
