@@ -23,11 +23,11 @@ LIB = os.path.join(HERE, "libmxfp6_gemm.so")
 NATIVE = os.path.join(HERE, "_native.so")
 PROBES_LIB = os.path.join(HERE, "libmxfp6_probes.so")
 SOURCES = ["api.hip", "dispatch.hip", "gemm_generic.hip", "gemm_tiled.hip", "gemm_tiled4.hip", "gemm_block.hip", "gemm_mid.hip", "gemm_skinny.hip", "gemm_ring.hip", "gemm_slice.hip", "quantize.hip"]
-# (source, object name, extra flags).  gemm_tiled.hip gives five objects: its host-side part, and the kernel
+# (source, object name, extra flags).  gemm_tiled.hip and gemm_block.hip give five objects each: the host-side part, and the kernel
 # instantiations of each pair of operand formats (the bulk of the build time; they compile side by side).  gemm_skinny.hip gives two:
 # on packed operands, and on a linear layer's activations.
 UNITS = [(src, src.replace(".hip", ""), []) for src in SOURCES] + [
-    ("gemm_tiled.hip", f"gemm_tiled_fmt{fmt}", [f"-DMXFP6_TILED_FMT={fmt}"]) for fmt in (22, 23, 32, 33)
+    (f"gemm_{k}.hip", f"gemm_{k}_fmt{fmt}", [f"-DMXFP6_{k.upper()}_FMT={fmt}"]) for k in ("tiled", "block") for fmt in (22, 23, 32, 33)
 ] + [("gemm_skinny.hip", "gemm_skinny_x", ["-DMXFP6_SKINNY_X"])]
 # what the measurement build compiles again (or in addition), with -DMXFP6_PROBES
 PROBE_UNITS = [("api.hip", "api_probes", ["-DMXFP6_PROBES"]), ("gemm_tiled.hip", "gemm_tiled_fmt22_probes", ["-DMXFP6_TILED_FMT=22", "-DMXFP6_PROBES"]),
@@ -72,7 +72,7 @@ def _build_native() -> str:
 def build(verbose: bool = True) -> str:
     os.makedirs(OBJ, exist_ok=True)
     # the units that take longest first
-    order = sorted(UNITS + PROBE_UNITS, key=lambda u: (u[1] != "gemm_block", not u[1].startswith("gemm_tiled_fmt"), u[1] not in ("gemm_skinny", "gemm_mid")))
+    order = sorted(UNITS + PROBE_UNITS, key=lambda u: ("_fmt" not in u[1], u[1] not in ("gemm_skinny", "gemm_mid")))
     with cf.ThreadPoolExecutor(max_workers=min(8, len(order))) as ex:
         objs = dict(zip((u[1] for u in order), ex.map(_compile, order)))
     product = [objs[u[1]] for u in UNITS]

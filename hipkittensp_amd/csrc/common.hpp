@@ -201,16 +201,12 @@ __device__ __forceinline__ void store_c(v4i v, const __amdgpu_buffer_rsrc_t& rsr
   __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, voff, soff, STREAM ? kNonTemporal : 0);
   asm volatile("s_nop 3" ::"v"(v) : "memory");
 }
-// Whether C, `rows` rows of `pitch` outputs, goes out non-temporally: where its rows start on lines, and where all of it is small beside the
-// L2s (32 MB).  Rows that start inside a line leave every line to two stores, and of a large C the L2s send out the first part before the
-// second has come.  us, non-temporal / through the L2s, fp32: 2000 x 8191 x 1056 52.4 / 42.8, 4096 x 11000 x 1024 113 / 82, 1000 x 5003 x 1056 (20 MB) 18.8 /
-// 20.2; bf16: 4096 x 11000 x 1024 69.6 / 64.1, 3500 x 5000 x 1024 (35 MB) 31.9 / 29.9, 2048 x 5000 x 1024 (20 MB) 18.9 / 20.4.
-constexpr size_t kStreamedPartLines = (size_t)24 << 20;
-template <typename OutT>
-__host__ __device__ inline bool streams_c(const void* C, int rows, size_t pitch, size_t limit = kStreamedPartLines) {
-  const size_t row = pitch * sizeof(OutT);
-  return (((uintptr_t)C | row) & 127) == 0 || rows * row <= limit;
-}
+// Whether C in whole lines, `rows` rows of `row` bytes, leaves non-temporally: where its rows start on lines, and up to 16 MB.  Rows that start inside a
+// line leave every line to two stores, and of a large C the L2s send out the first part before the second has come.  Through the L2s / non-temporally,
+// of the time in pieces, over 110 drawn shapes with such rows, block kernel: bf16 4 to 12 MB 0.99 / 0.97, 16 to 24 MB 0.98 / 1.02, above 0.98 / 1.02 (up to 1.3);
+// fp32 1.01 / 0.98, 0.99 / 1.03, above 0.97 / 1.27 (up to 1.9).
+constexpr size_t kLeavingPartLines = (size_t)16 << 20;
+__host__ __device__ inline bool c_leaves(const void* C, int rows, size_t row) { return (((uintptr_t)C | row) & 127) == 0 || rows * row <= kLeavingPartLines; }
 
 // Optional work fused into every kernel's epilogue, in fp32 before the output rounding:
 //   y = act(acc * row_scale[m] * col_scale[n] + bias[n])        (each factor / term only if its pointer is set)

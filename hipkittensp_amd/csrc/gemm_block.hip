@@ -43,6 +43,40 @@ struct BlockArgs {
   int fmt_c;
 };
 
+int cu_count_of_device() {
+  static int cus[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  if (cus[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
+    cus[dev] = n;
+  }
+  return cus[dev];
+}
+
+// Chunks of two K-tiles (PAIR, one workgroup per CU) or three slots of one K-tile (two workgroups per CU, one's waits are the
+// other's work).  While no CU gets a second workgroup: PAIR, but for K up to 1024, where filling its slots takes a good part of
+// the eight K-tiles there are (us, three slots / PAIR: 256 x 4096 x 512 5.9 / 6.4, 256^3 4.4 / 5.0, 384 x 2048 x 1024 7.4 / 7.4 and
+// 6.7 / 7.1 tile-major; 256 x 8192 x 1536 12.1 / 11.0, 512 x 4096 x 2048 15.4 / 13.3, tile-major 11.7 / 11.5; 32 x 20608 x 5632
+// 27.6 / 23.4 and 22.2 / 18.4), and up to 2048 with both operands tile-major (512 x 8192 x 2048 12.9 / 13.3, 512 x 4096 x 4096 17.9 /
+// 16.8).  Beyond: PAIR where its fewer line requests outweigh the second workgroup, with both operands row-major from K = 4096 on
+// (2048 x 4096 x 4096 49.5 / 43.8, 1536 x 4096 x 4096 41.2 / 41.1, 640 x 8192 x 2048 23.6 / 25.1), with one from 8192 on (1024 x 8192 x 8192
+// 70.1 / 64.9, 256 x 28672 x 8192 81.0 / 73.0, 2048 x 4096 x 4096 39.2 / 40.3), with none never (31.5 / 36.4).
+// (launch's and launch_fp6's `stages` = 3 or 6 forces one, for measurement.)
+int block_stages(const GemmArgs& g, int grid, int cus) {
+  const int row_major = !g.layout_a + !g.layout_b;
+  const int min_k = grid <= cus ? (row_major ? 1025 : 2049) : row_major == 2 ? 4096 : row_major == 1 ? 8192 : 0x7fffffff;
+  return g.K >= min_k ? 6 : 3;
+}
+int forced_stages(const GemmArgs& g) { return g.tile_rows == 3 || g.tile_rows == 6 ? g.tile_rows : 0; }
+
+}  // namespace
+
+#ifdef MXFP6_BLOCK_FMT  // ------------------------------------------------------------------------ one pair of operand formats
+
+namespace {
+
 // STAGES: ring slots, 3 (80 KB of LDS, two workgroups per CU), 4 (128 x 256 tiles) or 6, which is PAIR.  Loads run STAGES K-tiles
 // ahead of the MFMAs and have STAGES - 1 steps to land.
 // PAIR: three slots of two K-tiles (a chunk) each, 152 KB, one workgroup per CU.  What it is for is a row-major operand: the 96
@@ -74,10 +108,11 @@ struct BlockArgs {
 // rows 44.1 / 40.8.  What it costs stands at kStreamBytes.  Not row-major weights: 50.6 / 51.8, 96 rows 47.7 / 49.4, 128 x 8192 x 24576 45.0 / 47.5, unsplit 49.7 / 50.5 (with
 // activations for each layer 53.8 / 51.6, but 54.0 / 55.0 over 24 layers).  (An instantiation of its own: picked as the kernel runs, 1024 x 4096 x 14336
 // paid 58.6 / 59.5 for it.)
-// CFORM: how RAGGED stores C (CStore, ragged_c_form).
+// CFORM: how C is stored (CStore; block_c_form), one form to an instantiation: a choice at each store costs a short fp32 product 3 %, and of two copies
+// one comes through the instruction cache in vain (aligned rows, C of 4 to 12 MB, of the time as it comes: two copies 0.975, one 0.957).
 // 500 x 5003 x 2880: 17.0 us against 148.5 on the one-wave-per-tile kernel, which fetches every operand row again for each of
 // its 32 x 32 tiles, 4 bytes per lane.
-template <int FA, int FB, typename Out, int STAGES, int WN, bool FUSED, bool RAGGED = false, bool STREAM = false, int CFORM = kCOut>
+template <int FA, int FB, typename Out, int STAGES, int WN, bool FUSED, bool RAGGED = false, bool STREAM = false, int CFORM = kCPieces>
 __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_block_kernel(const BlockArgs args) {
   typedef typename Out::type OutT;
   static_assert((STAGES == 3 || STAGES == 4 || STAGES == 6) && (WN == 2 || WN == 4), "ring depth, tile width");
@@ -540,160 +575,112 @@ __global__ __launch_bounds__(2 * WN * 64, STAGES <= 3 ? 2 : WN / 2) void gemm_bl
       return;
     }
   }
-  // C as `FORM` says (CStore)
-  auto store_tile = [&]<int FORM>() __attribute__((always_inline)) {
-    constexpr bool LINES = FORM != kCPieces, OUT = FORM == kCOut;
-    constexpr int kRun = 16 / (int)sizeof(OutT);
-    const int row_l = wm * 64 + (LINES ? line_row<1>(lane) : r32), col_l = wn * 64 + (LINES ? line_piece<1>(lane) : h) * kRun;
-    const int voff = row_l * N2 + col_l * (int)sizeof(OutT);
-    // RAGGED: `n` consecutive outputs of a row, 16 bytes of them at C's element alignment or, across N, one by one
-    // (the lane's address once, the stores' places from it: 512 x 296 x 16960 19.6 / 19.0, 49 x 20832 x 672 fp32 7.8 / 7.5)
-    [[maybe_unused]] OutT* const lane_c = (OutT*)args.C + ((size_t)share * args.M + (size_t)pm * kBM + row_l) * ldc + (size_t)pn * kBN + col_l;
-    // 16 bytes of the lane, `row` rows and `col` columns on
-    auto put = [&](v4i v, int row, int col) __attribute__((always_inline)) {
-      const int m = row_l + row, n = col_l + col;
-      if constexpr (!RAGGED) {
-        if (!edge || (m < rows_a && n < rows_b)) store_c<OUT>(v, rC, voff + col * (int)sizeof(OutT), row * N2);
+  constexpr bool LINES = CFORM != kCPieces, OUT = CFORM == kCOut;
+  constexpr int kRun = 16 / (int)sizeof(OutT);
+  const int row_l = wm * 64 + (LINES ? line_row<1>(lane) : r32), col_l = wn * 64 + (LINES ? line_piece<1>(lane) : h) * kRun;
+  const int voff = row_l * N2 + col_l * (int)sizeof(OutT);
+  // RAGGED: `n` consecutive outputs of a row, 16 bytes of them at C's element alignment or, across N, one by one
+  // (the lane's address once, the stores' places from it: 512 x 296 x 16960 19.6 / 19.0, 49 x 20832 x 672 fp32 7.8 / 7.5)
+  [[maybe_unused]] OutT* const lane_c = (OutT*)args.C + ((size_t)share * args.M + (size_t)pm * kBM + row_l) * ldc + (size_t)pn * kBN + col_l;
+  // 16 bytes of the lane, `row` rows and `col` columns on
+  auto put = [&](v4i v, int row, int col) __attribute__((always_inline)) {
+    const int m = row_l + row, n = col_l + col;
+    if constexpr (!RAGGED) {
+      if (!edge || (m < rows_a && n < rows_b)) store_c<OUT>(v, rC, voff + col * (int)sizeof(OutT), row * N2);
+    } else {
+      if (m >= rows_a || n >= rows_b) return;
+      OutT* const p = lane_c + row * ldc + col;
+      if (n + kRun <= rows_b) {
+        typedef int v4i_element __attribute__((ext_vector_type(4), aligned(2)));
+        if constexpr (OUT) __builtin_nontemporal_store((v4i_element)v, reinterpret_cast<v4i_element*>(p));
+        else *reinterpret_cast<v4i_element*>(p) = (v4i_element)v;
       } else {
-        if (m >= rows_a || n >= rows_b) return;
-        OutT* const p = lane_c + row * ldc + col;
-        if (n + kRun <= rows_b) {
-          typedef int v4i_element __attribute__((ext_vector_type(4), aligned(2)));
-          if constexpr (OUT) __builtin_nontemporal_store((v4i_element)v, reinterpret_cast<v4i_element*>(p));
-          else *reinterpret_cast<v4i_element*>(p) = (v4i_element)v;
-        } else {
-          OutT o[kRun];
-          __builtin_memcpy(o, &v, 16);
+        OutT o[kRun];
+        __builtin_memcpy(o, &v, 16);
 #pragma unroll
-          for (int e = 0; e + 1 < kRun; e++)
-            if (n + e < rows_b) p[e] = o[e];
-        }
+        for (int e = 0; e + 1 < kRun; e++)
+          if (n + e < rows_b) p[e] = o[e];
       }
-    };
-    // four registers, 16 outputs (bf16) or 8 (fp32) of a row apart, of rows `row` on; `col` columns on
-    auto put4 = [&](v4i (&v)[2][2], int row, int col) __attribute__((always_inline)) {
-      constexpr int kApart = 2 * kRun;
-      if constexpr (LINES) {
+    }
+  };
+  // four registers, 16 outputs (bf16) or 8 (fp32) of a row apart, of rows `row` on; `col` columns on
+  auto put4 = [&](v4i (&v)[2][2], int row, int col) __attribute__((always_inline)) {
+    constexpr int kApart = 2 * kRun;
+    if constexpr (LINES) {
 #pragma unroll
-        for (int p = 0; p < 2; p++) pair_rows(v[p][0], v[p][1]);
+      for (int p = 0; p < 2; p++) pair_rows(v[p][0], v[p][1]);
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-          join_lines(v[0][t], v[1][t]);
-          put(v[0][t], row + t * 16, col);
-          put(v[1][t], row + t * 16 + 8, col);
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; q++) put(v[q >> 1][q & 1], row, col + q * kApart);
-      }
-    };
-    if constexpr (sizeof(OutT) == 2) {
-#pragma unroll
-      for (int i = 0; i < 2; i++) {
-        uint32_t pk[2][8];
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-          for (int e = 0; e < 8; e++) pk[j][e] = pack_bf16x2(acc[i][j][2 * e], acc[i][j][2 * e + 1]);
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-          for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int c = 0; c < 2; c++) {
-              // runs 2t and 2t+1 (dwords 4t+c and 4t+2+c): lower lanes keep run 2t and get the partner's, upper lanes run 2t+1
-              const auto x = __builtin_amdgcn_permlane32_swap(pk[j][4 * t + c], pk[j][4 * t + 2 + c], false, false);
-              pk[j][4 * t + c] = x[0], pk[j][4 * t + 2 + c] = x[1];
-            }
-        v4i v[2][2];
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-          for (int t = 0; t < 2; t++) v[j][t] = v4i{(int)pk[j][4 * t], (int)pk[j][4 * t + 1], (int)pk[j][4 * t + 2], (int)pk[j][4 * t + 3]};
-        put4(v, i * 32, 0);
+      for (int t = 0; t < 2; t++) {
+        join_lines(v[0][t], v[1][t]);
+        put(v[0][t], row + t * 16, col);
+        put(v[1][t], row + t * 16 + 8, col);
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-          v4i v[2][2];
-#pragma unroll
-          for (int q = 0; q < 4; q++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) v[q >> 1][q & 1][e] = __float_as_int(acc[i][j][4 * q + e]);
-          put4(v, i * 32, j * 32);
-        }
+      for (int q = 0; q < 4; q++) put(v[q >> 1][q & 1], row, col + q * kApart);
     }
   };
-  // Two copies, rather than a choice at each store, which costs a short fp32 product 3 %; of RAGGED's longer code one (FORM, launch_ragged)
-  if constexpr (RAGGED) store_tile.template operator()<CFORM>();
-  else if (streams_c<OutT>(args.C, args.M, N)) store_tile.template operator()<kCOut>();
-  else store_tile.template operator()<kCKept>();
-}
-
-int cu_count_of_device() {
-  static int cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (cus[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
-    cus[dev] = n;
+  if constexpr (sizeof(OutT) == 2) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      uint32_t pk[2][8];
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) pk[j][e] = pack_bf16x2(acc[i][j][2 * e], acc[i][j][2 * e + 1]);
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+          for (int c = 0; c < 2; c++) {
+            // runs 2t and 2t+1 (dwords 4t+c and 4t+2+c): lower lanes keep run 2t and get the partner's, upper lanes run 2t+1
+            const auto x = __builtin_amdgcn_permlane32_swap(pk[j][4 * t + c], pk[j][4 * t + 2 + c], false, false);
+            pk[j][4 * t + c] = x[0], pk[j][4 * t + 2 + c] = x[1];
+          }
+      v4i v[2][2];
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int t = 0; t < 2; t++) v[j][t] = v4i{(int)pk[j][4 * t], (int)pk[j][4 * t + 1], (int)pk[j][4 * t + 2], (int)pk[j][4 * t + 3]};
+      put4(v, i * 32, 0);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        v4i v[2][2];
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) v[q >> 1][q & 1][e] = __float_as_int(acc[i][j][4 * q + e]);
+        put4(v, i * 32, j * 32);
+      }
   }
-  return cus[dev];
 }
 
-// Chunks of two K-tiles (PAIR, one workgroup per CU) or three slots of one K-tile (two workgroups per CU, one's waits are the
-// other's work).  While no CU gets a second workgroup: PAIR, but for K up to 1024, where filling its slots takes a good part of
-// the eight K-tiles there are (us, three slots / PAIR: 256 x 4096 x 512 5.9 / 6.4, 256^3 4.4 / 5.0, 384 x 2048 x 1024 7.4 / 7.4 and
-// 6.7 / 7.1 tile-major; 256 x 8192 x 1536 12.1 / 11.0, 512 x 4096 x 2048 15.4 / 13.3, tile-major 11.7 / 11.5; 32 x 20608 x 5632
-// 27.6 / 23.4 and 22.2 / 18.4), and up to 2048 with both operands tile-major (512 x 8192 x 2048 12.9 / 13.3, 512 x 4096 x 4096 17.9 /
-// 16.8).  Beyond: PAIR where its fewer line requests outweigh the second workgroup, with both operands row-major from K = 4096 on
-// (2048 x 4096 x 4096 49.5 / 43.8, 1536 x 4096 x 4096 41.2 / 41.1, 640 x 8192 x 2048 23.6 / 25.1), with one from 8192 on (1024 x 8192 x 8192
-// 70.1 / 64.9, 256 x 28672 x 8192 81.0 / 73.0, 2048 x 4096 x 4096 39.2 / 40.3), with none never (31.5 / 36.4).
-// (launch's and launch_fp6's `stages` = 3 or 6 forces one, for measurement.)
-int block_stages(const GemmArgs& g, int grid, int cus) {
-  const int row_major = !g.layout_a + !g.layout_b;
-  const int min_k = grid <= cus ? (row_major ? 1025 : 2049) : row_major == 2 ? 4096 : row_major == 1 ? 8192 : 0x7fffffff;
-  return g.K >= min_k ? 6 : 3;
-}
-int forced_stages(const GemmArgs& g) { return g.tile_rows == 3 || g.tile_rows == 6 ? g.tile_rows : 0; }
 template <int FA, int FB, bool FUSED>
 hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, hipStream_t s) {
   const int cus = cu_count_of_device();
   const bool f32 = g.f32out || a.nsplit > 1;  // shares leave fp32 partial sums
-  const int grid = tiles * a.nsplit;
-  if (g.tile_cols == 256) {  // tiles of 128 x 256, eight waves, four slots
-    if (f32) gemm_block_kernel<FA, FB, OutF32, 4, 4, FUSED><<<grid, 512, 0, s>>>(a);
-    else gemm_block_kernel<FA, FB, OutBf16, 4, 4, FUSED><<<grid, 512, 0, s>>>(a);
-    return hipGetLastError();
-  }
+  const int grid = tiles * a.nsplit, form = block_c_form(g);
   if (stages == 0) stages = block_stages(g, grid, cus);
-  if (block_streams_weights(g) && (!f32 || !FUSED)) {
-    if (!f32) gemm_block_kernel<FA, FB, OutBf16, 6, 2, FUSED, false, true><<<grid, 256, 0, s>>>(a);
-    else if constexpr (!FUSED) gemm_block_kernel<FA, FB, OutF32, 6, 2, false, false, true><<<grid, 256, 0, s>>>(a);
-  } else if (stages == 6) {
-    if (f32) gemm_block_kernel<FA, FB, OutF32, 6, 2, FUSED><<<grid, 256, 0, s>>>(a);
-    else gemm_block_kernel<FA, FB, OutBf16, 6, 2, FUSED><<<grid, 256, 0, s>>>(a);
-  } else {
-    if (f32) gemm_block_kernel<FA, FB, OutF32, 3, 2, FUSED><<<grid, 256, 0, s>>>(a);
-    else gemm_block_kernel<FA, FB, OutBf16, 3, 2, FUSED><<<grid, 256, 0, s>>>(a);
-  }
+  auto with = [&]<typename Out, int STAGES, int WN, bool STREAM>() {
+    constexpr int kThreads = 2 * WN * 64;
+    if (form == kCOut) gemm_block_kernel<FA, FB, Out, STAGES, WN, FUSED, false, STREAM, kCOut><<<grid, kThreads, 0, s>>>(a);
+    else if (form == kCPieces) gemm_block_kernel<FA, FB, Out, STAGES, WN, FUSED, false, STREAM, kCPieces><<<grid, kThreads, 0, s>>>(a);
+    else gemm_block_kernel<FA, FB, Out, STAGES, WN, true, false, false, kCKept><<<grid, kThreads, 0, s>>>(a);  // fused or not: args.ep may be empty
+  };
+  auto with_out = [&]<typename Out>() {
+    if (g.tile_cols == 256) with.template operator()<Out, 4, 4, false>();  // tiles of 128 x 256, eight waves, four slots
+    else if ((sizeof(typename Out::type) == 2 || !FUSED) && block_streams_weights(g)) with.template operator()<Out, 6, 2, sizeof(typename Out::type) == 2 || !FUSED>();
+    else if (stages == 6) with.template operator()<Out, 6, 2, false>();
+    else with.template operator()<Out, 3, 2, false>();
+  };
+  if (f32) with_out.template operator()<OutF32>();
+  else with_out.template operator()<OutBf16>();
   return hipGetLastError();
-}
-// How a RAGGED instantiation stores C.  As it comes where that is little: below 4 MB, up to 64 rows, and the sums of a K split's shares, which are
-// read again at once (us, as it comes / whole lines through the L2s / whole lines non-temporal, fp32: 49 x 20832 x 672 7.45 / 7.75 / 7.5, 20 x 30001 x 672 7.35 /
-// 7.65 / 7.8, 64 x 20001 x 2080 13.1 / 13.35 / 13.4; 191 x 664 x 18624 18.6 / 18.85 / 18.85, 512 x 296 x 16960 19.05 / 19.2 / 19.2).  Else non-temporally where
-// its rows start on lines.  Where they do not, a line is two stores: bf16 up to 32 MB (1000 x 5003 x 1056, 9.5 MB, 17.1 / 17.1 / 16.6; 256 x 16001 x 1056 13.2 / 13.2 /
-// 12.8; 2000 x 8191 x 1056, 31 MB, 38.5 / 38.4 / 37.2; 6000 x 3001 x 672, 34 MB, 33.6 / 33.2 / 36.2); fp32 never (256 x 16001 x 1056, 16 MB, 13.4 / 12.2 /
-// 16.3; 1000 x 5003 x 1056, 19 MB, 16.5 / 15.5 / 18.6; 2000 x 8191 x 1056 36.3 / 34.2 / 49.3).  Over 70 drawn shapes of each type, of the time as it comes: bf16
-// 4 to 32 MB 1.00 / 0.97, above 1.00 / 1.04; fp32 8 to 12 MB 0.96 / 1.00, 12 to 20 MB 0.93 / 1.09, above 0.94 / 1.28.
-int ragged_c_form(const GemmArgs& g) {
-  const size_t row = (size_t)g.N * (g.f32out ? 4 : 2), bytes = g.M * row;
-  if (g.ksplit > 1 || g.M <= 64 || bytes < (size_t)4 << 20) return kCPieces;
-  if ((((uintptr_t)g.C | row) & 127) == 0) return kCOut;
-  return g.f32out ? kCKept : bytes <= (size_t)32 << 20 ? kCOut : kCPieces;
 }
 // RAGGED instantiations, the fused epilogue applied or not inside.  PAIR from K = 1920 on while no CU gets a second workgroup (us,
 // three slots / PAIR: 64 x 3001 x 1888 11.1 / 11.1, 500 x 5003 x 1056 13.2 / 13.6, 100 x 5003 x 2016 17.8 / 16.1), from 6144 on
@@ -706,7 +693,7 @@ hipError_t launch_ragged(const GemmArgs& g, const BlockArgs& a, int tiles, hipSt
     if (deep) gemm_block_kernel<FA, FB, Out, 6, 2, true, true, false, CFORM><<<grid, 256, 0, s>>>(a);
     else gemm_block_kernel<FA, FB, Out, 3, 2, true, true, false, CFORM><<<grid, 256, 0, s>>>(a);
   };
-  const int form = ragged_c_form(g);
+  const int form = block_c_form(g);
   if (g.f32out || a.nsplit > 1) {
     if (form == kCOut) with.template operator()<OutF32, kCOut>();
     else if (form == kCKept) with.template operator()<OutF32, kCKept>();
@@ -734,7 +721,28 @@ hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, 
   return launch<FA, FB, false>(g, a, tiles, stages, s);
 }
 
+
 }  // namespace
+
+#define MXFP6_PASTE2(a, b) a##b
+#define MXFP6_PASTE(a, b) MXFP6_PASTE2(a, b)
+hipError_t MXFP6_PASTE(launch_gemm_block_fmt, MXFP6_BLOCK_FMT)(const GemmArgs& g, hipStream_t s) {
+  constexpr int FA = MXFP6_BLOCK_FMT / 10, FB = MXFP6_BLOCK_FMT % 10;
+  static_assert((FA == 2 || FA == 3) && (FB == 2 || FB == 3), "MXFP6_BLOCK_FMT: 22, 23, 32 or 33");
+  const int bn = g.tile_cols == 256 ? 256 : 128, nsplit = g.ksplit > 1 ? g.ksplit : 1;
+  BlockArgs a{g.A, g.B, g.As, g.Bs, nsplit > 1 ? (void*)g.ks_part : g.C, g.M, g.N, g.K, (g.M + kBM - 1) / kBM, (g.N + bn - 1) / bn, g.layout_a, g.layout_b,
+              g.raster_group_m > 0 ? g.raster_group_m : kGroupM, g.raster_no_xcd_remap == 1 ? 0 : g.raster_no_xcd_remap == 2 ? 2 : 1, nsplit, g.ep, g.C_scale, g.fmt_c};
+  const int tiles = a.tiles_m * a.tiles_n;
+  if (g.ragged) {
+    if (nsplit > 1) a.ep = Epilogue{};  // the reduction applies it
+    return launch_ragged<FA, FB>(g, a, tiles, s);
+  }
+  return launch<FA, FB>(g, a, tiles, forced_stages(g), s);
+}
+#undef MXFP6_PASTE
+#undef MXFP6_PASTE2
+
+#else  // ---------------------------------------------------------------------------------------- the host-side object
 
 bool gemm_block_supports(const GemmArgs& g) {
   // N % 8 keeps every run of 8 bf16 outputs whole and aligned; K in whole K-tiles; 32-bit byte offsets
@@ -753,38 +761,46 @@ bool gemm_block_ragged_supports(const GemmArgs& g) {
 
 bool block_streams_weights(const GemmArgs& g) {
   const int split = g.ksplit > 1 ? g.ksplit : 1;
-  if (g.ragged || g.tile_cols == 256 || !g.layout_b || g.M > kBM || (size_t)g.N * (g.K / 4 * 3) < kStreamBytes) return false;
+  if (g.ragged || g.tile_cols == 256 || !g.layout_b || g.M > kBM || (size_t)g.N * (g.K / 4 * 3) < kStreamBytes || block_c_form(g) == kCKept) return false;
   if (split == 1 && (g.fmt_c || (g.f32out && epilogue_any(g.ep)))) return false;  // not built
   return (forced_stages(g) ? forced_stages(g) : block_stages(g, (g.N + 127) / 128 * split, cu_count_of_device())) == 6;
 }
 
+// How a RAGGED instantiation stores C.  As it comes where that is little: below 4 MB, up to 64 rows, and the sums of a K split's shares, which are
+// read again at once (us, as it comes / whole lines through the L2s / whole lines non-temporal, fp32: 49 x 20832 x 672 7.45 / 7.75 / 7.5, 20 x 30001 x 672 7.35 /
+// 7.65 / 7.8, 64 x 20001 x 2080 13.1 / 13.35 / 13.4; 191 x 664 x 18624 18.6 / 18.85 / 18.85, 512 x 296 x 16960 19.05 / 19.2 / 19.2).  Else non-temporally where
+// its rows start on lines.  Where they do not, a line is two stores: bf16 up to 32 MB (1000 x 5003 x 1056, 9.5 MB, 17.1 / 17.1 / 16.6; 256 x 16001 x 1056 13.2 / 13.2 /
+// 12.8; 2000 x 8191 x 1056, 31 MB, 38.5 / 38.4 / 37.2; 6000 x 3001 x 672, 34 MB, 33.6 / 33.2 / 36.2); fp32 never (256 x 16001 x 1056, 16 MB, 13.4 / 12.2 /
+// 16.3; 1000 x 5003 x 1056, 19 MB, 16.5 / 15.5 / 18.6; 2000 x 8191 x 1056 36.3 / 34.2 / 49.3).  Over 70 drawn shapes of each type, of the time as it comes: bf16
+// 4 to 32 MB 1.00 / 0.97, above 1.00 / 1.04; fp32 8 to 12 MB 0.96 / 1.00, 12 to 20 MB 0.93 / 1.09, above 0.94 / 1.28.
+static int ragged_c_form(const GemmArgs& g) {
+  const size_t row = (size_t)g.N * (g.f32out ? 4 : 2), bytes = g.M * row;
+  if (g.ksplit > 1 || g.M <= 64 || bytes < (size_t)4 << 20) return kCPieces;
+  if ((((uintptr_t)g.C | row) & 127) == 0) return kCOut;
+  return g.f32out ? kCKept : bytes <= (size_t)32 << 20 ? kCOut : kCPieces;
+}
 int block_c_form(const GemmArgs& g) {
   if (g.ragged) return ragged_c_form(g);
   if (g.ksplit > 1 || g.fmt_c) return kCPieces;
-  return (g.f32out ? streams_c<float>(g.C, g.M, g.N) : streams_c<uint16_t>(g.C, g.M, g.N)) ? kCOut : kCKept;
+  const size_t row = (size_t)g.N * (g.f32out ? 4 : 2), bytes = g.M * row;
+  const bool whole = (((uintptr_t)g.C | row) & 127) == 0;
+  return bytes < (size_t)(whole ? 2 : 4) << 20 ? kCPieces : c_leaves(g.C, g.M, row) ? kCOut : kCKept;
 }
+
+hipError_t launch_gemm_block_fmt22(const GemmArgs& g, hipStream_t s);
+hipError_t launch_gemm_block_fmt23(const GemmArgs& g, hipStream_t s);
+hipError_t launch_gemm_block_fmt32(const GemmArgs& g, hipStream_t s);
+hipError_t launch_gemm_block_fmt33(const GemmArgs& g, hipStream_t s);
 
 // g.ksplit > 1 (with g.ks_part): the K range of every output tile split between that many workgroups, then
 // ksplit_reduce_kernel (gemm_tiled.hip), which also applies a fused epilogue.  The caller has checked that the last share
 // is not empty (block_split_shares, dispatch.hip).
 hipError_t launch_gemm_block(const GemmArgs& g, hipStream_t s) {
-  const int bn = g.tile_cols == 256 ? 256 : 128, nsplit = g.ksplit > 1 ? g.ksplit : 1;
-  BlockArgs a{g.A, g.B, g.As, g.Bs, nsplit > 1 ? (void*)g.ks_part : g.C, g.M, g.N, g.K, (g.M + kBM - 1) / kBM, (g.N + bn - 1) / bn, g.layout_a, g.layout_b,
-              g.raster_group_m > 0 ? g.raster_group_m : kGroupM, g.raster_no_xcd_remap == 1 ? 0 : g.raster_no_xcd_remap == 2 ? 2 : 1, nsplit, g.ep, g.C_scale, g.fmt_c};
-  const int tiles = a.tiles_m * a.tiles_n, stages = forced_stages(g);
-  hipError_t e;
-  if (g.ragged) {
-    if (nsplit > 1) a.ep = Epilogue{};  // the reduction applies it
-    if (g.fmt_a == 2 && g.fmt_b == 2) e = launch_ragged<2, 2>(g, a, tiles, s);
-    else if (g.fmt_a == 2 && g.fmt_b == 3) e = launch_ragged<2, 3>(g, a, tiles, s);
-    else if (g.fmt_a == 3 && g.fmt_b == 2) e = launch_ragged<3, 2>(g, a, tiles, s);
-    else e = launch_ragged<3, 3>(g, a, tiles, s);
-  } else if (g.fmt_a == 2 && g.fmt_b == 2) e = launch<2, 2>(g, a, tiles, stages, s);
-  else if (g.fmt_a == 2 && g.fmt_b == 3) e = launch<2, 3>(g, a, tiles, stages, s);
-  else if (g.fmt_a == 3 && g.fmt_b == 2) e = launch<3, 2>(g, a, tiles, stages, s);
-  else e = launch<3, 3>(g, a, tiles, stages, s);
-  if (e == hipSuccess && nsplit > 1) e = launch_ksplit_reduce(g, s);
-  return e;
+  const hipError_t e = g.fmt_a == 2 ? (g.fmt_b == 2 ? launch_gemm_block_fmt22(g, s) : launch_gemm_block_fmt23(g, s))
+                                    : (g.fmt_b == 2 ? launch_gemm_block_fmt32(g, s) : launch_gemm_block_fmt33(g, s));
+  return e == hipSuccess && g.ksplit > 1 ? launch_ksplit_reduce(g, s) : e;
 }
+
+#endif  // MXFP6_BLOCK_FMT
 
 }  // namespace mxfp6

@@ -512,7 +512,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
   // tile meanwhile.  The stores count in vmcnt like the loads and retire in order with them, so the waits of
   // the K loop ("all but the newest batch") stay valid.
   // EDGE: the tile has fewer than 256 valid rows or columns; those stores are predicated per lane, and so are all of a C
-  // that goes through the L2s (streams_c; a third copy for those made the loop's code worse: 8192 x 8192 x 16384 e3m2 x e2m3 605 -> 619 us).
+  // that goes through the L2s (c_leaves; a third copy for those made the loop's code worse: 8192 x 8192 x 16384 e3m2 x e2m3 605 -> 619 us).
   typedef typename Out::type OutT;
   // Fused scales / bias / activation, on the accumulators themselves, before the epilogue proper.  Per 32x32 tile a
   // lane owns row wm * TM * 32 + 32 i + lane % 32 and columns 8 q + 4 h .. + 3 for q = 0..3; N % 8 == 0, so a run of
@@ -578,7 +578,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
     if constexpr (KSPLIT != 0 || sizeof(OutT) == 1) return true;
     else {
       const auto g = fresh_args();
-      return streams_c<OutT>(g->C, g->M, (size_t)g->N);
+      return c_leaves(g->C, g->M, (size_t)g->N * sizeof(OutT));
     }
   };
   auto epilogue = [&]<bool EDGE>(int rows_a, int rows_b, [[maybe_unused]] bool streamed) __attribute__((always_inline)) {

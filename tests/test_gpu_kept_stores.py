@@ -4,7 +4,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-LIMIT = 24 << 20  # bytes of C whose rows start inside lines
+LIMIT = 16 << 20  # bytes of C whose rows start inside lines
 
 
 # kernel (0: the block kernel's ragged instantiation), N, K, rows past a multiple of the tile
@@ -45,6 +45,21 @@ def test_large_output_matches_its_parts(kernel, N, K, rem, out):
     (2100, 7991, 1056, torch.bfloat16, 0, "PIECES"), (1100, 1024, 1056, torch.float32, 0, "OUT"), (1100, 1024, 1056, torch.float32, 1, "KEPT"),
     (2100, 8000, 1056, torch.bfloat16, 0, "OUT"), (2100, 8000, 1056, torch.bfloat16, 3, "PIECES")])
 def test_ragged_products_store_as_the_rule_says(route, M, N, K, out, shift, form):
+    check_form(route, 0, route.BLOCK, M, N, K, out, shift, form)
+
+
+# 2 MB of C whose rows start on lines, 4 and 16 MB of others, and an address inside a line; rings of three and six slots, the wide tile
+@pytest.mark.parametrize("M,N,out,shift,form", [
+    (255, 4096, torch.bfloat16, 0, "PIECES"), (256, 4096, torch.bfloat16, 0, "OUT"), (256, 4096, torch.bfloat16, 8, "PIECES"), (2100, 4096, torch.bfloat16, 0, "OUT"),
+    (2100, 4096, torch.bfloat16, 8, "KEPT"), (511, 4104, torch.bfloat16, 0, "PIECES"), (512, 4104, torch.bfloat16, 0, "OUT"), (2044, 4104, torch.bfloat16, 0, "OUT"),
+    (2045, 4104, torch.bfloat16, 0, "KEPT"), (127, 4096, torch.float32, 0, "PIECES"), (128, 4096, torch.float32, 0, "OUT"), (255, 4104, torch.float32, 0, "PIECES"),
+    (256, 4104, torch.float32, 0, "OUT"), (1022, 4104, torch.float32, 0, "OUT"), (1023, 4104, torch.float32, 0, "KEPT"), (1100, 4096, torch.float32, 4, "KEPT")])
+@pytest.mark.parametrize("kernel", [23, 24, 26])
+def test_block_kernel_stores_as_the_rule_says(route, kernel, M, N, out, shift, form):
+    check_form(route, kernel, kernel, M, N, 384, out, shift, form)
+
+
+def check_form(route, kernel, code, M, N, K, out, shift, form):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     import hipkittensp_amd as hk
@@ -55,8 +70,8 @@ def test_ragged_products_store_as_the_rule_says(route, M, N, K, out, shift, form
     B, Bs = hk.quantize(torch.randn(N, K, device="cuda", generator=g).mul_(0.05), 2)
     whole = torch.full((2 * pad + M * N,), 7.0, dtype=out, device="cuda")
     C = whole[pad + shift : pad + shift + M * N].view(M, N)
-    taken = route.gemm(A, B, As, Bs, C, M, N, K, k_split=1)
-    assert taken == route.BLOCK | getattr(route, form), hex(taken)
+    taken = route.gemm(A, B, As, Bs, C, M, N, K, kernel=kernel, k_split=1)
+    assert taken == code | getattr(route, form), hex(taken)
     assert (whole[: pad + shift] == 7).all() and (whole[pad + shift + M * N :] == 7).all()
     want = torch.empty(M, N, dtype=out, device="cuda")
     prev = tk.set_kernel(1)  # one wave per tile: the same sums
