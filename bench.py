@@ -556,7 +556,7 @@ CALIBRATION = [
 def calibration_sweep(hk, torch):
     """The sweep behind the kernel choice's calibration table (hipkittensp_amd/csrc/dispatch_table.inc): every candidate of the
     choice, forced, on a grid of shapes x four layout pairs, timed on the GPU's side with weights rotating through 400 MB
-    (probe_time_us), twice (the better counts), near ties with a K split once more (retime_k_split_ties, retime_level_decode).  `python -m hipkittensp_amd.calibrate` turns the JSON this prints into the
+    (probe_time_us), twice (the better counts), near ties with a K split once more (retime_k_split_ties).  `python -m hipkittensp_amd.calibrate` turns the JSON this prints into the
     table: per shape and candidate, measured time / the time model's figure."""
     import ctypes
 
@@ -603,16 +603,17 @@ def calibration_sweep(hk, torch):
         del row, tile
         torch.cuda.empty_cache()
     retime_k_split_ties(hk, torch, points)
-    retime_level_decode(hk, torch, points)
     return {"what": "calibration sweep of the kernel choice: measured microseconds per candidate (GPU-side timing, weights rotating through 400 MB; near ties with a K split, from 30 us on, with the activations rotating too)", "candidates": [c[0] for c in CANDIDATES],
             "device": torch.cuda.get_device_name(0), "cus": torch.cuda.get_device_properties(0).multi_processor_count, "points": points}
 
 
 def retime_k_split_ties(hk, torch, points):
     """Where a K split (the tiled kernel's or the block kernel's) is the best candidate of a calibration point or within 10 % of
-    it and the call takes 30 us or more, every candidate within 10 % is timed again as a program's calls.  probe_time_us has one A, which
-    the L2s keep from launch to launch; a program's next call has new activations, and the block kernel's K split pays more for them than
-    the tiled kernel's (256 x 8192 x 28672, tile-major weights, one A / three: block 67.6 / 71.3 us, tiled 256-row 69.1 / 69.2)."""
+    it and the call takes 30 us or more, every candidate within 10 % is timed again as a program's calls: runs of 100 on
+    three sets of activations and outputs in turn.  probe_time_us has one A, which the L2s keep from launch to launch; a
+    program's next call has new activations, and the block kernel's K split pays more for them than the tiled kernel's (256 x 8192 x
+    28672, tile-major weights, one A / three: block 67.6 / 71.3 us, tiled 256-row 69.1 / 69.2)."""
+    tk = hk.tk_kernel
     splits = {i for i, c in enumerate(CANDIDATES) if "k_split" in c[0]}
     ties = []
     for p in points:
@@ -621,32 +622,12 @@ def retime_k_split_ties(hk, torch, points):
         near = [i for i, t in known.items() if t <= 1.1 * best]
         if best >= 30 and len(near) > 1 and splits & set(near):
             ties.append((p, near))
-    retime(hk, torch, ties, 3)
-
-
-def retime_level_decode(hk, torch, points):
-    """Where the ring kernel and the block kernel's K split are the best candidates of a calibration point and within 3 % of each other, both
-    are timed again the same way, nine runs of each in turn: two single calibrations of such a point differ by as much as the two kernels."""
-    pair = [i for i, c in enumerate(CANDIDATES) if c[0] in ("block_k_split", "ring")]
-    level = []
-    for p in points:
-        times = [p["measured_us"][i] for i in pair]
-        if None not in times and min(times) <= 1.005 * min(t for t in p["measured_us"] if t is not None) and max(times) < 1.03 * min(times):
-            level.append((p, pair))
-    retime(hk, torch, level, 9)
-
-
-def retime(hk, torch, picked, runs):
-    """Times the candidates of (point, candidates) pairs again as a program's calls and keeps the median of `runs` runs in turn, each of 100 calls on
-    three sets of activations and outputs in turn."""
-    tk = hk.tk_kernel
     g = torch.Generator(device="cuda")
     g.manual_seed(1)
     last, weights, sets = None, None, 0
-    for p, near in sorted(picked, key=lambda t: (t[0]["N"], t[0]["K"])):
+    for p, near in sorted(ties, key=lambda t: (t[0]["N"], t[0]["K"])):
         M, N, K, la, lb = p["M"], p["N"], p["K"], p["layouts"] & 1, p["layouts"] >> 1
         if last != (N, K):
-            print(f"again: N = {N}, K = {K}", file=sys.stderr, flush=True)
             weights = None
             torch.cuda.empty_cache()
             sets, row, tile = weight_sets(hk, torch, N, K, g)
@@ -666,9 +647,9 @@ def retime(hk, torch, picked, runs):
             end.synchronize()
             tk.set_kernel(prev[0]), tk.set_k_split(prev[1])
             return start.elapsed_time(end) * 10
-        times = [[us(cand) for cand in near] for _ in range(runs)]
+        times = [[us(cand) for cand in near] for _ in range(3)]
         for j, cand in enumerate(near):
-            p["measured_us"][cand] = round(sorted(t[j] for t in times)[runs // 2], 2)
+            p["measured_us"][cand] = round(sorted(t[j] for t in times)[1], 2)
 
 
 def source_hash(kernel):
@@ -743,9 +724,8 @@ def main():
     p.add_argument("--sweep-settings", choices=["all", "default", "ksplit-order"], default="all",
                    help="with --raster-sweep: all raster settings, only the kernel's own (to compare schedules under a profiler), or the kernel's own and, as "
                         "xcd_remap=2, a K split's workgroups in tile-by-tile order instead of share by share (for shapes that take a K split)")
-    p.add_argument("--dispatch-sweep", choices=["small", "full", "offgrid", "offgrid2", "calibrate", "level"], default=None,
-                   help="only compare the automatic kernel choice with every forced kernel / tile shape / K split over a grid of shapes and print one JSON line (calibrate: time every candidate on the "
-                        "calibration grid; level: time again the committed sweep's points where the ring kernel and the block kernel's K split are level)")
+    p.add_argument("--dispatch-sweep", choices=["small", "full", "offgrid", "offgrid2", "calibrate"], default=None,
+                   help="only compare the automatic kernel choice with every forced kernel / tile shape / K split over a grid of shapes and print one JSON line")
     p.add_argument("--layouts", choices=["both", "row"], default="both", help="row: skip the decode run with tile-major weights (used for profiling one layout of the skinny kernel)")
     p.add_argument("--profile-kernels", action="store_true", help="only loops of the tiled kernel (8192^3, tile-major), the skinny kernel (configs[3], row-major) and the ring "
                                                                   "kernel (M = 64, tile-major weights), and a copy of known size: the run to put under rocprofv3 "
@@ -771,11 +751,6 @@ def main():
 
     if args.dispatch_sweep == "calibrate":
         print(json.dumps(calibration_sweep(hk, torch)))
-        return
-    if args.dispatch_sweep == "level":
-        sweep = json.load(open(os.path.join(ROOT, "hipkittensp_amd", "csrc", "dispatch_sweep.json")))
-        retime_level_decode(hk, torch, sweep["points"])
-        print(json.dumps(sweep))
         return
     if args.dispatch_sweep:
         print(json.dumps(dispatch_sweep(hk, torch, args.dispatch_sweep)))
