@@ -670,7 +670,7 @@ hipError_t launch(const GemmArgs& g, const BlockArgs& a, int tiles, int stages, 
     constexpr int kThreads = 2 * WN * 64;
     if (form == kCOut) gemm_block_kernel<FA, FB, Out, STAGES, WN, FUSED, false, STREAM, kCOut><<<grid, kThreads, 0, s>>>(a);
     else if (form == kCPieces) gemm_block_kernel<FA, FB, Out, STAGES, WN, FUSED, false, STREAM, kCPieces><<<grid, kThreads, 0, s>>>(a);
-    else gemm_block_kernel<FA, FB, Out, STAGES, WN, true, false, false, kCKept><<<grid, kThreads, 0, s>>>(a);  // fused or not: args.ep may be empty
+    else gemm_block_kernel<FA, FB, Out, STAGES, WN, FUSED, false, false, kCKept><<<grid, kThreads, 0, s>>>(a);
   };
   auto with_out = [&]<typename Out>() {
     if (g.tile_cols == 256) with.template operator()<Out, 4, 4, false>();  // tiles of 128 x 256, eight waves, four slots
