@@ -62,7 +62,7 @@ constexpr size_t kStreamWsMax = 128;
 
 hipError_t launch_tiled(const mxfp6::GemmArgs& g, hipStream_t s) {
 #ifdef MXFP6_PROBES
-  g_route |= mxfp6::tiled_streams_weights(g) ? kRouteStreamB : 0;
+  g_route |= (mxfp6::tiled_streams_weights(g) ? kRouteStreamB : 0) | mxfp6::tiled_c_form(g) * kRouteForm;
 #endif
   return mxfp6::launch_gemm_tiled(g, s);
 }

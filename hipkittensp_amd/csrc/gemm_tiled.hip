@@ -141,7 +141,9 @@ struct TiledArgs {
 // second tile row reads again.  Not with two tile rows (us, plain / non-temporal, N = 8192, K = 28672: 192 rows on tiles of 128 61.4 / 70.2), nor below that size
 // (256 x 4096 x 14336 36.5 / 37.5), nor row-major, where a line is read twice (128 rows 60.4 / 67.8).  (A kernel that picks the bit as it runs: 256 x 4096 x 14336
 // 39.4 / 41.2 in the same call.)
-template <int FA, int FB, typename Out, int TM, int TN, bool FUSED, int ABL = 0, int KSPLIT = 0>
+// KEPT: C goes through the L2s (c_leaves), else non-temporally.  (An instantiation: a third copy of the epilogue made the loop's code worse, 8192 x 8192 x
+// 16384 e3m2 x e2m3 605 -> 619 us, and one copy that picks at each store is predicated for whole tiles too.)
+template <int FA, int FB, typename Out, int TM, int TN, bool FUSED, int ABL = 0, int KSPLIT = 0, bool KEPT = false>
 __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs args) {
   typedef Shape<TM, TN> S;
   constexpr int kBM = S::BM, kBN = S::BN, OPA = S::OPA, OPA1 = S::OPA1, OPB = S::OPB, kLoadsInCompute = S::kLoadsInCompute;
@@ -511,8 +513,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
   // ~47 clocks per store instruction.)  Nothing here touches LDS, so the ring keeps streaming the next output
   // tile meanwhile.  The stores count in vmcnt like the loads and retire in order with them, so the waits of
   // the K loop ("all but the newest batch") stay valid.
-  // EDGE: the tile has fewer than 256 valid rows or columns; those stores are predicated per lane, and so are all of a C
-  // that goes through the L2s (c_leaves; a third copy for those made the loop's code worse: 8192 x 8192 x 16384 e3m2 x e2m3 605 -> 619 us).
+  // EDGE: the tile has fewer than 256 valid rows or columns; those stores are predicated per lane.
   typedef typename Out::type OutT;
   // Fused scales / bias / activation, on the accumulators themselves, before the epilogue proper.  Per 32x32 tile a
   // lane owns row wm * TM * 32 + 32 i + lane % 32 and columns 8 q + 4 h .. + 3 for q = 0..3; N % 8 == 0, so a run of
@@ -574,14 +575,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
       }
     }
   };
-  auto c_streams = [&]() __attribute__((always_inline)) {
-    if constexpr (KSPLIT != 0 || sizeof(OutT) == 1) return true;
-    else {
-      const auto g = fresh_args();
-      return c_leaves(g->C, g->M, (size_t)g->N * sizeof(OutT));
-    }
-  };
-  auto epilogue = [&]<bool EDGE>(int rows_a, int rows_b, [[maybe_unused]] bool streamed) __attribute__((always_inline)) {
+  auto epilogue = [&]<bool EDGE>(int rows_a, int rows_b) __attribute__((always_inline)) {
     const auto g = fresh_args();
     if constexpr (sizeof(OutT) == 1) {
       // C re-quantised to MXFP6 along N (the next GEMM's K): a wave's two tiles of a band at a time
@@ -620,13 +614,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
     auto store_rows = [&](v4i x, v4i y, int row, int col) __attribute__((always_inline)) {
       if constexpr (LINE) join_lines(x, y);
       constexpr int kNext = LINE ? 8 : 16;
-      if (!EDGE || streamed) {
-        if (!EDGE || (row_l + row < rows_a && col_l + col < rows_b)) store_c<true>(x, rC, voff + col * (int)sizeof(OutT), row * N2);
-        if (!EDGE || (row_l + row + kNext < rows_a && col_l + col < rows_b)) store_c<true>(y, rC, voff + col * (int)sizeof(OutT), (row + kNext) * N2);
-      } else {
-        if (row_l + row < rows_a && col_l + col < rows_b) store_c<false>(x, rC, voff + col * (int)sizeof(OutT), row * N2);
-        if (row_l + row + kNext < rows_a && col_l + col < rows_b) store_c<false>(y, rC, voff + col * (int)sizeof(OutT), (row + kNext) * N2);
-      }
+      if (!EDGE || (row_l + row < rows_a && col_l + col < rows_b)) store_c<!KEPT>(x, rC, voff + col * (int)sizeof(OutT), row * N2);
+      if (!EDGE || (row_l + row + kNext < rows_a && col_l + col < rows_b)) store_c<!KEPT>(y, rC, voff + col * (int)sizeof(OutT), (row + kNext) * N2);
     };
     if constexpr (sizeof(OutT) == 2) {
 #pragma unroll
@@ -694,9 +683,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_tiled_kernel(const TiledArgs arg
       {
         const auto g = fresh_args();
         const int rows_a = min(kBM, g->M - (tile_cur & 0xffff) * kBM), rows_b = min(kBN, g->N - (tile_cur >> 16) * kBN);
-        const bool streamed = c_streams();
-        if (rows_a == kBM && rows_b == kBN && streamed) epilogue.template operator()<false>(rows_a, rows_b, streamed);
-        else epilogue.template operator()<true>(rows_a, rows_b, streamed);
+        if (rows_a == kBM && rows_b == kBN) epilogue.template operator()<false>(rows_a, rows_b);
+        else epilogue.template operator()<true>(rows_a, rows_b);
       }
       if (tile_next < 0) break;
       p0 = (p0 + nk4) & 1;
@@ -916,6 +904,11 @@ bool tiled_streams_weights(const GemmArgs& g) {
   return g.ksplit > 1 && g.ks_part && g.M <= (g.tile_rows == 128 ? 128 : 256) && g.layout_b && (size_t)g.N * (g.K / 4 * 3) >= kStreamBytes;
 }
 
+int tiled_c_form(const GemmArgs& g) {
+  if ((g.ksplit > 1 && g.ks_part) || g.fmt_c) return kCPieces;
+  return c_leaves(g.C, g.M, (size_t)g.N * (g.f32out ? 4 : 2)) ? kCOut : kCKept;
+}
+
 hipError_t launch_gemm_tiled(const GemmArgs& g, hipStream_t s) {
   if (g.fmt_a == 2 && g.fmt_b == 2) return launch_gemm_tiled_fmt22(g, s);
   if (g.fmt_a == 2 && g.fmt_b == 3) return launch_gemm_tiled_fmt23(g, s);
@@ -959,6 +952,14 @@ static hipError_t launch(const GemmArgs& g, hipStream_t s) {
   if constexpr (sizeof(typename Out::type) == 1) {  // fp6 output: one instantiation, with the fused step (a no-op when nothing is fused)
     if (bm == 128) gemm_tiled_kernel<FA, FB, Out, 2, 2, true><<<grid, NW * 64, 0, s>>>(ta);
     else gemm_tiled_kernel<FA, FB, Out, 4, 2, true><<<grid, NW * 64, 0, s>>>(ta);
+  } else if (tiled_c_form(g) == kCKept && !g.ablation) {
+    auto kept = [&]<bool FUSED>() {
+      if (bn == 128) gemm_tiled_kernel<FA, FB, Out, 2, 1, FUSED, 0, 0, true><<<grid, NW * 64, 0, s>>>(ta);
+      else if (bm == 128) gemm_tiled_kernel<FA, FB, Out, 2, 2, FUSED, 0, 0, true><<<grid, NW * 64, 0, s>>>(ta);
+      else gemm_tiled_kernel<FA, FB, Out, 4, 2, FUSED, 0, 0, true><<<grid, NW * 64, 0, s>>>(ta);
+    };
+    if (epilogue_any(g.ep)) kept.template operator()<true>();
+    else kept.template operator()<false>();
   } else if (epilogue_any(g.ep)) {
     if (bn == 128) gemm_tiled_kernel<FA, FB, Out, 2, 1, true><<<grid, NW * 64, 0, s>>>(ta);
     else if (bm == 128) gemm_tiled_kernel<FA, FB, Out, 2, 2, true><<<grid, NW * 64, 0, s>>>(ta);

@@ -85,6 +85,7 @@ hipError_t launch_gemm_generic(const GemmArgs& g, hipStream_t s);
 bool gemm_tiled_supports(const GemmArgs& g);
 hipError_t launch_gemm_tiled(const GemmArgs& g, hipStream_t s);
 bool tiled_streams_weights(const GemmArgs& g);  // whether launch_gemm_tiled reads B with the non-temporal bit
+int tiled_c_form(const GemmArgs& g);            // how it stores C (CStore; kCPieces: a K split's sums, MXFP6)
 bool gemm_tiled4_supports(const GemmArgs& g);  // the 4-wave variant of the tiled kernel (selectable, never chosen automatically)
 hipError_t launch_gemm_tiled4(const GemmArgs& g, hipStream_t s);
 bool gemm_block_supports(const GemmArgs& g);  // 128 x 128 tiles, four waves in step (a few hundred to a few thousand rows of A)

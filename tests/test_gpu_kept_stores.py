@@ -59,6 +59,14 @@ def test_block_kernel_stores_as_the_rule_says(route, kernel, M, N, out, shift, f
     check_form(route, kernel, kernel, M, N, 384, out, shift, form)
 
 
+@pytest.mark.parametrize("M,N,out,shift,form", [
+    (2044, 4104, torch.bfloat16, 0, "OUT"), (2045, 4104, torch.bfloat16, 0, "KEPT"), (2100, 4096, torch.bfloat16, 0, "OUT"), (2100, 4096, torch.bfloat16, 8, "KEPT"),
+    (1022, 4104, torch.float32, 0, "OUT"), (1023, 4104, torch.float32, 0, "KEPT"), (1100, 4096, torch.float32, 4, "KEPT")])
+@pytest.mark.parametrize("kernel", [5, 6, 17])
+def test_tiled_kernel_stores_as_the_rule_says(route, kernel, M, N, out, shift, form):
+    check_form(route, kernel, kernel, M, N, 384, out, shift, form)
+
+
 def check_form(route, kernel, code, M, N, K, out, shift, form):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
