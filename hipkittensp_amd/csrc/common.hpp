@@ -190,11 +190,12 @@ template <int LINE>
 __device__ __forceinline__ int line_piece(int lane) { return (LINE ? lane >> 1 & 4 : 0) + (lane >> 3 & 2) + (lane >> 5); }
 
 // Stores 16 bytes per lane, non-temporal: lines that are whole go out to memory at once, under the rest of the kernel, and do not wait in the
-// L2s for the write-back at its end.
-// The registers stay as they are for four more cycles: a buffer store of 16 bytes reads its data a little after it has been issued.  The
-// compiler leaves two cycles where the store has no scalar offset and none where it has one, which is not enough (a v_mov of the first
-// dword right behind the store: the last four of every sixteen lanes stored the new value now and then).
-// STREAM false: the same through the L2s.
+// L2s for the write-back at its end.  STREAM false: the same through the L2s.
+// The registers stay as they are for four more cycles: a store of 16 bytes reads its data a little after it has been issued.  Where it has a scalar
+// offset, as half of these have, the compiler lets the next instruction write them (the instruction set's table of required waits excepts such
+// stores), and here a v_mov of the first dword right behind one changed what the last four of every sixteen lanes stored, now and then.  Where it has none --
+// the 16-byte stores through a pointer, in every kernel -- the compiler leaves two cycles, which is the table's wait, and no such store was seen to go
+// wrong.  A test disassembles the library for both distances.
 template <bool STREAM>
 __device__ __forceinline__ void store_c(v4i v, const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff) {
   constexpr int kNonTemporal = 2;
