@@ -159,8 +159,12 @@ __device__ __forceinline__ void store1(float* p, float a) { *p = a; }
 // and block kernel, tile-major operands: 8192 x 2048 x 512 17.1 / 12.2, 19.6 / 13.7; 1024 x 23552 x 512 26.2 / 22.2, 27.6 / 22.5; 6255 x 1920 x 1536
 // 24.3 / 21.5, 28.0 / 24.9; 4530 x 7936 x 2048 71.7 / 67.3, 78.5 / 75.0; 8192^3 287 / 280 (tiled).  (The same non-temporal in parts of 32 bytes: 19.7, 36.2;
 // 34.7, 56.6; 27.2, 35.7; 91, 95; 307; in parts of 64: 16.0, 16.1; 25.8, 26.2; 21.4, 25.1; 70, 78; 297.  Whole lines without it: 16.6, 19.0; 25.8, 27.2; 24.3,
-// 27.1; 71.1, 76.3; 284.)  A program that reads C in its next kernel keeps the gain or is level (2048 x 14336 x 1024 on the block kernel and the
-// quantiser 57.7 / 51.6, 512 x 2048 x 2048 12.4 / 12.6).
+// 27.1; 71.1, 76.3; 284.)
+// Little C is stored as it comes: the lanes' trades and the way to memory cost such a call more than they give (block_c_form, ragged_c_form; of the time as it
+// comes, whole lines non-temporally on the block kernel, by C's size below 1 MB, 1 to 2, 2 to 4 MB: rows on lines 1.01, 1.00, 0.98, others 1.07, 1.03, 1.02).
+// A program whose next kernel reads C keeps most of the gain (us, in pieces / as it is now, the quantiser or an elementwise add behind the kernel that the choice
+// takes): 512 x 2048 x 2048 12.6 / 12.6, 11.8 / 11.8; 1024 x 4096 x 1024 12.9 / 11.7, 12.4 / 11.6; 2048 x 4096 x 1024 17.5 / 15.6, 18.5 / 17.2; 4096 x 4096 x 2048
+// 35.2 / 33.2, 37.9 / 37.7; tiled 256 x 256, 2048 x 14336 x 1024 45.5 / 43.2, 50.6 / 51.7, 4096 x 14336 x 1024 87.1 / 81.0, 97.4 / 97.1.
 // How a tile kernel stores C: 16 bytes of 32 rows at a time, as the accumulators hold them; whole lines, through the L2s; whole lines, non-temporally
 enum CStore : int { kCPieces, kCKept, kCOut };
 // pair_rows: y holds what lies 32 bytes behind x's.  Afterwards x holds 64 contiguous bytes of rows 0 - 15 and y those of rows 16 - 31:
