@@ -129,7 +129,8 @@ def probes() -> ctypes.CDLL:
         L.mxfp6_probe_ksplit_plan.argtypes = [ci, ci, ci, ci, ci, ctypes.POINTER(ci)]
         for switch in (L.mxfp6_probe_block, L.mxfp6_probe_slice, L.mxfp6_probe_padded):
             switch.restype, switch.argtypes = ci, [ci]
-        L.mxfp6_probe_route.restype, L.mxfp6_probe_route.argtypes = ci, []
+        for report in (L.mxfp6_probe_route, L.mxfp6_probe_memory):
+            report.restype, report.argtypes = ci, []
         L.mxfp6_probe_candidate.restype = ci
         L.mxfp6_probe_candidate.argtypes = [ci] * 6 + [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ci)]
         L.mxfp6_probe_time_gemm.restype = ci

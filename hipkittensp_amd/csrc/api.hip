@@ -33,13 +33,14 @@ thread_local int g_slice = 0;                                 // mxfp6_probe_sli
 thread_local int g_padded = 0;                                // mxfp6_probe_padded: 1 = always, -1 = never
 thread_local int g_block = 1;                                 // mxfp6_probe_block: 0 keeps the block kernel out of the automatic choice
 thread_local int g_route = 0;                                 // mxfp6_probe_route
+thread_local int g_memory = 0;                                // mxfp6_probe_memory
 void note_route(int route) { g_route = route; }
 #else
 constexpr int g_slice = 0, g_padded = 0, g_block = 1;
 inline void note_route(int) {}
 #endif
 // What mxfp6_probe_route reports beside a kernel's code: the slice kernel's code, copies in front of the GEMM, quantised inside
-constexpr int kRouteSlice = 29, kRouteCopyA = 0x100, kRouteCopyB = 0x200, kRouteSplit = 0x400, kRouteX = 0x800, kRouteStreamB = 0x1000, kRouteForm = 0x2000;
+constexpr int kRouteSlice = 29, kRouteCopyA = 0x100, kRouteCopyB = 0x200, kRouteSplit = 0x400, kRouteX = 0x800;
 
 // Workspaces kept per (device, stream, kind): launches on one stream are ordered, so they can share one; it grows on
 // demand (old one returned to the allocator in stream order) and lives until mxfp6_release_workspaces().
@@ -62,13 +63,13 @@ constexpr size_t kStreamWsMax = 128;
 
 hipError_t launch_tiled(const mxfp6::GemmArgs& g, hipStream_t s) {
 #ifdef MXFP6_PROBES
-  g_route |= (mxfp6::tiled_streams_weights(g) ? kRouteStreamB : 0) | mxfp6::tiled_c_form(g) * kRouteForm;
+  g_memory = (mxfp6::tiled_streams_weights(g) ? 4 : 0) | mxfp6::tiled_c_form(g);
 #endif
   return mxfp6::launch_gemm_tiled(g, s);
 }
 hipError_t launch_block(const mxfp6::GemmArgs& g, hipStream_t s) {
 #ifdef MXFP6_PROBES
-  g_route |= (mxfp6::block_streams_weights(g) ? kRouteStreamB : 0) | mxfp6::block_c_form(g) * kRouteForm;
+  g_memory = (mxfp6::block_streams_weights(g) ? 4 : 0) | mxfp6::block_c_form(g);
 #endif
   return mxfp6::launch_gemm_block(g, s);
 }
@@ -880,6 +881,8 @@ int mxfp6_probe_padded(int mode) {
 }
 
 int mxfp6_probe_route(void) { return g_route; }
+
+int mxfp6_probe_memory(void) { return g_memory; }
 
 int mxfp6_probe_slice(int plan) {
   const int prev = g_slice;

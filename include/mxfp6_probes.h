@@ -104,9 +104,13 @@ int mxfp6_probe_padded(int mode);
 
 /* What the calling thread's last gemm, fused, fused_fp6 or linear call launched: the code of mxfp6_set_kernel of its GEMM kernel (2, 22 and 28
  * whatever their tiles and split, 29: the slice kernel, which mxfp6_kernel_choice reports as 22 or 27), plus 0x100 / 0x200 for a copy of A / of B
- * in front of it (A's also where the quantiser wrote it), 0x400 for a K split of the tiled, block, ring and slice kernels, 0x800 for activations quantised inside, 0x1000 for weights that the tiled or block
- * kernel reads with the non-temporal bit, and 0x2000 / 0x4000 for a C that they store in whole lines, through the L2s / non-temporally. */
+ * in front of it (A's also where the quantiser wrote it), 0x400 for a K split of the tiled, block, ring and slice kernels, 0x800 for activations quantised inside. */
 int mxfp6_probe_route(void);
+
+/* How the calling thread's last launch of the tiled or the block kernel goes to memory: C (or, with a K split, its shares' sums, or MXFP6) as the
+ * accumulators hold it (0), in whole lines through the L2s (1), in whole lines non-temporally (2); plus 4 where it reads the weights with the
+ * non-temporal bit. */
+int mxfp6_probe_memory(void);
 
 #ifdef __cplusplus
 }

@@ -22,8 +22,9 @@ class Route:
     settings of the measurement build count; kernel and k_split are set for the call."""
 
     TILED, SKINNY, BLOCK, RING, SLICE = 2, 3, 22, 28, 29
-    COPY_A, COPY_B, SPLIT, X, STREAM_B = 0x100, 0x200, 0x400, 0x800, 0x1000
-    FORM, PIECES, KEPT, OUT = 0x6000, 0, 0x2000, 0x4000  # how C is stored
+    COPY_A, COPY_B, SPLIT, X = 0x100, 0x200, 0x400, 0x800
+    PIECES, KEPT, OUT, STREAM_B = 0, 1, 2, 4  # memory: how the tiled or block kernel of the last call stored C and read B (mxfp6_probe_memory)
+    memory = 0
 
     def _run(self, kernel, k_split, call):
         import torch
@@ -34,6 +35,7 @@ class Route:
         prev = P.mxfp6_set_kernel(kernel), P.mxfp6_set_k_split(k_split)
         try:
             assert call(P, torch.cuda.current_stream().cuda_stream) == 0
+            self.memory = P.mxfp6_probe_memory()
             return P.mxfp6_probe_route()
         finally:
             P.mxfp6_set_kernel(prev[0]), P.mxfp6_set_k_split(prev[1])

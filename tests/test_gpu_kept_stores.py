@@ -79,7 +79,7 @@ def check_form(route, kernel, code, M, N, K, out, shift, form):
     whole = torch.full((2 * pad + M * N,), 7.0, dtype=out, device="cuda")
     C = whole[pad + shift : pad + shift + M * N].view(M, N)
     taken = route.gemm(A, B, As, Bs, C, M, N, K, kernel=kernel, k_split=1)
-    assert taken == code | getattr(route, form), hex(taken)
+    assert taken == code and route.memory == getattr(route, form), (taken, route.memory)
     assert (whole[: pad + shift] == 7).all() and (whole[pad + shift + M * N :] == 7).all()
     want = torch.empty(M, N, dtype=out, device="cuda")
     prev = tk.set_kernel(1)  # one wave per tile: the same sums

@@ -44,6 +44,6 @@ def test_one_tile_row_matches_two(operands, route, kernel, rows, shares, N, K, t
             tk.set_k_split(prev_split)
         res.append(C)
         if act is None:
-            taken = route.gemm(A[:M], B, As[:M], Bs, torch.empty_like(C), M, N, K, lb=tile_b, kernel=kernel, k_split=shares)
-            assert bool(taken & route.STREAM_B) == (tile_b == 1 and M <= rows), hex(taken)
+            route.gemm(A[:M], B, As[:M], Bs, torch.empty_like(C), M, N, K, lb=tile_b, kernel=kernel, k_split=shares)
+            assert bool(route.memory & route.STREAM_B) == (tile_b == 1 and M <= rows)
     assert torch.isfinite(res[2]).all() and torch.equal(res[0], res[2][:rows]) and torch.equal(res[1], res[2][: rows - 3])
