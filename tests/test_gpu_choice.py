@@ -70,3 +70,13 @@ def test_choice_of_small_products_with_weights_from_memory(hk, M, N, K, la, lb):
     """Within 8 %; the slice kernel, whose model knew weights from the cache only, was chosen here and 14 to 36 % behind."""
     ratios = ratios_to_the_best_forced_kernel(hk, M, N, K, la, lb, 1.08)
     assert min(ratios) <= 1.08, ratios
+
+
+@pytest.mark.parametrize("M,N,K,lb", [(2, 7552, 8320, 1), (35, 3584, 10624, 1), (11, 11392, 4352, 1), (46, 10880, 2688, 0)])
+def test_slice_kernel_with_weights_from_memory(hk, route, M, N, K, lb):
+    """Its modelled time from memory lies up to 5 % below the block kernel's, and it is 13 to 25 % faster: a margin there kept it out."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, asc = hk.quantize(torch.randn(M, K, device="cuda", generator=g), 2)
+    b, bsc = hk.quantize(torch.randn(N, K, device="cuda", generator=g) * 0.02, 2, lb)
+    C = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    assert route.gemm(a, b, asc, bsc, C, M, N, K, lb=lb) & 0xFF == route.SLICE
