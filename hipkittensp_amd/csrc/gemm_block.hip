@@ -693,15 +693,13 @@ hipError_t launch_ragged(const GemmArgs& g, const BlockArgs& a, int tiles, hipSt
     if (deep) gemm_block_kernel<FA, FB, Out, 6, 2, true, true, false, CFORM><<<grid, 256, 0, s>>>(a);
     else gemm_block_kernel<FA, FB, Out, 3, 2, true, true, false, CFORM><<<grid, 256, 0, s>>>(a);
   };
-  const int form = block_c_form(g);
-  if (g.f32out || a.nsplit > 1) {
-    if (form == kCOut) with.template operator()<OutF32, kCOut>();
-    else if (form == kCKept) with.template operator()<OutF32, kCKept>();
-    else with.template operator()<OutF32, kCPieces>();
-  } else {
-    if (form == kCOut) with.template operator()<OutBf16, kCOut>();
-    else with.template operator()<OutBf16, kCPieces>();
-  }
+  auto with_out = [&]<typename Out>(int form) {
+    if (form == kCOut) with.template operator()<Out, kCOut>();
+    else if (form == kCKept) with.template operator()<Out, kCKept>();
+    else with.template operator()<Out, kCPieces>();
+  };
+  if (g.f32out || a.nsplit > 1) with_out.template operator()<OutF32>(block_c_form(g));
+  else with_out.template operator()<OutBf16>(block_c_form(g));
   return hipGetLastError();
 }
 // fp6 output, the fused epilogue applied or not inside
@@ -770,14 +768,15 @@ bool block_streams_weights(const GemmArgs& g) {
 // read again at once (us, as it comes / whole lines through the L2s / whole lines non-temporal, fp32: 49 x 20832 x 672 7.45 / 7.75 / 7.5, 20 x 30001 x 672 7.35 /
 // 7.65 / 7.8, 64 x 20001 x 2080 13.1 / 13.35 / 13.4; 191 x 664 x 18624 18.6 / 18.85 / 18.85, 512 x 296 x 16960 19.05 / 19.2 / 19.2).  Else non-temporally where
 // its rows start on lines.  Where they do not, a line is two stores: bf16 up to 32 MB (1000 x 5003 x 1056, 9.5 MB, 17.1 / 17.1 / 16.6; 256 x 16001 x 1056 13.2 / 13.2 /
-// 12.8; 2000 x 8191 x 1056, 31 MB, 38.5 / 38.4 / 37.2; 6000 x 3001 x 672, 34 MB, 33.6 / 33.2 / 36.2); fp32 never (256 x 16001 x 1056, 16 MB, 13.4 / 12.2 /
+// 12.8; 2000 x 8191 x 1056, 31 MB, 38.5 / 38.4 / 37.2; not 6000 x 3001 x 672, 34 MB, 33.6 / 33.2 / 36.2, nor, through the L2s most with a short K, 3524 x 13814 x 288,
+// 93 MB, 47.6 / 42.3); fp32 never (256 x 16001 x 1056, 16 MB, 13.4 / 12.2 /
 // 16.3; 1000 x 5003 x 1056, 19 MB, 16.5 / 15.5 / 18.6; 2000 x 8191 x 1056 36.3 / 34.2 / 49.3).  Over 70 drawn shapes of each type, of the time as it comes: bf16
 // 4 to 32 MB 1.00 / 0.97, above 1.00 / 1.04; fp32 8 to 12 MB 0.96 / 1.00, 12 to 20 MB 0.93 / 1.09, above 0.94 / 1.28.
 static int ragged_c_form(const GemmArgs& g) {
   const size_t row = (size_t)g.N * (g.f32out ? 4 : 2), bytes = g.M * row;
   if (g.ksplit > 1 || g.M <= 64 || bytes < (size_t)4 << 20) return kCPieces;
   if ((((uintptr_t)g.C | row) & 127) == 0) return kCOut;
-  return g.f32out ? kCKept : bytes <= (size_t)32 << 20 ? kCOut : kCPieces;
+  return !g.f32out && bytes <= (size_t)32 << 20 ? kCOut : kCKept;
 }
 int block_c_form(const GemmArgs& g) {
   if (g.ragged) return ragged_c_form(g);
